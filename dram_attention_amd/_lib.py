@@ -33,6 +33,11 @@ SIGNATURES = {
          c_int64, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_int64, c_void_p,
          c_void_p],
     ),
+    "da_prefill_attention_f32": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64,
+         c_int64, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_int64, c_void_p, c_void_p],
+    ),
     "da_page_minmax": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int, c_int64, c_int, c_int, c_int, c_void_p, c_void_p],

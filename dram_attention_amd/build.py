@@ -25,6 +25,7 @@ SOURCES = (
     "decode_attention.hip",
     "stream_attention.hip",
     "prefill_attention.hip",
+    "prefill_attention_f32.hip",
 )
 # packed fp32 VALU ops are switched off for every device compile of this library
 HIPCC_FLAGS = (

@@ -1,0 +1,68 @@
+// Arguments of the causal prefill kernels (prefill_attention.hip for the 16-bit types,
+// prefill_attention_f32.hip) and the checks their entry points share.
+#pragma once
+#include "attention_core.hpp"
+
+namespace da {
+
+struct PrefillArgs {
+  const char *q, *k, *v;
+  char *out;
+  float *lse;  // (Hq, S) natural log, or null
+  int64_t q_tok_stride, q_head_stride;  // elements
+  int64_t k_tok_stride, k_head_stride;
+  int64_t v_tok_stride, v_head_stride;
+  int64_t o_tok_stride, o_head_stride;
+  int64_t seq_len;
+  int rep;          // query heads per kv head
+  int n_groups;     // workgroups that share a kv head's rows: rep / kHeads
+  int64_t n_row_blocks;
+  int heads_per_xcd;  // kv heads per die when they deal out evenly, else 0
+  float scale_log2;
+};
+
+constexpr int kXcds = 8;  // dies (XCDs) of the part; consecutive workgroup ids go to consecutive dies
+
+// Checks the operands of a prefill call and fills `a` (all but the grid's geometry).
+inline int prefill_args(PrefillArgs &a, const char *what, const void *q, int64_t q_tok_stride,
+                        int64_t q_head_stride, const void *k, int64_t k_tok_stride, int64_t k_head_stride,
+                        const void *v, int64_t v_tok_stride, int64_t v_head_stride, int64_t seq_len,
+                        int n_q_heads, int n_kv_heads, int dtype, float scale, void *out,
+                        int64_t o_tok_stride, int64_t o_head_stride, float *lse_out) {
+  DA_REQUIRE(n_q_heads > 0 && n_kv_heads > 0 && n_q_heads % n_kv_heads == 0,
+             "%s: %d query heads do not split over %d kv heads", what, n_q_heads, n_kv_heads);
+  DA_REQUIRE(seq_len >= 0, "%s: negative length", what);
+  DA_REQUIRE(dtype == DA_F32 || dtype == DA_F16 || dtype == DA_BF16, "%s: unknown dtype %d", what, dtype);
+  DA_REQUIRE(scale > 0.f, "%s: the softmax scale must be positive", what);
+  if (seq_len == 0) return DA_OK;
+  DA_REQUIRE(q && k && v && out, "%s: null pointer", what);
+  const int64_t e = elem_size(dtype);
+  for (int64_t stride : {q_tok_stride, q_head_stride, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride,
+                         o_tok_stride, o_head_stride})
+    DA_REQUIRE(stride * e % 16 == 0, "%s: rows must be 16-byte aligned", what);
+  DA_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 && (uintptr_t)out % 16 == 0,
+             "%s: rows must be 16-byte aligned", what);
+  // (a tile's byte offsets from its first row are formed in 32 bits)
+  const int64_t most = ((int64_t)1 << 24) / e;
+  if (k_tok_stride < 0 || v_tok_stride < 0 || k_tok_stride > most || v_tok_stride > most)
+    return fail(DA_ENOTSUP, "%s: key/value token strides of 0..2^24 bytes", what);
+  a.q = (const char *)q;
+  a.k = (const char *)k;
+  a.v = (const char *)v;
+  a.out = (char *)out;
+  a.lse = lse_out;
+  a.q_tok_stride = q_tok_stride;
+  a.q_head_stride = q_head_stride;
+  a.k_tok_stride = k_tok_stride;
+  a.k_head_stride = k_head_stride;
+  a.v_tok_stride = v_tok_stride;
+  a.v_head_stride = v_head_stride;
+  a.o_tok_stride = o_tok_stride;
+  a.o_head_stride = o_head_stride;
+  a.seq_len = seq_len;
+  a.rep = n_q_heads / n_kv_heads;
+  a.scale_log2 = scale * kLog2e;
+  return DA_OK;
+}
+
+}  // namespace da

@@ -35,7 +35,7 @@
 // die it runs on where the heads deal out evenly over the dies (see the kernel).
 #include <type_traits>
 
-#include "attention_core.hpp"
+#include "prefill_args.hpp"
 
 namespace da {
 
@@ -65,26 +65,9 @@ struct PrefillOps<F16> {
   static __device__ __forceinline__ uint32_t pack(float lo, float hi) { return pack_f16(lo, hi); }
 };
 
-struct PrefillArgs {
-  const char *q, *k, *v;
-  char *out;
-  float *lse;  // (Hq, S) natural log, or null
-  int64_t q_tok_stride, q_head_stride;  // elements
-  int64_t k_tok_stride, k_head_stride;
-  int64_t v_tok_stride, v_head_stride;
-  int64_t o_tok_stride, o_head_stride;
-  int64_t seq_len;
-  int rep;          // query heads per kv head
-  int n_groups;     // workgroups that share a kv head's rows: rep / kHeads
-  int64_t n_row_blocks;
-  int heads_per_xcd;  // kv heads per die when they deal out evenly, else 0
-  float scale_log2;
-};
-
 constexpr int kPfThreads = 512;
 constexpr int kPfWaves = 8;
 constexpr int kPfKeys = 64;  // keys per tile
-constexpr int kXcds = 8;     // dies (XCDs) of the part; consecutive workgroup ids go to consecutive dies
 
 // LDS layout of a tile.  K and V rows arrive by loads that write LDS directly
 // (global_load_lds_dwordx4: no staging registers, no LDS store instructions): a wave
@@ -389,43 +372,15 @@ extern "C" int da_prefill_attention(const void *q, int64_t q_tok_stride, int64_t
                                     int dtype, float scale, void *out, int64_t o_tok_stride,
                                     int64_t o_head_stride, float *lse_out, void *stream) {
   using namespace da;
-  DA_REQUIRE(n_q_heads > 0 && n_kv_heads > 0 && n_q_heads % n_kv_heads == 0,
-             "da_prefill_attention: %d query heads do not split over %d kv heads", n_q_heads,
-             n_kv_heads);
-  DA_REQUIRE(seq_len >= 0, "da_prefill_attention: negative length");
-  DA_REQUIRE(dtype == DA_F32 || dtype == DA_F16 || dtype == DA_BF16,
-             "da_prefill_attention: unknown dtype %d", dtype);
-  DA_REQUIRE(scale > 0.f, "da_prefill_attention: the softmax scale must be positive");
-  if (seq_len == 0) return DA_OK;
-  DA_REQUIRE(q && k && v && out, "da_prefill_attention: null pointer");
+  PrefillArgs a = {};
+  const int rc = prefill_args(a, "da_prefill_attention", q, q_tok_stride, q_head_stride, k, k_tok_stride,
+                              k_head_stride, v, v_tok_stride, v_head_stride, seq_len, n_q_heads, n_kv_heads,
+                              dtype, scale, out, o_tok_stride, o_head_stride, lse_out);
+  if (rc != DA_OK || seq_len == 0) return rc;
   if (dtype == DA_F32 || (head_dim != 64 && head_dim != 128))
     return fail(DA_ENOTSUP,
                 "da_prefill_attention: bf16 or fp16 with head_dim 64 or 128 (got dtype %d, head_dim %d)",
                 dtype, head_dim);
-  DA_REQUIRE(q_tok_stride % 8 == 0 && q_head_stride % 8 == 0 && k_tok_stride % 8 == 0 &&
-                 k_head_stride % 8 == 0 && v_tok_stride % 8 == 0 && v_head_stride % 8 == 0 &&
-                 o_tok_stride % 8 == 0 && o_head_stride % 8 == 0 && (uintptr_t)q % 16 == 0 &&
-                 (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 && (uintptr_t)out % 16 == 0,
-             "da_prefill_attention: rows must be 16-byte aligned");
-  if (k_tok_stride < 0 || v_tok_stride < 0 || k_tok_stride > (1 << 23) || v_tok_stride > (1 << 23))
-    return fail(DA_ENOTSUP, "da_prefill_attention: key/value token strides of 0..2^23 elements");
-  PrefillArgs a = {};
-  a.q = (const char *)q;
-  a.k = (const char *)k;
-  a.v = (const char *)v;
-  a.out = (char *)out;
-  a.lse = lse_out;
-  a.q_tok_stride = q_tok_stride;
-  a.q_head_stride = q_head_stride;
-  a.k_tok_stride = k_tok_stride;
-  a.k_head_stride = k_head_stride;
-  a.v_tok_stride = v_tok_stride;
-  a.v_head_stride = v_head_stride;
-  a.o_tok_stride = o_tok_stride;
-  a.o_head_stride = o_head_stride;
-  a.seq_len = seq_len;
-  a.rep = n_q_heads / n_kv_heads;
-  a.scale_log2 = scale * kLog2e;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == DA_BF16)
     return head_dim == 128 ? launch_prefill<BF16, 128>(a, n_kv_heads, s)

@@ -168,9 +168,50 @@ def prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
     """Causal attention over the prompt on the library's kernel (da_prefill_attention):
     (1,S,Hq,D), (1,S,Hkv,D) x 2 -> (1,S,Hq,D); fills ``lse`` (Hq, S) fp32 when given.
     Replaces flash_attn_func(xq, xk, xv, causal=True), reference dram_attention.py:136."""
+    out, args = _prefill_operands(xq, xk, xv, lse)
+    S, Hq, D = xq.shape[1:]
+    _lib.check(
+        _lib.load().da_prefill_attention(
+            *args, S, Hq, xk.shape[2], D, _lib.dtype_code(xq.dtype),
+            float(scale) if scale is not None else 1.0 / math.sqrt(D), out.data_ptr(),
+            out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None,
+            _lib.stream_ptr(xq.device)),
+        "da_prefill_attention")
+    return out
+
+
+def prefill_attention_f32_supported(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor) -> bool:
+    """Whether the library's fp32 prefill kernel takes these tensors as they are (it has no
+    backward, so operands that autograd follows stay with torch)."""
+    if not (xq.is_cuda and xq.shape[-1] in (64, 128)):
+        return False
+    return all(t.dtype == torch.float32 and t.is_cuda and t.stride(-1) == 1
+               and t.data_ptr() % 16 == 0 and t.stride(1) % 4 == 0 and t.stride(2) % 4 == 0
+               and not (t.requires_grad and torch.is_grad_enabled()) for t in (xq, xk, xv))
+
+
+def prefill_attention_f32(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
+                          scale: float | None = None,
+                          lse: torch.Tensor | None = None) -> torch.Tensor:
+    """:func:`prefill_attention` for an fp32 layer (da_prefill_attention_f32): fp32 products
+    and sums throughout."""
+    out, args = _prefill_operands(xq, xk, xv, lse)
+    if xq.dtype != torch.float32:
+        raise TypeError(f"prefill_attention_f32 takes float32, got {xq.dtype}")
+    S, Hq, D = xq.shape[1:]
+    _lib.check(
+        _lib.load().da_prefill_attention_f32(
+            *args, S, Hq, xk.shape[2], D, float(scale) if scale is not None else 1.0 / math.sqrt(D),
+            out.data_ptr(), out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None,
+            _lib.stream_ptr(xq.device)),
+        "da_prefill_attention_f32")
+    return out
+
+
+def _prefill_operands(xq, xk, xv, lse):
+    """Checks of the native prefill kernels; (output, pointer and stride arguments)."""
     bsz, S, Hq, D = xq.shape
     assert bsz == 1, "Only support batch size 1"
-    Hkv = xk.shape[2]
     for name, t in (("xq", xq), ("xk", xk), ("xv", xv)):
         _lib.require_gpu(t, name)
         if t.stride(-1) != 1:
@@ -178,19 +219,12 @@ def prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
     if xk.shape != xv.shape or xk.shape[1] != S or xk.shape[3] != D or not (
             xq.dtype == xk.dtype == xv.dtype):
         raise ValueError("query, keys and values must agree in length, head size and type")
-    out = torch.empty(1, S, Hq, D, dtype=xq.dtype, device=xq.device)
     if lse is not None and (lse.shape != (Hq, S) or lse.dtype != torch.float32
                             or not lse.is_contiguous()):
         raise ValueError("lse must be a contiguous fp32 tensor of shape (Hq, S)")
-    _lib.check(
-        _lib.load().da_prefill_attention(
-            xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1), xk.stride(2),
-            xv.data_ptr(), xv.stride(1), xv.stride(2), S, Hq, Hkv, D, _lib.dtype_code(xq.dtype),
-            float(scale) if scale is not None else 1.0 / math.sqrt(D), out.data_ptr(),
-            out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None,
-            _lib.stream_ptr(xq.device)),
-        "da_prefill_attention")
-    return out
+    out = torch.empty(1, S, Hq, D, dtype=xq.dtype, device=xq.device)
+    return out, (xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1),
+                 xk.stride(2), xv.data_ptr(), xv.stride(1), xv.stride(2))
 
 
 def causal_prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor,
@@ -204,11 +238,14 @@ def causal_prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tenso
                 block sized so that the scores torch may materialise for it (Hq x rows x S
                 fp32) stay within 1 GiB: at most 1024 rows, 64 at 128K tokens and 32
                 heads (any type, CPU too)
-      "auto"    native where it applies, else sdpa, else blocked."""
+      "auto"    native where it applies, the library's fp32 kernel for fp32 layers with
+                head_dim 64 or 128, else sdpa, else blocked."""
     if backend not in ("auto", "native", "sdpa", "blocked"):
         raise RuntimeError(f"Unsupported prefill backend: {backend}")
     if backend == "native" or (backend == "auto" and prefill_attention_supported(xq)):
         return prefill_attention(xq, xk, xv)
+    if backend == "auto" and prefill_attention_f32_supported(xq, xk, xv):
+        return prefill_attention_f32(xq, xk, xv)
     bsz, S, Hq, D = xq.shape
     Hkv = xk.shape[2]
     q = xq.transpose(1, 2)

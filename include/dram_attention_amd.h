@@ -79,6 +79,18 @@ int da_prefill_attention(const void *q, int64_t q_tok_stride, int64_t q_head_str
                          int64_t o_head_stride, float *lse_out, void *stream);
 
 /*
+ * Prefill in fp32 — the same attention for float operands (an fp32 layer), every
+ * product and sum in fp32 on the fp32 matrix instructions.  Operands, scale and lse_out
+ * as above; head_dim 64 or 128 (DA_ENOTSUP otherwise).  No workspace.
+ */
+int da_prefill_attention_f32(const float *q, int64_t q_tok_stride, int64_t q_head_stride,
+                             const float *k, int64_t k_tok_stride, int64_t k_head_stride,
+                             const float *v, int64_t v_tok_stride, int64_t v_head_stride,
+                             int64_t seq_len, int n_q_heads, int n_kv_heads, int head_dim,
+                             float scale, float *out, int64_t o_tok_stride, int64_t o_head_stride,
+                             float *lse_out, void *stream);
+
+/*
  * Subsystem 1 — per-page, per-channel min and max of the keys.
  * Replaces torch.aminmax + torch.stack in
  * dram_attention/topk_selector.py:31-34.

@@ -158,3 +158,31 @@ def test_module_prefill_stage_values_at_the_layer_shape(backend):
     assert out.shape == xq.shape and out.dtype == torch.bfloat16
     assert close(out.float(), want, ATOL, RTOL)
     assert isinstance(m.lru_cache, LRUCache) and m.dram_kv_cache_size == (S - 512 + 16) // 16 * 16
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D", [
+    (1, 4, 1, 64), (15, 8, 2, 64), (16, 4, 4, 128), (17, 6, 3, 64), (31, 2, 1, 128), (32, 3, 1, 64),
+    (33, 8, 1, 128), (63, 4, 2, 64), (65, 5, 5, 128), (1000, 8, 2, 64), (2049, 12, 3, 128),
+])
+def test_fp32_prefill_kernel_matches_dense_float64(S, Hq, Hkv, D):
+    """The fp32 kernel at the edges of its tiles (16 rows, 32 keys), every grouping of
+    heads and both head sizes, on rows cut out of a wider projection.  Bound: products and
+    sums of fp32, i.e. score errors of about sqrt(D) 2^-24 times the scores' size (|s| up to ~10 here),
+    which the exponential turns into relative errors of the weights: 1e-5."""
+    from dram_attention_amd.dram_attention import (causal_prefill_attention, prefill_attention_f32,
+                                                   prefill_attention_f32_supported)
+
+    g = torch.Generator(device=DEV).manual_seed(S)
+    qkv = torch.randn(1, S, Hq + 2 * Hkv, D, device=DEV, generator=g) * 1.5
+    xq, xk, xv = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
+    assert prefill_attention_f32_supported(xq, xk, xv)
+    lse = torch.empty(Hq, S, dtype=torch.float32, device=DEV)
+    out = prefill_attention_f32(xq, xk, xv, lse=lse)
+    assert same(causal_prefill_attention(xq, xk, xv), out)
+    rep = Hq // Hkv
+    mask = torch.ones(S, S, dtype=torch.bool, device=DEV).triu_(1)
+    for h in range(Hq):
+        q, k, v = xq[0, :, h].double(), xk[0, :, h // rep].double(), xv[0, :, h // rep].double()
+        s_ = (q @ k.t().contiguous() / math.sqrt(D)).masked_fill_(mask, float("-inf"))
+        assert close(out[0, :, h].double(), torch.softmax(s_, -1) @ v, 1e-5, 1e-5)
+        assert close(lse[h].double(), torch.logsumexp(s_, -1), 1e-5, 1e-5)
