@@ -26,6 +26,7 @@ SOURCES = (
     "stream_attention.hip",
     "prefill_attention.hip",
     "prefill_attention_f32.hip",
+    "model_rows.hip",
 )
 # packed fp32 VALU ops are switched off for every device compile of this library
 HIPCC_FLAGS = (

@@ -10,8 +10,9 @@ other call decodes one token.  ``start_pos`` of a decode call may be an int32
 device tensor, which keeps the step free of host reads so that it can be
 captured in a HIP graph the way examples/long-qa-chat/chat.py:238-249 does.
 
-Everything here is plumbing around the attention path (projections, rotary
-embedding, norms, SwiGLU): plain torch ops on the GPU.
+Projections are torch's linear layers; norms, rotary embedding and SwiGLU run in
+the kernels of ``model_kernels`` where those take the tensors, and in torch's
+operators otherwise (the CPU, autograd), with the same roundings.
 """
 from __future__ import annotations
 
@@ -23,6 +24,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import model_kernels as K
 from .dram_attention import DRAMAttention
 
 
@@ -119,9 +121,18 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x):
+        if K.takes(x, self.weight) and K.norm_fits(x):
+            return K.rms_norm(x, self.weight, self.eps)[0]
         x32 = x.float()
         normed = x32 * torch.rsqrt(x32.square().mean(-1, keepdim=True) + self.eps)
         return normed.to(x.dtype) * self.weight
+
+    def after_add(self, x, y):
+        """(norm of x + y, x + y)."""
+        if K.takes(x, y, self.weight) and K.norm_fits(x) and x.shape == y.shape:
+            return K.rms_norm(x, self.weight, self.eps, add=y)
+        total = x + y
+        return self(total), total
 
 
 class Attention(nn.Module):
@@ -160,7 +171,11 @@ class Attention(nn.Module):
         xq = self.wq(x).view(bsz, seqlen, self.n_heads, self.head_dim)
         xk = self.wk(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         xv = self.wv(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
-        xq, xk = apply_rope(xq, rope_rows), apply_rope(xk, rope_rows)
+        if (K.takes(xq, xk) and rope_rows.dtype == torch.float32 and rope_rows.is_contiguous()
+                and self.head_dim * xq.element_size() % 16 == 0):
+            K.rope_(xq, xk, rope_rows)          # the projections' own outputs, in place
+        else:
+            xq, xk = apply_rope(xq, rope_rows), apply_rope(xk, rope_rows)
         prefill = seqlen > 1 and not isinstance(start_pos, torch.Tensor) and start_pos == 0
         out = self.dram_attention(xq, xk, xv, start_pos=start_pos,
                                   stage="prefill" if prefill else "generate")
@@ -179,9 +194,14 @@ class FeedForward(nn.Module):
 
     def forward(self, x):
         if x.shape[1] <= self.ROWS_PER_PASS:
-            return self.w2(F.silu(self.w1(x)) * self.w3(x))
-        return torch.cat([self.w2(F.silu(self.w1(c)) * self.w3(c))
-                          for c in x.split(self.ROWS_PER_PASS, dim=1)], dim=1)
+            return self._slice(x)
+        return torch.cat([self._slice(c) for c in x.split(self.ROWS_PER_PASS, dim=1)], dim=1)
+
+    def _slice(self, x):
+        gate, up = self.w1(x), self.w3(x)
+        if K.takes(gate, up) and gate.numel() * gate.element_size() % 16 == 0:
+            return self.w2(K.swiglu_(gate, up))
+        return self.w2(F.silu(gate) * up)
 
 
 class TransformerBlock(nn.Module):
@@ -194,8 +214,9 @@ class TransformerBlock(nn.Module):
         self.ffn_norm = RMSNorm(args.dim, eps=args.norm_eps)
 
     def forward(self, x, start_pos, rope_rows):
-        h = x + self.attention(self.attention_norm(x), start_pos, rope_rows)
-        return h + self.feed_forward(self.ffn_norm(h))
+        normed, h = self.ffn_norm.after_add(
+            x, self.attention(self.attention_norm(x), start_pos, rope_rows))
+        return h + self.feed_forward(normed)
 
 
 class Transformer(nn.Module):

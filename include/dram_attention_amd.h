@@ -465,6 +465,24 @@ int da_pages_gather_attend(const void *dram, int64_t dram_head_stride_bytes,
                            int64_t c_capacity, void *workspace, size_t workspace_bytes,
                            void *stream);
 
+/*
+ * Row-wise parts of the model around the attention layers (evaluation/dram-attention/
+ * model.py of the reference), `rows` contiguous rows at a time; every operand 16-byte
+ * aligned, rows a multiple of 16 bytes (DA_ENOTSUP otherwise).
+ *
+ * da_rms_norm  (model.py:66-78): out = T(x * rsqrt(mean(x^2) + eps)) * weight.  With `add`
+ *   (and `sum_out`, both or neither) x is first replaced by x + add, which is written to
+ *   sum_out: the residual addition in front of the norm.  Rows of up to 32 KiB.
+ * da_rope_rows (model.py:126-136): rotates adjacent channel pairs of q (rows, Hq, D) and
+ *   k (rows, Hkv, D) in place; table (rows, D/2, 2) fp32 holds cosine and sine.
+ * da_swiglu    (model.py:236-245): out[i] = T(silu(gate[i])) * up[i]; out may be gate or up.
+ */
+int da_rms_norm(const void *x, const void *add, void *sum_out, const void *weight, float eps, void *out,
+                int64_t rows, int dim, int dtype, void *stream);
+int da_rope_rows(void *q, int64_t q_tok_stride, void *k, int64_t k_tok_stride, int n_q_heads,
+                 int n_kv_heads, int head_dim, const float *table, int64_t rows, int dtype, void *stream);
+int da_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

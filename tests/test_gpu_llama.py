@@ -225,3 +225,46 @@ def test_recall_harness_on_a_checkpoint_directory(tmp_path):
     (tmp_path / "params.json").write_text(json.dumps(dict(params, hidden=3)))
     with pytest.raises(ValueError, match="hidden"):
         E.load_model(str(tmp_path), 1100)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,dim", [(1, 8), (3, 256), (5, 1024), (4, 1032), (7, 4096), (2, 4104), (3, 8192)])
+def test_norm_and_swiglu_kernels_match_torch(rows, dim, dtype):
+    """The row kernels at the edges of their widths (a wave's rows, a block's, two, four and
+    eight vectors a lane) against the torch operators in the CPU branch of the same modules.
+    Bound: fp32 sums in another order may turn either of two roundings to the type, each by
+    one unit in the last place (up to 2^-7 of the value in bf16, 2^-10 in fp16)."""
+    tol = {torch.bfloat16: 2.0 ** -6, torch.float16: 2.0 ** -9, torch.float32: 3e-6}[dtype]
+    g = torch.Generator().manual_seed(rows * dim)
+    x, y = (torch.randn(1, rows, dim, generator=g).to(dtype) for _ in range(2))
+    norm = L.RMSNorm(dim, eps=1e-5).to(dtype)
+    with torch.no_grad():
+        norm.weight.copy_(1 + 0.1 * torch.randn(dim, generator=g))
+        want = norm(x)
+        want_sum_norm, want_sum = norm.after_add(x, y)
+        gate, up = x * 3, y * 2
+        want_glu = torch.nn.functional.silu(gate) * up
+        norm = norm.cuda()
+        assert L.K.takes(x.cuda(), norm.weight) and L.K.norm_fits(x)   # no fallback
+        got = norm(x.cuda())
+        got_norm, got_sum = norm.after_add(x.cuda(), y.cuda())
+        got_glu = L.K.swiglu_(gate.cuda(), up.cuda())
+    assert torch.equal(got_sum.cpu(), want_sum)
+    for a, b in ((got, want), (got_norm, want_sum_norm), (got_glu, want_glu)):
+        assert torch.allclose(a.cpu().float(), b.float(), rtol=tol, atol=tol * 1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(1, 4, 1, 128), (3, 8, 2, 64), (17, 6, 3, 16)])
+def test_rope_kernel_matches_torch(S, Hq, Hkv, D, dtype):
+    """In-place rotation of queries and keys against apply_rope on the CPU: fp32 products
+    that may be fused, which may turn one rounding to the type by a unit in the last place."""
+    g = torch.Generator().manual_seed(S)
+    xq, xk = torch.randn(1, S, Hq, D, generator=g).to(dtype), torch.randn(1, S, Hkv, D, generator=g).to(dtype)
+    rows = L.rope_table(D, 50, 1e4, True)[11:11 + S]
+    q, k = xq.cuda(), xk.cuda()
+    L.K.rope_(q, k, rows.cuda())
+    tol = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 1e-6}[dtype]
+    for got, x in ((q, xq), (k, xk)):
+        want = L.apply_rope(x, rows).float()
+        assert torch.allclose(got.cpu().float(), want, rtol=tol, atol=tol * 4)
