@@ -8,6 +8,11 @@
 // per lane; torch's operators made 6 passes for a norm, 9 for a rotation (most of them in
 // fp32) and 2 for the product.  Results are rounded where the torch operators they stand
 // for round: fp32 inside, the type T between.
+//
+// Measured at 8192 rows of dim 4096, hidden 14336, 32/8 heads of 128, bf16: norm 25 us, with
+// the addition in front 40 us; rotation of queries and keys 32 us (168 MB, 5.3 TB/s); SwiGLU
+// product 105 us (705 MB, 6.7 TB/s).  A prompt of 8192 tokens through two layers: 9.33 -> 7.48 ms;
+// a token through four layers from Python, 200 -> 72 launches: 2.35 -> 1.38 ms.
 #include "model_math.hpp"
 
 namespace da {
