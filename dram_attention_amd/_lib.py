@@ -104,6 +104,18 @@ SIGNATURES = {
         c_int,
         [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_int64, c_int, c_void_p]),
     "da_swiglu": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_void_p]),
+    "da_linear_qkv_rope": (
+        c_int,
+        [c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    "da_linear_swiglu": (
+        c_int,
+        [c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_int64, c_void_p, c_int, c_void_p]),
+    "da_linear_add": (
+        c_int, [c_void_p, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_void_p]),
+    "da_linear_logits": (
+        c_int, [c_void_p, c_void_p, c_float, c_int, c_void_p, c_int64, c_void_p, c_int, c_void_p]),
+    "da_argmax": (c_int, [c_void_p, c_int64, c_void_p, c_void_p]),
     "da_pages_gather_attend": (
         c_int,
         [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int, c_void_p, c_void_p,

@@ -27,6 +27,7 @@ SOURCES = (
     "prefill_attention.hip",
     "prefill_attention_f32.hip",
     "model_rows.hip",
+    "decode_linear.hip",
 )
 # packed fp32 VALU ops are switched off for every device compile of this library
 HIPCC_FLAGS = (

@@ -10,9 +10,10 @@ other call decodes one token.  ``start_pos`` of a decode call may be an int32
 device tensor, which keeps the step free of host reads so that it can be
 captured in a HIP graph the way examples/long-qa-chat/chat.py:238-249 does.
 
-Projections are torch's linear layers; norms, rotary embedding and SwiGLU run in
-the kernels of ``model_kernels`` where those take the tensors, and in torch's
-operators otherwise (the CPU, autograd), with the same roundings.
+Projections of a prompt are torch's linear layers; norms, rotary embedding and
+SwiGLU, and the whole block around the attention of a single token, run in the
+kernels of ``model_kernels`` where those take the tensors, and in torch's operators
+otherwise (the CPU, autograd, hooked or replaced modules), with the same roundings.
 """
 from __future__ import annotations
 
@@ -214,9 +215,31 @@ class TransformerBlock(nn.Module):
         self.ffn_norm = RMSNorm(args.dim, eps=args.norm_eps)
 
     def forward(self, x, start_pos, rope_rows):
-        normed, h = self.ffn_norm.after_add(
-            x, self.attention(self.attention_norm(x), start_pos, rope_rows))
+        if x.shape[0] == x.shape[1] == 1 and self._one_token_kernels(x, rope_rows):
+            a, f = self.attention, self.feed_forward
+            xq, xk, xv = K.linear_qkv_rope(x, self.attention_norm, a.wq.weight, a.wk.weight, a.wv.weight,
+                                           a.n_heads, a.n_kv_heads, a.head_dim, rope_rows)
+            out = a.dram_attention(xq, xk, xv, start_pos=start_pos, stage="generate")
+            h = K.linear_add(out, a.wo.weight, x)
+            return K.linear_add(K.linear_swiglu(h, self.ffn_norm, f.w1.weight, f.w3.weight), f.w2.weight, h)
+        attended = self.attention(self.attention_norm(x), start_pos, rope_rows)
+        if type(self.ffn_norm) is RMSNorm and K.bare(self.ffn_norm):
+            normed, h = self.ffn_norm.after_add(x, attended)
+        else:
+            h = x + attended
+            normed = self.ffn_norm(h)
         return h + self.feed_forward(normed)
+
+
+    def _one_token_kernels(self, x, rope_rows) -> bool:
+        """Whether the one-token kernels may stand for this block's modules."""
+        a, f = self.attention, self.feed_forward
+        return (type(a) is Attention and type(f) is FeedForward
+                and type(self.attention_norm) is RMSNorm and type(self.ffn_norm) is RMSNorm
+                and K.takes(x, self.attention_norm.weight, self.ffn_norm.weight)
+                and K.linears_fit(x, a.wq, a.wk, a.wv, a.wo, f.w1, f.w3, f.w2)
+                and K.bare(a, f, self.attention_norm, self.ffn_norm)
+                and rope_rows.dtype == torch.float32 and rope_rows.is_contiguous())
 
 
 class Transformer(nn.Module):
@@ -249,7 +272,11 @@ class Transformer(nn.Module):
             rows = self.rope[start_pos: start_pos + seqlen]
         for layer in self.layers:
             h = layer(h, start_pos, rows)
-        return self.output(self.norm(h[:, -1:, :])).float()
+        last = h[:, -1:, :]
+        if (last.shape[0] == 1 and K.takes(last, self.norm.weight) and K.linears_fit(last, self.output)
+                and type(self.norm) is RMSNorm and K.bare(self.norm)):
+            return K.linear_logits(last, self.norm, self.output.weight)
+        return self.output(self.norm(last)).float()
 
     def init_cache_from_files(self, cache_dir: str) -> int:
         """Load every layer's ``NN_cache.pth`` (examples/long-qa-chat/chat.py:214-233);
@@ -278,7 +305,10 @@ class GraphedDecoder:
 
     def _step(self):
         logits = self.model(self.token, self.pos)
-        self.token.copy_(logits.argmax(-1))
+        if logits.is_cuda:
+            K.argmax_into(logits, self.token)
+        else:
+            self.token.copy_(logits.argmax(-1))
         self.pos.add_(1)
         return logits
 

@@ -1,9 +1,12 @@
-"""The model's row-wise kernels (csrc/model_rows.hip) for tensors they take as they are;
-llama.py keeps torch's operators for everything else (the CPU, autograd, odd layouts)."""
+"""The model's row-wise kernels (csrc/model_rows.hip) and its linear layers for one token
+(csrc/decode_linear.hip), for tensors they take as they are; llama.py keeps torch's
+operators for everything else (the CPU, autograd, odd layouts)."""
 
 from __future__ import annotations
 
 import torch
+from torch import nn
+from torch.nn.modules import module as nn_module
 
 from . import _lib
 
@@ -55,3 +58,81 @@ def swiglu_(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
                               _lib.dtype_code(gate.dtype), _lib.stream_ptr(gate.device)),
         "da_swiglu")
     return gate
+
+
+def bare(*modules: nn.Module) -> bool:
+    """Whether calling these modules does nothing but their forward: nobody hooked them."""
+    if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
+MAX_LINEAR_ROW = 60 * 1024  # bytes of an input row the one-token layers hold in LDS
+
+
+def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
+    """Whether the one-token layers may stand for these nn.Linear modules (x: any tensor of
+    the step, for its type and device)."""
+    for m in linears:
+        if type(m) is not nn.Linear or m.bias is not None:
+            return False
+        w = m.weight
+        row = w.shape[1] * w.element_size()
+        if (w.dtype != x.dtype or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16
+                or row % 16 or row > MAX_LINEAR_ROW):
+            return False
+    return bare(*linears)
+
+
+def linear_qkv_rope(x, norm, wq, wk, wv, n_heads, n_kv_heads, head_dim, rope_row):
+    """Rotated queries and keys, and values, of one token: (1,1,Hq,D), (1,1,Hkv,D) x 2."""
+    out = torch.empty(n_heads + 2 * n_kv_heads, head_dim, dtype=x.dtype, device=x.device)
+    q, k, v = out.split((n_heads, n_kv_heads, n_kv_heads))
+    _lib.check(
+        _lib.load().da_linear_qkv_rope(
+            x.data_ptr(), norm.weight.data_ptr(), norm.eps, x.shape[-1], wq.data_ptr(), wk.data_ptr(),
+            wv.data_ptr(), n_heads, n_kv_heads, head_dim, rope_row.data_ptr(), q.data_ptr(), k.data_ptr(),
+            v.data_ptr(), _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
+        "da_linear_qkv_rope")
+    return q[None, None], k[None, None], v[None, None]
+
+
+def linear_swiglu(x, norm, w1, w3):
+    """silu(w1 n) * (w3 n), n the norm of x (1, 1, dim)."""
+    out = torch.empty(1, 1, w1.shape[0], dtype=x.dtype, device=x.device)
+    _lib.check(
+        _lib.load().da_linear_swiglu(
+            x.data_ptr(), norm.weight.data_ptr(), norm.eps, x.shape[-1], w1.data_ptr(), w3.data_ptr(),
+            w1.shape[0], out.data_ptr(), _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
+        "da_linear_swiglu")
+    return out
+
+
+def linear_add(x, w, residual):
+    """residual + w x for one token; x of any shape with w.shape[1] elements."""
+    out = torch.empty_like(residual)
+    _lib.check(
+        _lib.load().da_linear_add(
+            x.data_ptr(), w.shape[1], w.data_ptr(), w.shape[0], residual.data_ptr(), out.data_ptr(),
+            _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
+        "da_linear_add")
+    return out
+
+
+def linear_logits(x, norm, w):
+    """fp32 logits (1, 1, vocab) of the normed row x (1, 1, dim)."""
+    out = torch.empty(1, 1, w.shape[0], dtype=torch.float32, device=x.device)
+    _lib.check(
+        _lib.load().da_linear_logits(
+            x.data_ptr(), norm.weight.data_ptr(), norm.eps, x.shape[-1], w.data_ptr(), w.shape[0],
+            out.data_ptr(), _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
+        "da_linear_logits")
+    return out
+
+
+def argmax_into(logits: torch.Tensor, token: torch.Tensor) -> None:
+    """token (one int64) = index of the largest of the contiguous fp32 logits."""
+    _lib.check(
+        _lib.load().da_argmax(logits.data_ptr(), logits.numel(), token.data_ptr(),
+                              _lib.stream_ptr(logits.device)),
+        "da_argmax")

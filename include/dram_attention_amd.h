@@ -483,6 +483,32 @@ int da_rope_rows(void *q, int64_t q_tok_stride, void *k, int64_t k_tok_stride, i
                  int n_kv_heads, int head_dim, const float *table, int64_t rows, int dtype, void *stream);
 int da_swiglu(const void *gate, const void *up, void *out, int64_t n, int dtype, void *stream);
 
+/*
+ * The model's linear layers for ONE token (evaluation/dram-attention/model.py:138-245 at
+ * sequence length 1): y = T(W x), W (N, K) contiguous, fp32 accumulation, x of `dim` = K
+ * elements; with norm_weight x is first replaced by its RMS norm (as da_rms_norm gives it).
+ * Rows of x: a multiple of 16 bytes, up to 60 KiB (DA_ENOTSUP otherwise); x, norm_weight
+ * and the matrices 16-byte aligned.
+ *   qkv_rope  q, k = y rotated by rope_row (D/2, 2) fp32, v = y; q_out (Hq, D), k_out and
+ *             v_out (Hkv, D)
+ *   swiglu    out[i] = T(silu(y1[i])) * y3[i], i < hidden
+ *   add       out[i] = residual[i] + y[i], i < n_out; out may be residual
+ *   logits    out[i] = y[i] (rounded to T) as fp32, i < n_out
+ */
+int da_linear_qkv_rope(const void *x, const void *norm_weight, float eps, int dim, const void *wq,
+                       const void *wk, const void *wv, int n_q_heads, int n_kv_heads, int head_dim,
+                       const float *rope_row, void *q_out, void *k_out, void *v_out, int dtype, void *stream);
+int da_linear_swiglu(const void *x, const void *norm_weight, float eps, int dim, const void *w1, const void *w3,
+                     int64_t hidden, void *out, int dtype, void *stream);
+int da_linear_add(const void *x, int dim, const void *w, int64_t n_out, const void *residual, void *out,
+                  int dtype, void *stream);
+int da_linear_logits(const void *x, const void *norm_weight, float eps, int dim, const void *w, int64_t n_out,
+                     float *out, int dtype, void *stream);
+
+/* out[0] = index of the largest of n fp32 values (16-byte aligned): the lowest of equal ones, a NaN
+ * above everything (greedy decoding, examples/long-qa-chat/chat.py:255-262 of the reference). */
+int da_argmax(const float *x, int64_t n, int64_t *out, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

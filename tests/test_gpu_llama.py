@@ -268,3 +268,109 @@ def test_rope_kernel_matches_torch(S, Hq, Hkv, D, dtype):
     for got, x in ((q, xq), (k, xk)):
         want = L.apply_rope(x, rows).float()
         assert torch.allclose(got.cpu().float(), want, rtol=tol, atol=tol * 4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dim,n", [(8, 1), (256, 2), (520, 7), (2048, 66), (2056, 33), (4096, 257), (30720, 5)])
+def test_one_token_linear_kernels_match_torch(dim, n, dtype):
+    """The one-token layers at the edges of a wave's step (512 elements of 16 bits), of its
+    unrolled steps (2048) and at the longest row, odd and single output rows, against fp64
+    products of the same inputs.  Bound: sums of `dim` fp32 terms, then one turn of each
+    rounding to the type (a unit in the last place: 2^-7 of the value in bf16, 2^-10 in
+    fp16); silu and the product add one more each."""
+    if dim * (4 if dtype == torch.float32 else 2) > L.K.MAX_LINEAR_ROW:
+        dim //= 2
+    ulp = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 4e-6}[dtype]
+    g = torch.Generator().manual_seed(dim + n)
+
+    def draw(*shape, scale=1.0):
+        return (scale * torch.randn(*shape, generator=g)).to(dtype).cuda()
+
+    x, res = draw(1, 1, dim), draw(1, 1, n)
+    w, w3 = draw(n, dim, scale=dim ** -0.5), draw(n, dim, scale=dim ** -0.5)
+    norm = L.RMSNorm(dim).cuda().to(dtype)
+    with torch.no_grad():
+        norm.weight.copy_(draw(dim, scale=0.1) + 1)
+        xn = norm(x).double()
+
+        def rounded(t):
+            return t.to(dtype).double()
+
+        def near(got, want, ulps):
+            assert torch.allclose(got.double().flatten(), want.flatten(), rtol=ulps * ulp, atol=ulps * ulp * 0.3)
+
+        y, y3 = rounded(xn.flatten() @ w.double().t().contiguous()), rounded(xn.flatten() @ w3.double().t().contiguous())
+        near(L.K.linear_logits(x, norm, w), y, 2)
+        near(L.K.linear_swiglu(x, norm, w, w3), rounded(torch.nn.functional.silu(y)) * y3, 4)
+        near(L.K.linear_add(x, w, res), res.double().flatten() + rounded(x.double().flatten() @ w.double().t().contiguous()), 3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_one_token_qkv_kernel_matches_the_modules(dtype):
+    g = torch.Generator().manual_seed(3)
+    Hq, Hkv, D, dim = 6, 2, 64, 264
+    x = torch.randn(1, 1, dim, generator=g).to(dtype).cuda()
+    wq, wk, wv = ((torch.randn(h * D, dim, generator=g) / 16).to(dtype).cuda() for h in (Hq, Hkv, Hkv))
+    row = L.rope_table(D, 20, 1e4, False, device="cuda")[13:14]
+    norm = L.RMSNorm(dim).cuda().to(dtype)
+    with torch.no_grad():
+        q, k, v = L.K.linear_qkv_rope(x, norm, wq, wk, wv, Hq, Hkv, D, row)
+        xn = norm(x)
+        # one turn of the projection's rounding, spread over a pair by the rotation, one of the last
+        ulp = {torch.bfloat16: 2.0 ** -6, torch.float16: 2.0 ** -9, torch.float32: 4e-6}[dtype]
+        for got, w, h, rotated in ((q, wq, Hq, True), (k, wk, Hkv, True), (v, wv, Hkv, False)):
+            y = (xn.double() @ w.double().t().contiguous()).to(dtype).view(1, 1, h, D)
+            want = L.apply_rope(y, row) if rotated else y
+            assert got.shape == want.shape
+            assert torch.allclose(got.double(), want.double(), rtol=ulp, atol=ulp)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 16384, 16385, 128256])
+def test_argmax_kernel(n):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randint(-50, 50, (n,), generator=g, device="cuda").float() / 7      # many ties
+    token = torch.zeros(1, dtype=torch.int64, device="cuda")
+
+    def check():
+        L.K.argmax_into(x, token)
+        best = float("nan") if x.isnan().any() else x.max().item()
+        hits = (x.isnan() if best != best else x == best).nonzero()
+        assert token.item() == hits[0].item()
+
+    check()
+    x[n // 2] = float("inf")
+    check()
+    x[n - 1] = float("nan")
+    check()
+    x.fill_(float("-inf"))
+    check()
+
+
+def test_a_hooked_or_replaced_module_is_still_called():
+    """The one-token kernels leave out no module that somebody watches or has exchanged."""
+    args = small_args(torch.bfloat16)
+    model = build(args, 8)
+    prompt = torch.arange(600, device="cuda")[None] % args.vocab_size
+    model(prompt, 0)
+    seen = []
+    block = model.layers[1]
+    handles = [m.register_forward_hook(lambda mod, inp, out: seen.append(mod))
+               for m in (block.attention, block.feed_forward.w1, block.ffn_norm, model.output)]
+    token = torch.tensor([[5]], device="cuda")
+    model(token, 600)
+    assert set(seen) == {block.attention, block.feed_forward.w1, block.ffn_norm, model.output} and len(seen) == 4
+    for h in handles:
+        h.remove()
+
+    class Doubled(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner, self.calls = inner, 0
+
+        def forward(self, x):
+            self.calls += 1
+            return 2 * self.inner(x)
+
+    block.attention.wo = Doubled(block.attention.wo)
+    model(token, 601)
+    assert block.attention.wo.calls == 1
