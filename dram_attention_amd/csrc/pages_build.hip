@@ -8,21 +8,32 @@
 //
 // Bound: host link (every byte of K and V crosses it once, as posted writes);
 // algorithmic bytes = 2*S*Hkv*D*e read from HBM, the same written to the host,
-// N_hbm*page_bytes*Hkv written to HBM.
+// N_hbm*page_bytes*Hkv written to HBM.  Alone: 54.7 GB/s (9.8 ms for 537 MB).
+//
+// The grid is one-dimensional over (page, head) items, so that a caller that has other work
+// for the chip can ask for few workgroups: one moves about 7.6 GB/s, 32 fill the link.
+// Beside prefill attention every workgroup here keeps a compute unit from it (attention
+// takes a unit's whole register file), and a full link slows the misses of its caches:
+// 131072 tokens next to 138.1 ms of attention end after 138.9 ms with 2 workgroups, 139.4 with
+// 4, 139.7 with 8, 142.3 with one per page, against 148 ms one after the other; 8192 tokens next
+// to 0.60 ms after 0.82 ms with 8 or 16, 0.90 with 32, 1.08 with one per page, against 1.21 ms.
+// Loads and stores are streaming: nothing here is read again soon, and attention's keys
+// and values keep their place in the L2s (16 workgroups: +2.7 instead of +3.4 ms).
 #include "common.hpp"
 
 namespace da {
 
 __global__ void __launch_bounds__(256)
 pages_build_kernel(const char *__restrict__ k, const char *__restrict__ v, int64_t tok_stride_b,
-                   int64_t head_stride_b, int64_t n_pages, int page_size, int lanes,
+                   int64_t head_stride_b, int64_t n_pages, int n_heads, int page_size, int lanes,
                    char *__restrict__ dram, int64_t dram_head_stride, int64_t dram_page_stride,
                    char *__restrict__ hbm, int64_t hbm_head_stride, int64_t hbm_slot_stride,
                    int64_t first_resident, int64_t n_slots) {
-  const int h = blockIdx.y;
   const int tok_lanes = 2 * lanes;             // 16-byte lanes per token (K row, V row)
   const int page_vecs = page_size * tok_lanes;
-  for (int64_t p = blockIdx.x; p < n_pages; p += gridDim.x) {
+  for (int64_t item = blockIdx.x; item < n_pages * n_heads; item += gridDim.x) {
+    const int64_t p = item / n_heads;          // a page of every head, then the next page
+    const int h = (int)(item % n_heads);
     char *dst = dram ? dram + h * dram_head_stride + p * dram_page_stride : nullptr;
     const int64_t slot = p - first_resident;
     char *dst2 = (hbm && slot >= 0 && slot < n_slots)
@@ -37,15 +48,15 @@ pages_build_kernel(const char *__restrict__ k, const char *__restrict__ v, int64
           const int tok = j / tok_lanes, within = j % tok_lanes;
           const char *src = (within >= lanes ? v : k) + h * head_stride_b +
                             (p * page_size + tok) * tok_stride_b + (within % lanes) * 16;
-          r[u] = load16(src);
+          r[u] = load16_stream(src);
         }
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int j = j0 + u * 256;
         if (j < page_vecs) {
-          if (dst) store16(dst + (int64_t)j * 16, r[u]);
-          if (dst2) store16(dst2 + (int64_t)j * 16, r[u]);
+          if (dst) store16_stream(dst + (int64_t)j * 16, r[u]);
+          if (dst2) store16_stream(dst2 + (int64_t)j * 16, r[u]);
         }
       }
     }
@@ -54,12 +65,13 @@ pages_build_kernel(const char *__restrict__ k, const char *__restrict__ v, int64
 
 }  // namespace da
 
-extern "C" int da_pages_build(const void *k, const void *v, int64_t tok_stride, int64_t head_stride,
-                              int n_kv_heads, int64_t n_pages, int page_size, int head_dim,
-                              int dtype, void *dram, int64_t dram_head_stride_bytes,
-                              int64_t dram_page_stride_bytes, void *hbm,
-                              int64_t hbm_head_stride_bytes, int64_t hbm_slot_stride_bytes,
-                              int64_t first_resident_page, int64_t n_slots, void *stream) {
+extern "C" int da_pages_build_beside(const void *k, const void *v, int64_t tok_stride, int64_t head_stride,
+                                     int n_kv_heads, int64_t n_pages, int page_size, int head_dim,
+                                     int dtype, void *dram, int64_t dram_head_stride_bytes,
+                                     int64_t dram_page_stride_bytes, void *hbm,
+                                     int64_t hbm_head_stride_bytes, int64_t hbm_slot_stride_bytes,
+                                     int64_t first_resident_page, int64_t n_slots, int max_blocks,
+                                     void *stream) {
   using namespace da;
   DA_REQUIRE(n_kv_heads >= 0 && n_pages >= 0 && page_size > 0 && head_dim > 0 && n_slots >= 0,
              "da_pages_build: bad geometry");
@@ -80,11 +92,23 @@ extern "C" int da_pages_build(const void *k, const void *v, int64_t tok_stride, 
              "da_pages_build: operands must be 16-byte aligned");
   const int lanes = (int)(row_bytes / 16);
   DA_REQUIRE((int64_t)page_size * 2 * lanes <= 0x7fffffff, "da_pages_build: page too large");
-  const int64_t blocks = n_pages < 2048 ? n_pages : 2048;
-  dim3 grid((unsigned)blocks, n_kv_heads);
-  hipLaunchKernelGGL(pages_build_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const char *)k,
-                     (const char *)v, tok_stride * e, head_stride * e, n_pages, page_size, lanes,
+  const int64_t most = max_blocks > 0 ? max_blocks : 16384;
+  const int64_t items = n_pages * n_kv_heads;
+  hipLaunchKernelGGL(pages_build_kernel, dim3((unsigned)(items < most ? items : most)), dim3(256), 0,
+                     (hipStream_t)stream, (const char *)k, (const char *)v, tok_stride * e,
+                     head_stride * e, n_pages, n_kv_heads, page_size, lanes,
                      (char *)dram, dram_head_stride_bytes, dram_page_stride_bytes, (char *)hbm,
                      hbm_head_stride_bytes, hbm_slot_stride_bytes, first_resident_page, n_slots);
   return launch_status("da_pages_build");
+}
+
+extern "C" int da_pages_build(const void *k, const void *v, int64_t tok_stride, int64_t head_stride,
+                              int n_kv_heads, int64_t n_pages, int page_size, int head_dim,
+                              int dtype, void *dram, int64_t dram_head_stride_bytes,
+                              int64_t dram_page_stride_bytes, void *hbm,
+                              int64_t hbm_head_stride_bytes, int64_t hbm_slot_stride_bytes,
+                              int64_t first_resident_page, int64_t n_slots, void *stream) {
+  return da_pages_build_beside(k, v, tok_stride, head_stride, n_kv_heads, n_pages, page_size, head_dim, dtype,
+                               dram, dram_head_stride_bytes, dram_page_stride_bytes, hbm, hbm_head_stride_bytes,
+                               hbm_slot_stride_bytes, first_resident_page, n_slots, 0, stream);
 }

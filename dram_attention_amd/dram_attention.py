@@ -227,6 +227,36 @@ def _prefill_operands(xq, xk, xv, lse):
                  xk.stride(2), xv.data_ptr(), xv.stride(1), xv.stride(2))
 
 
+def store_build_blocks(q_shape, k_shape, dtype: torch.dtype) -> int:
+    """Workgroups that write the page store next to prefill attention: as few as are done
+    well within attention's time, because each takes a compute unit from it and a full
+    link slows it besides; at most the 32 that fill the link, which is what a prompt gets
+    whose store takes longer than its attention.  Rates: attention at 1 PFLOP/s, or 110
+    TFLOP/s in fp32; 7.6 GB/s to the host per workgroup, 3.7 beside fp32 attention, whose
+    workgroups leave room on a unit and then share it.  (Next to 138 ms of attention over
+    131072 tokens, 2, 4, 8 and 32 workgroups add 0.8, 1.2, 1.5 and 5 ms; next to 0.17 ms
+    over 4096, 8, 16 and 32 end after 0.45, 0.37 and 0.34 ms.)"""
+    _, S, Hq, D = q_shape
+    flops_per_s, bytes_per_s, esize = (1.1e14, 3.7e9, 4) if dtype == torch.float32 else (1e15, 7.6e9, 2)
+    attention_s = 2.0 * S * S * Hq * D / flops_per_s
+    store_bytes = 2.0 * S * k_shape[2] * D * esize
+    return max(2, min(32, math.ceil(store_bytes / bytes_per_s / (0.7 * attention_s))))
+
+
+_build_streams = {}
+
+
+def build_stream(device: torch.device) -> torch.cuda.Stream:
+    """The stream that page stores are written on next to prefill attention: one per device
+    for all layers (what it is given waits for its caller's stream and is waited for before
+    the call returns; a stream of its own would cost every new layer's first prompt
+    another 0.2 ms)."""
+    stream = _build_streams.get(device)
+    if stream is None:
+        stream = _build_streams.setdefault(device, torch.cuda.Stream(device=device))
+    return stream
+
+
 def causal_prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor,
                              backend: str = "auto") -> torch.Tensor:
     """Dense causal attention over the prompt, (1,S,Hq,D) -> (1,S,Hq,D), in place of
@@ -342,6 +372,10 @@ class DRAMAttention(torch.nn.Module):
     def init_cache(self, k_cache: torch.Tensor, v_cache: torch.Tensor):
         """Split the prompt's (1,S,Hkv,D) keys/values into the paged prefix and the
         local window, and build the page cache."""
+        self._build_cache(k_cache, v_cache)
+
+    def _build_cache(self, k_cache: torch.Tensor, v_cache: torch.Tensor, **build):
+        """init_cache; ``build``: where an LRUCache writes its page store."""
         bsz, seqlen, H, D = k_cache.shape
         assert bsz == 1, "Only support batch size 1"
         paged = (seqlen - self.local_cache_size + self.page_size) // self.page_size
@@ -359,6 +393,7 @@ class DRAMAttention(torch.nn.Module):
                 top_k=self.top_k // self.page_size,
                 lru_hbm_cache_size=self.lru_hbm_cache_size,
                 device=self.device,
+                **build,
             )
             self.link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
             if self.page_selector == "token_max":
@@ -413,13 +448,28 @@ class DRAMAttention(torch.nn.Module):
         bsz, seqlen, H, D = xq.shape
         assert bsz == 1, "Only support batch size 1"
         if stage == "prefill":
-            output = causal_prefill_attention(xq, xk, xv, self.prefill_backend)
-            self.init_cache(xk, xv)
-            return output
+            return self._prefill(xq, xk, xv)
         elif stage == "generate":
             return self._generate(xq, xk, xv, start_pos)
         else:
             raise RuntimeError(f"Unsupported stage: {stage}")
+
+    def _prefill(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor):
+        """Attention over the prompt and the caches built from it.  Where a library kernel
+        attends, the page store is written next to it, on a stream of its own: attention is
+        bound by the matrix cores, the store by the host link."""
+        if not (self.prefill_backend in ("auto", "native") and xk.is_cuda
+                and (prefill_attention_supported(xq) or prefill_attention_f32_supported(xq, xk, xv))):
+            output = causal_prefill_attention(xq, xk, xv, self.prefill_backend)
+            self.init_cache(xk, xv)
+            return output
+        self._build_cache(xk, xv, build_stream=build_stream(xk.device),
+                          build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype))
+        try:
+            return causal_prefill_attention(xq, xk, xv, self.prefill_backend)
+        finally:
+            if isinstance(self.lru_cache, LRUCache):
+                self.lru_cache.finish_build()
 
     def _generate(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, start_pos):
         """One decode step: select pages, update the LRU, then one attention pass

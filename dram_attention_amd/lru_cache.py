@@ -58,7 +58,14 @@ class LRUCache(torch.nn.Module):
         lru_hbm_cache_size: Optional[int] = None,
         hbm_kv_cache_fraction: float = 0.2,
         device: str = "cuda",
+        *,
+        build_stream: Optional[torch.cuda.Stream] = None,
+        build_blocks: int = 0,
     ):
+        """``build_stream``: where the page store is written, by at most ``build_blocks``
+        workgroups, next to what the caller issues on the current stream meanwhile; the
+        caller ends that with :meth:`finish_build` before anything reads or frees the
+        keys, the store or the slots.  By default the store is complete on return."""
         super().__init__()
         assert k_cache.shape == v_cache.shape, "Key and value cache shapes must match."
         num_kv_heads, dram_kv_cache_size, head_dim = k_cache.shape
@@ -100,6 +107,11 @@ class LRUCache(torch.nn.Module):
 
         # Start with the most recent pages resident: slot s holds page P - N + s.
         first = num_dram_pages - num_hbm_pages
+        slots = torch.arange(num_hbm_pages, dtype=torch.int64, device=device)
+        self.dram_page_to_hbm_page_mapping[:, first:] = slots
+        self.hbm_page_to_dram_page_mapping[:] = slots + first
+
+        self._build_stream = None
         row_bytes = head_dim * k_cache.element_size()
         if (k_cache.is_cuda and v_cache.is_cuda and row_bytes % 16 == 0 and num_dram_pages > 0
                 and k_cache.stride(-1) == 1 and v_cache.stride(-1) == 1
@@ -109,16 +121,24 @@ class LRUCache(torch.nn.Module):
             # one kernel packs every page into the pinned store and the resident ones into slots
             esz = k_cache.element_size()
             self._dram_device_ptr = _lib.device_visible_ptr(dram)
+            current = torch.cuda.current_stream(self.hbm_kv_cache.device)
+            stream = current if build_stream is None else build_stream
+            if build_stream is not None:
+                # (after the allocations above: their memory may still be in use by what the
+                # current stream was given before)
+                build_stream.wait_stream(current)
             _lib.check(
-                _lib.load().da_pages_build(
+                _lib.load().da_pages_build_beside(
                     k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(1), k_cache.stride(0),
                     num_kv_heads, num_dram_pages, page_size, head_dim, _lib.dtype_code(dtype),
                     self._dram_device_ptr, dram.stride(0) * esz, dram.stride(1) * esz,
                     self.hbm_kv_cache.data_ptr(), self.hbm_kv_cache.stride(0) * esz,
                     self.hbm_kv_cache.stride(1) * esz, first, num_hbm_pages,
-                    _lib.stream_ptr(self.hbm_kv_cache.device)),
+                    0 if build_stream is None else build_blocks, stream.cuda_stream),
                 "da_pages_build")
-            torch.cuda.current_stream(self.hbm_kv_cache.device).synchronize()  # host store complete
+            self._build_stream = stream
+            if build_stream is None:
+                self.finish_build()
         else:
             # host-resident or oddly shaped inputs: torch copies, then the slots from the store
             self._dram_device_ptr = None
@@ -130,12 +150,19 @@ class LRUCache(torch.nn.Module):
             if k_cache.is_cuda or v_cache.is_cuda:
                 torch.cuda.current_stream(self.hbm_kv_cache.device).synchronize()  # D2H copies
             self.hbm_kv_cache.copy_(dram[:, first:], non_blocking=True)
-        slots = torch.arange(num_hbm_pages, dtype=torch.int64, device=device)
-        self.dram_page_to_hbm_page_mapping[:, first:] = slots
-        self.hbm_page_to_dram_page_mapping[:] = slots + first
 
         self._scratch = None
         self._topk_idx = None
+
+    def finish_build(self) -> None:
+        """The page store is complete, on the host too, and the current stream is ordered
+        after it."""
+        stream, self._build_stream = self._build_stream, None
+        if stream is not None:
+            current = torch.cuda.current_stream(self.hbm_kv_cache.device)
+            if stream != current:
+                current.wait_stream(stream)
+            stream.synchronize()
 
     # -- internals ---------------------------------------------------------
     def _scratch_for(self, k: int) -> LruScratch:

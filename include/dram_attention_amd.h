@@ -121,6 +121,15 @@ int da_pages_build(const void *k, const void *v, int64_t tok_stride, int64_t hea
                    void *hbm, int64_t hbm_head_stride_bytes, int64_t hbm_slot_stride_bytes,
                    int64_t first_resident_page, int64_t n_slots, void *stream);
 
+/* The same with at most `max_blocks` workgroups (0 = no limit): for a build that runs next to
+ * other work on the chip.  One workgroup moves about 7.6 GB/s to the host, 32 fill the link. */
+int da_pages_build_beside(const void *k, const void *v, int64_t tok_stride, int64_t head_stride,
+                          int n_kv_heads, int64_t n_pages, int page_size, int head_dim,
+                          int dtype, void *dram, int64_t dram_head_stride_bytes,
+                          int64_t dram_page_stride_bytes, void *hbm,
+                          int64_t hbm_head_stride_bytes, int64_t hbm_slot_stride_bytes,
+                          int64_t first_resident_page, int64_t n_slots, int max_blocks, void *stream);
+
 /*
  * Subsystem 2 — Quest upper-bound page score
  *     score[n,h,l] = sum_d max(q[n,h,d]*mm[h,l,0,d], q[n,h,d]*mm[h,l,1,d]).

@@ -186,3 +186,33 @@ def test_fp32_prefill_kernel_matches_dense_float64(S, Hq, Hkv, D):
         s_ = (q @ k.t().contiguous() / math.sqrt(D)).masked_fill_(mask, float("-inf"))
         assert close(out[0, :, h].double(), torch.softmax(s_, -1) @ v, 1e-5, 1e-5)
         assert close(lse[h].double(), torch.logsumexp(s_, -1), 1e-5, 1e-5)
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,dtype", [
+    (600, 2, 2, 64, torch.bfloat16), (3000, 8, 2, 64, torch.float32), (9000, 32, 8, 128, torch.bfloat16),
+    (12345, 64, 8, 128, torch.float16),
+])
+def test_page_store_written_beside_attention_is_complete_on_return(S, Hq, Hkv, D, dtype):
+    """stage="prefill" writes the page store on a stream of its own while attention runs;
+    the host finds it complete when the call returns, slots and store equal init_cache's,
+    whatever number of workgroups the rule gives (32, the limit, to 2), twice in a row on one
+    module with the keys freed right after the call."""
+    from dram_attention_amd import DRAMAttention
+    from dram_attention_amd.dram_attention import causal_prefill_attention, store_build_blocks
+
+    assert 2 <= store_build_blocks((1, S, Hq, D), (1, S, Hkv, D), dtype) <= 32
+    m, ref = (DRAMAttention(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16,
+                            top_k=64, n_kv_heads=Hkv, head_dim=D, device=DEV, dtype=dtype) for _ in range(2))
+    for seed in (1, 2):
+        xq, xk, xv = draw(S, Hq, Hkv, D, dtype, seed)
+        out = m(xq, xk, xv, start_pos=0, stage="prefill")
+        store = m.lru_cache.dram_kv_cache.clone()          # read by the host, nothing waited for
+        want = causal_prefill_attention(xq, xk, xv)
+        ref.init_cache(xk, xv)
+        del xk, xv
+        junk = torch.full((S, Hkv, 4 * D), 7.0, device=DEV, dtype=dtype)   # takes the freed memory
+        assert same(store, ref.lru_cache.dram_kv_cache)
+        for name in ("hbm_kv_cache", "dram_page_to_hbm_page_mapping", "hbm_page_to_dram_page_mapping"):
+            assert same(getattr(m.lru_cache, name), getattr(ref.lru_cache, name))
+        assert same(out, want)
+        del junk
