@@ -18,6 +18,7 @@ LIB_PATH = HERE / "libdramattn.so"
 SOURCES = (
     "api.hip",
     "page_minmax.hip",
+    "cache_init.hip",
     "pages_build.hip",
     "page_score.hip",
     "topk_pages.hip",

@@ -85,31 +85,29 @@ class LRUCache(torch.nn.Module):
         self.top_k = top_k
 
         self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device)
-        self.register_buffer("current_step", torch.zeros(1, dtype=torch.int32, device=device))
-
+        assert num_hbm_pages <= num_dram_pages, "HBM cache size must be smaller than DRAM cache size."
         page_dim = page_size * 2 * head_dim
         dram = torch.empty((num_kv_heads, num_dram_pages, page_dim), dtype=dtype, device="cpu",
                            pin_memory=True)
+        self.register_buffer("current_step", torch.empty(1, dtype=torch.int32, device=device))
         self.register_buffer("dram_kv_cache", dram)
-        self.register_buffer(
-            "hbm_kv_cache",
-            torch.empty(num_kv_heads, num_hbm_pages, page_dim, dtype=dtype, device=device))
-        self.register_buffer(
-            "page_access_time",
-            torch.zeros(num_kv_heads, num_hbm_pages, dtype=torch.float32, device=device))
-        self.register_buffer(
-            "dram_page_to_hbm_page_mapping",
-            torch.full((num_kv_heads, num_dram_pages), -1, dtype=torch.int64, device=device))
-        self.register_buffer(
-            "hbm_page_to_dram_page_mapping",
-            torch.full((num_kv_heads, num_hbm_pages), -1, dtype=torch.int64, device=device))
-        assert num_hbm_pages <= num_dram_pages, "HBM cache size must be smaller than DRAM cache size."
+        for name, shape, kind in (
+                ("hbm_kv_cache", (num_kv_heads, num_hbm_pages, page_dim), dtype),
+                ("page_access_time", (num_kv_heads, num_hbm_pages), torch.float32),
+                ("dram_page_to_hbm_page_mapping", (num_kv_heads, num_dram_pages), torch.int64),
+                ("hbm_page_to_dram_page_mapping", (num_kv_heads, num_hbm_pages), torch.int64)):
+            self.register_buffer(name, torch.empty(shape, dtype=kind, device=device))
 
         # Start with the most recent pages resident: slot s holds page P - N + s.
         first = num_dram_pages - num_hbm_pages
-        slots = torch.arange(num_hbm_pages, dtype=torch.int64, device=device)
-        self.dram_page_to_hbm_page_mapping[:, first:] = slots
-        self.hbm_page_to_dram_page_mapping[:] = slots + first
+        current = torch.cuda.current_stream(self.hbm_kv_cache.device)
+        _lib.check(
+            _lib.load().da_page_cache_init(
+                self.current_step.data_ptr(), self.page_access_time.data_ptr(),
+                self.dram_page_to_hbm_page_mapping.data_ptr(),
+                self.hbm_page_to_dram_page_mapping.data_ptr(), num_kv_heads, num_dram_pages,
+                num_hbm_pages, current.cuda_stream),
+            "da_page_cache_init")
 
         self._build_stream = None
         row_bytes = head_dim * k_cache.element_size()
@@ -121,7 +119,6 @@ class LRUCache(torch.nn.Module):
             # one kernel packs every page into the pinned store and the resident ones into slots
             esz = k_cache.element_size()
             self._dram_device_ptr = _lib.device_visible_ptr(dram)
-            current = torch.cuda.current_stream(self.hbm_kv_cache.device)
             stream = current if build_stream is None else build_stream
             if build_stream is not None:
                 # (after the allocations above: their memory may still be in use by what the
@@ -148,7 +145,7 @@ class LRUCache(torch.nn.Module):
             paged[..., 1, :].copy_(
                 v_cache.reshape(num_kv_heads, num_dram_pages, page_size, head_dim), non_blocking=True)
             if k_cache.is_cuda or v_cache.is_cuda:
-                torch.cuda.current_stream(self.hbm_kv_cache.device).synchronize()  # D2H copies
+                current.synchronize()  # D2H copies
             self.hbm_kv_cache.copy_(dram[:, first:], non_blocking=True)
 
         self._scratch = None

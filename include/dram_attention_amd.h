@@ -103,6 +103,14 @@ int da_page_minmax(const void *k, int64_t k_head_stride, int64_t k_tok_stride,
                    int dtype, void *out, void *stream);
 
 /*
+ * Initial metadata of a page cache, lru_cache.py:143-189: current_step 0, access times 0
+ * (n_kv_heads, n_slots), slot s holds page n_pages - n_slots + s; maps (n_kv_heads, n_pages)
+ * and (n_kv_heads, n_slots), -1 = not resident.  All arrays contiguous.
+ */
+int da_page_cache_init(int32_t *current_step, float *access_time, int64_t *dram_to_hbm, int64_t *hbm_to_dram,
+                       int n_kv_heads, int64_t n_pages, int64_t n_slots, void *stream);
+
+/*
  * Subsystem 1b — build the paged KV store from the prompt's keys and values.
  * Replaces the torch copies of LRUCache.__init__, dram_attention/lru_cache.py:131-141
  * (interleaved page layout in the pinned store) and :191-209 (initial slots).

@@ -763,3 +763,22 @@ def test_lru_update_with_a_caller_stamp_and_more_slots_than_the_walk_orders_is_r
     lru_update(dram, time, d2h, h2d, idx, step, hbm, sc, bump_step=True)      # the bumped form runs
     torch.cuda.synchronize()
     assert step.item() == 2 and sc.miss_count.item() == K
+
+
+@pytest.mark.parametrize("H,P,N", [(1, 1, 0), (1, 1, 1), (3, 85, 85), (2, 128, 127), (8, 1000, 33)])
+def test_page_cache_init_kernel(H, P, N):
+    """Every slot holds one of the last N pages, nothing else is resident, no step taken;
+    the bytes around the arrays stay as they were."""
+    from dram_attention_amd import _lib
+
+    step = torch.full((3,), 7, dtype=torch.int32, device="cuda")
+    times = torch.full((H * N + 2,), 5.0, device="cuda")
+    d2h = torch.full((H * P + 2,), 99, dtype=torch.int64, device="cuda")
+    h2d = torch.full((H * N + 2,), 99, dtype=torch.int64, device="cuda")
+    _lib.check(_lib.load().da_page_cache_init(step[1:].data_ptr(), times[1:].data_ptr(), d2h[1:].data_ptr(),
+                                              h2d[1:].data_ptr(), H, P, N,
+                                              torch.cuda.current_stream().cuda_stream), "da_page_cache_init")
+    assert step.tolist() == [7, 0, 7]
+    assert times.tolist() == [5.0] + [0.0] * (H * N) + [5.0]
+    assert h2d.tolist() == [99] + list(range(P - N, P)) * H + [99]
+    assert d2h.tolist() == [99] + ([-1] * (P - N) + list(range(N))) * H + [99]
