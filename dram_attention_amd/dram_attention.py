@@ -378,11 +378,7 @@ class DRAMAttention(torch.nn.Module):
         """init_cache; ``build``: where an LRUCache writes its page store."""
         bsz, seqlen, H, D = k_cache.shape
         assert bsz == 1, "Only support batch size 1"
-        paged = (seqlen - self.local_cache_size + self.page_size) // self.page_size
-        self.dram_kv_cache_size = paged * self.page_size
-        tail = seqlen - self.dram_kv_cache_size
-        self.cache_k[:, :tail].copy_(k_cache[:, self.dram_kv_cache_size:], non_blocking=True)
-        self.cache_v[:, :tail].copy_(v_cache[:, self.dram_kv_cache_size:], non_blocking=True)
+        self.dram_kv_cache_size = self._paged_tokens(seqlen)
         prefix_k = k_cache[0, : self.dram_kv_cache_size].transpose(0, 1)
         prefix_v = v_cache[0, : self.dram_kv_cache_size].transpose(0, 1)
         if self.dram_kv_cache_size > self.lru_hbm_cache_size:
@@ -403,7 +399,14 @@ class DRAMAttention(torch.nn.Module):
                 raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
         else:
             self.lru_cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
+        tail = seqlen - self.dram_kv_cache_size
+        self.cache_k[:, :tail].copy_(k_cache[:, self.dram_kv_cache_size:], non_blocking=True)
+        self.cache_v[:, :tail].copy_(v_cache[:, self.dram_kv_cache_size:], non_blocking=True)
         self._workspace = None
+
+    def _paged_tokens(self, seqlen: int) -> int:
+        """Prompt tokens that go to the paged prefix; the rest is the local window."""
+        return (seqlen - self.local_cache_size + self.page_size) // self.page_size * self.page_size
 
     def _attend_selected(self, xq, xk, xv, cache_len, offset, idx, out):
         """The Quest baseline's attention (evaluation/quest/model.py:263-316): query head
@@ -458,18 +461,23 @@ class DRAMAttention(torch.nn.Module):
         """Attention over the prompt and the caches built from it.  Where a library kernel
         attends, the page store is written next to it, on a stream of its own: attention is
         bound by the matrix cores, the store by the host link."""
-        if not (self.prefill_backend in ("auto", "native") and xk.is_cuda
+        if not (self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
+                and self.prefill_backend in ("auto", "native") and xk.is_cuda
                 and (prefill_attention_supported(xq) or prefill_attention_f32_supported(xq, xk, xv))):
             output = causal_prefill_attention(xq, xk, xv, self.prefill_backend)
             self.init_cache(xk, xv)
             return output
-        self._build_cache(xk, xv, build_stream=build_stream(xk.device),
-                          build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype))
+        output = []
         try:
-            return causal_prefill_attention(xq, xk, xv, self.prefill_backend)
+            self._build_cache(
+                xk, xv, build_stream=build_stream(xk.device),
+                build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype),
+                beside=lambda: output.append(causal_prefill_attention(xq, xk, xv, self.prefill_backend)))
         finally:
-            if isinstance(self.lru_cache, LRUCache):
-                self.lru_cache.finish_build()
+            lru = getattr(self, "lru_cache", None)     # (none yet if the prompt was refused)
+            if isinstance(lru, LRUCache):
+                lru.finish_build()
+        return output[0]
 
     def _generate(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, start_pos):
         """One decode step: select pages, update the LRU, then one attention pass

@@ -7,7 +7,7 @@ DummyCache :24-37, LRUCache :40-265): same constructor, attributes, buffers and
 
 from __future__ import annotations
 
-from typing import NamedTuple, Optional
+from typing import Callable, NamedTuple, Optional
 
 import torch
 
@@ -61,11 +61,13 @@ class LRUCache(torch.nn.Module):
         *,
         build_stream: Optional[torch.cuda.Stream] = None,
         build_blocks: int = 0,
+        beside: Optional[Callable[[], None]] = None,
     ):
-        """``build_stream``: where the page store is written, by at most ``build_blocks``
-        workgroups, next to what the caller issues on the current stream meanwhile; the
-        caller ends that with :meth:`finish_build` before anything reads or frees the
-        keys, the store or the slots.  By default the store is complete on return."""
+        """``beside`` (with ``build_stream``): work that the caller issues on the current
+        stream as soon as the page store is being written, on ``build_stream`` and by at most
+        ``build_blocks`` workgroups; the rest of the construction is issued behind it.  The
+        caller then ends the build with :meth:`finish_build` before anything reads or frees
+        the keys, the store or the slots.  Without it the store is complete on return."""
         super().__init__()
         assert k_cache.shape == v_cache.shape, "Key and value cache shapes must match."
         num_kv_heads, dram_kv_cache_size, head_dim = k_cache.shape
@@ -84,7 +86,6 @@ class LRUCache(torch.nn.Module):
         self.num_hbm_pages = num_hbm_pages
         self.top_k = top_k
 
-        self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device)
         assert num_hbm_pages <= num_dram_pages, "HBM cache size must be smaller than DRAM cache size."
         page_dim = page_size * 2 * head_dim
         dram = torch.empty((num_kv_heads, num_dram_pages, page_dim), dtype=dtype, device="cpu",
@@ -101,14 +102,6 @@ class LRUCache(torch.nn.Module):
         # Start with the most recent pages resident: slot s holds page P - N + s.
         first = num_dram_pages - num_hbm_pages
         current = torch.cuda.current_stream(self.hbm_kv_cache.device)
-        _lib.check(
-            _lib.load().da_page_cache_init(
-                self.current_step.data_ptr(), self.page_access_time.data_ptr(),
-                self.dram_page_to_hbm_page_mapping.data_ptr(),
-                self.hbm_page_to_dram_page_mapping.data_ptr(), num_kv_heads, num_dram_pages,
-                num_hbm_pages, current.cuda_stream),
-            "da_page_cache_init")
-
         self._build_stream = None
         row_bytes = head_dim * k_cache.element_size()
         if (k_cache.is_cuda and v_cache.is_cuda and row_bytes % 16 == 0 and num_dram_pages > 0
@@ -119,11 +112,12 @@ class LRUCache(torch.nn.Module):
             # one kernel packs every page into the pinned store and the resident ones into slots
             esz = k_cache.element_size()
             self._dram_device_ptr = _lib.device_visible_ptr(dram)
-            stream = current if build_stream is None else build_stream
-            if build_stream is not None:
+            stream = current
+            if beside is not None:
                 # (after the allocations above: their memory may still be in use by what the
                 # current stream was given before)
-                build_stream.wait_stream(current)
+                stream = build_stream
+                stream.wait_stream(current)
             _lib.check(
                 _lib.load().da_pages_build_beside(
                     k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(1), k_cache.stride(0),
@@ -131,11 +125,9 @@ class LRUCache(torch.nn.Module):
                     self._dram_device_ptr, dram.stride(0) * esz, dram.stride(1) * esz,
                     self.hbm_kv_cache.data_ptr(), self.hbm_kv_cache.stride(0) * esz,
                     self.hbm_kv_cache.stride(1) * esz, first, num_hbm_pages,
-                    0 if build_stream is None else build_blocks, stream.cuda_stream),
+                    0 if beside is None else build_blocks, stream.cuda_stream),
                 "da_pages_build")
             self._build_stream = stream
-            if build_stream is None:
-                self.finish_build()
         else:
             # host-resident or oddly shaped inputs: torch copies, then the slots from the store
             self._dram_device_ptr = None
@@ -147,6 +139,23 @@ class LRUCache(torch.nn.Module):
             if k_cache.is_cuda or v_cache.is_cuda:
                 current.synchronize()  # D2H copies
             self.hbm_kv_cache.copy_(dram[:, first:], non_blocking=True)
+
+        try:
+            if beside is not None:
+                beside()
+            self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device)
+            _lib.check(
+                _lib.load().da_page_cache_init(
+                    self.current_step.data_ptr(), self.page_access_time.data_ptr(),
+                    self.dram_page_to_hbm_page_mapping.data_ptr(),
+                    self.hbm_page_to_dram_page_mapping.data_ptr(), num_kv_heads, num_dram_pages,
+                    num_hbm_pages, current.cuda_stream),
+                "da_page_cache_init")
+        except BaseException:
+            self.finish_build()     # nothing may go away under the kernel that is packing pages
+            raise
+        if beside is None:
+            self.finish_build()
 
         self._scratch = None
         self._topk_idx = None
