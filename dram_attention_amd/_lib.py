@@ -7,6 +7,7 @@ raises if it cannot be loaded; nothing falls back to torch or to the CPU.
 from __future__ import annotations
 
 import ctypes
+import struct
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -105,6 +106,7 @@ SIGNATURES = {
          c_void_p, c_int64, c_float, c_void_p, c_int64, c_void_p, c_void_p, c_size_t, c_void_p,
          c_void_p],
     ),
+    "da_decode_step": (c_int, [c_char_p, c_size_t, c_void_p]),
     "da_rms_norm": (
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "da_rope_rows": (
@@ -155,6 +157,10 @@ class PagedOverlap(ctypes.Structure):
         ("link_gbps", c_float),
         ("block_gbps", c_float),
     ]
+
+
+# struct da_decode_step_args of the header: 25 pointers, 7 int64, 10 int32, 3 floats, 1 int32
+DECODE_STEP_ARGS = struct.Struct("=25Q7q10i3fi")
 
 _lib = None
 

@@ -25,6 +25,7 @@ SOURCES = (
     "lru_update.hip",
     "decode_attention.hip",
     "stream_attention.hip",
+    "decode_step.hip",
     "prefill_attention.hip",
     "prefill_attention_f32.hip",
     "model_rows.hip",

@@ -18,7 +18,11 @@ import torch.nn.functional as F
 from . import _lib
 from .lru_cache import DummyCache, LRUCache
 from .lru_kernel import GATHER_BLOCKS, gather_attend_supported, host_link_gbps
-from .topk_selector import TokenMaxTopKSelector
+from .max_ip_kernel import DA_SCORE_ORDERED_BOUNDS, DA_SCORE_ROUND
+from .topk_selector import IPUpperboundTopKSelector, TokenMaxTopKSelector
+
+# da_page_score flags of a step by whether the summaries' bounds are ordered
+SCORE_FLAGS = {False: DA_SCORE_ROUND, True: DA_SCORE_ROUND | DA_SCORE_ORDERED_BOUNDS}
 
 
 class PagedPrefix:
@@ -484,7 +488,89 @@ class DRAMAttention(torch.nn.Module):
         over resident pages, local window and the new token (appended in place).
         The missed pages stream in on a side stream while attention already
         covers the local window and every slot that keeps its page."""
+        out = self._step_in_one_call(xq, xk, xv, start_pos)
+        if out is not None:
+            return out
         return self.attend_(xq, xk, xv, start_pos, self.select_(xq))
+
+    def _step_in_one_call(self, xq, xk, xv, start_pos):
+        """select_ and attend_ as one native call (da_decode_step) where everything has the
+        layout a layer is built with; None where anything differs, and the two methods, which
+        take or refuse it, do the step.  The same launches on the same operands."""
+        lru = self.lru_cache
+        cls = type(self)
+        if (type(lru) is not LRUCache or self.attention_scope != "resident" or not self.overlap_page_stream
+                or not self.attend_on_page_stream or cls.select_ is not DRAMAttention.select_
+                or cls.attend_ is not DRAMAttention.attend_):
+            return None
+        selector, buffers, own = lru.top_k_selector, lru._buffers, self._buffers
+        if type(selector) is not IPUpperboundTopKSelector:
+            return None
+        minmax, dram, hbm = selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"]
+        H, P, _, D = minmax.shape
+        N, page, dtype = lru.num_hbm_pages, lru.page_size, xq.dtype
+        if xq.dim() != 4:
+            return None
+        Hq = xq.shape[2]
+        rep, kp = Hq // H, min(lru.top_k, P)
+        times, d2h, h2d, step = (buffers["page_access_time"], buffers["dram_page_to_hbm_page_mapping"],
+                                 buffers["hbm_page_to_dram_page_mapping"], buffers["current_step"])
+        cache_k, cache_v = own["cache_k"], own["cache_v"]
+        capacity = cache_k.shape[1]
+        page_dim = page * 2 * D
+        if not (xq.shape == (1, 1, rep * H, D) and xk.shape == xv.shape == (1, 1, H, D) and kp > 0 and N > 0
+                and minmax.shape[2] == 2 and hbm.shape == (H, N, page_dim) and dram.shape == (H, P, page_dim)
+                and times.shape == h2d.shape == (H, N) and d2h.shape == (H, P)
+                and cache_k.shape == cache_v.shape == (1, capacity, H, D)
+                and times.dtype is torch.float32 and d2h.dtype is h2d.dtype is torch.int64
+                and step.dtype is torch.int32 and step.numel() == 1
+                and gather_attend_supported(Hq, H, D, page, dtype)):
+            return None
+        device = xq.device
+        for t in (xq, xk, xv, minmax, hbm, cache_k, cache_v):
+            if t.dtype is not dtype or t.device != device or not t.is_contiguous():
+                return None
+        for t in (times, d2h, h2d, step):
+            if t.device != device or not t.is_contiguous():
+                return None
+        if dram.dtype is not dtype or not dram.is_contiguous():
+            return None
+        if isinstance(start_pos, torch.Tensor):
+            if start_pos.dtype is not torch.int32 or start_pos.device != device:
+                return None
+            cache_len, cache_len_dev = -self.dram_kv_cache_size, start_pos.data_ptr()
+        else:
+            cache_len, cache_len_dev = int(start_pos) - self.dram_kv_cache_size, 0
+            if cache_len < 0 or cache_len >= capacity:
+                return None
+        total = rep * kp
+        scratch, idx, scores = lru._scratch_for(total), lru._topk_idx, selector._scores
+        if idx is None or idx.shape[1] != total:
+            idx = lru._topk_idx = torch.empty(H, total, dtype=torch.int64, device=device)
+        if scores is None or scores.shape[0] != rep:
+            scores = selector._scores = torch.empty(rep, H, P, dtype=torch.float32, device=device)
+        if scratch.slot_epoch.shape[1] != N:
+            return None
+        topk_ws = selector._workspace(scores, kp)
+        if self._workspace is None:
+            self._workspace = attention_workspace(Hq, H, D, dtype, N * page, capacity, total * page, device)
+        workspace = self._workspace
+        out = torch.empty(1, 1, Hq, D, dtype=dtype, device=device)
+        args = _lib.DECODE_STEP_ARGS.pack(
+            xq.data_ptr(), xk.data_ptr(), xv.data_ptr(), out.data_ptr(), minmax.data_ptr(), scores.data_ptr(),
+            idx.data_ptr(), 0 if topk_ws is None else topk_ws.data_ptr(), times.data_ptr(),
+            scratch.candidates.data_ptr(), step.data_ptr(), d2h.data_ptr(), h2d.data_ptr(),
+            scratch.hit_mask.data_ptr(), scratch.miss_page.data_ptr(), scratch.miss_slot.data_ptr(),
+            scratch.miss_count.data_ptr(), scratch.slot_epoch.data_ptr(), scratch.workspace.data_ptr(),
+            lru.page_stores()[1], hbm.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), cache_len_dev,
+            workspace.data_ptr(),
+            D, P, capacity, cache_len, 0 if topk_ws is None else topk_ws.numel(), scratch.workspace.numel(),
+            workspace.numel() * 4,
+            Hq, H, D, _lib.dtype_code(dtype), page, kp, N, scratch.candidates.shape[1],
+            SCORE_FLAGS[selector.bounds_are_ordered], max(1, min(self.stream_blocks // H, total)),
+            1.0 / math.sqrt(D), self.link_gbps, self.block_gbps, 0)
+        _lib.check(_lib.load().da_decode_step(args, len(args), _lib.stream_ptr(device)), "da_decode_step")
+        return out
 
     def select_(self, xq: torch.Tensor):
         """First half of a decode step: page scores, ordered top-k and the LRU update

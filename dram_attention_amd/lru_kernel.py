@@ -229,7 +229,7 @@ def host_link_gbps(device) -> float:
 def gather_attend_supported(n_q_heads: int, n_kv_heads: int, head_dim: int, page_size: int,
                             dtype: torch.dtype) -> bool:
     """Whether pages_gather_attend takes this shape (else: pages_gather + tail pass)."""
-    row = head_dim * torch.empty(0, dtype=dtype).element_size()
+    row = head_dim * dtype.itemsize
     return (row in (64, 128, 256, 512) and n_q_heads // n_kv_heads <= 8
             and page_size * 2 * row <= 16384 and n_kv_heads <= 64)
 

@@ -483,6 +483,43 @@ int da_pages_gather_attend(const void *dram, int64_t dram_head_stride_bytes,
                            void *stream);
 
 /*
+ * One whole decode step of a layer with a page cache: da_page_score, da_topk_pages_lru,
+ * da_lru_update (DA_LRU_BUMP_STEP) and da_decode_attention_paged (STREAM | FIRST |
+ * SECOND) on one argument block, in that order on `stream`; each of them checks its
+ * operands as when called alone.  For the layout a DRAMAttention layer has: every
+ * array contiguous, int64 maps and indexes, fp32 access times and scores.
+ * `args_bytes` = sizeof(da_decode_step_args).
+ */
+typedef struct da_decode_step_args {
+  const void *q;                    /* (Hq, D), head stride q_head_stride */
+  const void *new_k, *new_v;        /* (Hkv, D) */
+  void *out;                        /* (Hq, D) */
+  const void *minmax;               /* (Hkv, n_pages, 2, D) */
+  float *scores;                    /* (Hq/Hkv, Hkv, n_pages) */
+  int64_t *idx;                     /* (Hkv, Hq/Hkv * kp) */
+  void *topk_workspace;             /* as da_topk_pages */
+  float *access_time;               /* (Hkv, n_slots) */
+  int32_t *candidates;              /* as da_topk_pages_lru, k_cand entries per head */
+  int32_t *step;
+  int64_t *d2h, *h2d;               /* (Hkv, n_pages), (Hkv, n_slots) */
+  uint8_t *hit_mask;                /* (Hkv, Hq/Hkv * kp), as the two that follow; may be NULL */
+  int32_t *miss_page, *miss_slot, *miss_count, *slot_epoch;
+  void *lru_workspace;
+  const void *dram;                 /* (Hkv, n_pages, page_size*2*D), device-visible */
+  void *hbm;                        /* (Hkv, n_slots, page_size*2*D) */
+  void *cache_k, *cache_v;          /* (cache_rows, Hkv, D) */
+  const int32_t *cache_len_dev;     /* or NULL; cache_len is added to it */
+  void *workspace;                  /* as da_decode_attention_paged */
+  int64_t q_head_stride, n_pages, cache_rows, cache_len;
+  int64_t topk_workspace_bytes, lru_workspace_bytes, workspace_bytes;
+  int32_t n_q_heads, n_kv_heads, head_dim, dtype, page_size, kp, n_slots, k_cand, score_flags, gather_blocks;
+  float scale, link_gbps, block_gbps;
+  int32_t reserved;                 /* 0 */
+} da_decode_step_args;
+
+int da_decode_step(const da_decode_step_args *args, size_t args_bytes, void *stream);
+
+/*
  * Row-wise parts of the model around the attention layers (evaluation/dram-attention/
  * model.py of the reference), `rows` contiguous rows at a time; every operand 16-byte
  * aligned, rows a multiple of 16 bytes (DA_ENOTSUP otherwise).

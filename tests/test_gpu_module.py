@@ -824,3 +824,51 @@ def test_full_size_invariants(name, steps):
         xq, xk, xv = xq.to(DEV), xk.to(DEV), xv.to(DEV)
         out = m(xq, xk, xv, start_pos=w.prompt_tokens + t, stage="generate")
         check_invariants(m, w, xq, xk, xv, out, t, dram_dev)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,page,dtype", [(8, 2, 64, 16, torch.float32), (4, 4, 128, 32, torch.bfloat16),
+                                                 (14, 2, 64, 16, torch.float16)])
+def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
+    """forward(stage="generate") issues a whole step by one native call where a layer has the
+    layout it was built with; select_ + attend_ on a twin give the same bits, on host and on
+    device positions, and operands with another layout or a replaced buffer of another
+    type still take the two halves (strided queries, int32 access times)."""
+    from dram_attention_amd import DRAMAttention
+
+    S = 1500
+    g = torch.Generator(device=DEV).manual_seed(5)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    a, b = (DRAMAttention(12, 30 * page, 200, page, 6 * page, Hkv, D, device=DEV, dtype=dtype) for _ in range(2))
+    a.init_cache(k, v)
+    b.init_cache(k, v)
+
+    def check(t, xq, start):
+        xk, xv = rand(1, 1, Hkv, D), rand(1, 1, Hkv, D)
+        got = a(xq, xk, xv, start_pos=start, stage="generate")
+        want = b.attend_(xq, xk, xv, start, b.select_(xq))
+        assert same(got, want), t
+        for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
+                     "hbm_page_to_dram_page_mapping", "current_step"):
+            assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
+        assert same(a.cache_k, b.cache_k)
+
+    calls = []
+    one_call = a._step_in_one_call
+    a._step_in_one_call = lambda *args: calls.append(one_call(*args)) or calls[-1]
+    for t in range(3):
+        check(t, rand(1, 1, Hq, D), S + t)
+    check(3, rand(1, 1, Hq, D), torch.tensor([S + 3], dtype=torch.int32, device=DEV))
+    assert len(calls) == 4 and all(c is not None for c in calls)
+    check(4, rand(1, 1, Hq, 2 * D)[..., :D], S + 4)                 # strided rows
+    for m in (a, b):
+        m.lru_cache.page_access_time = m.lru_cache.page_access_time.to(torch.int32)
+    check(5, rand(1, 1, Hq, D), S + 5)
+    assert calls[4] is None and calls[5] is None
+    with pytest.raises(RuntimeError, match="one token per call"):
+        a(rand(1, 2, Hq, D), rand(1, 2, Hkv, D), rand(1, 2, Hkv, D), start_pos=S, stage="generate")
+    with pytest.raises(RuntimeError):                               # beyond the local cache
+        a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
