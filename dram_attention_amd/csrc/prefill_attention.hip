@@ -226,11 +226,9 @@ prefill_attention_kernel(const PrefillArgs a) {
   // One tile of 64 keys from LDS buffer `buf`; kMask: keys above a row are dropped.
   auto compute = [&](int tile, int buf, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
+    __builtin_amdgcn_iglp_opt(1);   // (measured: see the loop below)
     const char *kt = smem + buf * Sh::kBufBytes;
     pf_f32x16 st[2];
-    // (raised priority while a wave issues MFMAs: they go ahead of the vector work of the
-    // other wave on this SIMD, which fills the gaps; worth 0-2 % from run to run)
-    __builtin_amdgcn_s_setprio(3);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -239,7 +237,6 @@ prefill_attention_kernel(const PrefillArgs a) {
       for (int s = 0; s < kQSteps; ++s)
         st[half] = Ops::mma(*(const u32x4 *)(kt + k_at[s] + half * kHalfStep), qf[s], st[half]);
     }
-    __builtin_amdgcn_s_setprio(0);
     // register 4j + i of half `half`: key tile*64 + half*32 + 8j + 4g + i
     float smax = -INFINITY;
     if constexpr (kMask) {
@@ -282,7 +279,6 @@ prefill_attention_kernel(const PrefillArgs a) {
         pt[half * 2 + jj] = u32x4{Ops::pack(p[8 * jj], p[8 * jj + 1]), Ops::pack(p[8 * jj + 2], p[8 * jj + 3]),
                                   Ops::pack(p[8 * jj + 4], p[8 * jj + 5]), Ops::pack(p[8 * jj + 6], p[8 * jj + 7])};
     }
-    __builtin_amdgcn_s_setprio(3);
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {   // 16 keys each
 #pragma unroll
@@ -296,7 +292,6 @@ prefill_attention_kernel(const PrefillArgs a) {
         acc[b] = Ops::mma(va, pt[kk], acc[b]);
       }
     }
-    __builtin_amdgcn_s_setprio(0);
   };
 
   fetch(0, 0);
@@ -305,7 +300,24 @@ prefill_attention_kernel(const PrefillArgs a) {
 #pragma unroll
   for (int s = 0; s < kQSteps; ++s) asm volatile("" : "+v"(qf[s]));
   __syncthreads();                                  // (waits for this wave's tile loads first)
-  for (int tile = 0; tile < n_tiles; ++tile) {
+  // Tiles below the workgroup's first row, which every wave needs whole, go two a round:
+  // with the buffer known at compile time every LDS address is a register plus a constant,
+  // 12 vector additions fewer per tile and wave.  What this and the two changes that came
+  // with it give, in TFLOP/s (same bits): 135152 tokens, 32/8 heads, D 128: 1146 as it was, 1197
+  // with the rounds of two and without raised wave priority around the MFMAs (1123 with it:
+  // the other wave of the SIMD is the one to let in), 1211 with iglp_opt(1), which spreads the
+  // LDS reads between the MFMAs; 8192 tokens 1081 -> 1134, 4613 943 -> 998; 20000 tokens,
+  // 16/16 heads, D 64: 800 -> 912.
+  const int n_whole = (int)(m0 / kPfKeys) & ~1;
+  for (int tile = 0; tile < n_whole; tile += 2) {
+    fetch(tile + 1, 1);
+    compute(tile, 0, std::false_type{});
+    __syncthreads();
+    fetch(tile + 2, 0);                             // (there is one: the tiles of the block's own rows)
+    compute(tile + 1, 1, std::false_type{});
+    __syncthreads();
+  }
+  for (int tile = n_whole; tile < n_tiles; ++tile) {
     const int buf = tile & 1;
     // the other buffer was last read before the barrier that ended the previous round
     if (tile + 1 < n_tiles) fetch(tile + 1, buf ^ 1);
