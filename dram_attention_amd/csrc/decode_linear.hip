@@ -355,6 +355,17 @@ extern "C" int da_linear_logits(const void *x, const void *norm_weight, float ep
   return launch_linear<kEndLogits>("da_linear_logits", a, dtype, (hipStream_t)stream);
 }
 
+extern "C" int da_linear_block_tail(const void *attn, int attn_dim, const void *wo, const void *x, int dim,
+                                    const void *norm_weight, float eps, const void *w1, const void *w3,
+                                    int hidden, const void *w2, void *h, void *act, void *out, int dtype,
+                                    void *stream) {
+  int rc = da_linear_add(attn, attn_dim, wo, dim, x, h, dtype, stream);
+  if (rc) return rc;
+  rc = da_linear_swiglu(h, norm_weight, eps, dim, w1, w3, hidden, act, dtype, stream);
+  if (rc) return rc;
+  return da_linear_add(act, hidden, w2, dim, h, out, dtype, stream);
+}
+
 extern "C" int da_argmax(const float *x, int64_t n, int64_t *out, void *stream) {
   using namespace da;
   DA_REQUIRE(n > 0 && n <= 0x7fffffff, "da_argmax: 1 to 2^31 - 1 values");

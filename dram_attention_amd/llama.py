@@ -122,7 +122,7 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x):
-        if K.takes(x, self.weight) and K.norm_fits(x):
+        if K.takes(x, self.weight) and K.norm_fits(x, self.weight):
             return K.rms_norm(x, self.weight, self.eps)[0]
         x32 = x.float()
         normed = x32 * torch.rsqrt(x32.square().mean(-1, keepdim=True) + self.eps)
@@ -130,7 +130,7 @@ class RMSNorm(nn.Module):
 
     def after_add(self, x, y):
         """(norm of x + y, x + y)."""
-        if K.takes(x, y, self.weight) and K.norm_fits(x) and x.shape == y.shape:
+        if K.takes(x, y, self.weight) and K.norm_fits(x, self.weight) and x.shape == y.shape:
             return K.rms_norm(x, self.weight, self.eps, add=y)
         total = x + y
         return self(total), total
@@ -173,6 +173,8 @@ class Attention(nn.Module):
         xk = self.wk(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         xv = self.wv(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         if (K.takes(xq, xk) and rope_rows.dtype == torch.float32 and rope_rows.is_contiguous()
+                and rope_rows.device == xq.device
+                and bsz == 1 and rope_rows.shape == (seqlen, self.head_dim // 2, 2)
                 and self.head_dim * xq.element_size() % 16 == 0):
             K.rope_(xq, xk, rope_rows)          # the projections' own outputs, in place
         else:
@@ -200,7 +202,7 @@ class FeedForward(nn.Module):
 
     def _slice(self, x):
         gate, up = self.w1(x), self.w3(x)
-        if K.takes(gate, up) and gate.numel() * gate.element_size() % 16 == 0:
+        if K.takes(gate, up) and gate.shape == up.shape and gate.numel() * gate.element_size() % 16 == 0:
             return self.w2(K.swiglu_(gate, up))
         return self.w2(F.silu(gate) * up)
 
@@ -215,13 +217,17 @@ class TransformerBlock(nn.Module):
         self.ffn_norm = RMSNorm(args.dim, eps=args.norm_eps)
 
     def forward(self, x, start_pos, rope_rows):
-        if x.shape[0] == x.shape[1] == 1 and self._one_token_kernels(x, rope_rows):
-            a, f = self.attention, self.feed_forward
-            xq, xk, xv = K.linear_qkv_rope(x, self.attention_norm, a.wq.weight, a.wk.weight, a.wv.weight,
-                                           a.n_heads, a.n_kv_heads, a.head_dim, rope_rows)
-            out = a.dram_attention(xq, xk, xv, start_pos=start_pos, stage="generate")
-            h = K.linear_add(out, a.wo.weight, x)
-            return K.linear_add(K.linear_swiglu(h, self.ffn_norm, f.w1.weight, f.w3.weight), f.w2.weight, h)
+        if x.shape[0] == x.shape[1] == 1:
+            parts = self._modules
+            a, f, norm1, norm2 = (parts["attention"], parts["feed_forward"], parts["attention_norm"],
+                                  parts["ffn_norm"])
+            if self._one_token_kernels(a, f, norm1, norm2, x, rope_rows):
+                wq, wk, wv, wo = (a._modules[n]._parameters["weight"] for n in ("wq", "wk", "wv", "wo"))
+                w1, w2, w3 = (f._modules[n]._parameters["weight"] for n in ("w1", "w2", "w3"))
+                xq, xk, xv = K.linear_qkv_rope(x, norm1, wq, wk, wv, a.n_heads, a.n_kv_heads, a.head_dim,
+                                               rope_rows)
+                out = a.dram_attention(xq, xk, xv, start_pos=start_pos, stage="generate")
+                return K.block_tail(out, wo, x, norm2, w1, w3, w2)
         attended = self.attention(self.attention_norm(x), start_pos, rope_rows)
         if type(self.ffn_norm) is RMSNorm and K.bare(self.ffn_norm):
             normed, h = self.ffn_norm.after_add(x, attended)
@@ -231,15 +237,29 @@ class TransformerBlock(nn.Module):
         return h + self.feed_forward(normed)
 
 
-    def _one_token_kernels(self, x, rope_rows) -> bool:
-        """Whether the one-token kernels may stand for this block's modules."""
-        a, f = self.attention, self.feed_forward
-        return (type(a) is Attention and type(f) is FeedForward
-                and type(self.attention_norm) is RMSNorm and type(self.ffn_norm) is RMSNorm
-                and K.takes(x, self.attention_norm.weight, self.ffn_norm.weight)
-                and K.linears_fit(x, a.wq, a.wk, a.wv, a.wo, f.w1, f.w3, f.w2)
-                and K.bare(a, f, self.attention_norm, self.ffn_norm)
-                and rope_rows.dtype == torch.float32 and rope_rows.is_contiguous())
+    @staticmethod
+    def _one_token_kernels(a, f, norm1, norm2, x, rope_rows) -> bool:
+        """Whether the one-token kernels may stand for these modules of a block: the modules
+        are the block's own kinds, nobody watches them, and every shape is the one that the
+        kernels take for granted."""
+        if not (type(a) is Attention and type(f) is FeedForward and type(norm1) is type(norm2) is RMSNorm
+                and K.takes(x, norm1.weight, norm2.weight) and K.bare(a, f, norm1, norm2)
+                and rope_rows.dtype is torch.float32 and rope_rows.is_contiguous()
+                and rope_rows.device == x.device):
+            return False
+        am, fm, dim = a._modules, f._modules, x.shape[2]
+        wq, wk, wv, wo, w1, w2, w3 = am["wq"], am["wk"], am["wv"], am["wo"], fm["w1"], fm["w2"], fm["w3"]
+        if not K.linears_fit(x, wq, wk, wv, wo, w1, w3, w2):
+            return False
+        q_rows, kv_rows, hidden = a.n_heads * a.head_dim, a.n_kv_heads * a.head_dim, w1.out_features
+        return (dim * x.element_size() % 16 == 0
+                and (wq.out_features, wq.in_features) == (q_rows, dim)
+                and (wk.out_features, wk.in_features) == (wv.out_features, wv.in_features) == (kv_rows, dim)
+                and (wo.out_features, wo.in_features) == (dim, q_rows)
+                and (w3.out_features, w3.in_features) == (hidden, w1.in_features) == (hidden, dim)
+                and (w2.out_features, w2.in_features) == (dim, hidden)
+                and norm1.weight.shape == norm2.weight.shape == (dim,)
+                and rope_rows.shape == (1, a.head_dim // 2, 2) and a.head_dim % 2 == 0)
 
 
 class Transformer(nn.Module):
@@ -274,7 +294,8 @@ class Transformer(nn.Module):
             h = layer(h, start_pos, rows)
         last = h[:, -1:, :]
         if (last.shape[0] == 1 and K.takes(last, self.norm.weight) and K.linears_fit(last, self.output)
-                and type(self.norm) is RMSNorm and K.bare(self.norm)):
+                and type(self.norm) is RMSNorm and K.bare(self.norm)
+                and self.output.in_features == last.shape[2] and self.norm.weight.shape == last.shape[2:]):
             return K.linear_logits(last, self.norm, self.output.weight)
         return self.output(self.norm(last)).float()
 

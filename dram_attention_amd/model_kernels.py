@@ -23,9 +23,9 @@ def takes(*tensors: torch.Tensor) -> bool:
                for t in tensors)
 
 
-def norm_fits(x: torch.Tensor) -> bool:
+def norm_fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
     row = x.shape[-1] * x.element_size()
-    return row % 16 == 0 and row <= 32768
+    return weight.shape == x.shape[-1:] and x.numel() > 0 and row % 16 == 0 and row <= 32768
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, add: torch.Tensor | None = None):
@@ -73,13 +73,16 @@ MAX_LINEAR_ROW = 60 * 1024  # bytes of an input row the one-token layers hold in
 def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
     """Whether the one-token layers may stand for these nn.Linear modules (x: any tensor of
     the step, for its type and device)."""
+    dtype, device, esize = x.dtype, x.device, x.element_size()
     for m in linears:
-        if type(m) is not nn.Linear or m.bias is not None:
+        if type(m) is not nn.Linear:
             return False
-        w = m.weight
-        row = w.shape[1] * w.element_size()
-        if (w.dtype != x.dtype or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16
-                or row % 16 or row > MAX_LINEAR_ROW):
+        p = m._parameters
+        w = p["weight"]
+        row = m.in_features * esize
+        if (p["bias"] is not None or w.dtype is not dtype or w.device != device or not w.is_contiguous()
+                or w.shape != (m.out_features, m.in_features) or w.data_ptr() % 16 or row % 16
+                or row > MAX_LINEAR_ROW):
             return False
     return bare(*linears)
 
@@ -116,6 +119,21 @@ def linear_add(x, w, residual):
             x.data_ptr(), w.shape[1], w.data_ptr(), w.shape[0], residual.data_ptr(), out.data_ptr(),
             _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
         "da_linear_add")
+    return out
+
+
+def block_tail(attended, wo, x, norm, w1, w3, w2):
+    """The rest of a block behind attention's output, residuals included, as one call."""
+    dim, hidden = w2.shape
+    room = torch.empty(dim + hidden, dtype=x.dtype, device=x.device)
+    out = torch.empty_like(x)
+    h = room.data_ptr()
+    _lib.check(
+        _lib.load().da_linear_block_tail(
+            attended.data_ptr(), wo.shape[1], wo.data_ptr(), x.data_ptr(), dim, norm.weight.data_ptr(), norm.eps,
+            w1.data_ptr(), w3.data_ptr(), hidden, w2.data_ptr(), h, h + dim * x.element_size(), out.data_ptr(),
+            _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
+        "da_linear_block_tail")
     return out
 
 

@@ -559,6 +559,13 @@ int da_linear_add(const void *x, int dim, const void *w, int64_t n_out, const vo
 int da_linear_logits(const void *x, const void *norm_weight, float eps, int dim, const void *w, int64_t n_out,
                      float *out, int dtype, void *stream);
 
+/* What follows attention in a block, in one call (three launches): h = x + wo attn, then
+ * out = h + w2 (T(silu(w1 n)) * (w3 n)) with n the RMS norm of h.  attn (attn_dim), x, h and out
+ * (dim), act (hidden: room for the feed-forward row). */
+int da_linear_block_tail(const void *attn, int attn_dim, const void *wo, const void *x, int dim,
+                         const void *norm_weight, float eps, const void *w1, const void *w3, int hidden,
+                         const void *w2, void *h, void *act, void *out, int dtype, void *stream);
+
 /* out[0] = index of the largest of n fp32 values (16-byte aligned): the lowest of equal ones, a NaN
  * above everything (greedy decoding, examples/long-qa-chat/chat.py:255-262 of the reference). */
 int da_argmax(const float *x, int64_t n, int64_t *out, void *stream);

@@ -245,7 +245,7 @@ def test_norm_and_swiglu_kernels_match_torch(rows, dim, dtype):
         gate, up = x * 3, y * 2
         want_glu = torch.nn.functional.silu(gate) * up
         norm = norm.cuda()
-        assert L.K.takes(x.cuda(), norm.weight) and L.K.norm_fits(x)   # no fallback
+        assert L.K.takes(x.cuda(), norm.weight) and L.K.norm_fits(x, norm.weight)   # no fallback
         got = norm(x.cuda())
         got_norm, got_sum = norm.after_add(x.cuda(), y.cuda())
         got_glu = L.K.swiglu_(gate.cuda(), up.cuda())
@@ -374,3 +374,26 @@ def test_a_hooked_or_replaced_module_is_still_called():
     block.attention.wo = Doubled(block.attention.wo)
     model(token, 601)
     assert block.attention.wo.calls == 1
+    # shapes that do not belong together are torch's to refuse, as before
+    model.layers[0].attention.wk = torch.nn.Linear(args.dim, 8, bias=False, device="cuda", dtype=args.dtype)
+    with pytest.raises(RuntimeError):
+        model(token, 602)
+    with pytest.raises(RuntimeError), torch.no_grad():
+        L.RMSNorm(64).cuda()(torch.randn(2, 32, device="cuda"))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_block_tail_kernel_equals_its_three_parts(dtype):
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def draw(*shape):
+        return (torch.randn(*shape, device="cuda", generator=g) / 8).to(dtype)
+
+    dim, attn, hidden = 264, 384, 520
+    x, att = draw(1, 1, dim), draw(1, 1, 6, 64)
+    wo, w1, w3, w2 = draw(dim, attn), draw(hidden, dim), draw(hidden, dim), draw(dim, hidden)
+    norm = L.RMSNorm(dim).cuda().to(dtype)
+    with torch.no_grad():
+        h = L.K.linear_add(att, wo, x)
+        want = L.K.linear_add(L.K.linear_swiglu(h, norm, w1, w3), w2, h)
+        assert torch.equal(L.K.block_tail(att, wo, x, norm, w1, w3, w2), want)
