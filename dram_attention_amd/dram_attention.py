@@ -19,6 +19,7 @@ from . import _lib
 from .lru_cache import DummyCache, LRUCache
 from .lru_kernel import GATHER_BLOCKS, gather_attend_supported, host_link_gbps
 from .max_ip_kernel import DA_SCORE_ORDERED_BOUNDS, DA_SCORE_ROUND
+from .model_kernels import unobserved
 from .topk_selector import IPUpperboundTopKSelector, TokenMaxTopKSelector
 
 # da_page_score flags of a step by whether the summaries' bounds are ordered
@@ -186,11 +187,13 @@ def prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
 
 def prefill_attention_f32_supported(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor) -> bool:
     """Whether the library's fp32 prefill kernel takes these tensors as they are (it has no
-    backward, so operands that autograd follows stay with torch)."""
-    if not (xq.is_cuda and xq.shape[-1] in (64, 128)):
+    backward and no other derivative, so operands that autograd or a transform follows stay
+    with torch, as do token strides above the kernel's 2^24 bytes)."""
+    if not (xq.is_cuda and xq.shape[-1] in (64, 128) and unobserved()):
         return False
-    return all(t.dtype == torch.float32 and t.is_cuda and t.stride(-1) == 1
-               and t.data_ptr() % 16 == 0 and t.stride(1) % 4 == 0 and t.stride(2) % 4 == 0
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_cuda
+               and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.stride(1) % 4 == 0
+               and t.stride(2) % 4 == 0 and t.stride(1) <= 1 << 22
                and not (t.requires_grad and torch.is_grad_enabled()) for t in (xq, xk, xv))
 
 
@@ -382,10 +385,10 @@ class DRAMAttention(torch.nn.Module):
         """init_cache; ``build``: where an LRUCache writes its page store."""
         bsz, seqlen, H, D = k_cache.shape
         assert bsz == 1, "Only support batch size 1"
-        self.dram_kv_cache_size = self._paged_tokens(seqlen)
-        prefix_k = k_cache[0, : self.dram_kv_cache_size].transpose(0, 1)
-        prefix_v = v_cache[0, : self.dram_kv_cache_size].transpose(0, 1)
-        if self.dram_kv_cache_size > self.lru_hbm_cache_size:
+        paged = self._paged_tokens(seqlen)
+        prefix_k = k_cache[0, :paged].transpose(0, 1)
+        prefix_v = v_cache[0, :paged].transpose(0, 1)
+        if paged > self.lru_hbm_cache_size:
             self.lru_cache = LRUCache(
                 k_cache=prefix_k,
                 v_cache=prefix_v,
@@ -403,6 +406,7 @@ class DRAMAttention(torch.nn.Module):
                 raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
         else:
             self.lru_cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
+        self.dram_kv_cache_size = paged     # (only now: a prompt that was refused changes nothing)
         tail = seqlen - self.dram_kv_cache_size
         self.cache_k[:, :tail].copy_(k_cache[:, self.dram_kv_cache_size:], non_blocking=True)
         self.cache_v[:, :tail].copy_(v_cache[:, self.dram_kv_cache_size:], non_blocking=True)
@@ -501,7 +505,8 @@ class DRAMAttention(torch.nn.Module):
         cls = type(self)
         if (type(lru) is not LRUCache or self.attention_scope != "resident" or not self.overlap_page_stream
                 or not self.attend_on_page_stream or cls.select_ is not DRAMAttention.select_
-                or cls.attend_ is not DRAMAttention.attend_):
+                or cls.attend_ is not DRAMAttention.attend_ or "select_" in self.__dict__
+                or "attend_" in self.__dict__):
             return None
         selector, buffers, own = lru.top_k_selector, lru._buffers, self._buffers
         if type(selector) is not IPUpperboundTopKSelector:

@@ -172,8 +172,8 @@ class Attention(nn.Module):
         xq = self.wq(x).view(bsz, seqlen, self.n_heads, self.head_dim)
         xk = self.wk(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         xv = self.wv(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
-        if (K.takes(xq, xk) and rope_rows.dtype == torch.float32 and rope_rows.is_contiguous()
-                and rope_rows.device == xq.device
+        if (K.takes(xq, xk) and K.plain_linears(self.wq, self.wk) and rope_rows.dtype == torch.float32
+                and rope_rows.is_contiguous() and rope_rows.device == xq.device
                 and bsz == 1 and rope_rows.shape == (seqlen, self.head_dim // 2, 2)
                 and self.head_dim * xq.element_size() % 16 == 0):
             K.rope_(xq, xk, rope_rows)          # the projections' own outputs, in place
@@ -202,8 +202,9 @@ class FeedForward(nn.Module):
 
     def _slice(self, x):
         gate, up = self.w1(x), self.w3(x)
-        if K.takes(gate, up) and gate.shape == up.shape and gate.numel() * gate.element_size() % 16 == 0:
-            return self.w2(K.swiglu_(gate, up))
+        if (K.takes(gate, up) and K.plain_linears(self.w1) and gate.shape == up.shape
+                and gate.numel() * gate.element_size() % 16 == 0):
+            return self.w2(K.swiglu_(gate, up))     # in w1's own output
         return self.w2(F.silu(gate) * up)
 
 
@@ -326,7 +327,7 @@ class GraphedDecoder:
 
     def _step(self):
         logits = self.model(self.token, self.pos)
-        if logits.is_cuda:
+        if K.takes(logits) and logits.dtype == torch.float32 and logits.numel() == logits.shape[-1]:
             K.argmax_into(logits, self.token)
         else:
             self.token.copy_(logits.argmax(-1))

@@ -49,6 +49,8 @@ class LRUCache(torch.nn.Module):
         hbm_page_to_dram_page_mapping   (H, num_hbm_pages) int64
     """
 
+    _build_stream = None    # the stream the page store is being written on (see finish_build)
+
     def __init__(
         self,
         k_cache: torch.Tensor,
@@ -102,7 +104,6 @@ class LRUCache(torch.nn.Module):
         # Start with the most recent pages resident: slot s holds page P - N + s.
         first = num_dram_pages - num_hbm_pages
         current = torch.cuda.current_stream(self.hbm_kv_cache.device)
-        self._build_stream = None
         row_bytes = head_dim * k_cache.element_size()
         if (k_cache.is_cuda and v_cache.is_cuda and row_bytes % 16 == 0 and num_dram_pages > 0
                 and k_cache.stride(-1) == 1 and v_cache.stride(-1) == 1

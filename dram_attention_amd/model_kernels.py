@@ -6,21 +6,33 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as nn_module
 
 from . import _lib
 
 _TYPES = (torch.bfloat16, torch.float16, torch.float32)
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def unobserved() -> bool:
+    """Whether nothing but the tensors' values depends on which operators run: no forward-mode
+    differentiation (which torch.no_grad leaves on), vmap or other transform, dispatch mode,
+    tracer or compiler would have to see them."""
+    return (forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
+            and not torch.compiler.is_compiling())
 
 
 def takes(*tensors: torch.Tensor) -> bool:
-    """Whether the kernels apply: contiguous, aligned GPU tensors of one type, and no
-    autograd or autocast that would have to see the operation."""
+    """Whether the kernels apply: plain, contiguous, aligned GPU tensors of one type, and no
+    autograd, autocast or transform that would have to see the operation."""
     x = tensors[0]
-    if not x.is_cuda or x.dtype not in _TYPES or torch.is_grad_enabled() or torch.is_autocast_enabled():
+    if (not x.is_cuda or x.dtype not in _TYPES or torch.is_grad_enabled() or torch.is_autocast_enabled()
+            or not unobserved()):
         return False
-    return all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
-               for t in tensors)
+    return all(type(t) in _PLAIN and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def norm_fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -61,10 +73,17 @@ def swiglu_(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 
 def bare(*modules: nn.Module) -> bool:
-    """Whether calling these modules does nothing but their forward: nobody hooked them."""
+    """Whether calling these modules does nothing but their class's forward: nobody hooked
+    them or gave one of them a forward of its own."""
     if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
+
+
+def plain_linears(*modules: nn.Module) -> bool:
+    """Whether the outputs of these modules are fresh tensors that nobody else holds, so
+    that they may be changed in place: torch's own nn.Linear, unwatched."""
+    return all(type(m) is nn.Linear for m in modules) and bare(*modules)
 
 
 MAX_LINEAR_ROW = 60 * 1024  # bytes of an input row the one-token layers hold in LDS
@@ -80,7 +99,8 @@ def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
         p = m._parameters
         w = p["weight"]
         row = m.in_features * esize
-        if (p["bias"] is not None or w.dtype is not dtype or w.device != device or not w.is_contiguous()
+        if (p["bias"] is not None or type(w) not in _PLAIN or w.dtype is not dtype or w.device != device
+                or not w.is_contiguous()
                 or w.shape != (m.out_features, m.in_features) or w.data_ptr() % 16 or row % 16
                 or row > MAX_LINEAR_ROW):
             return False

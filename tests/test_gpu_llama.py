@@ -397,3 +397,48 @@ def test_block_tail_kernel_equals_its_three_parts(dtype):
         h = L.K.linear_add(att, wo, x)
         want = L.K.linear_add(L.K.linear_swiglu(h, norm, w1, w3), w2, h)
         assert torch.equal(L.K.block_tail(att, wo, x, norm, w1, w3, w2), want)
+
+
+@pytest.mark.parametrize("length", [1, 600])
+def test_a_watched_projection_keeps_its_output(length):
+    """What a forward hook keeps of a projection is what the projection returned: rotation
+    and SwiGLU work in place only on outputs that nobody else holds."""
+    args = small_args(torch.bfloat16)
+    model = build(args, 9)
+    model(torch.arange(600, device="cuda")[None] % args.vocab_size, 0)
+    a, f = model.layers[0].attention, model.layers[0].feed_forward
+    kept = {}
+    for name, m in (("wq", a.wq), ("wk", a.wk), ("w1", f.w1)):
+        m.register_forward_hook(lambda mod, inp, out, name=name: kept.__setitem__(name, (inp[0], out)))
+    tokens = torch.arange(length, device="cuda")[None] % args.vocab_size
+    model(tokens, 600 if length == 1 else 0)
+    for name, (x, out) in kept.items():
+        assert torch.equal(torch.nn.functional.linear(x, dict(wq=a.wq, wk=a.wk, w1=f.w1)[name].weight), out), name
+
+
+def test_an_instance_forward_is_still_called():
+    args = small_args(torch.bfloat16)
+    model = build(args, 10)
+    model(torch.arange(600, device="cuda")[None] % args.vocab_size, 0)
+    calls, w2 = [], model.layers[1].feed_forward.w2
+    inner = w2.forward
+    w2.forward = lambda x: (calls.append(1), inner(x))[1]
+    model(torch.tensor([[5]], device="cuda"), 600)
+    assert calls == [1]
+
+
+def test_transforms_see_the_norm_as_torch_operators():
+    """vmap, forward-mode derivatives and tracing, which no_grad leaves on, get torch's
+    operators, so that what they compute is not lost."""
+    from torch.autograd import forward_ad
+
+    norm = L.RMSNorm(64).cuda()
+    x, t = torch.randn(2, 3, 64, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).unbind(0)
+    with torch.no_grad():
+        want = norm(x)
+        assert torch.allclose(torch.vmap(norm)(x), want, atol=1e-6)
+        with forward_ad.dual_level():
+            tangent = forward_ad.unpack_dual(norm(forward_ad.make_dual(x, t))).tangent
+        assert tangent is not None and torch.isfinite(tangent).all() and tangent.abs().max() > 0
+        traced = torch.jit.trace(norm, (x,), check_trace=False)
+        assert torch.allclose(traced(t), norm(t), atol=1e-6)

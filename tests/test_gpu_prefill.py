@@ -216,3 +216,17 @@ def test_page_store_written_beside_attention_is_complete_on_return(S, Hq, Hkv, D
             assert same(getattr(m.lru_cache, name), getattr(ref.lru_cache, name))
         assert same(out, want)
         del junk
+
+
+def test_a_refused_prompt_leaves_the_layer_as_it_was():
+    from dram_attention_amd import DRAMAttention
+
+    m = DRAMAttention(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16,
+                      top_k=64, n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16)
+    xq, xk, xv = draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    m(xq, xk, xv, start_pos=0, stage="prefill")
+    cache, paged = m.lru_cache, m.dram_kv_cache_size
+    xq, xk, xv = draw(2000, 4, 2, 64, torch.bfloat16, 2)
+    with pytest.raises(ValueError):
+        m(xq, xk.half(), xv.half(), start_pos=0, stage="prefill")
+    assert m.lru_cache is cache and m.dram_kv_cache_size == paged
