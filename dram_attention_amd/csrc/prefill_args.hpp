@@ -17,11 +17,9 @@ struct PrefillArgs {
   int rep;          // query heads per kv head
   int n_groups;     // workgroups that share a kv head's rows: rep / kHeads
   int64_t n_row_blocks;
-  int heads_per_xcd;  // kv heads per die when they deal out evenly, else 0
+  int n_kv_heads;
   float scale_log2;
 };
-
-constexpr int kXcds = 8;  // dies (XCDs) of the part; consecutive workgroup ids go to consecutive dies
 
 // Checks the operands of a prefill call and fills `a` (all but the grid's geometry).
 inline int prefill_args(PrefillArgs &a, const char *what, const void *q, int64_t q_tok_stride,
@@ -61,6 +59,7 @@ inline int prefill_args(PrefillArgs &a, const char *what, const void *q, int64_t
   a.o_head_stride = o_head_stride;
   a.seq_len = seq_len;
   a.rep = n_q_heads / n_kv_heads;
+  a.n_kv_heads = n_kv_heads;
   a.scale_log2 = scale * kLog2e;
   return DA_OK;
 }
