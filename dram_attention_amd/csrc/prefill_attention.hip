@@ -9,7 +9,8 @@
 //
 // Work split: a 512-thread workgroup, one per CU, owns kHeads query heads of one kv
 // head (the GQA group, or a part of it) times 256/kHeads consecutive query rows;
-// each of its eight waves owns 32 query rows of one head (two waves per SIMD: the
+// each of its eight waves owns 32 query rows of one head (for short prompts: four pairs of
+// waves do; two waves per SIMD: the
 // registers of a wave allow no more, and with eight waves on one tile instead of two
 // workgroups of four on two the CU loads half as many tile rows).  All waves walk the
 // same keys, so one tile of K and V in LDS serves the whole group.  Per tile
@@ -32,6 +33,10 @@
 // is only raised when a score clears it by kRescaleSlack (as in the decode
 // kernels), per-lane partial sums, everything in the log2 domain.
 // Workgroups take the longest rows first, the kv heads in turn (see the kernel).
+//
+// Short prompts (see launch_prefill): half of the waves walk the even tiles and the other
+// half the odd ones, for the same rows, and the second half's state is merged into the
+// first's at the end, in fp32 through LDS.
 #include <type_traits>
 
 #include "prefill_args.hpp"
@@ -76,7 +81,7 @@ constexpr int kPfKeys = 64;  // keys per tile
 // lanes that read one column of 16 rows (K rows as MFMA operands), and the 8 rows x 64
 // bytes of a transposing read of V, then fall on distinct banks; 16 bytes of padding
 // per block shift consecutive blocks by one bank group.
-template <int kD>
+template <int kD, int kSplit>
 struct PrefillShared {
   static constexpr int kRowBytes = kD * 2;
   static constexpr int kRows = 1024 / kRowBytes;          // rows per block: 4 (D 128) or 8 (D 64)
@@ -85,9 +90,14 @@ struct PrefillShared {
   static constexpr int kBlocks = kPfKeys / kRows;         // blocks per tile (K, and V)
   static constexpr int kKBytes = kBlocks * kBlock;
   static constexpr int kBufBytes = 2 * kKBytes;           // K tile, then V tile
-  static constexpr int kOutRow = kD * 2 + 16;             // epilogue staging
-  static constexpr int kOutBytes = kPfWaves * 32 * kOutRow;
-  static constexpr int kBytes = 2 * kBufBytes > kOutBytes ? 2 * kBufBytes : kOutBytes;
+  // epilogue: output rows of the waves that store; ahead of them, with two key groups, the
+  // second group's fp32 state (output, maximum, sum: 16 bytes per lane and step)
+  static constexpr int kOutRow = kD * 2 + 16;
+  static constexpr int kStashSteps = kD / 8 + 1;
+  static constexpr int kStashBytes = kSplit > 1 ? kPfWaves / 2 * kStashSteps * 1024 : 0;
+  static constexpr int kOutBytes = kStashBytes + kPfWaves / kSplit * 32 * kOutRow;
+  static constexpr int kTileBytes = 2 * kSplit * kBufBytes;
+  static constexpr int kBytes = kTileBytes > kOutBytes ? kTileBytes : kOutBytes;
   // column swizzle of row rr of a block (a multiple of the chunk index's high bits)
   static __host__ __device__ constexpr int swizzle(int rr) { return kD == 128 ? 4 * rr : 2 * (rr >> 1); }
   // byte offset of chunk cc of row r of a tile
@@ -96,14 +106,15 @@ struct PrefillShared {
   }
 };
 
-template <typename T, int kD, int kHeads>
+template <typename T, int kD, int kHeads, int kSplit>
 __global__ void __launch_bounds__(kPfThreads, 1)
 prefill_attention_kernel(const PrefillArgs a) {
   using Ops = PrefillOps<T>;
-  using Sh = PrefillShared<kD>;
+  using Sh = PrefillShared<kD, kSplit>;
   static_assert(kD == 64 || kD == 128, "head sizes of 64 and 128");
   static_assert(kHeads == 1 || kHeads == 2 || kHeads == 4, "1, 2 or 4 query heads per workgroup");
-  constexpr int kRowBlocks = kPfWaves / kHeads;       // 32-row blocks per workgroup
+  static_assert(kSplit == 1 || kSplit == 2, "all keys in one group of waves, or in two");
+  constexpr int kRowBlocks = kPfWaves / kHeads / kSplit;  // 32-row blocks per workgroup
   constexpr int kBlockRows = 32 * kRowBlocks;
   constexpr int kQSteps = kD / 16;                    // MFMAs of S^T per 32 keys
   constexpr int kCBlocks = kD / 32;                   // 32-channel blocks of O^T
@@ -129,10 +140,12 @@ prefill_attention_kernel(const PrefillArgs a) {
   const int hq = hk * a.rep + hg * kHeads + wave % kHeads;
   const int64_t S = a.seq_len;
   const int64_t m0 = rb * kBlockRows;                       // first row of the workgroup
-  const int64_t row0 = m0 + (wave / kHeads) * 32;           // first row of this wave
+  const int64_t row0 = m0 + (wave / kHeads % kRowBlocks) * 32;  // first row of this wave
+  const int kgroup = kSplit > 1 ? __builtin_amdgcn_readfirstlane(wave) / (kHeads * kRowBlocks) : 0;  // whose tiles: kgroup, + kSplit, ...
   const int64_t my_row = row0 + c;
   const int64_t last_key = (m0 + kBlockRows < S ? m0 + kBlockRows : S) - 1;  // last key any wave needs
   const int n_tiles = (int)(last_key / kPfKeys) + 1;
+  const int n_rounds = (n_tiles + kSplit - 1) / kSplit;     // a round: kSplit tiles side by side
   // keys beyond this wave's last row are masked for all of its rows
   const int64_t wave_last_key = row0 + 31 < S ? row0 + 31 : S - 1;
 
@@ -151,7 +164,7 @@ prefill_attention_kernel(const PrefillArgs a) {
   const char *vbase = a.v + (int64_t)hk * a.v_head_stride * T::kBytes;
   const int64_t k_tok_b = a.k_tok_stride * T::kBytes, v_tok_b = a.v_tok_stride * T::kBytes;
 
-  // Tile loads.  Wave w brings blocks w, w + 4, ... of K and of V; lane L of the wave
+  // Tile loads.  Wave w brings blocks w, w + 8, ... of K and of V; lane L of the wave
   // owns place L of a block, i.e. row L / kChunks and the chunk whose swizzled column is
   // L % kChunks.  Offsets inside a tile fit 32 bits (checked by the launcher).
   constexpr int kBlocksPerWave = Sh::kBlocks / kPfWaves;
@@ -191,19 +204,25 @@ prefill_attention_kernel(const PrefillArgs a) {
     }
   };
 
-  // LDS addresses of this lane's operands inside a tile.  K, as the A operand of S^T:
+  auto fetch_round = [&](int round, int phase) {
+    fetch(round * kSplit, phase * kSplit);
+    if constexpr (kSplit > 1)
+      if (round * kSplit + 1 < n_tiles) fetch(round * kSplit + 1, phase * kSplit + 1);
+  };
+
+  // LDS addresses of this lane's operands inside a round's tiles.  K, as the A operand of S^T:
   // row c of a half, chunk 2s + g.  V, for the transposing load: lane i of a 16-lane
   // group addresses key t0 + i/4, channels c0 + 4*(i%4) .. +3 and receives channel
   // c0 + i of keys t0..t0+3; t0 = 4g (+8, +16 per group of keys), c0 = 32b + 16*((lane/16)%2).
   int k_at[kQSteps], v_at[kCBlocks];
 #pragma unroll
-  for (int s2 = 0; s2 < kQSteps; ++s2) k_at[s2] = Sh::at(c, 2 * s2 + g);
+  for (int s2 = 0; s2 < kQSteps; ++s2) k_at[s2] = kgroup * Sh::kBufBytes + Sh::at(c, 2 * s2 + g);
   {
     const int i16 = lane & 15;
 #pragma unroll
     for (int b = 0; b < kCBlocks; ++b)
-      v_at[b] = Sh::kKBytes + Sh::at(4 * g + (i16 >> 2), 4 * b + 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1)) +
-                (i16 & 1) * 8;
+      v_at[b] = kgroup * Sh::kBufBytes + Sh::kKBytes +
+                Sh::at(4 * g + (i16 >> 2), 4 * b + 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1)) + (i16 & 1) * 8;
   }
   constexpr int kHalfStep = (32 / Sh::kRows) * Sh::kBlock;   // 32 rows further down a tile
   constexpr int kKeys16 = (16 / Sh::kRows) * Sh::kBlock;     // 16 rows
@@ -216,11 +235,11 @@ prefill_attention_kernel(const PrefillArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
 
-  // One tile of 64 keys from LDS buffer `buf`; kMask: keys above a row are dropped.
-  auto compute = [&](int tile, int buf, auto mask_tag) {
+  // One tile of 64 keys from the buffers of `phase`; kMask: keys above a row are dropped.
+  auto compute = [&](int tile, int phase, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
     __builtin_amdgcn_iglp_opt(1);   // (measured: see the loop below)
-    const char *kt = smem + buf * Sh::kBufBytes;
+    const char *kt = smem + phase * kSplit * Sh::kBufBytes;
     pf_f32x16 st[2];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -287,7 +306,7 @@ prefill_attention_kernel(const PrefillArgs a) {
     }
   };
 
-  fetch(0, 0);
+  fetch_round(0, 0);
   // The query rows have arrived before the loop starts (they were requested ahead of
   // tile 0): inside the loop nothing then waits for a load except the tile's own.
 #pragma unroll
@@ -301,31 +320,62 @@ prefill_attention_kernel(const PrefillArgs a) {
   // the other wave of the SIMD is the one to let in), 1211 with iglp_opt(1), which spreads the
   // LDS reads between the MFMAs; 8192 tokens 1081 -> 1134, 4613 943 -> 998; 20000 tokens,
   // 16/16 heads, D 64: 800 -> 912.
-  const int n_whole = (int)(m0 / kPfKeys) & ~1;
-  for (int tile = 0; tile < n_whole; tile += 2) {
-    fetch(tile + 1, 1);
-    compute(tile, 0, std::false_type{});
+  const int n_whole = (int)(m0 / kPfKeys) / kSplit & ~1;
+  for (int round = 0; round < n_whole; round += 2) {
+    fetch_round(round + 1, 1);
+    compute(round * kSplit + kgroup, 0, std::false_type{});
     __syncthreads();
-    fetch(tile + 2, 0);                             // (there is one: the tiles of the block's own rows)
-    compute(tile + 1, 1, std::false_type{});
+    fetch_round(round + 2, 0);                      // (there is one: the tiles of the block's own rows)
+    compute((round + 1) * kSplit + kgroup, 1, std::false_type{});
     __syncthreads();
   }
-  for (int tile = n_whole; tile < n_tiles; ++tile) {
-    const int buf = tile & 1;
-    // the other buffer was last read before the barrier that ended the previous round
-    if (tile + 1 < n_tiles) fetch(tile + 1, buf ^ 1);
+  for (int round = n_whole; round < n_rounds; ++round) {
+    const int phase = round & 1, tile = round * kSplit + kgroup;
+    // the other buffers were last read before the barrier that ended the previous round
+    if (round + 1 < n_rounds) fetch_round(round + 1, phase ^ 1);
     const int64_t t0 = (int64_t)tile * kPfKeys;
-    if (t0 <= wave_last_key) {                     // else: every key of the tile is masked for this wave
-      if (t0 + kPfKeys - 1 > row0) compute(tile, buf, std::true_type{});
-      else compute(tile, buf, std::false_type{});
+    if (t0 <= wave_last_key) {                     // else: no such tile, or masked whole for this wave
+      if (t0 + kPfKeys - 1 > row0) compute(tile, phase, std::true_type{});
+      else compute(tile, phase, std::false_type{});
     }
-    __syncthreads();                                // tile + 1 has landed, and everyone is done with `buf`
+    __syncthreads();                                // the next round has landed; everyone is done with this one
+  }
+
+  // ---- two key groups: the second hands its state to the first, which merges
+  if constexpr (kSplit > 1) {
+    char *stash = smem + (wave % (kPfWaves / 2)) * Sh::kStashSteps * 1024 + lane * 16;
+    if (kgroup == 1) {                              // (the last barrier retired every read of the tiles)
+#pragma unroll
+      for (int b = 0; b < kCBlocks; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *(float4 *)(stash + (4 * b + j) * 1024) =
+              make_float4(acc[b][4 * j], acc[b][4 * j + 1], acc[b][4 * j + 2], acc[b][4 * j + 3]);
+      *(float2 *)(stash + 4 * kCBlocks * 1024) = make_float2(m, l);
+    }
+    __syncthreads();
+    if (kgroup == 1) return;
+    const float2 other = *(const float2 *)(stash + 4 * kCBlocks * 1024);
+    const float mx = fmaxf(m, other.x);             // (finite: this group had tile 0)
+    const float mine = fast_exp2(m - mx), theirs = fast_exp2(other.x - mx);
+    m = mx;
+    l = l * mine + other.y * theirs;
+#pragma unroll
+    for (int b = 0; b < kCBlocks; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 o = *(const float4 *)(stash + (4 * b + j) * 1024);
+        acc[b][4 * j] = acc[b][4 * j] * mine + o.x * theirs;
+        acc[b][4 * j + 1] = acc[b][4 * j + 1] * mine + o.y * theirs;
+        acc[b][4 * j + 2] = acc[b][4 * j + 2] * mine + o.z * theirs;
+        acc[b][4 * j + 3] = acc[b][4 * j + 3] * mine + o.w * theirs;
+      }
   }
 
   // ---- epilogue: normalise, transpose through LDS, store rows of 16-byte lanes
   l += __shfl_xor(l, 32, 64);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  char *ot = smem + wave * 32 * Sh::kOutRow;     // (the last barrier retired every read of the tiles)
+  char *ot = smem + Sh::kStashBytes + wave * 32 * Sh::kOutRow;     // (the last barrier retired every read of the tiles)
 #pragma unroll
   for (int b = 0; b < kCBlocks; ++b)
 #pragma unroll
@@ -349,22 +399,36 @@ prefill_attention_kernel(const PrefillArgs a) {
     a.lse[(int64_t)hq * S + my_row] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
-template <typename T, int kD>
-static int launch_prefill(PrefillArgs a, hipStream_t s) {
-  const int heads = a.rep % 4 == 0 ? 4 : (a.rep % 2 == 0 ? 2 : 1);
-  const int block_rows = 32 * (kPfWaves / heads);
+template <typename T, int kD, int kSplit>
+static int launch_prefill_split(PrefillArgs a, int heads, hipStream_t s) {
   a.n_groups = a.rep / heads;
-  a.n_row_blocks = ceil_div(a.seq_len, block_rows);
+  a.n_row_blocks = ceil_div(a.seq_len, 32 * (kPfWaves / heads / kSplit));
   const int64_t blocks = a.n_row_blocks * a.n_groups * a.n_kv_heads;
   if (blocks > 0x7fffffff) return fail(DA_ENOTSUP, "da_prefill_attention: %lld workgroups", (long long)blocks);
   const dim3 grid((unsigned)blocks);
-  if (heads == 4)
-    hipLaunchKernelGGL((prefill_attention_kernel<T, kD, 4>), grid, dim3(kPfThreads), 0, s, a);
-  else if (heads == 2)
-    hipLaunchKernelGGL((prefill_attention_kernel<T, kD, 2>), grid, dim3(kPfThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL((prefill_attention_kernel<T, kD, 1>), grid, dim3(kPfThreads), 0, s, a);
+#define DA_PREFILL(kHeads) \
+  hipLaunchKernelGGL((prefill_attention_kernel<T, kD, kHeads, kSplit>), grid, dim3(kPfThreads), 0, s, a)
+  if (heads == 4) DA_PREFILL(4);
+  else if (heads == 2) DA_PREFILL(2);
+  else DA_PREFILL(1);
+#undef DA_PREFILL
   return launch_status("da_prefill_attention");
+}
+
+// One group of waves or two over the keys.  Two halve what a workgroup holds of the rows, and
+// its serial chain of tiles, for twice the tile loads per product.  So they are for prompts
+// whose workgroups of one group are all on the chip at once (one per compute unit) and wait
+// for the longest chain; at D 64, where a tile load costs half as much, also a little beyond.
+// One group against two, us:
+//   D 128   32/8 heads: 700 tokens (88 workgroups) 22.5 / 17.8, 2048 (256) 53.5 / 45.2, 2400 (304) 64.8 / 67.0,
+//           4613 173 / 193; 24/8: 2300 (216) 57.2 / 44.3; 8/2: 8192 (256) 184 / 140, 12000 (376) 303 / 309
+//   D 64    16/4: 3100 (196) 51.4 / 31.9, 5500 (344) 93.9 / 88.2, 6500 (408) 109 / 113; 8/2: 11000 (344) 182 / 168
+template <typename T, int kD>
+static int launch_prefill(const PrefillArgs &a, hipStream_t s) {
+  const int heads = a.rep % 4 == 0 ? 4 : (a.rep % 2 == 0 ? 2 : 1);
+  const int64_t blocks = ceil_div(a.seq_len, 32 * (kPfWaves / heads)) * (a.rep / heads) * a.n_kv_heads;
+  return blocks <= (kD == 64 ? 360 : 256) ? launch_prefill_split<T, kD, 2>(a, heads, s)
+                                          : launch_prefill_split<T, kD, 1>(a, heads, s);
 }
 
 }  // namespace da

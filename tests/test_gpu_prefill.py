@@ -75,6 +75,32 @@ def test_prefill_attention_matches_dense_causal_softmax(S, Hq, Hkv, D, dtype):
     assert close(lse, want_lse, 1e-3, 1e-4)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [
+    # few workgroups: two groups of waves share the keys of 32, 64 or 128 rows; lengths around
+    # their tiles and blocks, down to a second group without a tile
+    (1, 4, 1, 128), (32, 4, 1, 128), (33, 4, 1, 64), (64, 8, 2, 64), (65, 4, 1, 128), (97, 6, 3, 64),
+    (128, 2, 1, 128), (129, 5, 5, 128), (191, 4, 2, 128), (193, 3, 3, 64), (257, 12, 3, 128), (385, 14, 2, 64),
+    (1030, 10, 5, 64),
+    # 256 and 258 workgroups at D 128, 360 and 362 at D 64: the last on this side, the first beyond
+    (128, 512, 128, 128), (129, 344, 86, 128), (257, 128, 128, 128), (257, 129, 129, 128), (129, 258, 129, 128),
+    (128, 720, 180, 64), (65, 724, 181, 64), (257, 180, 180, 64), (300, 181, 181, 64),
+])
+def test_prefill_attention_on_both_sides_of_the_key_split(S, Hq, Hkv, D, dtype):
+    """Peaked scores, so that the groups' maxima differ.  Against the dense fp32 softmax: the
+    weights' and the output's rounding, 2^-9 each of the value in bf16 and 2^-12 in fp16, and
+    sums of weights near one; the tolerance of the contract covers them, fp16 gets an eighth."""
+    from dram_attention_amd.dram_attention import prefill_attention
+
+    xq, xk, xv = draw(S, Hq, Hkv, D, dtype, S + Hq, spread=1.7)
+    lse = torch.empty(Hq, S, dtype=torch.float32, device=DEV)
+    out = prefill_attention(xq, xk, xv, lse=lse)
+    want, want_lse = dense_causal(xq, xk, xv)
+    factor = 1.0 if dtype == torch.bfloat16 else 0.125
+    assert close(out.float(), want, ATOL * factor, RTOL * factor)
+    assert close(lse, want_lse, 1e-3, 1e-4)
+
+
 def test_prefill_attention_takes_strided_views_and_peaked_scores():
     """Rows taken out of a fused (S, Hq + 2 Hkv, D) projection, and scores spread widely
     enough that the running maximum moves many times."""
