@@ -21,8 +21,9 @@
 // operands of four steps, and its four consecutive channels 4c .. +3 of a V row its A
 // operands of four channel blocks (block b, row c is channel 4c + b).
 //
-// Measured: 126-128 TFLOP/s (0.80-0.82 of 157) at 32/8 heads, D 128, 9200 and 30000 tokens;
-// 0.75 ms = 116 TFLOP/s at 8/2 heads, D 64, 9200 tokens, where torch's operators took 4.27 ms.
+// Measured: 133 TFLOP/s (0.85 of 157; a large fp32 matrix product of the library: 154) at 32/8
+// heads, D 128, 9200 tokens; 0.69 ms = 126 TFLOP/s at 8/2 heads, D 64, 9200 tokens, where
+// torch's operators took 4.27 ms.
 //
 // Tiles are double-buffered and travel global memory -> LDS directly, in the blocks of
 // 1024 bytes with swizzled columns that prefill_attention.hip explains.
@@ -113,17 +114,32 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
   const int ld_col = (lane % Sh::kChunks) ^ Sh::swizzle(ld_row);
   typedef __attribute__((address_space(1))) const void *GlobalPtr;
   typedef __attribute__((address_space(3))) void *LdsPtr;
+  const uint32_t k_rel = (uint32_t)(ld_row * k_tok_b) + ld_col * 16;   // (fit 32 bits: checked by the launcher)
+  const uint32_t v_rel = (uint32_t)(ld_row * v_tok_b) + ld_col * 16;
   auto fetch = [&](int tile, int buf) {
+    const int64_t t0 = (int64_t)tile * kPfsKeys;
     char *kt = smem + buf * Sh::kBufBytes;
+    if (t0 + kPfsKeys - 1 <= last_key) {            // a whole tile: one base, constant offsets
+      const char *kt0 = kbase + t0 * k_tok_b, *vt0 = vbase + t0 * v_tok_b;
 #pragma unroll
-    for (int u = 0; u < kBlocksPerWave; ++u) {
-      const int blk = wave_u + u * kPfsWaves;
-      int64_t tok = (int64_t)tile * kPfsKeys + blk * Sh::kRows + ld_row;
-      if (tok > last_key) tok = last_key;   // in bounds; such keys are masked
-      __builtin_amdgcn_global_load_lds((GlobalPtr)(kbase + tok * k_tok_b + ld_col * 16),
-                                       (LdsPtr)(kt + blk * Sh::kBlock), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((GlobalPtr)(vbase + tok * v_tok_b + ld_col * 16),
-                                       (LdsPtr)(kt + Sh::kKBytes + blk * Sh::kBlock), 16, 0, 0);
+      for (int u = 0; u < kBlocksPerWave; ++u) {
+        const int blk = wave_u + u * kPfsWaves;
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(kt0 + (int64_t)blk * Sh::kRows * k_tok_b + k_rel),
+                                         (LdsPtr)(kt + blk * Sh::kBlock), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(vt0 + (int64_t)blk * Sh::kRows * v_tok_b + v_rel),
+                                         (LdsPtr)(kt + Sh::kKBytes + blk * Sh::kBlock), 16, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kBlocksPerWave; ++u) {
+        const int blk = wave_u + u * kPfsWaves;
+        int64_t tok = t0 + blk * Sh::kRows + ld_row;
+        if (tok > last_key) tok = last_key;         // in bounds; such keys are masked
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(kbase + tok * k_tok_b + ld_col * 16),
+                                         (LdsPtr)(kt + blk * Sh::kBlock), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(vbase + tok * v_tok_b + ld_col * 16),
+                                         (LdsPtr)(kt + Sh::kKBytes + blk * Sh::kBlock), 16, 0, 0);
+      }
     }
   };
 
@@ -147,6 +163,7 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
 
   auto compute = [&](int tile, int buf, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
+    __builtin_amdgcn_iglp_opt(1);   // (measured: see the loop below)
     const char *kt = smem + buf * Sh::kBufBytes;
     pf_f32x4 st[2];
 #pragma unroll
@@ -214,7 +231,22 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
 #pragma unroll
   for (int t = 0; t < kQChunks; ++t) asm volatile("" : "+v"(qf[t]));  // (arrived before the loop)
   __syncthreads();
-  for (int tile = 0; tile < n_tiles; ++tile) {
+  // Tiles below the workgroup's first row, which every wave needs whole, go two a round, as
+  // in prefill_attention.hip: with the buffer known at compile time LDS addresses are a
+  // register plus a constant, and a whole tile's loads one base plus constants (a 64-bit
+  // product per lane and load before).  iglp_opt(1) spreads the LDS reads between the MFMAs.
+  // us as it was / with the rounds / and iglp_opt (same bits): 9200 tokens, 8/2 heads, D 64: 743 /
+  // 696 / 687; 1800: 82.9 / 75.6 / 72.9; 9000, 16/4: 1381 / 1298 / 1281; 9200, 32/8, D 128: 5518 / 5325 / 5222.
+  const int n_whole = (int)(m0 / kPfsKeys) & ~1;
+  for (int tile = 0; tile < n_whole; tile += 2) {
+    fetch(tile + 1, 1);
+    compute(tile, 0, std::false_type{});
+    __syncthreads();
+    fetch(tile + 2, 0);                             // (there is one: the tiles of the block's own rows)
+    compute(tile + 1, 1, std::false_type{});
+    __syncthreads();
+  }
+  for (int tile = n_whole; tile < n_tiles; ++tile) {
     const int buf = tile & 1;
     if (tile + 1 < n_tiles) fetch(tile + 1, buf ^ 1);
     const int64_t t0 = (int64_t)tile * kPfsKeys;
