@@ -33,10 +33,13 @@ __device__ __forceinline__ void rotate_pair(float &even, float &odd, float c, fl
 }
 
 // x / (1 + exp(-x)); for the 16-bit types the hardware exponential and reciprocal (each
-// within an ulp or two of fp32), which the rounding of the result swallows.
+// within an ulp or two of fp32), which the rounding of the result swallows.  The reciprocal
+// is taken of a sixteenth: v_rcp_f32 gives zero for 1 / d below 2^-126, i.e. for x between
+// -88.7 and -87.3, where x / d is still a normal number of the type.
 template <typename T>
 __device__ __forceinline__ float silu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
+  const float d = 1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x);
+  return (x * 0.0625f) * __builtin_amdgcn_rcpf(d * 0.0625f);
 }
 template <>
 __device__ __forceinline__ float silu<F32>(float x) { return x / (1.f + expf(-x)); }

@@ -254,6 +254,25 @@ def test_norm_and_swiglu_kernels_match_torch(rows, dim, dtype):
         assert torch.allclose(a.cpu().float(), b.float(), rtol=tol, atol=tol * 1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu_keeps_its_smallest_results(dtype):
+    """Gates far below zero, where exp(-x) nears the largest float and its reciprocal leaves
+    the normal numbers before the product does, and beyond, in the row kernel and in the one-token
+    layer.  Bound: one turn of the rounding to the type; half the type's smallest step."""
+    gate = torch.tensor([-60.0, -80.0, -86.5, -87.0, -87.5, -88.0, -88.5, -89.0, -1e4, 0.0, 3.0, 100.0,
+                         -1e-3, 1e-3, -20.0, -40.0], dtype=dtype)
+    up = torch.linspace(-2, 2, 16).to(dtype)
+    want = (torch.nn.functional.silu(gate) * up).double()
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0
+    got = L.K.swiglu_(gate.cuda(), up.cuda()).cpu().double()
+    assert torch.allclose(got, want, rtol=2.0 ** -7, atol=tiny), (got, want)
+    norm = L.RMSNorm(8, eps=0.0).cuda().to(dtype)           # of ones: ones
+    w1, w3 = (torch.nn.functional.pad(t[:, None], (0, 7)).cuda() for t in (gate, up))
+    with torch.no_grad():
+        got = L.K.linear_swiglu(torch.ones(1, 1, 8, dtype=dtype, device="cuda"), norm, w1, w3).flatten().cpu().double()
+    assert torch.allclose(got, want, rtol=2.0 ** -7, atol=tiny), (got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("S,Hq,Hkv,D", [(1, 4, 1, 128), (3, 8, 2, 64), (17, 6, 3, 16)])
 def test_rope_kernel_matches_torch(S, Hq, Hkv, D, dtype):
