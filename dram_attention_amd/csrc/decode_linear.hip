@@ -120,16 +120,14 @@ decode_linear_kernel(const LinearArgs a) {
       for (int j = threadIdx.x; j < vecs; j += kLinThreads) {
         float f[T::kVec];
         unpack<T>(load16(a.x + (int64_t)j * 16), f);
-#pragma unroll
-        for (int i = 0; i < T::kVec; ++i) ss = fmaf(f[i], f[i], ss);
+        ss += sum_of_squares<T>(f);
       }
       ss = group_sum<64>(ss);
       __shared__ float part[kLinWaves];
       if (lane == 0) part[wave] = ss;
       __syncthreads();
-      ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < kLinWaves; ++i) ss += part[i];
+      static_assert(kLinWaves == 4, "the waves' sums in pairs");
+      ss = (part[0] + part[1]) + (part[2] + part[3]);
       inv = rms_scale(ss, a.dim, a.eps);
     }
     const int padded = (steps + kLinUnroll - 1) / kLinUnroll * kLinUnroll * 64;

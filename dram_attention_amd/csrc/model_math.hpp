@@ -21,8 +21,29 @@ __device__ __forceinline__ u32x4 pack_vec<F32>(const float *f) {
                __builtin_bit_cast(uint32_t, f[2]), __builtin_bit_cast(uint32_t, f[3])};
 }
 
+// Of one 16-byte vector, in pairs: what a lane adds up one after the other is then a few vectors.
+template <typename T>
+__device__ __forceinline__ float sum_of_squares(const float *f) {
+  float s[T::kVec / 2];
+#pragma unroll
+  for (int i = 0; i < T::kVec / 2; ++i) s[i] = fmaf(f[2 * i], f[2 * i], f[2 * i + 1] * f[2 * i + 1]);
+#pragma unroll
+  for (int n = T::kVec / 4; n >= 1; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) s[i] += s[i + n];
+  return s[0];
+}
+
+// 1 / sqrt(mean + eps): the hardware's root with one Newton step, its residual 1 - v r^2
+// formed by fused multiply-adds.  Without the step, and with all squares of a lane in one
+// chain, the fp32 norm is 4-6 % further from float64 than torch's operators (5.2-5.3e-8 against
+// 5.0e-8 in the 2-norm).
 __device__ __forceinline__ float rms_scale(float sum_of_squares, int dim, float eps) {
-  return rsqrtf(sum_of_squares / (float)dim + eps);
+  const float v = sum_of_squares / (float)dim + eps;
+  const float r = rsqrtf(v);
+  const float h = v * r;
+  const float e = fmaf(-fmaf(v, r, -h), r, fmaf(-h, r, 1.f));
+  return e == e ? fmaf(0.5f * r, e, r) : r;   // (v of 0, infinity or NaN: as the root gives it)
 }
 
 // (even, odd) turned by the angle whose cosine and sine are c and s.

@@ -44,8 +44,7 @@ rms_norm_kernel(const char *__restrict__ x, const char *__restrict__ add, char *
         for (int i = 0; i < T::kVec; ++i) f[u][i] = round_to<T>(f[u][i] + g[i]);
         if (live) store16(sum_out + base + (int64_t)j * 16, pack_vec<T>(f[u]));
       }
-#pragma unroll
-      for (int i = 0; i < T::kVec; ++i) ss = fmaf(f[u][i], f[u][i], ss);
+      ss += sum_of_squares<T>(f[u]);
     }
   }
   ss = group_sum<64>(ss);
@@ -53,9 +52,8 @@ rms_norm_kernel(const char *__restrict__ x, const char *__restrict__ add, char *
     __shared__ float part[kRowThreads / 64];
     if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = ss;
     __syncthreads();
-    ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < kRowThreads / 64; ++i) ss += part[i];
+    static_assert(kRowThreads / 64 == 4, "the waves' sums in pairs");
+    ss = (part[0] + part[1]) + (part[2] + part[3]);
   }
   const float inv = rms_scale(ss, dim, eps);
 #pragma unroll

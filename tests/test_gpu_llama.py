@@ -254,6 +254,28 @@ def test_norm_and_swiglu_kernels_match_torch(rows, dim, dtype):
         assert torch.allclose(a.cpu().float(), b.float(), rtol=tol, atol=tol * 1e-2)
 
 
+@pytest.mark.parametrize("dim", [64, 256, 1024, 4096, 8192])
+def test_fp32_norm_is_its_roundings_from_float64(dim):
+    """Roundings of half a unit in the last place at most: 2.3e-8 in the 2-norm for each of the two
+    products; 2.7e-8 for the scale and, halved by the root, for the sum of squares, the mean and the
+    sum with eps, which all lie about 1 here: 4.9e-8 together, and 4 % for the sum's inner roundings.
+    Rows whose mean is zero, overflows or is not a number come out as the torch operators
+    give them."""
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    x = torch.randn(1, 2 ** 24 // dim, dim, device="cuda", generator=g)
+    norm = L.RMSNorm(dim, eps=1e-5).cuda()
+    with torch.no_grad():
+        norm.weight.copy_(1 + 0.1 * torch.randn(dim, device="cuda", generator=g))
+        x64 = x.double()
+        want = x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + 1e-5) * norm.weight.double()
+        assert ((norm(x).double() - want).norm() / want.norm()).item() < 5.1e-8
+        odd = torch.zeros(1, 5, dim, device="cuda")
+        odd[0, 1:, 0] = torch.tensor([1e30, float("inf"), float("nan"), 1e-30])
+        for eps in (0.0, 1e-5):
+            bare = L.RMSNorm(dim, eps=eps)
+            assert torch.allclose(bare.cuda()(odd).cpu(), bare.cpu()(odd.cpu()), rtol=1e-6, equal_nan=True)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_swiglu_keeps_its_smallest_results(dtype):
     """Gates far below zero, where exp(-x) nears the largest float and its reciprocal leaves
