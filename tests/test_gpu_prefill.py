@@ -214,6 +214,31 @@ def test_fp32_prefill_kernel_matches_dense_float64(S, Hq, Hkv, D):
         assert close(lse[h].double(), torch.logsumexp(s_, -1), 1e-5, 1e-5)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_fp32_prefill_sums_are_short_chains(D):
+    """Summands that lose half of what lies below the sum's last place when they are added one
+    after the other.  Sum of the weights, by the log-sum-exp: one addition to the running sum per
+    tile of 32 keys (and five in and behind it), half a unit in the last place each, and that of the result
+    (9, to 2^-21).  Output at D 64: equal weights, so chains of 16 tiles, one addition per 4 keys,
+    and of S / 512 chains."""
+    from dram_attention_amd.dram_attention import prefill_attention_f32
+
+    S = 8192
+    odd = 1.0 + 502 * 2.0 ** -23
+    q, k = torch.zeros(1, S, 4, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV)
+    out = prefill_attention_f32(q, k, torch.full((1, S, 1, D), odd, device=DEV))
+    if D == 64:
+        assert (out.double() / odd - 1).abs().max().item() < (128 + S / 512 + 4) * 2.0 ** -24
+    q[..., 0] = 1.0
+    k[:, 32:, :, 0] = math.log(odd) * math.sqrt(D)       # the first tile's scores, zero, stay the reference
+    lse = torch.empty(4, S, device=DEV)
+    prefill_attention_f32(q, k, out[:, :, :1].contiguous(), lse=lse)
+    n = torch.arange(1, S + 1, device=DEV, dtype=torch.float64)
+    weight = (k[0, 32, 0, 0].double() / math.sqrt(D)).exp()
+    want = (n.clamp(max=32) + (n - 32).clamp(min=0) * weight).log()
+    assert (lse.double() - want).abs().max().item() < (S / 32 + 5 + 8) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("S,Hq,Hkv,D,dtype", [
     (600, 2, 2, 64, torch.bfloat16), (3000, 8, 2, 64, torch.float32), (9000, 32, 8, 128, torch.bfloat16),
     (12345, 64, 8, 128, torch.float16),
