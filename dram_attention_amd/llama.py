@@ -228,15 +228,20 @@ class TransformerBlock(nn.Module):
                 xq, xk, xv = K.linear_qkv_rope(x, norm1, wq, wk, wv, a.n_heads, a.n_kv_heads, a.head_dim,
                                                rope_rows)
                 out = a.dram_attention(xq, xk, xv, start_pos=start_pos, stage="generate")
-                return K.block_tail(out, wo, x, norm2, w1, w3, w2)
-        attended = self.attention(self.attention_norm(x), start_pos, rope_rows)
+                if K.row_fits(out, x, wo.shape[1]):
+                    return K.block_tail(out, wo, x, norm2, w1, w3, w2)
+                # (an attention module of its own kind, or a hook, returned something else)
+                return self._tail(x, a.wo(out.reshape(1, 1, -1)))
+        return self._tail(x, self.attention(self.attention_norm(x), start_pos, rope_rows))
+
+    def _tail(self, x, attended):
+        """Residuals and feed-forward behind attention's projected output."""
         if type(self.ffn_norm) is RMSNorm and K.bare(self.ffn_norm):
             normed, h = self.ffn_norm.after_add(x, attended)
         else:
             h = x + attended
             normed = self.ffn_norm(h)
         return h + self.feed_forward(normed)
-
 
     @staticmethod
     def _one_token_kernels(a, f, norm1, norm2, x, rope_rows) -> bool:

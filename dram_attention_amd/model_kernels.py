@@ -107,6 +107,13 @@ def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
     return bare(*linears)
 
 
+def row_fits(row, x: torch.Tensor, n: int) -> bool:
+    """Whether ``row``, which any module may have made, is what the one-token layers read: n
+    elements of x's type on x's device, in place one after the other."""
+    return (type(row) is torch.Tensor and row.dtype is x.dtype and row.device == x.device and row.numel() == n
+            and row.is_contiguous() and row.data_ptr() % 16 == 0)
+
+
 def linear_qkv_rope(x, norm, wq, wk, wv, n_heads, n_kv_heads, head_dim, rope_row):
     """Rotated queries and keys, and values, of one token: (1,1,Hq,D), (1,1,Hkv,D) x 2."""
     out = torch.empty(n_heads + 2 * n_kv_heads, head_dim, dtype=x.dtype, device=x.device)

@@ -468,6 +468,39 @@ def test_an_instance_forward_is_still_called():
     assert calls == [1]
 
 
+def test_a_hook_may_exchange_the_attention_output_of_a_token():
+    """What a forward hook (or an attention module of another kind) returns reaches the
+    projection as any tensor reaches it: strided and broadcast outputs with their own values, another type
+    or size refused.  Against the same call with a feed-forward that is watched, which leaves the
+    one-token kernels out: one turn of a rounding to the type here or there, 2^-6 of the largest logit."""
+    args = small_args(torch.bfloat16)
+    token = torch.tensor([[5]], device="cuda")
+    prompt = torch.arange(600, device="cuda")[None] % args.vocab_size
+
+    def strided(out):
+        wide = torch.full((*out.shape[:-1], 2 * out.shape[-1]), 7.0, dtype=out.dtype, device="cuda")
+        wide[..., ::2] = out
+        return wide[..., ::2]
+
+    def run(change, watched):
+        model = build(args, 11)
+        model(prompt, 0)
+        block = model.layers[1]
+        if watched:
+            block.feed_forward.register_forward_hook(lambda mod, inp, out: None)
+        block.attention.dram_attention.register_forward_hook(lambda mod, inp, out: change(out))
+        return model(token, 600)
+
+    for change in (strided, lambda out: out.new_ones(()).expand_as(out), lambda out: out.transpose(2, 3),
+                   lambda out: torch.nn.Parameter(out.flatten()[1:].new_zeros(out.numel() + 1)[1:].view_as(out))):
+        got, want = run(change, False), run(change, True)
+        assert (got - want).abs().max() <= 2.0 ** -6 * want.abs().max()
+    for change in (lambda out: out.float(), lambda out: out[:, :, :-1], lambda out: out.cpu()):
+        for watched in (False, True):
+            with pytest.raises(RuntimeError):
+                run(change, watched)
+
+
 def test_transforms_see_the_norm_as_torch_operators():
     """vmap, forward-mode derivatives and tracing, which no_grad leaves on, get torch's
     operators, so that what they compute is not lost."""
