@@ -332,7 +332,8 @@ class GraphedDecoder:
 
     def _step(self):
         logits = self.model(self.token, self.pos)
-        if K.takes(logits) and logits.dtype == torch.float32 and logits.numel() == logits.shape[-1]:
+        if (K.takes(logits) and logits.dtype == torch.float32 and logits.numel() == logits.shape[-1]
+                and K.is_token(self.token, logits)):
             K.argmax_into(logits, self.token)
         else:
             self.token.copy_(logits.argmax(-1))

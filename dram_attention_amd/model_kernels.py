@@ -175,6 +175,12 @@ def linear_logits(x, norm, w):
     return out
 
 
+def is_token(token, logits: torch.Tensor) -> bool:
+    """Whether the arg-max kernel may write ``token``: one plain int64 on the logits' device."""
+    return (type(token) is torch.Tensor and token.dtype == torch.int64 and token.numel() == 1
+            and token.device == logits.device)
+
+
 def argmax_into(logits: torch.Tensor, token: torch.Tensor) -> None:
     """token (one int64) = index of the largest of the contiguous fp32 logits."""
     _lib.check(

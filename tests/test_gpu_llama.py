@@ -387,6 +387,22 @@ def test_argmax_kernel(n):
     check()
 
 
+def test_greedy_decoding_writes_no_further_than_its_token():
+    """A caller's token of another type (int32 is one that embeddings take) is written by torch: the
+    arg-max kernel writes eight bytes."""
+    args = small_args(torch.bfloat16)
+    model = build(args, 12)
+    model(torch.arange(600, device="cuda")[None] % args.vocab_size, 0)
+    dec = L.GraphedDecoder(model, 600, 5)
+    around = torch.full((4,), -7, dtype=torch.int32, device="cuda")
+    around[1] = 5
+    dec.token = around[1:2].view(1, 1)
+    with torch.no_grad():
+        for _ in range(4):              # eager, captured, replayed
+            logits = dec.step()
+            assert around.tolist() == [-7, logits.argmax(-1).item(), -7, -7]
+
+
 def test_a_hooked_or_replaced_module_is_still_called():
     """The one-token kernels leave out no module that somebody watches or has exchanged."""
     args = small_args(torch.bfloat16)
