@@ -330,6 +330,7 @@ class GraphedDecoder:
         self.graph = None
         self.logits = None
 
+    @torch.no_grad()        # (the caller's mode would otherwise keep the arg-max from its kernel)
     def _step(self):
         logits = self.model(self.token, self.pos)
         if (K.takes(logits) and logits.dtype == torch.float32 and logits.numel() == logits.shape[-1]

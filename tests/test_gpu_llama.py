@@ -387,6 +387,22 @@ def test_argmax_kernel(n):
     check()
 
 
+def test_greedy_decoding_chooses_by_the_argmax_kernel_in_any_grad_mode(monkeypatch):
+    args = small_args(torch.bfloat16)
+    calls, argmax_into = [], L.K.argmax_into
+    monkeypatch.setattr(L.K, "argmax_into", lambda logits, token: calls.append(1) or argmax_into(logits, token))
+    for grad in (True, False):
+        model = build(args, 13)
+        model(torch.arange(600, device="cuda")[None] % args.vocab_size, 0)
+        calls.clear()
+        with torch.set_grad_enabled(grad):
+            dec = L.GraphedDecoder(model, 600, 5)
+            for _ in range(3):
+                logits = dec.step()
+                assert dec.token.item() == logits.argmax(-1).item() and not logits.requires_grad
+        assert len(calls) == 2          # the eager step and the captured one
+
+
 def test_greedy_decoding_writes_no_further_than_its_token():
     """A caller's token of another type (int32 is one that embeddings take) is written by torch: the
     arg-max kernel writes eight bytes."""
