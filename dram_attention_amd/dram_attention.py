@@ -382,34 +382,43 @@ class DRAMAttention(torch.nn.Module):
         self._build_cache(k_cache, v_cache)
 
     def _build_cache(self, k_cache: torch.Tensor, v_cache: torch.Tensor, **build):
-        """init_cache; ``build``: where an LRUCache writes its page store."""
+        """init_cache; ``build``: where an LRUCache writes its page store.  The layer changes only
+        when every part is made, so a prompt that is refused leaves it as it was."""
         bsz, seqlen, H, D = k_cache.shape
         assert bsz == 1, "Only support batch size 1"
         paged = self._paged_tokens(seqlen)
         prefix_k = k_cache[0, :paged].transpose(0, 1)
         prefix_v = v_cache[0, :paged].transpose(0, 1)
-        if paged > self.lru_hbm_cache_size:
-            self.lru_cache = LRUCache(
-                k_cache=prefix_k,
-                v_cache=prefix_v,
-                page_size=self.page_size,
-                top_k=self.top_k // self.page_size,
-                lru_hbm_cache_size=self.lru_hbm_cache_size,
-                device=self.device,
-                **build,
-            )
-            self.link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
-            if self.page_selector == "token_max":
-                self.lru_cache.top_k_selector = TokenMaxTopKSelector(
-                    prefix_k, self.lru_cache.num_dram_pages, device=self.device)
-            elif self.page_selector != "bound":
-                raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
-        else:
-            self.lru_cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
-        self.dram_kv_cache_size = paged     # (only now: a prompt that was refused changes nothing)
-        tail = seqlen - self.dram_kv_cache_size
-        self.cache_k[:, :tail].copy_(k_cache[:, self.dram_kv_cache_size:], non_blocking=True)
-        self.cache_v[:, :tail].copy_(v_cache[:, self.dram_kv_cache_size:], non_blocking=True)
+        link_gbps, cache = self.link_gbps, None
+        try:
+            if paged > self.lru_hbm_cache_size:
+                if self.page_selector not in ("bound", "token_max"):
+                    raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
+                cache = LRUCache(
+                    k_cache=prefix_k,
+                    v_cache=prefix_v,
+                    page_size=self.page_size,
+                    top_k=self.top_k // self.page_size,
+                    lru_hbm_cache_size=self.lru_hbm_cache_size,
+                    device=self.device,
+                    **build,
+                )
+                link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
+                if self.page_selector == "token_max":
+                    cache.top_k_selector = TokenMaxTopKSelector(
+                        prefix_k, cache.num_dram_pages, device=self.device)
+            else:
+                cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
+            tail = seqlen - paged
+            window_k, window_v = self.cache_k[:, :tail], self.cache_v[:, :tail]
+            # (both shapes are refused here or neither copy is)
+            tail_k, tail_v = k_cache[:, paged:].expand_as(window_k), v_cache[:, paged:].expand_as(window_v)
+            window_k.copy_(tail_k, non_blocking=True)
+            window_v.copy_(tail_v, non_blocking=True)
+        finally:
+            if isinstance(cache, LRUCache):
+                cache.finish_build()
+        self.lru_cache, self.link_gbps, self.dram_kv_cache_size = cache, link_gbps, paged
         self._workspace = None
 
     def _paged_tokens(self, seqlen: int) -> int:
@@ -476,15 +485,10 @@ class DRAMAttention(torch.nn.Module):
             self.init_cache(xk, xv)
             return output
         output = []
-        try:
-            self._build_cache(
-                xk, xv, build_stream=build_stream(xk.device),
-                build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype),
-                beside=lambda: output.append(causal_prefill_attention(xq, xk, xv, self.prefill_backend)))
-        finally:
-            lru = getattr(self, "lru_cache", None)     # (none yet if the prompt was refused)
-            if isinstance(lru, LRUCache):
-                lru.finish_build()
+        self._build_cache(
+            xk, xv, build_stream=build_stream(xk.device),
+            build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype),
+            beside=lambda: output.append(causal_prefill_attention(xq, xk, xv, self.prefill_backend)))
         return output[0]
 
     def _generate(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, start_pos):

@@ -281,3 +281,38 @@ def test_a_refused_prompt_leaves_the_layer_as_it_was():
     with pytest.raises(ValueError):
         m(xq, xk.half(), xv.half(), start_pos=0, stage="prefill")
     assert m.lru_cache is cache and m.dram_kv_cache_size == paged
+
+
+@pytest.mark.parametrize("stage", ["prefill", "init_cache"])
+@pytest.mark.parametrize("why", ["unknown selector", "failing selector", "shorter than the window", "values cut short"])
+def test_a_prompt_refused_late_leaves_the_layer_decoding_as_before(why, stage, monkeypatch):
+    """Refusals behind the construction of the page cache: the layer keeps its cache, prefix length
+    and local window, and its next token is that of a layer that never saw the prompt."""
+    from dram_attention_amd import DRAMAttention, dram_attention
+
+    m, ref = (DRAMAttention(max_output_length=8, lru_hbm_cache_size=256, local_cache_size=256, page_size=16,
+                            top_k=64, n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    xq, xk, xv = draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    m.init_cache(xk, xv)
+    ref.init_cache(xk, xv)
+    cache = m.lru_cache
+    length = {"shorter than the window": 100, "values cut short": 400}.get(why, 2000)
+    q, k, v = draw(length, 4, 2, 64, torch.bfloat16, 2)
+    if why == "values cut short":       # (a static cache: 160 of its tokens are paged)
+        v = v[:, :-8]
+    if why == "unknown selector":
+        m.page_selector = "none of them"
+    if why == "failing selector":
+        m.page_selector = "token_max"
+
+        def failing(*args, **kwargs):
+            raise RuntimeError("out of memory")
+
+        monkeypatch.setattr(dram_attention, "TokenMaxTopKSelector", failing)
+    with pytest.raises((RuntimeError, ValueError)):
+        m.init_cache(k, v) if stage == "init_cache" else m(q, k, v, start_pos=0, stage="prefill")
+    m.page_selector = "bound"
+    assert m.lru_cache is cache and m.dram_kv_cache_size == ref.dram_kv_cache_size
+    xq, xk, xv = draw(1, 4, 2, 64, torch.bfloat16, 3)
+    assert same(m(xq, xk, xv, start_pos=1000, stage="generate"), ref(xq, xk, xv, start_pos=1000, stage="generate"))
+    assert same(m.cache_k, ref.cache_k) and same(m.cache_v, ref.cache_v)
