@@ -394,6 +394,8 @@ class DRAMAttention(torch.nn.Module):
             if paged > self.lru_hbm_cache_size:
                 if self.page_selector not in ("bound", "token_max"):
                     raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
+                # (measured ahead of the store, which may be crossing the link when LRUCache returns)
+                link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
                 cache = LRUCache(
                     k_cache=prefix_k,
                     v_cache=prefix_v,
@@ -403,7 +405,6 @@ class DRAMAttention(torch.nn.Module):
                     device=self.device,
                     **build,
                 )
-                link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
                 if self.page_selector == "token_max":
                     cache.top_k_selector = TokenMaxTopKSelector(
                         prefix_k, cache.num_dram_pages, device=self.device)

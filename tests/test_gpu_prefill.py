@@ -283,6 +283,24 @@ def test_a_refused_prompt_leaves_the_layer_as_it_was():
     assert m.lru_cache is cache and m.dram_kv_cache_size == paged
 
 
+def test_the_host_link_is_timed_while_no_store_is_being_written(monkeypatch):
+    """The rate is kept for the whole process: it must not come from copies that shared the link
+    with a page store on its way."""
+    from dram_attention_amd import DRAMAttention, LRUCache, dram_attention
+
+    being_built, at_timing = [], []
+    init, finish = LRUCache.__init__, LRUCache.finish_build
+    monkeypatch.setattr(LRUCache, "__init__", lambda self, *a, **kw: being_built.append(1) or init(self, *a, **kw))
+    monkeypatch.setattr(LRUCache, "finish_build", lambda self: finish(self) or being_built.clear())
+    monkeypatch.setattr(dram_attention, "host_link_gbps", lambda device: at_timing.append(len(being_built)) or 50.0)
+    m = DRAMAttention(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16,
+                      top_k=64, n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16)
+    xq, xk, xv = draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    m(xq, xk, xv, start_pos=0, stage="prefill")
+    m.init_cache(xk, xv)
+    assert at_timing == [0, 0] and m.link_gbps == 0.95 * 50.0
+
+
 @pytest.mark.parametrize("stage", ["prefill", "init_cache"])
 @pytest.mark.parametrize("why", ["unknown selector", "failing selector", "shorter than the window", "values cut short"])
 def test_a_prompt_refused_late_leaves_the_layer_decoding_as_before(why, stage, monkeypatch):
