@@ -92,19 +92,23 @@ MAX_LINEAR_ROW = 60 * 1024  # bytes of an input row the one-token layers hold in
 def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
     """Whether the one-token layers may stand for these nn.Linear modules (x: any tensor of
     the step, for its type and device)."""
+    # (hooks first: pruning and weight normalisation keep the class, move the parameter and put
+    # the weight together in a pre-hook)
+    if not bare(*linears):
+        return False
     dtype, device, esize = x.dtype, x.device, x.element_size()
     for m in linears:
         if type(m) is not nn.Linear:
             return False
         p = m._parameters
-        w = p["weight"]
+        w = p.get("weight")
         row = m.in_features * esize
-        if (p["bias"] is not None or type(w) not in _PLAIN or w.dtype is not dtype or w.device != device
+        if (p.get("bias", m) is not None or type(w) not in _PLAIN or w.dtype is not dtype or w.device != device
                 or not w.is_contiguous()
                 or w.shape != (m.out_features, m.in_features) or w.data_ptr() % 16 or row % 16
                 or row > MAX_LINEAR_ROW):
             return False
-    return bare(*linears)
+    return True
 
 
 def row_fits(row, x: torch.Tensor, n: int) -> bool:

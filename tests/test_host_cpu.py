@@ -79,6 +79,29 @@ def test_no_cpu_fallback():
         LRUCache(torch.zeros(2, 60, 8), torch.zeros(2, 60, 8), page_size=16, top_k=2)
 
 
+@pytest.mark.parametrize("change", ["prune", "weight_norm", "spectral_norm", "own weight", "own bias"])
+def test_linears_that_make_their_weights_are_left_to_torch(change):
+    """Modules whose class is nn.Linear but whose weight or bias is no parameter (any longer)."""
+    from torch.nn.utils import prune, spectral_norm, weight_norm
+
+    from dram_attention_amd import model_kernels as K
+
+    x, plain, m = torch.zeros(1, 1, 16), *(torch.nn.Linear(16, 8, bias=False) for _ in range(2))
+    assert K.linears_fit(x, plain, m)
+    if change == "prune":
+        prune.random_unstructured(m, "weight", 0.5)
+    elif change == "own weight":
+        del m.weight
+        m.weight = torch.zeros(8, 16)
+    elif change == "own bias":
+        del m.bias
+        m.bias = torch.ones(8)
+    else:
+        dict(weight_norm=weight_norm, spectral_norm=spectral_norm)[change](m)
+    assert type(m) is torch.nn.Linear and m(x).shape == (1, 1, 8)
+    assert not K.linears_fit(x, plain, m)
+
+
 def test_package_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "dram_attention_amd")
     for name in os.listdir(pkg):
