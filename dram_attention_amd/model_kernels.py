@@ -19,9 +19,10 @@ def unobserved() -> bool:
     """Whether nothing but the tensors' values depends on which operators run: no forward-mode
     differentiation (which torch.no_grad leaves on), vmap or other transform, dispatch mode,
     tracer or compiler would have to see them."""
-    return (forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
-            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
-            and not torch.compiler.is_compiling())
+    # (the compiler first: it cannot follow the other questions)
+    return (not torch.compiler.is_compiling()
+            and forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None)
 
 
 def takes(*tensors: torch.Tensor) -> bool:

@@ -500,6 +500,20 @@ def test_an_instance_forward_is_still_called():
     assert calls == [1]
 
 
+def test_norm_and_feed_forward_compile_as_one_graph():
+    args = small_args(torch.float32)
+    block = build(args, 14).layers[0]
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x, y = (torch.randn(1, 5, args.dim, device="cuda", generator=g) for _ in range(2))
+
+    def f(x, y):
+        normed, total = block.ffn_norm.after_add(x, y)
+        return total + block.feed_forward(block.attention_norm(normed))
+
+    with torch.no_grad():
+        assert torch.allclose(torch.compile(f, fullgraph=True, backend="eager")(x, y), f(x, y), atol=1e-5, rtol=1e-5)
+
+
 def test_a_hook_may_exchange_the_attention_output_of_a_token():
     """What a forward hook (or an attention module of another kind) returns reaches the
     projection as any tensor reaches it: strided and broadcast outputs with their own values, another type

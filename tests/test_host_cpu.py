@@ -102,6 +102,17 @@ def test_linears_that_make_their_weights_are_left_to_torch(change):
     assert not K.linears_fit(x, plain, m)
 
 
+def test_compiled_code_is_asked_for_its_operators_without_a_graph_break():
+    from dram_attention_amd import model_kernels as K
+
+    def f(x):
+        return x + 1 if K.unobserved() else x - 1
+
+    x = torch.zeros(3)
+    assert torch.equal(f(x), x + 1)
+    assert torch.equal(torch.compile(f, fullgraph=True, backend="eager")(x), x - 1)
+
+
 def test_package_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "dram_attention_amd")
     for name in os.listdir(pkg):
