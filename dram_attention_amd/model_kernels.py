@@ -8,6 +8,7 @@ import torch
 from torch import nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as nn_module
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -17,12 +18,20 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 def unobserved() -> bool:
     """Whether nothing but the tensors' values depends on which operators run: no forward-mode
-    differentiation (which torch.no_grad leaves on), vmap or other transform, dispatch mode,
-    tracer or compiler would have to see them."""
+    differentiation (which torch.no_grad leaves on), vmap or other transform, dispatch or
+    function mode, tracer or compiler would have to see them."""
     # (the compiler first: it cannot follow the other questions)
     return (not torch.compiler.is_compiling()
             and forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
-            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None)
+            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
+            and not (torch._C._len_torch_function_stack() and _function_mode_watches()))
+
+
+def _function_mode_watches() -> bool:
+    """Whether a function mode other than torch.device(...) and torch.set_default_device, which
+    only say where new tensors are born, is on."""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+               for i in range(torch._C._len_torch_function_stack()))
 
 
 def takes(*tensors: torch.Tensor) -> bool:

@@ -500,6 +500,25 @@ def test_an_instance_forward_is_still_called():
     assert calls == [1]
 
 
+def test_a_function_mode_sees_the_operators_of_a_token():
+    """What a mode that counts calls sees of a decode step: the projections of every layer."""
+    from torch.overrides import TorchFunctionMode
+
+    class Count(TorchFunctionMode):
+        linears = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.linears += func is torch.nn.functional.linear
+            return func(*args, **(kwargs or {}))
+
+    args = small_args(torch.bfloat16)
+    model = build(args, 15)
+    model(torch.arange(600, device="cuda")[None] % args.vocab_size, 0)
+    with Count() as count:
+        model(torch.tensor([[5]], device="cuda"), 600)
+    assert count.linears == 7 * args.n_layers + 1
+
+
 def test_norm_and_feed_forward_compile_as_one_graph():
     args = small_args(torch.float32)
     block = build(args, 14).layers[0]

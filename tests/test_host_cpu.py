@@ -113,6 +113,25 @@ def test_compiled_code_is_asked_for_its_operators_without_a_graph_break():
     assert torch.equal(torch.compile(f, fullgraph=True, backend="eager")(x), x - 1)
 
 
+def test_function_modes_are_observers_and_device_contexts_are_not():
+    from torch.overrides import TorchFunctionMode
+
+    from dram_attention_amd import model_kernels as K
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with torch.device("cpu"):
+        assert K.unobserved()
+        with Watch():
+            assert not K.unobserved()
+            with torch.device("cpu"):
+                assert not K.unobserved()
+        assert K.unobserved()
+    assert K.unobserved()
+
+
 def test_package_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "dram_attention_amd")
     for name in os.listdir(pkg):
