@@ -239,6 +239,18 @@ def test_fp32_prefill_sums_are_short_chains(D):
     assert (lse.double() - want).abs().max().item() < (S / 32 + 5 + 8) * 2.0 ** -24
 
 
+def test_fp32_prompt_under_autocast_is_torchs():
+    """Autocast turns scaled dot products to its type; 2e-2 is that type's tolerance here."""
+    from dram_attention_amd.dram_attention import causal_prefill_attention
+
+    xq, xk, xv = draw(300, 4, 4, 64, torch.float32, 1)
+    want = causal_prefill_attention(xq, xk, xv)
+    assert want.dtype == torch.float32
+    with torch.no_grad(), torch.autocast("cuda", torch.bfloat16):
+        got = causal_prefill_attention(xq, xk, xv)
+    assert got.dtype == torch.bfloat16 and close(got, want, ATOL, RTOL)
+
+
 @pytest.mark.parametrize("S,Hq,Hkv,D,dtype", [
     (600, 2, 2, 64, torch.bfloat16), (3000, 8, 2, 64, torch.float32), (9000, 32, 8, 128, torch.bfloat16),
     (12345, 64, 8, 128, torch.float16),
