@@ -188,11 +188,15 @@ def prefill_attention(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
 def prefill_attention_f32_supported(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor) -> bool:
     """Whether the library's fp32 prefill kernel takes these tensors as they are (it has no
     backward and no other derivative, so operands that autograd or a transform follows stay
-    with torch, as do token strides above the kernel's 2^24 bytes, and autocast, under which
-    torch attends in the 16-bit type)."""
+    with torch, as do token strides above the kernel's 2^24 bytes, several sequences, keys of
+    another length, and autocast, under which torch attends in the 16-bit type)."""
     if not (xq.is_cuda and xq.shape[-1] in (64, 128) and unobserved() and not torch.is_autocast_enabled()):
         return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_cuda
+    if not (xq.dim() == xk.dim() == 4 and xq.shape[0] == xk.shape[0] == 1 and xk.shape == xv.shape
+            and xk.shape[1] == xq.shape[1] and xk.shape[3] == xq.shape[3]
+            and xk.shape[2] > 0 and xq.shape[2] % xk.shape[2] == 0):
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.device == xq.device
                and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.stride(1) % 4 == 0
                and t.stride(2) % 4 == 0 and t.stride(1) <= 1 << 22
                and not (t.requires_grad and torch.is_grad_enabled()) for t in (xq, xk, xv))

@@ -239,6 +239,23 @@ def test_fp32_prefill_sums_are_short_chains(D):
     assert (lse.double() - want).abs().max().item() < (S / 32 + 5 + 8) * 2.0 ** -24
 
 
+def test_fp32_prompts_of_other_shapes_are_torchs():
+    """Several sequences, and keys that reach beyond the queries (row i looks at keys 0..i), against the
+    single-sequence kernel and the blocked form: fp32 both, 1e-5.  Heads that do not split are refused."""
+    from dram_attention_amd.dram_attention import causal_prefill_attention, prefill_attention_f32
+
+    parts = [draw(70, 4, 2, 64, torch.float32, seed) for seed in (1, 2)]
+    both = causal_prefill_attention(*(torch.cat(t) for t in zip(*parts)))
+    for got, (xq, xk, xv) in zip(both, parts):
+        assert close(got, prefill_attention_f32(xq, xk, xv)[0], 1e-5, 1e-5)
+    xq, xk, xv = parts[0]
+    want = causal_prefill_attention(xq[:, :50].contiguous(), xk, xv, "blocked")
+    assert close(causal_prefill_attention(xq[:, :50].contiguous(), xk, xv), want, 1e-5, 1e-5)
+    assert close(want, prefill_attention_f32(xq, xk, xv)[:, :50], 1e-5, 1e-5)
+    with pytest.raises(RuntimeError):
+        causal_prefill_attention(xq[:, :, :3].contiguous(), xk, xv)
+
+
 def test_fp32_prompt_under_autocast_is_torchs():
     """Autocast turns scaled dot products to its type; 2e-2 is that type's tolerance here."""
     from dram_attention_amd.dram_attention import causal_prefill_attention
