@@ -512,14 +512,11 @@ class DRAMAttention(torch.nn.Module):
         layout a layer is built with; None where anything differs, and the two methods, which
         take or refuse it, do the step.  The same launches on the same operands."""
         lru = self.lru_cache
-        cls = type(self)
         if (type(lru) is not LRUCache or self.attention_scope != "resident" or not self.overlap_page_stream
-                or not self.attend_on_page_stream or cls.select_ is not DRAMAttention.select_
-                or cls.attend_ is not DRAMAttention.attend_ or "select_" in self.__dict__
-                or "attend_" in self.__dict__):
+                or not self.attend_on_page_stream):
             return None
         selector, buffers, own = lru.top_k_selector, lru._buffers, self._buffers
-        if type(selector) is not IPUpperboundTopKSelector:
+        if type(selector) is not IPUpperboundTopKSelector or not self._steps_by_its_own_methods(lru, selector):
             return None
         minmax, dram, hbm = selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"]
         H, P, _, D = minmax.shape
@@ -586,6 +583,15 @@ class DRAMAttention(torch.nn.Module):
             1.0 / math.sqrt(D), self.link_gbps, self.block_gbps, 0)
         _lib.check(_lib.load().da_decode_step(args, len(args), _lib.stream_ptr(device)), "da_decode_step")
         return out
+
+    def _steps_by_its_own_methods(self, lru, selector) -> bool:
+        """Whether the methods a step is made of are this module's: neither a subclass, nor an
+        exchanged method of a class, the layer, its page cache or its selector would be passed by."""
+        cls, layer, cache, ranking = type(self), self.__dict__, lru.__dict__, selector.__dict__
+        return ((cls.select_, cls.attend_, LRUCache.select_, LRUCache.update_, LRUCache.views,
+                 IPUpperboundTopKSelector.top_k_for_lru, IPUpperboundTopKSelector.scores) == _STEP_METHODS
+                and not ("select_" in layer or "attend_" in layer or "select_" in cache or "update_" in cache
+                         or "views" in cache or "top_k_for_lru" in ranking or "scores" in ranking))
 
     def select_(self, xq: torch.Tensor):
         """First half of a decode step: page scores, ordered top-k and the LRU update
@@ -699,3 +705,7 @@ class DRAMAttention(torch.nn.Module):
         main.wait_stream(side)                      # the pages have landed
         attend(P.SECOND)
         return (out, None) if defer_merge else out
+
+
+_STEP_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, LRUCache.select_, LRUCache.update_, LRUCache.views,
+                 IPUpperboundTopKSelector.top_k_for_lru, IPUpperboundTopKSelector.scores)

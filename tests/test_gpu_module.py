@@ -872,3 +872,41 @@ def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
         a(rand(1, 2, Hq, D), rand(1, 2, Hkv, D), rand(1, 2, Hkv, D), start_pos=S, stage="generate")
     with pytest.raises(RuntimeError):                               # beyond the local cache
         a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
+
+
+def test_an_exchanged_method_of_a_step_is_called(monkeypatch):
+    """Whatever the step is made of, on the instances, on the classes or in a subclass."""
+    from dram_attention_amd import DRAMAttention, LRUCache
+    from dram_attention_amd.topk_selector import IPUpperboundTopKSelector
+
+    class Halves(DRAMAttention):
+        def select_(self, xq):
+            calls.append("subclass")
+            return super().select_(xq)
+
+    g = torch.Generator(device=DEV).manual_seed(6)
+    xq, xk, xv = (torch.randn(1, 1000, h, 64, device=DEV, generator=g).bfloat16() for h in (4, 2, 2))
+    layer, halves = (cls(16, 256, 256, 16, 64, 2, 64, device=DEV) for cls in (DRAMAttention, Halves))
+    layer.init_cache(xk, xv)
+    halves.init_cache(xk, xv)
+    calls = []
+
+    def step(m=layer):
+        calls.clear()
+        m(xq[:, :1], xk[:, :1], xv[:, :1], start_pos=1000, stage="generate")
+        return calls
+
+    assert step() == [] and step(halves) == ["subclass"]
+    cache, selector = layer.lru_cache, layer.lru_cache.top_k_selector
+    for owner, name in ((layer, "select_"), (layer, "attend_"), (cache, "select_"), (cache, "update_"),
+                        (cache, "views"), (selector, "top_k_for_lru"), (selector, "scores"),
+                        (DRAMAttention, "select_"), (DRAMAttention, "attend_"), (LRUCache, "select_"),
+                        (LRUCache, "update_"), (LRUCache, "views"), (IPUpperboundTopKSelector, "top_k_for_lru"),
+                        (IPUpperboundTopKSelector, "scores")):
+        inner = getattr(owner, name)
+        with monkeypatch.context() as patch:
+            patch.setattr(owner, name, lambda *a, **kw: calls.append(name) or inner(*a, **kw))
+            assert name in step(), (owner, name)
+        if not isinstance(owner, type):
+            delattr(owner, name)        # (the bound method that monkeypatch left on the instance)
+    assert step() == []
