@@ -483,8 +483,10 @@ class DRAMAttention(torch.nn.Module):
     def _prefill(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor):
         """Attention over the prompt and the caches built from it.  Where a library kernel
         attends, the page store is written next to it, on a stream of its own: attention is
-        bound by the matrix cores, the store by the host link."""
-        if not (self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
+        bound by the matrix cores, the store by the host link.  An init_cache of somebody's
+        own is called, behind attention."""
+        if not (type(self).init_cache is _INIT_CACHE and "init_cache" not in self.__dict__
+                and self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
                 and self.prefill_backend in ("auto", "native") and xk.is_cuda
                 and (prefill_attention_supported(xq) or prefill_attention_f32_supported(xq, xk, xv))):
             output = causal_prefill_attention(xq, xk, xv, self.prefill_backend)
@@ -709,3 +711,4 @@ class DRAMAttention(torch.nn.Module):
 
 _STEP_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, LRUCache.select_, LRUCache.update_, LRUCache.views,
                  IPUpperboundTopKSelector.top_k_for_lru, IPUpperboundTopKSelector.scores)
+_INIT_CACHE = DRAMAttention.init_cache

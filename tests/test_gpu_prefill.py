@@ -312,6 +312,36 @@ def test_a_refused_prompt_leaves_the_layer_as_it_was():
     assert m.lru_cache is cache and m.dram_kv_cache_size == paged
 
 
+def test_an_init_cache_of_its_own_gets_the_prompt(monkeypatch):
+    """In a subclass, on the layer or in the class's place: called once, with the prompt's keys and values."""
+    from dram_attention_amd import DRAMAttention
+
+    class Own(DRAMAttention):
+        def init_cache(self, k_cache, v_cache):
+            given.append((k_cache, v_cache))
+            super().init_cache(k_cache, v_cache)
+
+    xq, xk, xv = draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    sizes = dict(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16, top_k=64,
+                 n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16)
+    given, ref = [], DRAMAttention(**sizes)
+    want = ref(xq, xk, xv, start_pos=0, stage="prefill")
+    for where in ("subclass", "layer", "class"):
+        given.clear()
+        m = (Own if where == "subclass" else DRAMAttention)(**sizes)
+        with monkeypatch.context() as patch:
+            if where == "layer":
+                inner = m.init_cache
+                m.init_cache = lambda k, v: given.append((k, v)) or inner(k, v)
+            if where == "class":
+                init_cache = DRAMAttention.init_cache
+                patch.setattr(DRAMAttention, "init_cache",
+                              lambda self, k, v: given.append((k, v)) or init_cache(self, k, v))
+            assert same(m(xq, xk, xv, start_pos=0, stage="prefill"), want)
+        assert len(given) == 1 and given[0][0] is xk and given[0][1] is xv, where
+        assert same(m.lru_cache.dram_kv_cache, ref.lru_cache.dram_kv_cache)
+
+
 def test_the_host_link_is_timed_while_no_store_is_being_written(monkeypatch):
     """The rate is kept for the whole process: it must not come from copies that shared the link
     with a page store on its way."""
