@@ -250,7 +250,7 @@ def store_build_blocks(q_shape, k_shape, dtype: torch.dtype) -> int:
     over 4096, 8, 16 and 32 end after 0.45, 0.37 and 0.34 ms.)"""
     _, S, Hq, D = q_shape
     flops_per_s, bytes_per_s, esize = (1.1e14, 3.7e9, 4) if dtype == torch.float32 else (1e15, 7.6e9, 2)
-    attention_s = 2.0 * S * S * Hq * D / flops_per_s
+    attention_s = max(1e-9, 2.0 * S * S * Hq * D / flops_per_s)    # (no queries: attention refuses them)
     store_bytes = 2.0 * S * k_shape[2] * D * esize
     return max(2, min(32, math.ceil(store_bytes / bytes_per_s / (0.7 * attention_s))))
 

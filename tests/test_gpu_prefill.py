@@ -309,6 +309,8 @@ def test_a_refused_prompt_leaves_the_layer_as_it_was():
     xq, xk, xv = draw(2000, 4, 2, 64, torch.bfloat16, 2)
     with pytest.raises(ValueError):
         m(xq, xk.half(), xv.half(), start_pos=0, stage="prefill")
+    with pytest.raises(ValueError):
+        m(xq[:, :0], xk, xv, start_pos=0, stage="prefill")
     assert m.lru_cache is cache and m.dram_kv_cache_size == paged
 
 

@@ -132,6 +132,15 @@ def test_function_modes_are_observers_and_device_contexts_are_not():
     assert K.unobserved()
 
 
+def test_store_build_blocks_stays_within_its_limits():
+    """2 to 32 for prompts of any length, and for a call without queries, which attention refuses."""
+    from dram_attention_amd.dram_attention import store_build_blocks
+
+    for S in (0, 1, 300, 10 ** 4, 10 ** 7):
+        for dtype in (torch.bfloat16, torch.float32):
+            assert 2 <= store_build_blocks((1, S, 4, 64), (1, max(S, 1000), 2, 64), dtype) <= 32
+
+
 def test_package_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "dram_attention_amd")
     for name in os.listdir(pkg):
