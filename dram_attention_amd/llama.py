@@ -173,7 +173,7 @@ class Attention(nn.Module):
         xk = self.wk(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         xv = self.wv(x).view(bsz, seqlen, self.n_kv_heads, self.head_dim)
         if (K.takes(xq, xk) and K.plain_linears(self.wq, self.wk) and rope_rows.dtype == torch.float32
-                and rope_rows.is_contiguous() and rope_rows.device == xq.device
+                and rope_rows.is_contiguous() and rope_rows.device == xq.device and rope_rows.data_ptr() % 16 == 0
                 and bsz == 1 and rope_rows.shape == (seqlen, self.head_dim // 2, 2)
                 and self.head_dim * xq.element_size() % 16 == 0):
             K.rope_(xq, xk, rope_rows)          # the projections' own outputs, in place

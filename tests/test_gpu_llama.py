@@ -519,6 +519,24 @@ def test_a_function_mode_sees_the_operators_of_a_token():
     assert count.linears == 7 * args.n_layers + 1
 
 
+def test_rotation_takes_a_table_that_starts_anywhere():
+    """Rows of a table four bytes off the kernels' alignment: torch's operators, the same values but
+    for products that may be fused (a turn of the rounding: 2^-7)."""
+    args = small_args(torch.bfloat16)
+    attention = build(args, 16).layers[0].attention
+    seen = []
+    attention.dram_attention.register_forward_pre_hook(lambda mod, inp: seen.append(inp))
+    x = torch.randn(1, 200, args.dim, device="cuda", dtype=torch.bfloat16,
+                    generator=torch.Generator(device="cuda").manual_seed(1))
+    rows = L.rope_table(attention.head_dim, 200, 1e4, False, device="cuda")
+    odd = torch.empty(rows.numel() + 1, device="cuda")[1:].view(rows.shape).copy_(rows)
+    with torch.no_grad():
+        attention(x, 0, rows)
+        attention(x, 0, odd)
+    for a, b in zip(*seen):
+        assert torch.allclose(a.float(), b.float(), rtol=2.0 ** -7, atol=2.0 ** -9)
+
+
 def test_norm_and_feed_forward_compile_as_one_graph():
     args = small_args(torch.float32)
     block = build(args, 14).layers[0]
