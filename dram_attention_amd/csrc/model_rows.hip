@@ -95,7 +95,7 @@ rope_rows_kernel(char *__restrict__ q, int64_t q_tok_b, char *__restrict__ k, in
 
 template <typename T>
 __global__ void __launch_bounds__(kRowThreads)
-swiglu_kernel(const char *__restrict__ gate, const char *__restrict__ up, char *__restrict__ out, int64_t vecs) {
+swiglu_kernel(const char *gate, const char *up, char *out, int64_t vecs) {   // (out may be gate or up)
   const int64_t j = (int64_t)blockIdx.x * kRowThreads + threadIdx.x;
   if (j >= vecs) return;
   float a[T::kVec], b[T::kVec];

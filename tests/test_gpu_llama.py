@@ -537,6 +537,22 @@ def test_rotation_takes_a_table_that_starts_anywhere():
         assert torch.allclose(a.float(), b.float(), rtol=2.0 ** -7, atol=2.0 ** -9)
 
 
+@pytest.mark.parametrize("n", [8, 2056, 100000])
+def test_swiglu_in_place_of_either_operand(n):
+    from dram_attention_amd import _lib
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    gate, up = (torch.randn(n, device="cuda", generator=g).bfloat16() for _ in range(2))
+    results = []
+    for place in (None, 0, 1):
+        operands = [gate.clone(), up.clone()]
+        out = torch.empty_like(gate) if place is None else operands[place]
+        _lib.check(_lib.load().da_swiglu(operands[0].data_ptr(), operands[1].data_ptr(), out.data_ptr(), n,
+                                         _lib.dtype_code(gate.dtype), _lib.stream_ptr(gate.device)), "da_swiglu")
+        results.append(out)
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
 def test_norm_and_feed_forward_compile_as_one_graph():
     args = small_args(torch.float32)
     block = build(args, 14).layers[0]
