@@ -22,16 +22,17 @@
 // operands of four channel blocks (block b, row c is channel 4c + b).
 //
 // Measured: 133 TFLOP/s (0.85 of 157; a large fp32 matrix product of the library: 154) at 32/8
-// heads, D 128, 9200 tokens; 0.70 ms = 124 TFLOP/s at 8/2 heads, D 64, 9200 tokens, where
+// heads, D 128, 9200 tokens; 0.70 ms = 125 TFLOP/s at 8/2 heads, D 64, 9200 tokens, where
 // torch's operators took 4.27 ms.
 //
-// Sums: a lane adds its eight weights of a tile in pairs before they join its running sum, and
-// at D 64 the output sums of each kPfsChain tiles, which the matrix cores add up one key group
-// after the other, are added to a second set of registers.  Distance to float64 (2-norm, 8/2
-// heads, N(0, 1) queries and values, keys with outlier channels) at 1756 / 2001 / 9200 tokens:
-// 5.1 / 5.3 / 8.5e-7 in single chains, 4.5 / 4.6 / 5.4e-7 like this; torch's blocked operators 4.6 / 4.7 /
-// 8.4e-7.  At D 128 (1756 to 9000 tokens) the weights' pairs are enough: 6.1 to 8.4e-7 against
-// torch's 6.1 to 8.5e-7.  It costs 1.6 % at 9200 tokens (689 -> 700 us) and 3 us at 1756.
+// Sums: a score is the sum of two chains of MFMAs, over every other 16 channels each, and a lane
+// adds its eight weights of a tile in pairs before they join its running sum.  Distance to
+// float64 (2-norm; N(0, 1) queries and values, keys with outlier channels) in single chains / like
+// this / of torch's blocked operators, in 1e-7: 8/2 heads, D 64: 1756 tokens 5.1 / 4.2 / 4.7, 3000 5.9
+// / 5.0 / 5.5, 9200 8.5 / 7.6 / 8.4; 16/4 2500: 5.5 / 4.7 / 5.3; 32/8, D 128: 1800 5.9 / 4.5 / 5.9, 9000 8.5 /
+// 7.4 / 8.5.  It costs 1 % at 9200 tokens of 8/2 heads (688 -> 695 us) and nothing at D 128.  (Output
+// sums of 16 tiles joining a second set of registers: 4.6, 4.9, 5.4, but the kernel then fills the
+// register file, and the page store beside it takes 5 % more of the call.)
 //
 // Tiles are double-buffered and travel global memory -> LDS directly, in the blocks of
 // 1024 bytes with swizzled columns that prefill_attention.hip explains.
@@ -47,7 +48,6 @@ constexpr int kPfsThreads = 256;
 constexpr int kPfsWaves = 4;
 constexpr int kPfsRows = 16;  // query rows of a wave
 constexpr int kPfsKeys = 32;  // keys per tile
-constexpr int kPfsChain = 16;     // tiles (a power of two) whose output sums are one chain, at D 64
 constexpr int kPfsCus = 256;      // compute units of the part
 constexpr int kPfsResident = 4;   // workgroups of one launch a unit holds at once (two at D 128)
 
@@ -69,14 +69,13 @@ struct PrefillSharedF32 {
 };
 
 template <int kD, int kHeads>
-__global__ void __launch_bounds__(kPfsThreads, kD == 64 ? kPfsResident : 2)
+__global__ void __launch_bounds__(kPfsThreads, 2)
 prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
   using Sh = PrefillSharedF32<kD>;
   static_assert(kD == 64 || kD == 128, "head sizes of 64 and 128");
   constexpr int kBlockRows = kPfsRows * kPfsWaves / kHeads;
   constexpr int kQChunks = kD / 16;     // 16-byte query chunks per lane
   constexpr int kCGroups = kD / 64;     // groups of 64 output channels
-  constexpr bool kTwoSums = kD == 64;   // output sums in two levels
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -170,40 +169,32 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
   for (int b = 0; b < 4 * kCGroups; ++b)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[b][i] = 0.f;
-  pf_f32x4 total[kTwoSums ? 4 * kCGroups : 1];   // (two levels: of the chains that are complete)
-#pragma unroll
-  for (int b = 0; b < (kTwoSums ? 4 * kCGroups : 1); ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) total[b][i] = 0.f;
-  auto end_chain = [&]() {
-#pragma unroll
-    for (int b = 0; b < 4 * kCGroups; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        total[b][i] += acc[b][i];
-        acc[b][i] = 0.f;
-      }
-  };
 
   auto compute = [&](int tile, int buf, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
     __builtin_amdgcn_iglp_opt(1);   // (measured: see the loop below)
     const char *kt = smem + buf * Sh::kBufBytes;
-    pf_f32x4 st[2];
+    pf_f32x4 st[2], odd[2];   // the channels' sums in two chains (chunks of 16 in turn)
 #pragma unroll
     for (int half = 0; half < 2; ++half)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) st[half][i] = 0.f;
+      for (int i = 0; i < 4; ++i) st[half][i] = odd[half][i] = 0.f;
 #pragma unroll
-    for (int t = 0; t < kQChunks; ++t) {
-      const u32x4 k0 = *(const u32x4 *)(kt + k_at[t]);
-      const u32x4 k1 = *(const u32x4 *)(kt + k_at[t] + kHalfStep);
+    for (int t = 0; t < kQChunks; t += 2) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {   // the two halves in turn: each chain's latency hides the other's
-        st[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(as_f32(k0[i]), as_f32(qf[t][i]), st[0], 0, 0, 0);
-        st[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(as_f32(k1[i]), as_f32(qf[t][i]), st[1], 0, 0, 0);
+      for (int u = 0; u < 2; ++u) {
+        const u32x4 k0 = *(const u32x4 *)(kt + k_at[t + u]);
+        const u32x4 k1 = *(const u32x4 *)(kt + k_at[t + u] + kHalfStep);
+        pf_f32x4 *const s = u ? odd : st;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // the two halves in turn: each chain's latency hides the other's
+          s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(as_f32(k0[i]), as_f32(qf[t + u][i]), s[0], 0, 0, 0);
+          s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(as_f32(k1[i]), as_f32(qf[t + u][i]), s[1], 0, 0, 0);
+        }
       }
     }
+    st[0] += odd[0];
+    st[1] += odd[1];
     float smax = -INFINITY;
     if constexpr (kMask) {
       const int lim = (int)(my_row - ((int64_t)tile * kPfsKeys + 4 * g));  // key offset <= lim stays
@@ -228,10 +219,7 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
 #pragma unroll
       for (int b = 0; b < 4 * kCGroups; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[b][i] *= alpha;
-          if constexpr (kTwoSums) total[b][i] *= alpha;
-        }
+        for (int i = 0; i < 4; ++i) acc[b][i] *= alpha;
     }
 #pragma unroll
     for (int half = 0; half < 2; ++half)
@@ -269,8 +257,6 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
     __syncthreads();
     fetch(tile + 2, 0);                             // (there is one: the tiles of the block's own rows)
     compute(tile + 1, 1, std::false_type{});
-    if constexpr (kTwoSums)
-      if ((tile + 2) % kPfsChain == 0) end_chain();
     __syncthreads();
   }
   for (int tile = n_whole; tile < n_tiles; ++tile) {
@@ -284,10 +270,6 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
     __syncthreads();
   }
 
-  if constexpr (kTwoSums) {                         // (the chain that was begun)
-#pragma unroll
-    for (int b = 0; b < 4 * kCGroups; ++b) acc[b] += total[b];
-  }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   const float inv = l > 0.f ? 1.f / l : 0.f;

@@ -217,26 +217,30 @@ def test_fp32_prefill_kernel_matches_dense_float64(S, Hq, Hkv, D):
 @pytest.mark.parametrize("D", [64, 128])
 def test_fp32_prefill_sums_are_short_chains(D):
     """Summands that lose half of what lies below the sum's last place when they are added one
-    after the other.  Sum of the weights, by the log-sum-exp: one addition to the running sum per
-    tile of 32 keys (and five in and behind it), half a unit in the last place each, and that of the result
-    (9, to 2^-21).  Output at D 64: equal weights, so chains of 16 tiles, one addition per 4 keys,
-    and of S / 512 chains."""
+    after the other, seen in the log-sum-exp.  Sum of the weights: one addition to the running sum per tile of
+    32 keys (and five in and behind it), half a unit in the last place each, and that of the result
+    (9, to 2^-21).  A single score: half the channels in a chain lie a binade below the whole sum and lose
+    nothing; the chains' sum, the scale, the product with ln 2 and the two logarithms remain, half a unit each."""
     from dram_attention_amd.dram_attention import prefill_attention_f32
 
     S = 8192
     odd = 1.0 + 502 * 2.0 ** -23
-    q, k = torch.zeros(1, S, 4, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV)
-    out = prefill_attention_f32(q, k, torch.full((1, S, 1, D), odd, device=DEV))
-    if D == 64:
-        assert (out.double() / odd - 1).abs().max().item() < (128 + S / 512 + 4) * 2.0 ** -24
+    q, k, v = torch.zeros(1, S, 4, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV), torch.ones(1, S, 1, D, device=DEV)
     q[..., 0] = 1.0
     k[:, 32:, :, 0] = math.log(odd) * math.sqrt(D)       # the first tile's scores, zero, stay the reference
     lse = torch.empty(4, S, device=DEV)
-    prefill_attention_f32(q, k, out[:, :, :1].contiguous(), lse=lse)
+    prefill_attention_f32(q, k, v, lse=lse)
     n = torch.arange(1, S + 1, device=DEV, dtype=torch.float64)
     weight = (k[0, 32, 0, 0].double() / math.sqrt(D)).exp()
     want = (n.clamp(max=32) + (n - 32).clamp(min=0) * weight).log()
     assert (lse.double() - want).abs().max().item() < (S / 32 + 5 + 8) * 2.0 ** -24
+
+    term = 1.0 + 0.49 * D * 2.0 ** -24                   # 0.49 of the last place of sums in D/2 .. D
+    k = torch.full((1, 1, 1, D), term, device=DEV)
+    lse = torch.empty(4, 1, device=DEV)
+    prefill_attention_f32(torch.ones(1, 1, 4, D, device=DEV), k, v[:, :1].contiguous(), lse=lse)
+    want = D * k[0, 0, 0, 0].double().item() / math.sqrt(D)
+    assert (lse.double() / want - 1).abs().max().item() < 5 * 2.0 ** -24
 
 
 def test_fp32_prompts_of_other_shapes_are_torchs():
