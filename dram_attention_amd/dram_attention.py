@@ -190,16 +190,21 @@ def prefill_attention_f32_supported(xq: torch.Tensor, xk: torch.Tensor, xv: torc
     backward and no other derivative, so operands that autograd or a transform follows stay
     with torch, as do token strides above the kernel's 2^24 bytes, several sequences, keys of
     another length, and autocast, under which torch attends in the 16-bit type)."""
-    if not (xq.is_cuda and xq.shape[-1] in (64, 128) and unobserved() and not torch.is_autocast_enabled()):
+    q_shape, k_shape = xq.shape, xk.shape
+    if not xq.is_cuda or not len(q_shape) == len(k_shape) == 4 or xv.shape != k_shape:
         return False
-    if not (xq.dim() == xk.dim() == 4 and xq.shape[0] == xk.shape[0] == 1 and xk.shape == xv.shape
-            and xk.shape[1] == xq.shape[1] and xk.shape[3] == xq.shape[3]
-            and xk.shape[2] > 0 and xq.shape[2] % xk.shape[2] == 0):
+    (bsz, S, Hq, D), (n_seqs, Skv, Hkv, Dk) = q_shape, k_shape
+    if not (bsz == n_seqs == 1 and Skv == S and Dk == D and D in (64, 128) and Hkv > 0 and Hq % Hkv == 0
+            and unobserved() and not torch.is_autocast_enabled()):
         return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.device == xq.device
-               and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.stride(1) % 4 == 0
-               and t.stride(2) % 4 == 0 and t.stride(1) <= 1 << 22
-               and not (t.requires_grad and torch.is_grad_enabled()) for t in (xq, xk, xv))
+    device, grad = xq.device, torch.is_grad_enabled()
+    for t in (xq, xk, xv):
+        stride = t.stride()
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype is not torch.float32 or t.device != device
+                or stride[3] != 1 or stride[1] % 4 or stride[2] % 4 or stride[1] > 1 << 22 or t.data_ptr() % 16
+                or (grad and t.requires_grad)):
+            return False
+    return True
 
 
 def prefill_attention_f32(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
@@ -417,15 +422,23 @@ class DRAMAttention(torch.nn.Module):
                 cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
             tail = seqlen - paged
             window_k, window_v = self.cache_k[:, :tail], self.cache_v[:, :tail]
-            # (both shapes are refused here or neither copy is)
-            tail_k, tail_v = k_cache[:, paged:].expand_as(window_k), v_cache[:, paged:].expand_as(window_v)
+            tail_k, tail_v = k_cache[:, paged:], v_cache[:, paged:]
+            if not tail_k.shape == tail_v.shape == window_k.shape:
+                # (both are refused here or neither is)
+                tail_k, tail_v = tail_k.expand_as(window_k), tail_v.expand_as(window_v)
             window_k.copy_(tail_k, non_blocking=True)
             window_v.copy_(tail_v, non_blocking=True)
+            # Nothing refuses the prompt from here on.  The old cache is taken apart while the
+            # new store is on its way, but for its own store, in pinned memory, which launches
+            # of the last steps may still be reading until finish_build has waited.
+            held = self._modules.get("lru_cache")
+            held = None if held is None else held._buffers.get("dram_kv_cache")
+            self.lru_cache, self.link_gbps, self.dram_kv_cache_size = cache, link_gbps, paged
+            self._workspace = None
         finally:
             if isinstance(cache, LRUCache):
                 cache.finish_build()
-        self.lru_cache, self.link_gbps, self.dram_kv_cache_size = cache, link_gbps, paged
-        self._workspace = None
+        del held
 
     def _paged_tokens(self, seqlen: int) -> int:
         """Prompt tokens that go to the paged prefix; the rest is the local window."""

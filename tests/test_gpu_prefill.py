@@ -348,6 +348,23 @@ def test_an_init_cache_of_its_own_gets_the_prompt(monkeypatch):
         assert same(m.lru_cache.dram_kv_cache, ref.lru_cache.dram_kv_cache)
 
 
+def test_the_old_page_store_outlives_the_launches_that_read_it(monkeypatch):
+    """A second prompt on a layer: the first one's store, which the last decode steps read by address,
+    is let go only when the host has waited for what was launched."""
+    import weakref
+
+    from dram_attention_amd import DRAMAttention, LRUCache
+
+    m = DRAMAttention(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16,
+                      top_k=64, n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16)
+    xq, xk, xv = draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    m(xq, xk, xv, start_pos=0, stage="prefill")
+    old, held, finish = weakref.ref(m.lru_cache.dram_kv_cache), [], LRUCache.finish_build
+    monkeypatch.setattr(LRUCache, "finish_build", lambda self: finish(self) or held.append(old() is not None))
+    m(xq, xk, xv, start_pos=0, stage="prefill")
+    assert held == [True] and old() is None
+
+
 def test_the_host_link_is_timed_while_no_store_is_being_written(monkeypatch):
     """The rate is kept for the whole process: it must not come from copies that shared the link
     with a page store on its way."""
