@@ -248,8 +248,10 @@ class TransformerBlock(nn.Module):
         """Whether the one-token kernels may stand for these modules of a block: the modules
         are the block's own kinds, nobody watches them, and every shape is the one that the
         kernels take for granted."""
-        if not (type(a) is Attention and type(f) is FeedForward and type(norm1) is type(norm2) is RMSNorm
-                and K.takes(x, norm1.weight, norm2.weight) and K.bare(a, f, norm1, norm2)
+        if not (type(a) is Attention and type(f) is FeedForward and type(norm1) is type(norm2) is RMSNorm):
+            return False
+        weight1, weight2 = norm1._parameters.get("weight"), norm2._parameters.get("weight")
+        if not (K.takes(x, weight1, weight2) and K.bare(a, f, norm1, norm2)
                 and rope_rows.dtype is torch.float32 and rope_rows.is_contiguous()
                 and rope_rows.device == x.device):
             return False
@@ -264,7 +266,7 @@ class TransformerBlock(nn.Module):
                 and (wo.out_features, wo.in_features) == (dim, q_rows)
                 and (w3.out_features, w3.in_features) == (hidden, w1.in_features) == (hidden, dim)
                 and (w2.out_features, w2.in_features) == (dim, hidden)
-                and norm1.weight.shape == norm2.weight.shape == (dim,)
+                and weight1.shape == weight2.shape == (dim,)
                 and rope_rows.shape == (1, a.head_dim // 2, 2) and a.head_dim % 2 == 0)
 
 

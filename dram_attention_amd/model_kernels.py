@@ -14,6 +14,10 @@ from . import _lib
 
 _TYPES = (torch.bfloat16, torch.float16, torch.float32)
 _PLAIN = (torch.Tensor, nn.Parameter)
+# (asked several times for every layer of a token)
+_transform_level = torch._C._functorch.maybe_current_level
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_tracing_state = torch._C._get_tracing_state
 
 
 def unobserved() -> bool:
@@ -22,16 +26,15 @@ def unobserved() -> bool:
     function mode, tracer or compiler would have to see them."""
     # (the compiler first: it cannot follow the other questions)
     return (not torch.compiler.is_compiling()
-            and forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
-            and not torch._C._len_torch_dispatch_stack() and torch._C._get_tracing_state() is None
-            and not (torch._C._len_torch_function_stack() and _function_mode_watches()))
+            and forward_ad._current_level < 0 and _transform_level() is None
+            and not _dispatch_modes() and _tracing_state() is None
+            and not (_function_modes() and _function_mode_watches()))
 
 
 def _function_mode_watches() -> bool:
     """Whether a function mode other than torch.device(...) and torch.set_default_device, which
     only say where new tensors are born, is on."""
-    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
-               for i in range(torch._C._len_torch_function_stack()))
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(_function_modes()))
 
 
 def takes(*tensors: torch.Tensor) -> bool:
@@ -41,8 +44,12 @@ def takes(*tensors: torch.Tensor) -> bool:
     if (not x.is_cuda or x.dtype not in _TYPES or torch.is_grad_enabled() or torch.is_autocast_enabled()
             or not unobserved()):
         return False
-    return all(type(t) in _PLAIN and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
-               and t.data_ptr() % 16 == 0 for t in tensors)
+    dtype, device = x.dtype, x.device
+    for t in tensors:
+        if (type(t) not in _PLAIN or t.dtype is not dtype or t.device != device or not t.is_contiguous()
+                or t.data_ptr() % 16):
+            return False
+    return True
 
 
 def norm_fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -87,7 +94,10 @@ def bare(*modules: nn.Module) -> bool:
     them or gave one of them a forward of its own."""
     if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules)
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+            return False
+    return True
 
 
 def plain_linears(*modules: nn.Module) -> bool:
