@@ -318,8 +318,9 @@ prefill_attention_kernel(const PrefillArgs a) {
   // with it give, in TFLOP/s (same bits): 135152 tokens, 32/8 heads, D 128: 1146 as it was, 1197
   // with the rounds of two and without raised wave priority around the MFMAs (1123 with it:
   // the other wave of the SIMD is the one to let in), 1211 with iglp_opt(1), which spreads the
-  // LDS reads between the MFMAs; 8192 tokens 1081 -> 1134, 4613 943 -> 998; 20000 tokens,
-  // 16/16 heads, D 64: 800 -> 912.
+  // LDS reads between the MFMAs; 8192 tokens 1081 -> 1134, 4613 943 -> 998; 20000 tokens, 16/16
+  // heads, D 64: 800 -> 912 (old and new in turn on one box; over boxes and operands the 135152-token
+  // prompt runs at 1149 to 1221, 4613 tokens back to back at 990 to 1009, one launch alone at 973).
   const int n_whole = (int)(m0 / kPfKeys) / kSplit & ~1;
   for (int round = 0; round < n_whole; round += 2) {
     fetch_round(round + 1, 1);
