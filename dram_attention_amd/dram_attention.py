@@ -399,7 +399,7 @@ class DRAMAttention(torch.nn.Module):
         paged = self._paged_tokens(seqlen)
         prefix_k = k_cache[0, :paged].transpose(0, 1)
         prefix_v = v_cache[0, :paged].transpose(0, 1)
-        link_gbps, cache = self.link_gbps, None
+        link_gbps = cache = held = None
         try:
             if paged > self.lru_hbm_cache_size:
                 if self.page_selector not in ("bound", "token_max"):
@@ -431,10 +431,10 @@ class DRAMAttention(torch.nn.Module):
             # Nothing refuses the prompt from here on.  The old cache is taken apart while the
             # new store is on its way, but for its own store, in pinned memory, which launches
             # of the last steps may still be reading until finish_build has waited.
-            held = self._modules.get("lru_cache")
-            held = None if held is None else held._buffers.get("dram_kv_cache")
-            self.lru_cache, self.link_gbps, self.dram_kv_cache_size = cache, link_gbps, paged
-            self._workspace = None
+            if link_gbps is not None:
+                held, self.link_gbps = self._modules.get("lru_cache"), link_gbps
+                held = None if held is None else held._buffers.get("dram_kv_cache")
+            self.lru_cache, self.dram_kv_cache_size, self._workspace = cache, paged, None
         finally:
             if isinstance(cache, LRUCache):
                 cache.finish_build()
@@ -498,8 +498,8 @@ class DRAMAttention(torch.nn.Module):
         attends, the page store is written next to it, on a stream of its own: attention is
         bound by the matrix cores, the store by the host link.  An init_cache of somebody's
         own is called, behind attention."""
-        if not (type(self).init_cache is _INIT_CACHE and "init_cache" not in self.__dict__
-                and self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
+        if not (self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
+                and type(self).init_cache is _INIT_CACHE and "init_cache" not in self.__dict__
                 and self.prefill_backend in ("auto", "native") and xk.is_cuda
                 and (prefill_attention_supported(xq) or prefill_attention_f32_supported(xq, xk, xv))):
             output = causal_prefill_attention(xq, xk, xv, self.prefill_backend)
