@@ -39,6 +39,13 @@ SIGNATURES = {
         [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64,
          c_int64, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_int64, c_void_p, c_void_p],
     ),
+    "da_prefill_attention_f32_workspace_bytes": (c_size_t, [c_int64, c_int, c_int, c_int]),
+    "da_prefill_attention_f32_split": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64,
+         c_int64, c_int, c_int, c_int, c_float, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
+         c_size_t, c_void_p],
+    ),
     "da_page_minmax": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int, c_int64, c_int, c_int, c_int, c_void_p, c_void_p],

@@ -28,6 +28,7 @@ SOURCES = (
     "decode_step.hip",
     "prefill_attention.hip",
     "prefill_attention_f32.hip",
+    "prefill_attention_f32_split.hip",
     "model_rows.hip",
     "decode_linear.hip",
 )

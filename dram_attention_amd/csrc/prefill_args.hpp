@@ -19,7 +19,23 @@ struct PrefillArgs {
   int64_t n_row_blocks;
   int n_kv_heads;
   float scale_log2;
+  // fp32 only: words of which one is not zero where the prompt's operands do not split into three
+  // bf16 parts (null: nobody looked); the plain kernel then runs if gate_runs_if_set, the split one if not
+  const uint32_t *gate;
+  int n_gate;
+  int gate_runs_if_set;
 };
+
+// Whether this launch is not the one that does the prompt (the whole workgroup calls it).
+__device__ __forceinline__ bool prefill_gate(const PrefillArgs &a) {
+  if (a.gate == nullptr) return false;
+  uint32_t any = 0;
+  for (int i = threadIdx.x; i < a.n_gate; i += blockDim.x) any |= a.gate[i];
+  return (__syncthreads_or((int)any) != 0) != (a.gate_runs_if_set != 0);
+}
+
+// The kernel on fp32 instructions (prefill_attention_f32.hip), head_dim 64 or 128.
+int launch_prefill_f32(const PrefillArgs &a, int head_dim, hipStream_t s);
 
 // Checks the operands of a prefill call and fills `a` (all but the grid's geometry).
 inline int prefill_args(PrefillArgs &a, const char *what, const void *q, int64_t q_tok_stride,

@@ -72,6 +72,7 @@ template <int kD, int kHeads>
 __global__ void __launch_bounds__(kPfsThreads, 2)
 prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
   using Sh = PrefillSharedF32<kD>;
+  if (prefill_gate(a)) return;
   static_assert(kD == 64 || kD == 128, "head sizes of 64 and 128");
   constexpr int kBlockRows = kPfsRows * kPfsWaves / kHeads;
   constexpr int kQChunks = kD / 16;     // 16-byte query chunks per lane
@@ -289,7 +290,7 @@ prefill_attention_f32_kernel(const PrefillArgs a, const int n_kv_heads) {
 }
 
 template <int kD>
-static int launch_prefill_f32(PrefillArgs a, int n_kv_heads, hipStream_t s) {
+static int launch_prefill_f32_of(PrefillArgs a, int n_kv_heads, hipStream_t s) {
   const int heads = a.rep % 4 == 0 ? 4 : (a.rep % 2 == 0 ? 2 : 1);
   a.n_groups = a.rep / heads;
   a.n_row_blocks = ceil_div(a.seq_len, kPfsRows * kPfsWaves / heads);
@@ -306,6 +307,11 @@ static int launch_prefill_f32(PrefillArgs a, int n_kv_heads, hipStream_t s) {
   return launch_status("da_prefill_attention_f32");
 }
 
+int launch_prefill_f32(const PrefillArgs &a, int head_dim, hipStream_t s) {
+  return head_dim == 128 ? launch_prefill_f32_of<128>(a, a.n_kv_heads, s)
+                         : launch_prefill_f32_of<64>(a, a.n_kv_heads, s);
+}
+
 }  // namespace da
 
 extern "C" int da_prefill_attention_f32(const float *q, int64_t q_tok_stride, int64_t q_head_stride,
@@ -320,7 +326,7 @@ extern "C" int da_prefill_attention_f32(const float *q, int64_t q_tok_stride, in
                               k_head_stride, v, v_tok_stride, v_head_stride, seq_len, n_q_heads, n_kv_heads,
                               DA_F32, scale, out, o_tok_stride, o_head_stride, lse_out);
   if (rc != DA_OK || seq_len == 0) return rc;
-  if (head_dim == 128) return launch_prefill_f32<128>(a, n_kv_heads, (hipStream_t)stream);
-  if (head_dim == 64) return launch_prefill_f32<64>(a, n_kv_heads, (hipStream_t)stream);
-  return fail(DA_ENOTSUP, "da_prefill_attention_f32: head_dim 64 or 128 (got %d)", head_dim);
+  if (head_dim != 64 && head_dim != 128)
+    return fail(DA_ENOTSUP, "da_prefill_attention_f32: head_dim 64 or 128 (got %d)", head_dim);
+  return launch_prefill_f32(a, head_dim, (hipStream_t)stream);
 }

@@ -210,18 +210,28 @@ def prefill_attention_f32_supported(xq: torch.Tensor, xk: torch.Tensor, xv: torc
 def prefill_attention_f32(xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor, *,
                           scale: float | None = None,
                           lse: torch.Tensor | None = None) -> torch.Tensor:
-    """:func:`prefill_attention` for an fp32 layer (da_prefill_attention_f32): fp32 products
-    and sums throughout."""
+    """:func:`prefill_attention` for an fp32 layer: fp32 products and sums throughout
+    (da_prefill_attention_f32), and for a prompt of some length, where there is memory for its keys
+    and values in three bf16 parts each, the products of those parts, which are as exact
+    (da_prefill_attention_f32_split)."""
     out, args = _prefill_operands(xq, xk, xv, lse)
     if xq.dtype != torch.float32:
         raise TypeError(f"prefill_attention_f32 takes float32, got {xq.dtype}")
     S, Hq, D = xq.shape[1:]
-    _lib.check(
-        _lib.load().da_prefill_attention_f32(
-            *args, S, Hq, xk.shape[2], D, float(scale) if scale is not None else 1.0 / math.sqrt(D),
-            out.data_ptr(), out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None,
-            _lib.stream_ptr(xq.device)),
-        "da_prefill_attention_f32")
+    lib, Hkv = _lib.load(), xk.shape[2]
+    args += (S, Hq, Hkv, D, float(scale) if scale is not None else 1.0 / math.sqrt(D), out.data_ptr(),
+             out.stride(1), out.stride(2), lse.data_ptr() if lse is not None else None)
+    need = lib.da_prefill_attention_f32_workspace_bytes(S, Hq, Hkv, D)
+    if need:
+        try:
+            room = torch.empty(need, dtype=torch.uint8, device=xq.device)
+        except torch.cuda.OutOfMemoryError:
+            need = 0
+    if need:
+        _lib.check(lib.da_prefill_attention_f32_split(*args, room.data_ptr(), need, _lib.stream_ptr(xq.device)),
+                   "da_prefill_attention_f32_split")
+    else:
+        _lib.check(lib.da_prefill_attention_f32(*args, _lib.stream_ptr(xq.device)), "da_prefill_attention_f32")
     return out
 
 

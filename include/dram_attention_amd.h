@@ -91,6 +91,23 @@ int da_prefill_attention_f32(const float *q, int64_t q_tok_stride, int64_t q_hea
                              float *lse_out, void *stream);
 
 /*
+ * The same, faster for all but short prompts: every operand as the sum of three bf16 numbers,
+ * products of those on the bf16 matrix instructions, sums in fp32; no further from float64 than
+ * the form above, which does the prompt after all where an operand is not finite, above 2^60 or
+ * (but for 0) below 2^-100 (decided on the device).
+ *   workspace: 16-byte aligned, 4096 + ceil(S / 64) * Hkv * 768 * D bytes; contents may be anything.
+ *              da_prefill_attention_f32_workspace_bytes is that size, or 0 where the prompt is so
+ *              short that the form above is the faster one
+ */
+size_t da_prefill_attention_f32_workspace_bytes(int64_t seq_len, int n_q_heads, int n_kv_heads, int head_dim);
+int da_prefill_attention_f32_split(const float *q, int64_t q_tok_stride, int64_t q_head_stride,
+                                   const float *k, int64_t k_tok_stride, int64_t k_head_stride,
+                                   const float *v, int64_t v_tok_stride, int64_t v_head_stride,
+                                   int64_t seq_len, int n_q_heads, int n_kv_heads, int head_dim,
+                                   float scale, float *out, int64_t o_tok_stride, int64_t o_head_stride,
+                                   float *lse_out, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Subsystem 1 — per-page, per-channel min and max of the keys.
  * Replaces torch.aminmax + torch.stack in
  * dram_attention/topk_selector.py:31-34.

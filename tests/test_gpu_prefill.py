@@ -243,6 +243,78 @@ def test_fp32_prefill_sums_are_short_chains(D):
     assert (lse.double() / want - 1).abs().max().item() < 5 * 2.0 ** -24
 
 
+def _split_prefill(xq, xk, xv):
+    """da_prefill_attention_f32_split itself, whatever the length, in a workspace of NaN bytes."""
+    from dram_attention_amd import _lib
+
+    S, Hq, D = xq.shape[1:]
+    Hkv = xk.shape[2]
+    out, lse = torch.empty(1, S, Hq, D, device=DEV), torch.empty(Hq, S, device=DEV)
+    room = torch.full((4096 + -(-S // 64) * Hkv * 768 * D,), 255, dtype=torch.uint8, device=DEV)
+    _lib.check(_lib.load().da_prefill_attention_f32_split(
+        xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1), xk.stride(2), xv.data_ptr(),
+        xv.stride(1), xv.stride(2), S, Hq, Hkv, D, 1 / math.sqrt(D), out.data_ptr(), out.stride(1), out.stride(2),
+        lse.data_ptr(), room.data_ptr(), room.numel(), _lib.stream_ptr(xq.device)), "split")
+    return out, lse
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D", [
+    (1, 4, 1, 64), (2, 1, 1, 128), (31, 8, 2, 128), (32, 2, 1, 64), (33, 3, 1, 64), (63, 6, 3, 128), (64, 4, 4, 64),
+    (65, 4, 2, 128), (127, 8, 2, 64), (128, 5, 5, 128), (129, 7, 1, 64), (200, 12, 3, 128), (1283, 8, 2, 64),
+])
+def test_fp32_prefill_in_three_parts_matches_dense_float64(S, Hq, Hkv, D):
+    """The kernel on bf16 parts at the edges of its tiles (32 rows, 32 and 64 keys), every grouping of heads
+    and both head sizes, on rows cut out of a wider projection.  Bound: that of the fp32 kernel's test (the
+    parts are exact, what is left out of a product is a quarter of one fp32 rounding)."""
+    g = torch.Generator(device=DEV).manual_seed(S)
+    qkv = torch.randn(1, S, Hq + 2 * Hkv, D, device=DEV, generator=g) * 1.5
+    xq, xk, xv = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
+    out, lse = _split_prefill(xq, xk, xv)
+    mask = torch.ones(S, S, dtype=torch.bool, device=DEV).triu_(1)
+    for h in range(Hq):
+        q, k, v = xq[0, :, h].double(), xk[0, :, h // (Hq // Hkv)].double(), xv[0, :, h // (Hq // Hkv)].double()
+        s_ = (q @ k.t().contiguous() / math.sqrt(D)).masked_fill_(mask, float("-inf"))
+        assert close(out[0, :, h].double(), torch.softmax(s_, -1) @ v, 1e-5, 1e-5)
+        assert close(lse[h].double(), torch.logsumexp(s_, -1), 1e-5, 1e-5)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38, 2.0 ** 61, 1e-35, 1e-42])
+def test_fp32_prefill_operands_that_do_not_split(value, D):
+    """One element of the queries, keys or values, first or last, outside what three parts stand for: the bits of
+    the kernel on fp32 instructions."""
+    from dram_attention_amd import _lib
+
+    S, Hq, Hkv = 70, 4, 2
+    for which in range(3):
+        for at in (0, -1):
+            ops = list(draw(S, Hq, Hkv, D, torch.float32, 3))
+            ops[which].view(-1)[at] = value
+            out, lse = _split_prefill(*ops)
+            want, want_lse = torch.empty_like(out), torch.empty_like(lse)
+            q, k, v = ops
+            _lib.check(_lib.load().da_prefill_attention_f32(
+                q.data_ptr(), q.stride(1), q.stride(2), k.data_ptr(), k.stride(1), k.stride(2), v.data_ptr(),
+                v.stride(1), v.stride(2), S, Hq, Hkv, D, 1 / math.sqrt(D), want.data_ptr(), want.stride(1),
+                want.stride(2), want_lse.data_ptr(), _lib.stream_ptr(q.device)), "plain")
+            assert same(out, want) and same(lse, want_lse)
+
+
+def test_fp32_prefill_splits_to_the_ends_of_its_range():
+    """Values of 2^60 and 2^-100, scores of products of the two: still float64's result to 1e-5."""
+    S, D = 40, 64
+    xq, xk, xv = (x.clone() for x in draw(S, 2, 1, D, torch.float32, 4))
+    xv[0, ::3] *= 2.0 ** 57
+    xv[0, 1::3] = 2.0 ** -100
+    xq[..., 0], xk[..., 0] = 2.0 ** 60, 2.0 ** -58
+    out, _ = _split_prefill(xq, xk, xv)
+    mask = torch.ones(S, S, dtype=torch.bool, device=DEV).triu_(1)
+    for h in range(2):
+        s_ = (xq[0, :, h].double() @ xk[0, :, 0].double().t().contiguous() / math.sqrt(D)).masked_fill_(mask, float("-inf"))
+        want = torch.softmax(s_, -1) @ xv[0, :, 0].double()
+        assert ((out[0, :, h].double() - want).abs() <= 1e-5 * want.abs().amax(-1, keepdim=True)).all()
+
+
 def test_fp32_prompts_of_other_shapes_are_torchs():
     """Several sequences, and keys that reach beyond the queries (row i looks at keys 0..i), against the
     single-sequence kernel and the blocked form: fp32 both, 1e-5.  Heads that do not split are refused."""
