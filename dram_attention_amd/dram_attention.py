@@ -254,20 +254,24 @@ def _prefill_operands(xq, xk, xv, lse):
                  xk.stride(2), xv.data_ptr(), xv.stride(1), xv.stride(2))
 
 
-def store_build_blocks(q_shape, k_shape, dtype: torch.dtype) -> int:
-    """Workgroups that write the page store next to prefill attention: as few as are done
-    well within attention's time, because each takes a compute unit from it and a full
-    link slows it besides; at most the 32 that fill the link, which is what a prompt gets
-    whose store takes longer than its attention.  Rates: attention at 1 PFLOP/s, or 110
-    TFLOP/s in fp32; 7.6 GB/s to the host per workgroup, 3.7 beside fp32 attention, whose
-    workgroups leave room on a unit and then share it.  (Next to 138 ms of attention over
-    131072 tokens, 2, 4, 8 and 32 workgroups add 0.8, 1.2, 1.5 and 5 ms; next to 0.17 ms
-    over 4096, 8, 16 and 32 end after 0.45, 0.37 and 0.34 ms.)"""
+def store_build_blocks(q_shape, k_shape, dtype: torch.dtype, page_size: int = 16) -> int:
+    """Workgroups that write the page store of the keys (and values) of ``k_shape`` next to prefill
+    attention.  Each takes a compute unit from it, and once the writes fill the link (57 GB/s)
+    every miss of attention's caches waits behind them: 9000 tokens, 32/8 heads, D 128, bf16, in us by
+    workgroups: 6 910, 8 755, 12 949, 32 1054; 4000 of those heads in fp32: 5 756, 8 860, 16 973.  So
+    there are as many as fill the link but a little, by the bytes each has in flight (a page, up to
+    16 KB), or fewer where the store is done in 0.6 of attention's time all the same (20000 tokens in bf16:
+    5 3045, 6 2990, 8 3006, 12 3651; 50000 tokens, 28/4 heads: 2 to 16 within 0.5 %, 32 4 % more).  Where
+    the store takes several times as long as attention, it gets the whole link: 12000 tokens, 16/16 heads,
+    D 64: 8 1170, 32 995.  Rates: attention at 1 PFLOP/s, or 190 TFLOP/s in fp32; 5.4 GB/s to the host per
+    workgroup beside it, 4 with pages of 4 KB."""
     _, S, Hq, D = q_shape
-    flops_per_s, bytes_per_s, esize = (1.1e14, 3.7e9, 4) if dtype == torch.float32 else (1e15, 7.6e9, 2)
+    flops_per_s, esize = (1.9e14, 4) if dtype == torch.float32 else (1e15, 2)
     attention_s = max(1e-9, 2.0 * S * S * Hq * D / flops_per_s)    # (no queries: attention refuses them)
-    store_bytes = 2.0 * S * k_shape[2] * D * esize
-    return max(2, min(32, math.ceil(store_bytes / bytes_per_s / (0.7 * attention_s))))
+    page_bytes = page_size * 2 * D * esize
+    bytes_per_s, most = (5.4e9, 6) if page_bytes >= 16384 else (5.4e9, 8) if page_bytes >= 8192 else (4e9, 12)
+    blocks = math.ceil(2.0 * k_shape[1] * k_shape[2] * D * esize / bytes_per_s / (0.6 * attention_s))
+    return max(2, min(most if blocks < 3 * most else 32, blocks))
 
 
 _build_streams = {}
@@ -518,7 +522,8 @@ class DRAMAttention(torch.nn.Module):
         output = []
         self._build_cache(
             xk, xv, build_stream=build_stream(xk.device),
-            build_blocks=store_build_blocks(xq.shape, xk.shape, xq.dtype),
+            build_blocks=store_build_blocks(xq.shape, (1, self._paged_tokens(xk.shape[1]), *xk.shape[2:]), xq.dtype,
+                                            self.page_size),
             beside=lambda: output.append(causal_prefill_attention(xq, xk, xv, self.prefill_backend)))
         return output[0]
 
