@@ -1,14 +1,14 @@
 // One decode step of one layer as one call: page scores, ordered top-k with the list of
 // least recent slots, LRU update, then page stream, attention and merge (the sequence of
 // DRAMAttention.forward's generate stage, dram_attention/dram_attention.py:144-238 of the
-// reference).  Host code only: it issues the launches of the five entry points it calls, on
-// the operands of one argument block.
+// reference).  Host code only: it issues the launches of the entry points it stands for, on the
+// operands of one argument block, selection and LRU update as one where their sizes allow.
 //
 // What it saves is the caller's time: a step of the small layers takes 35 us of the GPU and
 // 86 us of Python that marshals five calls of 18 to 33 arguments.  With one call: 34 us a step
 // for the fp32 layer over 8K tokens (85 before), 435 us a token for four 2048-wide model layers
 // launched from Python (674 before).
-#include "common.hpp"
+#include "topk_rows.hpp"
 
 extern "C" int da_decode_step(const da_decode_step_args *a, size_t args_bytes, void *stream) {
   using namespace da;
@@ -22,15 +22,20 @@ extern "C" int da_decode_step(const da_decode_step_args *a, size_t args_bytes, v
                          rep, H, a->n_pages, D, a->dtype, a->scores, (int64_t)H * a->n_pages, a->n_pages, DA_F32,
                          a->score_flags, stream);
   if (rc) return rc;
-  rc = da_topk_pages_lru(a->scores, (int64_t)H * a->n_pages, a->n_pages, rep, rep, H, a->n_pages, a->kp, a->idx, K,
-                         K, a->kp, DA_I64, a->access_time, a->n_slots, DA_TIME_F32, a->n_slots, a->k_cand,
-                         a->candidates, a->step, a->topk_workspace, a->topk_workspace_bytes, stream);
-  if (rc) return rc;
-  rc = da_lru_update(a->idx, K, DA_I64, H, K, a->n_pages, a->n_slots, a->step, DA_LRU_BUMP_STEP, a->access_time,
-                     a->n_slots, DA_TIME_F32, a->d2h, a->n_pages, a->h2d, a->n_slots, DA_I64, a->hit_mask,
-                     a->miss_page, a->miss_slot, a->miss_count, a->slot_epoch, a->candidates, a->k_cand,
-                     a->lru_workspace, a->lru_workspace_bytes, stream);
-  if (rc) return rc;
+  if (topk_lru_in_one_launch(*a)) {
+    rc = launch_topk_lru(*a, (hipStream_t)stream);
+    if (rc) return rc;
+  } else {
+    rc = da_topk_pages_lru(a->scores, (int64_t)H * a->n_pages, a->n_pages, rep, rep, H, a->n_pages, a->kp, a->idx, K,
+                           K, a->kp, DA_I64, a->access_time, a->n_slots, DA_TIME_F32, a->n_slots, a->k_cand,
+                           a->candidates, a->step, a->topk_workspace, a->topk_workspace_bytes, stream);
+    if (rc) return rc;
+    rc = da_lru_update(a->idx, K, DA_I64, H, K, a->n_pages, a->n_slots, a->step, DA_LRU_BUMP_STEP, a->access_time,
+                       a->n_slots, DA_TIME_F32, a->d2h, a->n_pages, a->h2d, a->n_slots, DA_I64, a->hit_mask,
+                       a->miss_page, a->miss_slot, a->miss_count, a->slot_epoch, a->candidates, a->k_cand,
+                       a->lru_workspace, a->lru_workspace_bytes, stream);
+    if (rc) return rc;
+  }
   const int64_t e = elem_size(a->dtype), page = (int64_t)a->page_size * 2 * D;
   da_paged_overlap o = {};
   o.page_size = a->page_size;

@@ -21,7 +21,7 @@
 // reference's literal serial walk on one lane per head.
 //
 // Bound: latency; algorithmic bytes are the metadata only.
-#include "lru_keys.hpp"
+#include "topk_rows.hpp"
 
 namespace da {
 
@@ -50,32 +50,51 @@ __device__ __forceinline__ void atomic_min_signed(int64_t *p, int64_t v) {
 constexpr int64_t kMarkerBase = -(int64_t(1) << 30);
 
 template <typename IdxT, typename MapT, typename TimeT>
-__global__ void __launch_bounds__(kSelThreads)
-lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int K,
-                  int64_t n_dram_pages, int n_hbm, int32_t *step_ptr, int bump,
-                  TimeT *time_all, int64_t time_head_stride, MapT *d2h_all,
-                  int64_t d2h_head_stride, MapT *h2d_all, int64_t h2d_head_stride,
-                  uint8_t *hit_mask, int32_t *miss_page_out, int32_t *miss_slot_out,
-                  int32_t *miss_count, int32_t *slot_epoch_all, int32_t *ticket, int serial,
-                  const int32_t *cand_all_in, int k_cand) {
-  const int32_t *cand_all = cand_all_in;
-  __shared__ LruShared sm;
+struct LruArgs {
+  const IdxT *idx;
+  int64_t idx_head_stride;
+  int K;
+  int64_t n_dram_pages;
+  int n_hbm;
+  int32_t *step_ptr;
+  int bump;
+  TimeT *time;
+  int64_t time_head_stride;
+  MapT *d2h;
+  int64_t d2h_head_stride;
+  MapT *h2d;
+  int64_t h2d_head_stride;
+  uint8_t *hit_mask;
+  int32_t *miss_page_out, *miss_slot_out, *miss_count, *slot_epoch, *ticket;
+  int serial;
+  const int32_t *cand;
+  int k_cand;
+};
+
+// The update of kv head h.  kShared: requests and candidate list come from other workgroups of
+// this launch.
+template <bool kShared, typename IdxT, typename MapT, typename TimeT>
+__device__ __forceinline__ void lru_update_block(const LruArgs<IdxT, MapT, TimeT> &a, const int h, const int n_heads,
+                                                 LruShared &sm) {
+  const int K = a.K, n_hbm = a.n_hbm, bump = a.bump, serial = a.serial, k_cand = a.k_cand;
+  const int64_t n_dram_pages = a.n_dram_pages;
+  int32_t *const step_ptr = a.step_ptr, *const ticket = a.ticket, *const miss_count = a.miss_count;
+  const int32_t *cand_all = a.cand;
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
-  const int h = blockIdx.x;
-  const IdxT *idx = idx_all + h * idx_head_stride;
-  TimeT *time = time_all + h * time_head_stride;
-  MapT *d2h = d2h_all + h * d2h_head_stride;
-  MapT *h2d = h2d_all + h * h2d_head_stride;
-  uint8_t *hit = hit_mask ? hit_mask + (int64_t)h * K : nullptr;
-  int32_t *mpage = miss_page_out + (int64_t)h * K;
-  int32_t *mslot = miss_slot_out + (int64_t)h * K;
-  int32_t *slot_epoch = slot_epoch_all ? slot_epoch_all + (int64_t)h * n_hbm : nullptr;
+  const IdxT *idx = a.idx + h * a.idx_head_stride;
+  TimeT *time = a.time + h * a.time_head_stride;
+  MapT *d2h = a.d2h + h * a.d2h_head_stride;
+  MapT *h2d = a.h2d + h * a.h2d_head_stride;
+  uint8_t *hit = a.hit_mask ? a.hit_mask + (int64_t)h * K : nullptr;
+  int32_t *mpage = a.miss_page_out + (int64_t)h * K;
+  int32_t *mslot = a.miss_slot_out + (int64_t)h * K;
+  int32_t *slot_epoch = a.slot_epoch ? a.slot_epoch + (int64_t)h * n_hbm : nullptr;
 
   // Every wave reads the step for itself and waits for the value right here
   // (and for the stamp of the candidate list, requested with it).
-  int32_t stamp_read = cand_all != nullptr ? cand_all[(int64_t)gridDim.x * k_cand + h] : 0;
+  int32_t stamp_read = cand_all != nullptr ? load_between<kShared>(cand_all + (int64_t)n_heads * k_cand + h) : 0;
   int32_t step_read = *step_ptr;
   asm volatile("" : "+v"(step_read), "+v"(stamp_read)::"memory");  // the values have arrived: what follows cannot pass the reads
   const int32_t step_before = __builtin_amdgcn_readfirstlane(step_read);
@@ -96,7 +115,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
   auto draw_ticket = [&]() {
     if (bump && t == 0) {
       const int32_t done = atomicAdd(ticket, 1);
-      if (done == (int32_t)gridDim.x - 1) {
+      if (done == n_heads - 1) {
         *step_ptr = step;
         *ticket = 0;
       }
@@ -106,7 +125,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
   if (serial) {
     // -- literal restatement of the reference's three launches ---------------
     for (int k = t; k < K; k += kSelThreads) {
-      const int64_t p = (int64_t)idx[k];
+      const int64_t p = (int64_t)load_between<kShared>(idx + k);
       if (p < 0 || p >= n_dram_pages) continue;
       const int64_t s = (int64_t)d2h[p];
       if (s >= 0) time[s] = now;
@@ -118,7 +137,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
     if (t == 0) {
       int ep = 0, m = 0;
       for (int k = 0; k < K; ++k) {
-        const int64_t p = (int64_t)idx[k];
+        const int64_t p = (int64_t)load_between<kShared>(idx + k);
         if (p < 0 || p >= n_dram_pages) {
           if (hit) hit[k] = 0;
           continue;
@@ -164,7 +183,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
     const bool use_bitmap = K <= kLruTableMaxK && n_hbm <= kLruBitmapSlots;
     int32_t ahead_slot = -1, ahead_old = kNotFetched;
     if (use_bitmap && cand_all != nullptr && t < k_cand) {
-      ahead_slot = cand_all[(int64_t)h * k_cand + t];
+      ahead_slot = load_between<kShared>(cand_all + (int64_t)h * k_cand + t);
       if (ahead_slot < 0 || ahead_slot >= n_hbm) ahead_slot = -1;  // not a slot: ignored
       if (ahead_slot >= 0) ahead_old = (int32_t)h2d[ahead_slot];   // (page ids fit 32 bits)
     }
@@ -195,7 +214,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
 #pragma unroll
       for (int r = 0; r < kRounds; ++r) {
         const int k = r * kSelThreads + t;
-        page_of[r] = k < K ? (int64_t)idx[k] : -1;
+        page_of[r] = k < K ? (int64_t)load_between<kShared>(idx + k) : -1;
       }
 #pragma unroll
       for (int r = 0; r < kRounds; ++r) {
@@ -252,7 +271,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
     } else {
     // -- phase A: touch hits, mark the first occurrence of every missed page --
     for (int k = t; k < K; k += kSelThreads) {
-      const int64_t p = (int64_t)idx[k];
+      const int64_t p = (int64_t)load_between<kShared>(idx + k);
       if (p < 0 || p >= n_dram_pages) continue;
       const int64_t s = (int64_t)d2h[p];
       if (s >= 0)
@@ -268,7 +287,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
       bool first = false;
       int64_t p = -1;
       if (k < K) {
-        p = (int64_t)idx[k];
+        p = (int64_t)load_between<kShared>(idx + k);
         if (p >= 0 && p < n_dram_pages) first = (int64_t)d2h[p] == kMarkerBase + k;
         if (hit) hit[k] = (p >= 0 && p < n_dram_pages && !first) ? 1 : 0;
       }
@@ -294,7 +313,7 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
       for (int base = 0; base < k_cand && kept < (uint32_t)m; base += kSelThreads) {
         const int i = base + t;
         const bool ahead = use_bitmap && base == 0;
-        int32_t slot = ahead ? ahead_slot : i < k_cand ? cand_all[(int64_t)h * k_cand + i] : -1;
+        int32_t slot = ahead ? ahead_slot : i < k_cand ? load_between<kShared>(cand_all + (int64_t)h * k_cand + i) : -1;
         if (slot >= n_hbm) slot = -1;
         const bool untouched =
             slot >= 0 && (use_bitmap ? !((sm.touched[slot >> 5] >> (slot & 31)) & 1u) : time[slot] != now);
@@ -337,6 +356,13 @@ lru_update_kernel(const IdxT *__restrict__ idx_all, int64_t idx_head_stride, int
 
 }
 
+template <typename IdxT, typename MapT, typename TimeT>
+__global__ void __launch_bounds__(kSelThreads)
+lru_update_kernel(const LruArgs<IdxT, MapT, TimeT> a) {
+  __shared__ LruShared sm;
+  lru_update_block<false>(a, blockIdx.x, gridDim.x, sm);
+}
+
 // One 256-thread block per (entry, head), striding over the head's miss list.
 // Every lane moves 16 bytes at a time with all of a page's loads issued before
 // the first store, so a wave keeps several KiB of host-link reads in flight.
@@ -376,14 +402,89 @@ static void launch_lru_time(int time_type, dim3 grid, hipStream_t s, const void 
                             int k_cand) {
   if (time_type == DA_TIME_F32)
     hipLaunchKernelGGL((lru_update_kernel<IdxT, MapT, float>), grid, dim3(kSelThreads), 0, s,
-                       (const IdxT *)idx, idx_hs, K, P, n_hbm, step, bump, (float *)time, time_hs,
-                       (MapT *)d2h, d2h_hs, (MapT *)h2d, h2d_hs, hit, mp, ms, mc, se, ticket, serial,
-                       cand, k_cand);
+                       LruArgs<IdxT, MapT, float>{(const IdxT *)idx, idx_hs, K, P, n_hbm, step, bump, (float *)time,
+                                                  time_hs, (MapT *)d2h, d2h_hs, (MapT *)h2d, h2d_hs, hit, mp, ms, mc,
+                                                  se, ticket, serial, cand, k_cand});
   else
     hipLaunchKernelGGL((lru_update_kernel<IdxT, MapT, int32_t>), grid, dim3(kSelThreads), 0, s,
-                       (const IdxT *)idx, idx_hs, K, P, n_hbm, step, bump, (int32_t *)time,
-                       time_hs, (MapT *)d2h, d2h_hs, (MapT *)h2d, h2d_hs, hit, mp, ms, mc, se, ticket,
-                       serial, cand, k_cand);
+                       LruArgs<IdxT, MapT, int32_t>{(const IdxT *)idx, idx_hs, K, P, n_hbm, step, bump,
+                                                    (int32_t *)time, time_hs, (MapT *)d2h, d2h_hs, (MapT *)h2d, h2d_hs,
+                                                    hit, mp, ms, mc, se, ticket, serial, cand, k_cand});
+}
+
+// The selection and the update it feeds as one launch: per kv head one workgroup for every score
+// row, one for the list of least recent slots, and whichever of them is done last goes on to the
+// update.  What they hand over, the requests and the list, is written through to memory and read
+// from there (a few KB per head), which takes almost as long as the launch of the update that it
+// saves; the caller, who has one launch less to issue, gains more.  A step of the fp32 layer over
+// 8K tokens 32.5 -> 31.6 us (a host thread's part of it 36 -> 33), a token of four 2048-wide layers
+// launched from Python 344 -> 331 us; steps that stream for 60 us and more are as they were.
+struct TopkRowsArgs {
+  const float *scores;  // (rows, heads, pages)
+  int n_rows, n_pages, kp;
+};
+__global__ void __launch_bounds__(kSelThreads)
+topk_lru_update_kernel(const TopkRowsArgs r, const LruCandidateArgs cand,
+                       const LruArgs<int64_t, int64_t, float> a, uint32_t *__restrict__ arrivals) {
+  __shared__ LruShared sm;
+  __shared__ uint32_t arrived;
+  const int n = blockIdx.x, h = blockIdx.y;
+  if (n >= r.n_rows) {
+    lru_candidates_block<true, float>(cand, h, sm.sel);
+  } else {
+    const float *row = r.scores + ((int64_t)n * gridDim.y + h) * r.n_pages;
+    ScoreKey key{row, ((uintptr_t)row & 15) == 0};
+    int64_t *dst = const_cast<int64_t *>(a.idx) + h * a.idx_head_stride + (int64_t)n * r.kp;
+    select_sorted(key, r.n_pages, r.kp, sm.sel,
+                  direct([=](uint32_t rank, uint32_t page) { store_between<true>(dst + rank, (int64_t)page); }));
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every store of this wave has reached memory
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    arrived = __hip_atomic_fetch_add(arrivals + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (arrived == gridDim.x - 1) store_between<true>(arrivals + h, 0u);  // ready for the next launch
+  }
+  __syncthreads();
+  if (arrived != gridDim.x - 1) return;
+  lru_update_block<true>(a, h, gridDim.y, sm);
+}
+
+constexpr int kLruTicketWords = 2;  // of the update's workspace; the arrivals follow, a word per head
+
+bool topk_lru_in_one_launch(const da_decode_step_args &a) {
+  const int64_t K = (int64_t)(a.n_q_heads / a.n_kv_heads) * a.kp;
+  // (longer rows take two launches, more requests than slots the serial walk)
+  return a.n_pages <= kSelRegKeys * kSelThreads && a.kp <= kSelMaxK && K <= a.n_slots && K <= kLruMaxK &&
+         a.candidates != nullptr && a.k_cand > 0 &&
+         a.lru_workspace_bytes >= (int64_t)sizeof(uint32_t) * (kLruTicketWords + a.n_kv_heads);
+}
+
+int launch_topk_lru(const da_decode_step_args &a, hipStream_t s) {
+  const int rep = a.n_q_heads / a.n_kv_heads, K = rep * a.kp;
+  DA_REQUIRE(a.n_pages >= 0 && a.kp <= a.n_pages, "da_decode_step: kp %d exceeds the %lld pages of a row", a.kp,
+             (long long)a.n_pages);
+  DA_REQUIRE(a.scores && a.idx && a.access_time && a.step && a.d2h && a.h2d && a.miss_page && a.miss_slot &&
+                 a.miss_count && a.lru_workspace,
+             "da_decode_step: null pointer");
+  DA_REQUIRE(a.k_cand <= a.n_slots && a.k_cand <= kSelMaxK, "da_decode_step: %d candidates of %d slots (at most %d)",
+             a.k_cand, a.n_slots, kSelMaxK);
+  if (a.n_kv_heads > 65535) return fail(DA_ENOTSUP, "da_decode_step: head count out of range");
+  const TopkRowsArgs r = {a.scores, rep, (int)a.n_pages, a.kp};
+  LruCandidateArgs cand = {};
+  cand.access_time = a.access_time;
+  cand.time_head_stride = a.n_slots;
+  cand.n_slots = a.n_slots;
+  cand.k_cand = a.k_cand;
+  cand.out = a.candidates;
+  cand.step = a.step;
+  cand.n_heads = a.n_kv_heads;
+  const LruArgs<int64_t, int64_t, float> u = {
+      a.idx, K, K, a.n_pages, a.n_slots, a.step, 1, a.access_time, a.n_slots, a.d2h, a.n_pages, a.h2d, a.n_slots,
+      a.hit_mask, a.miss_page, a.miss_slot, a.miss_count, a.slot_epoch, (int32_t *)a.lru_workspace, 0, a.candidates,
+      a.k_cand};
+  hipLaunchKernelGGL(topk_lru_update_kernel, dim3(rep + 1, a.n_kv_heads), dim3(kSelThreads), 0, s, r, cand, u,
+                     (uint32_t *)a.lru_workspace + kLruTicketWords);
+  return launch_status("da_decode_step(selection)");
 }
 
 }  // namespace da

@@ -5,53 +5,9 @@
 //
 // Bound: latency (a row is a few tens of KiB and stays in L2); algorithmic
 // bytes = rows*P*4 read + rows*kp*8 written.
-#include "lru_keys.hpp"
+#include "topk_rows.hpp"
 
 namespace da {
-
-struct ScoreKey {
-  const float *row;
-  bool aligned;  // row starts on a 16-byte boundary
-  __device__ __forceinline__ uint32_t operator()(int i) const { return float_order_key(row[i]); }
-  __device__ __forceinline__ void load4(int i, uint32_t *k) const {
-    float4 v;
-    if (aligned) {
-      v = *(const float4 *)(row + i);
-    } else {
-      v = make_float4(row[i], row[i + 1], row[i + 2], row[i + 3]);
-    }
-    k[0] = float_order_key(v.x);
-    k[1] = float_order_key(v.y);
-    k[2] = float_order_key(v.z);
-    k[3] = float_order_key(v.w);
-  }
-};
-
-// The k_cand least recently used slots of kv head h, in eviction order, into
-// out[h, 0..k_cand).  Independent of this step's scores, so it rides along with
-// the top-k launch (one more workgroup per head) and the LRU update that follows
-// only has to drop the slots it touched from this list.
-struct LruCandidateArgs {
-  const void *access_time;  // (Hkv, n_slots), fp32 or int32; null: no candidates
-  int64_t time_head_stride;
-  int time_is_i32;
-  int n_slots, k_cand;
-  int32_t *out;  // (Hkv, k_cand) lists, then Hkv stamp words
-  const int32_t *step;  // the LRU step counter: its value now is the list's stamp
-  int n_heads;
-};
-
-template <typename TimeT>
-__device__ __forceinline__ void lru_candidates_block(const LruCandidateArgs &c, int h,
-                                                     SelectShared &sm) {
-  LeastRecentKey<TimeT> key{(const TimeT *)c.access_time + h * c.time_head_stride};
-  int32_t *dst = c.out + (int64_t)h * c.k_cand;
-  // The stamp says which state of the access times the list describes: the update
-  // that consumes the list compares it with the step it reads.
-  if (threadIdx.x == 0) c.out[(int64_t)c.n_heads * c.k_cand + h] = *c.step;
-  select_sorted(key, c.n_slots, c.k_cand, sm,
-                direct([=](uint32_t rank, uint32_t slot) { dst[rank] = (int32_t)slot; }));
-}
 
 template <typename IdxT>
 __global__ void __launch_bounds__(kSelThreads)
@@ -64,9 +20,9 @@ topk_pages_kernel(const float *__restrict__ scores, int64_t row_stride, int64_t 
   const int h = blockIdx.y;
   if (n >= n_rows) {
     if (cand.time_is_i32)
-      lru_candidates_block<int32_t>(cand, h, sm);
+      lru_candidates_block<false, int32_t>(cand, h, sm);
     else
-      lru_candidates_block<float>(cand, h, sm);
+      lru_candidates_block<false, float>(cand, h, sm);
     return;
   }
   const float *row = scores + n * row_stride + h * head_stride;
@@ -161,9 +117,9 @@ topk_merge_kernel(const uint32_t *__restrict__ cand_key, const uint32_t *__restr
     // parts of the 1M shape fill the device exactly (64 rows x 4 parts on 256
     // compute units, one workgroup each), and eight more would run as a second round.
     if (cand.time_is_i32)
-      lru_candidates_block<int32_t>(cand, h, sm);
+      lru_candidates_block<false, int32_t>(cand, h, sm);
     else
-      lru_candidates_block<float>(cand, h, sm);
+      lru_candidates_block<false, float>(cand, h, sm);
     return;
   }
   const int64_t base = ((int64_t)n * gridDim.y + h) * n_parts * kp;

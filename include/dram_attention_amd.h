@@ -502,8 +502,10 @@ int da_pages_gather_attend(const void *dram, int64_t dram_head_stride_bytes,
 /*
  * One whole decode step of a layer with a page cache: da_page_score, da_topk_pages_lru,
  * da_lru_update (DA_LRU_BUMP_STEP) and da_decode_attention_paged (STREAM | FIRST |
- * SECOND) on one argument block, in that order on `stream`; each of them checks its
- * operands as when called alone.  For the layout a DRAMAttention layer has: every
+ * SECOND) on one argument block, in that order on `stream`, with the operands and results that
+ * each has when called alone; top-k and LRU update are one launch where rows are of up to
+ * 16384 pages and a head has no more requests than slots (the words of lru_workspace behind the
+ * first two, zeroed once as the rest, then count a head's workgroups in).  For the layout a DRAMAttention layer has: every
  * array contiguous, int64 maps and indexes, fp32 access times and scores.
  * `args_bytes` = sizeof(da_decode_step_args).
  */

@@ -874,6 +874,35 @@ def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
         a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
 
 
+@pytest.mark.parametrize("Hq,Hkv,slots,kp,S", [
+    (8, 2, 24, 6, 1500),     # as many requests as slots
+    (8, 2, 20, 6, 1500),     # more: the serial walk, a launch of its own
+    (4, 4, 40, 1, 1500),     # one page a head
+    (16, 2, 400, 40, 9000),  # eight rows a head, lists ordered by the radix sort's neighbour
+    (8, 1, 600, 70, 12000),  # lists beyond the short sort, more candidates than misses
+    (62, 62, 8, 2, 700), (63, 63, 8, 2, 700),   # the last number of heads the arrivals have words for, and one more
+])
+def test_selection_and_update_in_one_launch(Hq, Hkv, slots, kp, S):
+    """Bits of the separate launches, step by step, at the edges of the rule that joins them."""
+    from dram_attention_amd import DRAMAttention
+
+    D, page = 64, 16
+    g = torch.Generator(device=DEV).manual_seed(7)
+    k, v = (torch.randn(1, S, Hkv, D, device=DEV, generator=g).bfloat16() for _ in range(2))
+    a, b = (DRAMAttention(8, slots * page, 200, page, kp * page, Hkv, D, device=DEV) for _ in range(2))
+    a.init_cache(k, v)
+    b.init_cache(k, v)
+    for t in range(6):
+        xq, xk, xv = (torch.randn(1, 1, h, D, device=DEV, generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
+        got = a(xq, xk, xv, start_pos=S + t, stage="generate")
+        assert same(got, b.attend_(xq, xk, xv, S + t, b.select_(xq))), t
+        for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
+                     "hbm_page_to_dram_page_mapping", "current_step", "_topk_idx"):
+            assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
+        for name in ("miss_count", "candidates", "slot_epoch", "hit_mask"):
+            assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
+
+
 def test_an_exchanged_method_of_a_step_is_called(monkeypatch):
     """Whatever the step is made of, on the instances, on the classes or in a subclass."""
     from dram_attention_amd import DRAMAttention, LRUCache
