@@ -114,6 +114,8 @@ SIGNATURES = {
          c_void_p],
     ),
     "da_decode_step": (c_int, [c_char_p, c_size_t, c_void_p]),
+    "da_decode_steps_supported": (c_int, [c_char_p, c_int, c_size_t]),
+    "da_decode_steps": (c_int, [c_char_p, c_int, c_size_t, c_void_p]),
     "da_rms_norm": (
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "da_rope_rows": (

@@ -28,6 +28,7 @@
 
 #include "attention_mfma.hpp"
 #include "page_stream.hpp"
+#include "topk_rows.hpp"
 
 namespace da {
 
@@ -45,9 +46,8 @@ constexpr int kMergeStats = 2048;  // (max, sum) pairs staged in LDS
 enum MergeMode { kMergeAll = 0, kMergePre = 1, kMergeFinal = 2 };
 
 template <typename T>
-__global__ void __launch_bounds__(kMergeThreads)
-decode_attention_merge_kernel(const AttnArgs a, int mode, int head_dim, char *__restrict__ out,
-                              int64_t out_head_stride, float *__restrict__ lse_out) {
+__device__ __forceinline__ void merge_block(const AttnArgs &a, int mode, int head_dim, char *__restrict__ out,
+                                            int64_t out_head_stride, float *__restrict__ lse_out) {
   const int hq = blockIdx.x;
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -175,6 +175,35 @@ decode_attention_merge_kernel(const AttnArgs a, int mode, int head_dim, char *__
     lse_out[hq] = lt > 0.f ? (mx + __builtin_amdgcn_logf(lt)) * kLn2 : -INFINITY;
 }
 
+template <typename T>
+__global__ void __launch_bounds__(kMergeThreads)
+decode_attention_merge_kernel(const AttnArgs a, int mode, int head_dim, char *__restrict__ out,
+                              int64_t out_head_stride, float *__restrict__ lse_out) {
+  merge_block<T>(a, mode, head_dim, out, out_head_stride, lse_out);
+}
+
+// The final merges of several layers' steps, layers of the same sizes: what differs between them.
+struct MergeLayer {
+  float *part_ml, *part_acc;
+  const int32_t *miss_count, *c_len_dev;
+  int64_t c_len;
+  char *out;
+};
+struct MergeBatch {
+  MergeLayer layer[kStepBatch];
+};
+template <typename T>
+__global__ void __launch_bounds__(kMergeThreads)
+decode_attention_merge_layers_kernel(AttnArgs a, const MergeBatch batch, int head_dim, int64_t out_head_stride) {
+  const MergeLayer &l = batch.layer[blockIdx.y];
+  a.part_ml = l.part_ml;
+  a.part_acc = l.part_acc;
+  a.miss_count = l.miss_count;
+  a.c_len_dev = l.c_len_dev;
+  a.c_len = l.c_len;
+  merge_block<T>(a, kMergeAll, head_dim, l.out, out_head_stride, nullptr);
+}
+
 // The matrix-core form of the pass, for the shapes it takes.
 template <typename T, int kD>
 static void launch_tile(const AttnArgs &a, int n_launch, int n_kv_heads, hipStream_t s) {
@@ -274,6 +303,47 @@ static int launch_attention(const AttnArgs &a, int dtype, int phase, int n_kv_he
   }
 #undef DA_ATTN_MERGE
 #undef DA_ATTN_LAUNCH
+  return DA_OK;
+}
+
+// The merges behind launches of DA_PHASE_STREAM | DA_PHASE_FIRST that da_decode_attention_paged has
+// issued, and checked, for n steps of the same sizes.
+int launch_merge_layers(const da_decode_step_args *steps, int n, hipStream_t s) {
+  const da_decode_step_args &g = *steps;
+  const int D = g.head_dim, rep = g.n_q_heads / g.n_kv_heads;
+  const ChunkPlan p = plan_chunks(g.n_kv_heads, lanes_of(D, g.dtype), (int64_t)g.n_slots * g.page_size, g.cache_rows,
+                                  (int64_t)rep * g.kp * g.page_size);
+  AttnArgs a = {};
+  a.rep = rep;
+  a.n_q_heads = g.n_q_heads;
+  a.c_capacity = g.cache_rows;
+  a.new_k = (const char *)g.new_k;     // (every step has a new token)
+  a.chunk = p.chunk;
+  a.n_pchunks = p.n_p;
+  a.n_lchunks = p.n_l;
+  a.n_tchunks = p.n_t;
+  a.pre_chunk = p.pre_chunk();
+  a.gather_chunk0 = p.gather_chunk0();
+  a.gather_blocks = g.gather_blocks;
+  for (int first = 0; first < n; first += kStepBatch) {
+    const int count = n - first < kStepBatch ? n - first : kStepBatch;
+    MergeBatch batch;
+    for (int i = 0; i < count; ++i) {
+      const da_decode_step_args &l = steps[first + i];
+      float *acc = (float *)l.workspace;
+      batch.layer[i] = {acc + (size_t)p.total() * g.n_q_heads * D, acc, l.miss_count, l.cache_len_dev, l.cache_len,
+                        (char *)l.out};
+    }
+    const dim3 grid(g.n_q_heads, count);
+#define DA_MERGE(T) \
+  hipLaunchKernelGGL(decode_attention_merge_layers_kernel<T>, grid, dim3(kMergeThreads), 0, s, a, batch, D, D)
+    if (g.dtype == DA_BF16) DA_MERGE(BF16);
+    else if (g.dtype == DA_F16) DA_MERGE(F16);
+    else DA_MERGE(F32);
+#undef DA_MERGE
+    const int rc = launch_status("da_decode_steps(merge)");
+    if (rc) return rc;
+  }
   return DA_OK;
 }
 

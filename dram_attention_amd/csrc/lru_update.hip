@@ -419,34 +419,42 @@ static void launch_lru_time(int time_type, dim3 grid, hipStream_t s, const void 
 // saves; the caller, who has one launch less to issue, gains more.  A step of the fp32 layer over
 // 8K tokens 32.5 -> 31.6 us (a host thread's part of it 36 -> 33), a token of four 2048-wide layers
 // launched from Python 344 -> 331 us; steps that stream for 60 us and more are as they were.
-struct TopkRowsArgs {
+struct TopkLruLayer {
   const float *scores;  // (rows, heads, pages)
   int n_rows, n_pages, kp;
+  LruCandidateArgs cand;
+  LruArgs<int64_t, int64_t, float> update;
+  uint32_t *arrivals;   // one per head, zero between launches
 };
+template <int kLayers>
+struct TopkLruBatch {
+  TopkLruLayer layer[kLayers];
+};
+template <int kLayers>
 __global__ void __launch_bounds__(kSelThreads)
-topk_lru_update_kernel(const TopkRowsArgs r, const LruCandidateArgs cand,
-                       const LruArgs<int64_t, int64_t, float> a, uint32_t *__restrict__ arrivals) {
+topk_lru_update_kernel(const TopkLruBatch<kLayers> batch) {
   __shared__ LruShared sm;
   __shared__ uint32_t arrived;
+  const TopkLruLayer &l = batch.layer[kLayers > 1 ? blockIdx.z : 0];
   const int n = blockIdx.x, h = blockIdx.y;
-  if (n >= r.n_rows) {
-    lru_candidates_block<true, float>(cand, h, sm.sel);
+  if (n >= l.n_rows) {
+    lru_candidates_block<true, float>(l.cand, h, sm.sel);
   } else {
-    const float *row = r.scores + ((int64_t)n * gridDim.y + h) * r.n_pages;
+    const float *row = l.scores + ((int64_t)n * gridDim.y + h) * l.n_pages;
     ScoreKey key{row, ((uintptr_t)row & 15) == 0};
-    int64_t *dst = const_cast<int64_t *>(a.idx) + h * a.idx_head_stride + (int64_t)n * r.kp;
-    select_sorted(key, r.n_pages, r.kp, sm.sel,
+    int64_t *dst = const_cast<int64_t *>(l.update.idx) + h * l.update.idx_head_stride + (int64_t)n * l.kp;
+    select_sorted(key, l.n_pages, l.kp, sm.sel,
                   direct([=](uint32_t rank, uint32_t page) { store_between<true>(dst + rank, (int64_t)page); }));
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every store of this wave has reached memory
   __syncthreads();
   if (threadIdx.x == 0) {
-    arrived = __hip_atomic_fetch_add(arrivals + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (arrived == gridDim.x - 1) store_between<true>(arrivals + h, 0u);  // ready for the next launch
+    arrived = __hip_atomic_fetch_add(l.arrivals + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (arrived == gridDim.x - 1) store_between<true>(l.arrivals + h, 0u);  // ready for the next launch
   }
   __syncthreads();
   if (arrived != gridDim.x - 1) return;
-  lru_update_block<true>(a, h, gridDim.y, sm);
+  lru_update_block<true>(l.update, h, gridDim.y, sm);
 }
 
 constexpr int kLruTicketWords = 2;  // of the update's workspace; the arrivals follow, a word per head
@@ -459,7 +467,7 @@ bool topk_lru_in_one_launch(const da_decode_step_args &a) {
          a.lru_workspace_bytes >= (int64_t)sizeof(uint32_t) * (kLruTicketWords + a.n_kv_heads);
 }
 
-int launch_topk_lru(const da_decode_step_args &a, hipStream_t s) {
+static int topk_lru_layer(const da_decode_step_args &a, TopkLruLayer &l) {
   const int rep = a.n_q_heads / a.n_kv_heads, K = rep * a.kp;
   DA_REQUIRE(a.n_pages >= 0 && a.kp <= a.n_pages, "da_decode_step: kp %d exceeds the %lld pages of a row", a.kp,
              (long long)a.n_pages);
@@ -469,22 +477,44 @@ int launch_topk_lru(const da_decode_step_args &a, hipStream_t s) {
   DA_REQUIRE(a.k_cand <= a.n_slots && a.k_cand <= kSelMaxK, "da_decode_step: %d candidates of %d slots (at most %d)",
              a.k_cand, a.n_slots, kSelMaxK);
   if (a.n_kv_heads > 65535) return fail(DA_ENOTSUP, "da_decode_step: head count out of range");
-  const TopkRowsArgs r = {a.scores, rep, (int)a.n_pages, a.kp};
-  LruCandidateArgs cand = {};
-  cand.access_time = a.access_time;
-  cand.time_head_stride = a.n_slots;
-  cand.n_slots = a.n_slots;
-  cand.k_cand = a.k_cand;
-  cand.out = a.candidates;
-  cand.step = a.step;
-  cand.n_heads = a.n_kv_heads;
-  const LruArgs<int64_t, int64_t, float> u = {
-      a.idx, K, K, a.n_pages, a.n_slots, a.step, 1, a.access_time, a.n_slots, a.d2h, a.n_pages, a.h2d, a.n_slots,
-      a.hit_mask, a.miss_page, a.miss_slot, a.miss_count, a.slot_epoch, (int32_t *)a.lru_workspace, 0, a.candidates,
-      a.k_cand};
-  hipLaunchKernelGGL(topk_lru_update_kernel, dim3(rep + 1, a.n_kv_heads), dim3(kSelThreads), 0, s, r, cand, u,
-                     (uint32_t *)a.lru_workspace + kLruTicketWords);
+  l.scores = a.scores;
+  l.n_rows = rep;
+  l.n_pages = (int)a.n_pages;
+  l.kp = a.kp;
+  l.cand = {};
+  l.cand.access_time = a.access_time;
+  l.cand.time_head_stride = a.n_slots;
+  l.cand.n_slots = a.n_slots;
+  l.cand.k_cand = a.k_cand;
+  l.cand.out = a.candidates;
+  l.cand.step = a.step;
+  l.cand.n_heads = a.n_kv_heads;
+  l.update = {a.idx, K, K, a.n_pages, a.n_slots, a.step, 1, a.access_time, a.n_slots, a.d2h, a.n_pages, a.h2d,
+              a.n_slots, a.hit_mask, a.miss_page, a.miss_slot, a.miss_count, a.slot_epoch, (int32_t *)a.lru_workspace,
+              0, a.candidates, a.k_cand};
+  l.arrivals = (uint32_t *)a.lru_workspace + kLruTicketWords;
+  return DA_OK;
+}
+
+template <int kLayers>
+static int launch_topk_lru_batch(const da_decode_step_args *a, int n, hipStream_t s) {
+  TopkLruBatch<kLayers> batch;
+  for (int i = 0; i < n; ++i) {
+    const int rc = topk_lru_layer(a[i], batch.layer[i]);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(topk_lru_update_kernel<kLayers>,
+                     dim3(a->n_q_heads / a->n_kv_heads + 1, a->n_kv_heads, n), dim3(kSelThreads), 0, s, batch);
   return launch_status("da_decode_step(selection)");
+}
+
+int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s) {
+  if (n == 1) return launch_topk_lru_batch<1>(a, 1, s);
+  for (int i = 0; i < n; i += kStepBatch) {
+    const int rc = launch_topk_lru_batch<kStepBatch>(a + i, n - i < kStepBatch ? n - i : kStepBatch, s);
+    if (rc) return rc;
+  }
+  return DA_OK;
 }
 
 }  // namespace da

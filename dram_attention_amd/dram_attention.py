@@ -540,7 +540,16 @@ class DRAMAttention(torch.nn.Module):
     def _step_in_one_call(self, xq, xk, xv, start_pos):
         """select_ and attend_ as one native call (da_decode_step) where everything has the
         layout a layer is built with; None where anything differs, and the two methods, which
-        take or refuse it, do the step.  The same launches on the same operands."""
+        take or refuse it, do the step.  The same results on the same operands."""
+        step = self._step_args(xq, xk, xv, start_pos)
+        if step is None:
+            return None
+        args, out = step
+        _lib.check(_lib.load().da_decode_step(args, len(args), _lib.stream_ptr(xq.device)), "da_decode_step")
+        return out
+
+    def _step_args(self, xq, xk, xv, start_pos):
+        """(argument block of da_decode_step, output) of a step that one native call can do, else None."""
         lru = self.lru_cache
         if (type(lru) is not LRUCache or self.attention_scope != "resident" or not self.overlap_page_stream
                 or not self.attend_on_page_stream):
@@ -611,8 +620,7 @@ class DRAMAttention(torch.nn.Module):
             Hq, H, D, _lib.dtype_code(dtype), page, kp, N, scratch.candidates.shape[1],
             SCORE_FLAGS[selector.bounds_are_ordered], max(1, min(self.stream_blocks // H, total)),
             1.0 / math.sqrt(D), self.link_gbps, self.block_gbps, 0)
-        _lib.check(_lib.load().da_decode_step(args, len(args), _lib.stream_ptr(device)), "da_decode_step")
-        return out
+        return args, out
 
     def _steps_by_its_own_methods(self, lru, selector) -> bool:
         """Whether the methods a step is made of are this module's: neither a subclass, nor an

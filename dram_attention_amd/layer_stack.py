@@ -4,18 +4,19 @@ The reference's model walks its layers one after the other on one stream
 (evaluation/dram-attention/model.py:265-274, 305-317); each layer's decode step
 is page scoring, ordered top-k and the LRU update (no host-link traffic), then
 the page stream and attention (bound by the host link).  In an attention-only
-stack the layers' queries do not depend on each other, so the first half of
-layer i+1 can run while layer i's pages are still crossing the host link: the
-link then never waits for a selection.
+stack the layers' queries do not depend on each other, so nothing has to wait for
+another layer.
 
-``AttentionStack.generate`` issues the first halves (and the final merge of each
-layer's attention partials) on a side stream and the page stream + attention
-launches on the caller's stream, tied together by events;
-every layer runs exactly the launches it runs alone, on its own buffers, so the
-results have the same bits as stepping the layers one by one.  All streams have
-the default priority.  The step has no host synchronisation and can be
-captured into one HIP graph per model step (the side stream forks from and
-joins the capturing stream).
+``AttentionStack.generate`` steps layers of one size by one native call: all
+layers' selections, in few launches, then the page streams one behind the other, then
+all merges in a launch (csrc/decode_step.hip has the figures).  Layers that call
+does not take (rows beyond 16384 pages, different sizes, exchanged methods) are stepped
+on two streams: the first halves, and the final merge of each layer's attention
+partials, on a side stream next to the page stream + attention launches on the caller's
+stream, tied together by events.  Either way the results have the bits of stepping the
+layers one by one, on their own buffers.  All streams have the default priority.  The step
+has no host synchronisation and can be captured into one HIP graph per model step (the
+side stream forks from and joins the capturing stream).
 """
 
 from __future__ import annotations
@@ -24,13 +25,13 @@ from typing import List, Sequence
 
 import torch
 
+from . import _lib
 from .dram_attention import DRAMAttention
 
 
 class AttentionStack(torch.nn.Module):
     """``layers``: DRAMAttention modules whose caches are initialised (each with its
-    own page cache); ``pipelined``: overlap layer i's page stream with the
-    selection of the layers after it."""
+    own page cache); ``pipelined``: step the layers together, as above, and not one by one."""
 
     def __init__(self, layers: Sequence[DRAMAttention], pipelined: bool = True):
         super().__init__()
@@ -51,6 +52,9 @@ class AttentionStack(torch.nn.Module):
         if not self.pipelined or n < 2 or not xqs[0].is_cuda:
             return [layer(xq, xk, xv, start_pos=start_pos, stage="generate")
                     for layer, xq, xk, xv in zip(self.layers, xqs, xks, xvs)]
+        outs = self._together(xqs, xks, xvs, start_pos)
+        if outs is not None:
+            return outs
         dev = xqs[0].device
         main = torch.cuda.current_stream(dev)
         if self._side is None:
@@ -85,3 +89,22 @@ class AttentionStack(torch.nn.Module):
                     merge()
         main.wait_stream(side)          # join: every merge has written its output
         return outs
+
+    def _together(self, xqs, xks, xvs, start_pos):
+        """The whole model step as one native call (da_decode_steps), or None where that does not take it:
+        a layer whose own step is none that one call does, layers of different sizes."""
+        layers, device = self.layers, xqs[0].device
+        if (len(set(map(id, layers))) < len(layers) or not all(type(m) is DRAMAttention for m in layers)
+                or any(xq.device != device for xq in xqs)):
+            return None
+        steps = []
+        for m, xq, xk, xv in zip(layers, xqs, xks, xvs):
+            step = m._step_args(xq, xk, xv, start_pos)
+            if step is None:
+                return None
+            steps.append(step)
+        lib, args = _lib.load(), b"".join(args for args, _ in steps)
+        if not lib.da_decode_steps_supported(args, len(steps), len(args)):
+            return None
+        _lib.check(lib.da_decode_steps(args, len(steps), len(args), _lib.stream_ptr(device)), "da_decode_steps")
+        return [out for _, out in steps]

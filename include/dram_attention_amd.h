@@ -539,6 +539,16 @@ typedef struct da_decode_step_args {
 int da_decode_step(const da_decode_step_args *args, size_t args_bytes, void *stream);
 
 /*
+ * A step of each of n_steps layers whose queries do not depend on each other: the results of
+ * da_decode_step on every block, in fewer launches.  The blocks differ in pointers, cache_len, scale,
+ * rates and score flags only, top-k and LRU update are one launch (both said by
+ * da_decode_steps_supported; DA_ENOTSUP before anything is launched otherwise), and no two share a
+ * buffer that a step writes.  `args_bytes` = n_steps * sizeof(da_decode_step_args).
+ */
+int da_decode_steps_supported(const da_decode_step_args *args, int n_steps, size_t args_bytes);
+int da_decode_steps(const da_decode_step_args *args, int n_steps, size_t args_bytes, void *stream);
+
+/*
  * Row-wise parts of the model around the attention layers (evaluation/dram-attention/
  * model.py of the reference), `rows` contiguous rows at a time; every operand 16-byte
  * aligned, rows a multiple of 16 bytes (DA_ENOTSUP otherwise).

@@ -194,3 +194,40 @@ def test_stack_argument_checks_and_short_stacks():
         stack.generate([q.to(DEV)], [k.to(DEV)], [], w.prompt_tokens)
     (out,) = stack.generate([q.to(DEV)], [k.to(DEV)], [v.to(DEV)], w.prompt_tokens)
     check_step(layers[0], oracles[0], q, k, v, w.prompt_tokens, out, 0, 2e-2, 1e-2)
+
+
+@pytest.mark.parametrize("n,dtype,sizes", [
+    (2, torch.float32, None), (8, torch.bfloat16, None), (9, torch.float16, None),   # a batch of launches, one more
+    (3, torch.bfloat16, (200, 200, 216)),                                            # layers of different sizes
+])
+def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, sizes):
+    """Bits of the serial order for every layer, its caches and what its next step starts from."""
+    from dram_attention_amd import AttentionStack, DRAMAttention
+
+    Hq, Hkv, D, S = 8, 2, 64, 1500
+    g = torch.Generator(device=DEV).manual_seed(n)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    stacks = []
+    prompts = [(rand(1, S, Hkv, D), rand(1, S, Hkv, D)) for _ in range(n)]
+    for pipelined in (True, False):
+        layers = [DRAMAttention(6, 480, local, 16, 96, Hkv, D, device=DEV, dtype=dtype)
+                  for local in sizes or [200] * n]
+        for m, (k, v) in zip(layers, prompts):
+            m.init_cache(k, v)
+        stacks.append(AttentionStack(layers, pipelined=pipelined))
+    together = []
+    inner = stacks[0]._together
+    stacks[0]._together = lambda *a: together.append(inner(*a)) or together[-1]
+    for t in range(4):
+        xqs, xks, xvs = ([rand(1, 1, h, D) for _ in range(n)] for h in (Hq, Hkv, Hkv))
+        pos = S + t if t % 2 else torch.tensor([S + t], dtype=torch.int32, device=DEV)
+        got, want = (s.generate(xqs, xks, xvs, pos) for s in stacks)
+        assert (together[t] is None) == (sizes is not None)
+        for a, b, x, y in zip(stacks[0].layers, stacks[1].layers, got, want):
+            assert same(x, y) and same(a.cache_k, b.cache_k) and same(a.cache_v, b.cache_v)
+            for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
+                         "hbm_page_to_dram_page_mapping", "current_step"):
+                assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
