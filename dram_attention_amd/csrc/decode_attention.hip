@@ -306,69 +306,38 @@ static int launch_attention(const AttnArgs &a, int dtype, int phase, int n_kv_he
   return DA_OK;
 }
 
-// The merges behind launches of DA_PHASE_STREAM | DA_PHASE_FIRST that da_decode_attention_paged has
-// issued, and checked, for n steps of the same sizes.
-int launch_merge_layers(const da_decode_step_args *steps, int n, hipStream_t s) {
-  const da_decode_step_args &g = *steps;
-  const int D = g.head_dim, rep = g.n_q_heads / g.n_kv_heads;
-  const ChunkPlan p = plan_chunks(g.n_kv_heads, lanes_of(D, g.dtype), (int64_t)g.n_slots * g.page_size, g.cache_rows,
-                                  (int64_t)rep * g.kp * g.page_size);
-  AttnArgs a = {};
-  a.rep = rep;
-  a.n_q_heads = g.n_q_heads;
-  a.c_capacity = g.cache_rows;
-  a.new_k = (const char *)g.new_k;     // (every step has a new token)
-  a.chunk = p.chunk;
-  a.n_pchunks = p.n_p;
-  a.n_lchunks = p.n_l;
-  a.n_tchunks = p.n_t;
-  a.pre_chunk = p.pre_chunk();
-  a.gather_chunk0 = p.gather_chunk0();
-  a.gather_blocks = g.gather_blocks;
-  for (int first = 0; first < n; first += kStepBatch) {
-    const int count = n - first < kStepBatch ? n - first : kStepBatch;
-    MergeBatch batch;
-    for (int i = 0; i < count; ++i) {
-      const da_decode_step_args &l = steps[first + i];
-      float *acc = (float *)l.workspace;
-      batch.layer[i] = {acc + (size_t)p.total() * g.n_q_heads * D, acc, l.miss_count, l.cache_len_dev, l.cache_len,
-                        (char *)l.out};
-    }
-    const dim3 grid(g.n_q_heads, count);
-#define DA_MERGE(T) \
-  hipLaunchKernelGGL(decode_attention_merge_layers_kernel<T>, grid, dim3(kMergeThreads), 0, s, a, batch, D, D)
-    if (g.dtype == DA_BF16) DA_MERGE(BF16);
-    else if (g.dtype == DA_F16) DA_MERGE(F16);
-    else DA_MERGE(F32);
-#undef DA_MERGE
-    const int rc = launch_status("da_decode_steps(merge)");
-    if (rc) return rc;
+// The final merges of n <= kStepBatch layers of the same sizes, behind launches of DA_PHASE_STREAM | DA_PHASE_FIRST.
+int launch_merge_layers(const PreparedAttention *p, const da_decode_step_args *steps, int n, hipStream_t s) {
+  MergeBatch batch;
+  for (int i = 0; i < n; ++i) {
+    const AttnArgs &a = p[i].a;
+    batch.layer[i] = {a.part_ml, a.part_acc, a.miss_count, a.c_len_dev, a.c_len, (char *)steps[i].out};
   }
-  return DA_OK;
+  const dim3 grid(p->a.n_q_heads, n);
+  const int D = p->head_dim;
+#define DA_MERGE(T) \
+  hipLaunchKernelGGL(decode_attention_merge_layers_kernel<T>, grid, dim3(kMergeThreads), 0, s, p->a, batch, D, D)
+  if (p->dtype == DA_BF16) DA_MERGE(BF16);
+  else if (p->dtype == DA_F16) DA_MERGE(F16);
+  else DA_MERGE(F32);
+#undef DA_MERGE
+  return launch_status("da_decode_steps(merge)");
 }
 
-}  // namespace da
-
-extern "C" size_t da_decode_attention_workspace_bytes(int n_q_heads, int n_kv_heads,
-                                                      int head_dim, int dtype, int64_t p_len,
-                                                      int64_t c_capacity, int64_t miss_tokens) {
-  using namespace da;
-  if (n_q_heads <= 0 || n_kv_heads <= 0 || p_len < 0 || c_capacity < 0 || miss_tokens < 0)
-    return 0;
-  const int lanes = lanes_of(head_dim, dtype);
-  if (!lanes) return 0;
-  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
-  return attn_workspace_bytes(n_q_heads, head_dim, p.total()) + 16;
-}
-
-extern "C" int da_decode_attention_paged(
-    const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int dtype,
-    const void *pk, const void *pv, int64_t p_tok_stride, int64_t p_head_stride, int64_t p_len,
-    void *ck, void *cv, int64_t c_tok_stride, int64_t c_head_stride, int64_t c_capacity,
-    int64_t c_len, const int32_t *c_len_dev, const void *new_k, const void *new_v,
-    int64_t new_head_stride, float scale, void *out, int64_t out_head_stride, float *lse_out,
-    void *workspace, size_t workspace_bytes, const da_paged_overlap *overlap, void *stream) {
-  using namespace da;
+// Checks the operands of a call and fills in what its launches take.
+int prepare_attention(const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int dtype, const void *pk,
+    const void *pv, int64_t p_tok_stride, int64_t p_head_stride, int64_t p_len, void *ck, void *cv, int64_t
+    c_tok_stride, int64_t c_head_stride, int64_t c_capacity, int64_t c_len, const int32_t *c_len_dev, const void
+    *new_k, const void *new_v, int64_t new_head_stride, float scale, void *out, void *workspace, size_t
+    workspace_bytes, const da_paged_overlap *overlap, PreparedAttention &prepared) {
+  prepared = {};
+  AttnArgs &a = prepared.a;
+  GatherAttendArgs &g = prepared.g;
+  int &phase = prepared.phase;
+  float &link_gbps = prepared.link_gbps, &block_gbps = prepared.block_gbps;
+  prepared.n_kv_heads = n_kv_heads;
+  prepared.head_dim = head_dim;
+  prepared.dtype = dtype;
   DA_REQUIRE(n_q_heads > 0 && n_kv_heads > 0 && n_q_heads % n_kv_heads == 0,
              "da_decode_attention: %d query heads do not split over %d kv heads", n_q_heads,
              n_kv_heads);
@@ -402,7 +371,6 @@ extern "C" int da_decode_attention_paged(
              "da_decode_attention: rows must be 16-byte aligned");
   if (n_kv_heads > 65535) return fail(DA_ENOTSUP, "da_decode_attention: too many kv heads");
 
-  AttnArgs a = {};
   a.q = (const char *)q;
   a.q_head_stride = q_head_stride;
   a.rep = n_q_heads / n_kv_heads;
@@ -423,7 +391,7 @@ extern "C" int da_decode_attention_paged(
   a.new_head_stride = new_head_stride;
   a.scale_log2 = scale * kLog2e;
   a.n_q_heads = n_q_heads;
-  int phase = 3;
+  phase = 3;
   int64_t miss_tokens = 0;
   if (overlap) {
     DA_REQUIRE(overlap->page_size > 0 && p_len % overlap->page_size == 0,
@@ -474,10 +442,7 @@ extern "C" int da_decode_attention_paged(
              "da_decode_attention: workspace must be 16-byte aligned");
   a.part_acc = (float *)workspace;
   a.part_ml = a.part_acc + (size_t)p.total() * n_q_heads * head_dim;
-  hipStream_t s = (hipStream_t)stream;
   if (p.n_p + p.n_l == 0) return fail(DA_EINVAL, "da_decode_attention: no key/value rows at all");
-  GatherAttendArgs g = {};
-  float link_gbps = 0.f, block_gbps = 0.f;
   if (phase & DA_PHASE_STREAM) {
     DA_REQUIRE(overlap->link_gbps >= 0.f && overlap->block_gbps >= 0.f,
                "da_decode_attention: negative rate in the overlap description");
@@ -518,16 +483,48 @@ extern "C" int da_decode_attention_paged(
     g.part_ml = a.part_ml;
     g.chunk0 = a.gather_chunk0;
   }
+  prepared.lanes = lanes;
+  return DA_OK;
+}
+
+}  // namespace da
+
+extern "C" size_t da_decode_attention_workspace_bytes(int n_q_heads, int n_kv_heads,
+                                                      int head_dim, int dtype, int64_t p_len,
+                                                      int64_t c_capacity, int64_t miss_tokens) {
+  using namespace da;
+  if (n_q_heads <= 0 || n_kv_heads <= 0 || p_len < 0 || c_capacity < 0 || miss_tokens < 0)
+    return 0;
+  const int lanes = lanes_of(head_dim, dtype);
+  if (!lanes) return 0;
+  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
+  return attn_workspace_bytes(n_q_heads, head_dim, p.total()) + 16;
+}
+
+extern "C" int da_decode_attention_paged(const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int dtype,
+    const void *pk, const void *pv, int64_t p_tok_stride, int64_t p_head_stride, int64_t p_len,
+    void *ck, void *cv, int64_t c_tok_stride, int64_t c_head_stride, int64_t c_capacity,
+    int64_t c_len, const int32_t *c_len_dev, const void *new_k, const void *new_v,
+    int64_t new_head_stride, float scale, void *out, int64_t out_head_stride, float *lse_out,
+    void *workspace, size_t workspace_bytes, const da_paged_overlap *overlap, void *stream) {
+  using namespace da;
+  PreparedAttention p;
+  const int rc = prepare_attention(q, q_head_stride, n_q_heads, n_kv_heads, head_dim, dtype, pk, pv, p_tok_stride,
+                                   p_head_stride, p_len, ck, cv, c_tok_stride, c_head_stride, c_capacity, c_len,
+                                   c_len_dev, new_k, new_v, new_head_stride, scale, out, workspace, workspace_bytes,
+                                   overlap, p);
+  if (rc) return rc;
+  hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
     case DA_F32:
-      return launch_attention<F32>(a, dtype, phase, n_kv_heads, lanes, head_dim, out,
-                                   out_head_stride, lse_out, &g, link_gbps, block_gbps, s);
+      return launch_attention<F32>(p.a, dtype, p.phase, n_kv_heads, p.lanes, head_dim, out, out_head_stride,
+                                   lse_out, &p.g, p.link_gbps, p.block_gbps, s);
     case DA_F16:
-      return launch_attention<F16>(a, dtype, phase, n_kv_heads, lanes, head_dim, out,
-                                   out_head_stride, lse_out, &g, link_gbps, block_gbps, s);
+      return launch_attention<F16>(p.a, dtype, p.phase, n_kv_heads, p.lanes, head_dim, out, out_head_stride,
+                                   lse_out, &p.g, p.link_gbps, p.block_gbps, s);
     default:
-      return launch_attention<BF16>(a, dtype, phase, n_kv_heads, lanes, head_dim, out,
-                                    out_head_stride, lse_out, &g, link_gbps, block_gbps, s);
+      return launch_attention<BF16>(p.a, dtype, p.phase, n_kv_heads, p.lanes, head_dim, out, out_head_stride,
+                                    lse_out, &p.g, p.link_gbps, p.block_gbps, s);
   }
 }
 

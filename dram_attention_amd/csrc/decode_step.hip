@@ -10,13 +10,14 @@
 // launched from Python (674 before).
 //
 // Several layers whose queries do not depend on each other (da_decode_steps): all layers' scores,
-// all selections and updates in a launch, the page streams one behind the other, all merges in a
-// launch.  The stream of a layer waits for the host link and everything else is a chain of short
+// all selections and updates in a launch, all page streams in a launch (stream_attention.hip), all
+// merges in a launch, eight layers at a time.  The stream of a layer waits for the host link and everything else is a chain of short
 // launches; a second queue that takes the chains of the other layers beside the stream hides them,
 // but each hand-over between queues of a graph idles 9 us and a selection beside a stream takes
 // three times as long and slows it.  us a model step in one graph, two queues / this: 4 layers of
-// 64K tokens, 32/8 heads 363 / 332; 4 of 128K 612 / 591; 3 of 250K 391 / 376; 5 of 12K, 28/4 217 / 169;
-// 4 of 20K, 16/16, D 64 153 / 107; 2 of 8K, 16/4, D 64 87 / 50.
+// 64K tokens, 32/8 heads 363 / 309; 4 of 128K 612 / 570; 3 of 250K 391 / 361; 5 of 12K, 28/4 217 / 130;
+// 4 of 20K, 16/16, D 64 153 / 96; 2 of 8K, 16/4, D 64 87 / 48.
+#include "page_stream.hpp"
 #include "topk_rows.hpp"
 
 namespace da {
@@ -48,9 +49,8 @@ static int select_and_update(const da_decode_step_args &a, void *stream) {
                        a.lru_workspace_bytes, stream);
 }
 
-static int stream_and_attend(const da_decode_step_args &a, int phase, void *stream) {
-  const int H = a.n_kv_heads, D = a.head_dim;
-  const int64_t e = elem_size(a.dtype), page = (int64_t)a.page_size * 2 * D;
+static da_paged_overlap overlap_of(const da_decode_step_args &a, int phase) {
+  const int64_t e = elem_size(a.dtype), page = (int64_t)a.page_size * 2 * a.head_dim;
   da_paged_overlap o = {};
   o.page_size = a.page_size;
   o.phase = phase;
@@ -59,7 +59,7 @@ static int stream_and_attend(const da_decode_step_args &a, int phase, void *stre
   o.epoch = a.step;
   o.miss_slot = a.miss_slot;
   o.miss_count = a.miss_count;
-  o.miss_capacity = a.n_q_heads / H * a.kp;
+  o.miss_capacity = a.n_q_heads / a.n_kv_heads * a.kp;
   o.gather_blocks = a.gather_blocks;
   o.dram = a.dram;
   o.dram_head_stride_bytes = a.n_pages * page * e;
@@ -70,11 +70,29 @@ static int stream_and_attend(const da_decode_step_args &a, int phase, void *stre
   o.miss_page = a.miss_page;
   o.link_gbps = a.link_gbps;
   o.block_gbps = a.block_gbps;
+  return o;
+}
+
+static int stream_and_attend(const da_decode_step_args &a, int phase, void *stream) {
+  const int H = a.n_kv_heads, D = a.head_dim;
+  const da_paged_overlap o = overlap_of(a, phase);
   const char *hbm = (const char *)a.hbm;
   return da_decode_attention_paged(
-      a.q, a.q_head_stride, a.n_q_heads, H, D, a.dtype, hbm, hbm + D * e, 2 * D, a.n_slots * page,
-      (int64_t)a.n_slots * a.page_size, a.cache_k, a.cache_v, (int64_t)H * D, D, a.cache_rows, a.cache_len,
-      a.cache_len_dev, a.new_k, a.new_v, D, a.scale, a.out, D, nullptr, a.workspace, a.workspace_bytes, &o, stream);
+      a.q, a.q_head_stride, a.n_q_heads, H, D, a.dtype, hbm, hbm + D * elem_size(a.dtype), 2 * D,
+      (int64_t)a.n_slots * a.page_size * 2 * D, (int64_t)a.n_slots * a.page_size, a.cache_k, a.cache_v, (int64_t)H * D,
+      D, a.cache_rows, a.cache_len, a.cache_len_dev, a.new_k, a.new_v, D, a.scale, a.out, D, nullptr, a.workspace,
+      a.workspace_bytes, &o, stream);
+}
+
+static int prepare_step(const da_decode_step_args &a, PreparedAttention &p) {
+  const int H = a.n_kv_heads, D = a.head_dim;
+  const da_paged_overlap o = overlap_of(a, DA_PHASE_STREAM | DA_PHASE_FIRST);
+  const char *hbm = (const char *)a.hbm;
+  return prepare_attention(
+      a.q, a.q_head_stride, a.n_q_heads, H, D, a.dtype, hbm, hbm + D * elem_size(a.dtype), 2 * D,
+      (int64_t)a.n_slots * a.page_size * 2 * D, (int64_t)a.n_slots * a.page_size, a.cache_k, a.cache_v, (int64_t)H * D,
+      D, a.cache_rows, a.cache_len, a.cache_len_dev, a.new_k, a.new_v, D, a.scale, a.out, a.workspace,
+      a.workspace_bytes, &o, p);
 }
 
 // Whether two steps differ in nothing but their operands' places.
@@ -114,15 +132,30 @@ extern "C" int da_decode_steps(const da_decode_step_args *a, int n_steps, size_t
              "da_decode_steps: argument blocks of %zu bytes, expected %d of %zu", args_bytes, n_steps, sizeof(*a));
   if (!da_decode_steps_supported(a, n_steps, args_bytes))
     return fail(DA_ENOTSUP, "da_decode_steps: layers of the same sizes, whose selection and update are one launch");
-  for (int i = 0; i < n_steps; ++i) {
-    const int rc = scores_of(a[i], stream);
+  PreparedAttention p[kStepBatch];
+  for (int i = 0; i < n_steps; ++i) {     // (every block is looked at before the first launch)
+    const int rc = prepare_step(a[i], p[0]);
     if (rc) return rc;
   }
-  int rc = launch_topk_lru(a, n_steps, (hipStream_t)stream);
-  if (rc) return rc;
-  for (int i = 0; i < n_steps; ++i) {
-    rc = stream_and_attend(a[i], DA_PHASE_STREAM | DA_PHASE_FIRST, stream);
+  hipStream_t s = (hipStream_t)stream;
+  for (; n_steps > 0; a += kStepBatch, n_steps -= kStepBatch) {
+    const int n = n_steps < kStepBatch ? n_steps : kStepBatch;
+    int rc = DA_OK;
+    for (int i = 0; i < n && rc == DA_OK; ++i) {
+      rc = prepare_step(a[i], p[i]);
+      if (rc == DA_OK) rc = scores_of(a[i], stream);
+    }
+    if (rc) return rc;
+    rc = launch_topk_lru(a, n, s);
+    if (rc) return rc;
+    if (stream_layers_supported(p[0])) {
+      rc = launch_stream_layers(p, n, s);
+    } else {
+      for (int i = 0; i < n && rc == DA_OK; ++i) rc = stream_and_attend(a[i], DA_PHASE_STREAM | DA_PHASE_FIRST, stream);
+    }
+    if (rc) return rc;
+    rc = launch_merge_layers(p, a, n, s);
     if (rc) return rc;
   }
-  return launch_merge_layers(a, n_steps, (hipStream_t)stream);
+  return DA_OK;
 }

@@ -509,12 +509,7 @@ static int launch_topk_lru_batch(const da_decode_step_args *a, int n, hipStream_
 }
 
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s) {
-  if (n == 1) return launch_topk_lru_batch<1>(a, 1, s);
-  for (int i = 0; i < n; i += kStepBatch) {
-    const int rc = launch_topk_lru_batch<kStepBatch>(a + i, n - i < kStepBatch ? n - i : kStepBatch, s);
-    if (rc) return rc;
-  }
-  return DA_OK;
+  return n == 1 ? launch_topk_lru_batch<1>(a, 1, s) : launch_topk_lru_batch<kStepBatch>(a, n, s);
 }
 
 }  // namespace da

@@ -218,4 +218,24 @@ int launch_stream_attend(const AttnArgs &a, const GatherAttendArgs &g, int dtype
                          int n_chunks, int n_kv_heads, float link_gbps, float block_gbps,
                          hipStream_t s);
 
+// What the launches of one attention call take (decode_attention.hip).
+struct PreparedAttention {
+  AttnArgs a;
+  GatherAttendArgs g;
+  int n_kv_heads, head_dim, dtype, lanes, phase;
+  float link_gbps, block_gbps;
+};
+int prepare_attention(const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int
+                      dtype, const void *pk, const void *pv, int64_t p_tok_stride, int64_t p_head_stride, int64_t
+                      p_len, void *ck, void *cv, int64_t c_tok_stride, int64_t c_head_stride, int64_t c_capacity,
+                      int64_t c_len, const int32_t *c_len_dev, const void *new_k, const void *new_v, int64_t
+                      new_head_stride, float scale, void *out, void *workspace, size_t workspace_bytes, const
+                      da_paged_overlap *overlap, PreparedAttention &prepared);
+
+// The same of n <= kStepBatch layers' steps (DA_PHASE_STREAM | DA_PHASE_FIRST, same sizes) in one launch, where
+// the matrix-core form of the pass takes them, and their final merges in another.
+bool stream_layers_supported(const PreparedAttention &p);
+int launch_stream_layers(const PreparedAttention *p, int n, hipStream_t s);
+int launch_merge_layers(const PreparedAttention *p, const da_decode_step_args *steps, int n, hipStream_t s);
+
 }  // namespace da

@@ -7,6 +7,7 @@
 
 #include "attention_mfma.hpp"
 #include "page_stream.hpp"
+#include "topk_rows.hpp"
 
 namespace da {
 
@@ -47,6 +48,11 @@ struct StreamRates {
   float link_bytes_per_us, block_bytes_per_us;
 };
 constexpr float kDefaultLinkGBps = 54.f, kDefaultBlockGBps = 30.f;
+// (1 GB/s = 1000 bytes per microsecond; 0 = the rates of the box this was tuned on)
+static StreamRates stream_rates(float link_gbps, float block_gbps) {
+  return {(link_gbps > 0.f ? link_gbps : kDefaultLinkGBps) * 1000.f,
+          (block_gbps > 0.f ? block_gbps : kDefaultBlockGBps) * 1000.f};
+}
 __device__ __forceinline__ bool stream_hides_few_blocks(int64_t stream_bytes, int64_t chunk_bytes,
                                                         int n_chunks, int n_core,
                                                         const StreamRates &r) {
@@ -109,6 +115,69 @@ decode_stream_attend_tile_kernel(const AttnArgs a, const GatherAttendArgs g, con
   }
 }
 
+// The same for several layers whose steps do not depend on each other.  The stream blocks go
+// through the layers one after the other, each on the range it has of a layer's lists when the
+// layer is alone (so the partial results are the same): a block that is done with its range goes
+// on at once, and neither the end of a layer's stream, which waits for its slowest block, nor the start of
+// the next, 7 us until the first page has come over the link, leaves the link idle.
+// Attention: next to a stream that hides it the core blocks walk the chunks of all layers;
+// otherwise they take their chunk of the first layer and the blocks behind them one chunk each.
+// us a model step with a launch per layer / this: 4 layers of 64K tokens, 32/8 heads 332 / 309; 8 of 128K 1167 /
+// 1115; 5 of 12K, 28/4 169 / 130; 3 of 30K, 64/8, fp16 157 / 138; 2 of 8K, 16/4, D 64 50 / 48.
+struct StreamLayers {
+  AttnArgs a[kStepBatch];
+  GatherAttendArgs g[kStepBatch];
+};
+static_assert(sizeof(StreamLayers) <= 3900, "kernel arguments: 4 KiB");
+template <typename T, int kLanes, int kRowsAttn, int kRowsGather>
+__global__ void __launch_bounds__(kAttnThreads)
+decode_stream_attend_layers_kernel(const StreamLayers layers, const int n_layers, const int g_blocks,
+                                   const int n_core, const int n_chunks, const StreamRates rates) {
+  const int n_kv_heads = layers.g[0].n_kv_heads;
+  const int b = blockIdx.x;
+  const int per_head = g_blocks + n_core;
+  const int n_first = per_head * n_kv_heads;
+  if (b < n_first && b % per_head < g_blocks) {
+    for (int i = 0; i < n_layers; ++i) {
+      gather_attend_block<T, kLanes, kRowsGather>(layers.g[i], b / per_head * g_blocks + b % per_head,
+                                                  g_blocks * n_kv_heads);
+      __syncthreads();  // the block's LDS is used again
+    }
+    return;
+  }
+  int64_t missed = 0;
+  for (int i = 0; i < n_layers; ++i)
+    for (int hh = 0; hh < n_kv_heads; ++hh) missed += layers.g[i].miss_count[hh];
+  const bool few = stream_hides_few_blocks(missed * layers.g[0].page_vecs * 16,
+                                           (int64_t)layers.a[0].chunk * kLanes * 16 * 2, n_chunks * n_layers,
+                                           n_core, rates);
+  if (b < n_first) {
+    const int h = b / per_head, first = b % per_head - g_blocks;
+    if (!few) {
+      attention_tile_block<T, kLanes * 8, kRowsAttn>(layers.a[0], first, h);
+      return;
+    }
+    for (int i = 0; i < n_layers; ++i)
+      for (int c = first; c < n_chunks; c += n_core) {
+        attention_tile_block<T, kLanes * 8, kRowsAttn, true>(layers.a[i], c, h);
+        __syncthreads();
+      }
+    return;
+  }
+  if (few) return;
+  // (first layer: the chunks behind the core blocks'; the others: all)
+  int at = b - n_first, i = 0, skip = n_core;
+  const int first_layer = (n_chunks - n_core) * n_kv_heads;
+  if (at >= first_layer) {
+    at -= first_layer;
+    i = 1 + at / (n_chunks * n_kv_heads);
+    at %= n_chunks * n_kv_heads;
+    skip = 0;
+  }
+  const int rest = n_chunks - skip;
+  attention_tile_block<T, kLanes * 8, kRowsAttn>(layers.a[i], skip + at % rest, at / rest);
+}
+
 template <typename T, int kLanes>
 static void launch_stream_attend(AttnArgs a, const GatherAttendArgs &g, int g_blocks, int n_chunks,
                                  int n_kv_heads, const StreamRates &rates, hipStream_t s) {
@@ -163,14 +232,45 @@ static int dispatch_stream_attend(const AttnArgs &a, const GatherAttendArgs &g, 
 int launch_stream_attend(const AttnArgs &a, const GatherAttendArgs &g, int dtype, int lanes,
                          int n_chunks, int n_kv_heads, float link_gbps, float block_gbps,
                          hipStream_t s) {
-  // 1 GB/s = 1000 bytes per microsecond; 0 = the rates of the box this was tuned on
-  const StreamRates rates = {(link_gbps > 0.f ? link_gbps : kDefaultLinkGBps) * 1000.f,
-                             (block_gbps > 0.f ? block_gbps : kDefaultBlockGBps) * 1000.f};
+  const StreamRates rates = stream_rates(link_gbps, block_gbps);
   switch (dtype) {
     case DA_F32: return dispatch_stream_attend<F32>(a, g, lanes, n_chunks, n_kv_heads, rates, s);
     case DA_F16: return dispatch_stream_attend<F16>(a, g, lanes, n_chunks, n_kv_heads, rates, s);
     default: return dispatch_stream_attend<BF16>(a, g, lanes, n_chunks, n_kv_heads, rates, s);
   }
+}
+
+bool stream_layers_supported(const PreparedAttention &p) {
+  return (p.lanes == 8 || p.lanes == 16) &&
+         tile_pass_supported(p.dtype, p.head_dim, p.a.rep, p.a.slot_epoch != nullptr, p.a.page_size);
+}
+
+template <typename T, int kLanes>
+static int launch_layers(const PreparedAttention *p, int n, hipStream_t s) {
+  const int n_kv_heads = p->n_kv_heads, g_blocks = p->a.gather_blocks;
+  const int n_chunks = p->a.n_pchunks + p->a.n_lchunks;
+  const StreamRates rates = stream_rates(p->link_gbps, p->block_gbps);
+  int n_core = 64 / n_kv_heads > 1 ? 64 / n_kv_heads : 1;   // as for one layer
+  if (n_core > n_chunks) n_core = n_chunks;
+  StreamLayers layers;
+  for (int i = 0; i < n; ++i) {
+    layers.a[i] = p[i].a;
+    layers.a[i].chunk_base = 0;
+    layers.g[i] = p[i].g;
+  }
+  const dim3 grid((g_blocks + n_chunks * n) * n_kv_heads, 1, 1);
+  if (p->a.rep > 4)
+    hipLaunchKernelGGL((decode_stream_attend_layers_kernel<T, kLanes, 8, 8>), grid, dim3(kAttnThreads), 0, s, layers, n,
+                       g_blocks, n_core, n_chunks, rates);
+  else
+    hipLaunchKernelGGL((decode_stream_attend_layers_kernel<T, kLanes, 4, 4>), grid, dim3(kAttnThreads), 0, s, layers, n,
+                       g_blocks, n_core, n_chunks, rates);
+  return launch_status("da_decode_steps(page stream + first pass)");
+}
+
+int launch_stream_layers(const PreparedAttention *p, int n, hipStream_t s) {
+  if (p->dtype == DA_BF16) return p->lanes == 16 ? launch_layers<BF16, 16>(p, n, s) : launch_layers<BF16, 8>(p, n, s);
+  return p->lanes == 16 ? launch_layers<F16, 16>(p, n, s) : launch_layers<F16, 8>(p, n, s);
 }
 
 template <typename T, int kLanes>

@@ -66,12 +66,9 @@ __device__ __forceinline__ void lru_candidates_block(const LruCandidateArgs &c, 
 
 // Ordered top-k of every row, the list of least recent slots and the LRU update of a decode step
 // as one launch (lru_update.hip).  Whether a step's sizes allow it, and the launch itself, whose
-// operands it checks: of n layers of the same sizes, kStepBatch to a launch.
+// operands it checks, of n <= kStepBatch layers of the same sizes.
 constexpr int kStepBatch = 8;
 bool topk_lru_in_one_launch(const da_decode_step_args &a);
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s);
-
-// The final merges of n layers' attention partials (decode_attention.hip).
-int launch_merge_layers(const da_decode_step_args *steps, int n, hipStream_t s);
 
 }  // namespace da

@@ -8,8 +8,8 @@ stack the layers' queries do not depend on each other, so nothing has to wait fo
 another layer.
 
 ``AttentionStack.generate`` steps layers of one size by one native call: all
-layers' selections, in few launches, then the page streams one behind the other, then
-all merges in a launch (csrc/decode_step.hip has the figures).  Layers that call
+layers' selections, then all page streams and attention passes in a launch, then all
+merges in a launch, eight layers at a time (csrc/decode_step.hip has the figures).  Layers that call
 does not take (rows beyond 16384 pages, different sizes, exchanged methods) are stepped
 on two streams: the first halves, and the final merge of each layer's attention
 partials, on a side stream next to the page stream + attention launches on the caller's
