@@ -68,7 +68,7 @@ def check_tile_scorer_listing(text: str) -> int:
         (never inside a loop that also holds such a write)."""
     import re
 
-    heads = list(re.finditer(r"^(_ZN2da22page_score_tile_kernel[^\s:]*):", text, re.M))
+    heads = list(re.finditer(r"^(_ZN2da(?:22page_score_tile|29page_score_tile_layers)_kernel[^\s:]*):", text, re.M))
     if not heads:
         raise RuntimeError("no page_score_tile_kernel in the listing of page_score.hip")
     names = [m.group(1) for m in heads]

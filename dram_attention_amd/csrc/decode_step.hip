@@ -9,14 +9,14 @@
 // for the fp32 layer over 8K tokens (85 before), 435 us a token for four 2048-wide model layers
 // launched from Python (674 before).
 //
-// Several layers whose queries do not depend on each other (da_decode_steps): all layers' scores,
-// all selections and updates in a launch, all page streams in a launch (stream_attention.hip), all
-// merges in a launch, eight layers at a time.  The stream of a layer waits for the host link and everything else is a chain of short
+// Several layers whose queries do not depend on each other (da_decode_steps): all scores in a
+// launch, all selections and updates in a launch, all page streams in a launch
+// (stream_attention.hip), all merges in a launch, eight layers at a time.  The stream of a layer waits for the host link and everything else is a chain of short
 // launches; a second queue that takes the chains of the other layers beside the stream hides them,
 // but each hand-over between queues of a graph idles 9 us and a selection beside a stream takes
 // three times as long and slows it.  us a model step in one graph, two queues / this: 4 layers of
-// 64K tokens, 32/8 heads 363 / 309; 4 of 128K 612 / 570; 3 of 250K 391 / 361; 5 of 12K, 28/4 217 / 130;
-// 4 of 20K, 16/16, D 64 153 / 96; 2 of 8K, 16/4, D 64 87 / 48.
+// 64K tokens, 32/8 heads 363 / 302 (309 with a launch of scores per layer); 4 of 128K 612 / 561; 3 of 250K
+// 391 / 356; 5 of 12K, 28/4 217 / 115 (130); 4 of 20K, 16/16, D 64 153 / 89 (96); 2 of 8K, 16/4, D 64 87 / 45 (48).
 #include "page_stream.hpp"
 #include "topk_rows.hpp"
 
@@ -36,8 +36,11 @@ static int scores_of(const da_decode_step_args &a, void *stream) {
                        stream);
 }
 
+// (Rows of more than 4096 pages keep the two launches: their steps stream for so long that the caller's
+// time is hidden, and on the GPU the hand-over is 0.4 us slower there than a launch: 128K tokens 160.8 /
+// 161.5 us; 3064 pages 81.2 / 81.0; 513 pages 32.5 / 31.6.)
 static int select_and_update(const da_decode_step_args &a, void *stream) {
-  if (topk_lru_in_one_launch(a)) return launch_topk_lru(&a, 1, (hipStream_t)stream);
+  if (a.n_pages <= 4096 && topk_lru_in_one_launch(a)) return launch_topk_lru(&a, 1, (hipStream_t)stream);
   const int H = a.n_kv_heads, rep = a.n_q_heads / H, K = rep * a.kp;
   const int rc = da_topk_pages_lru(a.scores, (int64_t)H * a.n_pages, a.n_pages, rep, rep, H, a.n_pages, a.kp, a.idx, K,
                                    K, a.kp, DA_I64, a.access_time, a.n_slots, DA_TIME_F32, a.n_slots, a.k_cand,
@@ -141,10 +144,11 @@ extern "C" int da_decode_steps(const da_decode_step_args *a, int n_steps, size_t
   for (; n_steps > 0; a += kStepBatch, n_steps -= kStepBatch) {
     const int n = n_steps < kStepBatch ? n_steps : kStepBatch;
     int rc = DA_OK;
-    for (int i = 0; i < n && rc == DA_OK; ++i) {
-      rc = prepare_step(a[i], p[i]);
-      if (rc == DA_OK) rc = scores_of(a[i], stream);
-    }
+    for (int i = 0; i < n && rc == DA_OK; ++i) rc = prepare_step(a[i], p[i]);
+    if (rc) return rc;
+    bool scored = false;
+    rc = launch_score_layers(a, n, &scored, s);
+    for (int i = 0; i < n && rc == DA_OK && !scored; ++i) rc = scores_of(a[i], stream);
     if (rc) return rc;
     rc = launch_topk_lru(a, n, s);
     if (rc) return rc;

@@ -418,7 +418,7 @@ static void launch_lru_time(int time_type, dim3 grid, hipStream_t s, const void 
 // from there (a few KB per head), which takes almost as long as the launch of the update that it
 // saves; the caller, who has one launch less to issue, gains more.  A step of the fp32 layer over
 // 8K tokens 32.5 -> 31.6 us (a host thread's part of it 36 -> 33), a token of four 2048-wide layers
-// launched from Python 344 -> 331 us; steps that stream for 60 us and more are as they were.
+// launched from Python 344 -> 331 us; steps that stream for 60 us and more gain nothing (decode_step.hip).
 struct TopkLruLayer {
   const float *scores;  // (rows, heads, pages)
   int n_rows, n_pages, kp;

@@ -67,11 +67,11 @@ __device__ __forceinline__ float slice_bound<F16>(const float *q, const float *m
 }
 
 template <typename T, int kLanes, int kRows, int kUnroll, typename OutT>
-__global__ void __launch_bounds__(256)
-page_score_vec_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t q_head_stride,
-                      const char *__restrict__ mm, int n_rows, int64_t n_pages,
-                      OutT *__restrict__ out, int64_t out_row_stride, int64_t out_head_stride,
-                      int round_out, int rounds) {
+__device__ __forceinline__ void page_score_vec_block(const char *__restrict__ q, int64_t q_row_stride,
+                                                     int64_t q_head_stride, const char *__restrict__ mm, int n_rows,
+                                                     int64_t n_pages, OutT *__restrict__ out, int64_t out_row_stride,
+                                                     int64_t out_head_stride, int round_out, int rounds,
+                                                     const int row0) {
   constexpr int V = T::kVec;
   constexpr int kGroups = 64 / kLanes;  // pages per wave step
   constexpr int kRowBytes = kLanes * 16;
@@ -80,7 +80,6 @@ page_score_vec_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t 
   const int c = lane % kLanes;
   const int g = lane / kLanes;
   const int h = blockIdx.y;
-  const int row0 = blockIdx.z * kRows;
 
   float qf[kRows][V];
 #pragma unroll
@@ -131,6 +130,27 @@ page_score_vec_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t 
     }
   }
   }  // rounds
+}
+
+template <typename T, int kLanes, int kRows, int kUnroll, typename OutT>
+__global__ void __launch_bounds__(256)
+page_score_vec_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t q_head_stride,
+                      const char *__restrict__ mm, int n_rows, int64_t n_pages,
+                      OutT *__restrict__ out, int64_t out_row_stride, int64_t out_head_stride,
+                      int round_out, int rounds) {
+  page_score_vec_block<T, kLanes, kRows, kUnroll, OutT>(q, q_row_stride, q_head_stride, mm, n_rows, n_pages, out,
+                                                        out_row_stride, out_head_stride, round_out, rounds,
+                                                        blockIdx.z * kRows);
+}
+
+// Several layers of the same sizes (blockIdx.z), up to kRows query rows each.
+template <typename T, int kLanes, int kRows>
+__global__ void __launch_bounds__(256)
+page_score_vec_layers_kernel(const ScoreLayers l, int64_t q_row_stride, int64_t q_head_stride, int n_rows,
+                             int64_t n_pages, int64_t out_row_stride, int64_t out_head_stride, int round_out) {
+  const int i = blockIdx.z;
+  page_score_vec_block<T, kLanes, kRows, 2, float>(l.q[i], q_row_stride, q_head_stride, l.mm[i], n_rows, n_pages,
+                                                   l.out[i], out_row_stride, out_head_stride, round_out, 1, 0);
 }
 
 // Generic path: any head_dim, any strides.  One wave per page, lanes stride
@@ -262,6 +282,65 @@ static int dispatch_out(const void *q, int64_t qrs, int64_t qhs, const void *mm,
   typedef typename Storage<T>::type O;
   return launch_page_score<T, O>(q, qrs, qhs, mm, mhs, mps, mrs, n_rows, n_heads, n_pages,
                                  head_dim, (O *)out, ors, ohs, round_out, ordered, s);
+}
+
+template <typename T, int kLanes>
+static void launch_vec_layers(const ScoreLayers &l, int n, const da_decode_step_args &a, hipStream_t s) {
+  const int H = a.n_kv_heads, rep = a.n_q_heads / H;
+  const int64_t P = a.n_pages, hs = a.q_head_stride;
+  const dim3 grid((unsigned)ceil_div(P, 4 * (64 / kLanes) * 2), H, n);
+  const int round_out = a.dtype == DA_F32 ? 0 : a.score_flags & DA_SCORE_ROUND;
+  if (rep <= 4)
+    hipLaunchKernelGGL((page_score_vec_layers_kernel<T, kLanes, 4>), grid, dim3(256), 0, s, l, hs, hs * rep, rep, P,
+                       H * P, P, round_out);
+  else
+    hipLaunchKernelGGL((page_score_vec_layers_kernel<T, kLanes, 8>), grid, dim3(256), 0, s, l, hs, hs * rep, rep, P,
+                       H * P, P, round_out);
+}
+
+// The scores of n <= kStepBatch layers of the same sizes as one launch where every layer takes the same
+// kernel and one workgroup all its query rows; *done says whether.  Same kernels' bodies, same bits.
+int launch_score_layers(const da_decode_step_args *a, int n, bool *done, hipStream_t s) {
+  *done = false;
+  const int H = a->n_kv_heads, D = a->head_dim, rep = a->n_q_heads / H;
+  const int lanes = D * elem_size(a->dtype) / 16;
+  const int64_t P = a->n_pages, hs = a->q_head_stride;
+  if (n < 2 || rep > 8 || (D != 64 && D != 128) || hs % 8 || H > 65535 || P < 1) return DA_OK;
+  ScoreLayers l = {};
+  for (int i = 0; i < n; ++i) {
+    if (!a[i].q || !a[i].minmax || !a[i].scores || (uintptr_t)a[i].q % 16 || (uintptr_t)a[i].minmax % 16 ||
+        a[i].q_head_stride != hs || a[i].score_flags != a->score_flags)
+      return DA_OK;
+    l.q[i] = (const char *)a[i].q;
+    l.mm[i] = (const char *)a[i].minmax;
+    l.out[i] = a[i].scores;
+  }
+  if (a->score_flags & ~(DA_SCORE_ROUND | DA_SCORE_ORDERED_BOUNDS)) return DA_OK;
+  *done = true;
+  if (a->dtype == DA_BF16 && (a->score_flags & DA_SCORE_ORDERED_BOUNDS) &&
+      page_score_tile_supported(D, P, H * P, P, l.out[0], l.q[0], l.mm[0], hs, hs * rep)) {
+    const int round_out = a->score_flags & DA_SCORE_ROUND;
+#define DA_TILE_LAYERS(kQ, kRows) \
+  launch_page_score_tile<kQ, kRows>(nullptr, hs, hs * rep, nullptr, rep, H, P, nullptr, H * P, P, round_out, s, &l, n)
+    if (D == 64) {
+      if (rep > 4) DA_TILE_LAYERS(2, 8);
+      else DA_TILE_LAYERS(2, 4);
+    } else {
+      if (rep > 4) DA_TILE_LAYERS(4, 8);
+      else DA_TILE_LAYERS(4, 4);
+    }
+#undef DA_TILE_LAYERS
+  } else if (a->dtype == DA_F32) {
+    if (lanes == 16) launch_vec_layers<F32, 16>(l, n, *a, s);
+    else launch_vec_layers<F32, 32>(l, n, *a, s);
+  } else if (a->dtype == DA_F16) {
+    if (lanes == 8) launch_vec_layers<F16, 8>(l, n, *a, s);
+    else launch_vec_layers<F16, 16>(l, n, *a, s);
+  } else {
+    if (lanes == 8) launch_vec_layers<BF16, 8>(l, n, *a, s);
+    else launch_vec_layers<BF16, 16>(l, n, *a, s);
+  }
+  return launch_status("da_decode_steps(scores)");
 }
 
 }  // namespace da

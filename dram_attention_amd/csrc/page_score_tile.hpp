@@ -40,7 +40,7 @@
 //
 #pragma once
 
-#include "common.hpp"
+#include "topk_rows.hpp"
 
 namespace da {
 
@@ -95,11 +95,11 @@ __device__ inline float page_score_exact_bf16(const char *q_row, const char *mn,
 }
 
 template <int kQ, int kRows, int kSteps, bool kMulti>
-__global__ void __launch_bounds__(256, 2)
-page_score_tile_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t q_head_stride,
-                       const char *__restrict__ mm, int n_rows, int64_t n_pages,
-                       float *__restrict__ out, int64_t out_row_stride, int64_t out_head_stride,
-                       int round_out, int rounds) {
+__device__ __forceinline__ void page_score_tile_block(const char *__restrict__ q, int64_t q_row_stride,
+                                                      int64_t q_head_stride, const char *__restrict__ mm,
+                                                      int n_rows, int64_t n_pages, float *__restrict__ out,
+                                                      int64_t out_row_stride, int64_t out_head_stride,
+                                                      int round_out, int rounds, const int row0) {
   static_assert(kQ == 1 || kQ == 2 || kQ == 4, "rows of 64, 128 or 256 bytes");
   static_assert(kRows == 4 || kRows == 8, "4 or 8 query rows per block");
   static_assert(kSteps % 4 == 0, "an accumulator collects four steps");
@@ -117,7 +117,6 @@ page_score_tile_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t
   const int part = j % kQ;
   const int chunk = part + kQ * kb;
   const int h = blockIdx.y;
-  const int row0 = blockIdx.z * kRows;
 
   // The only registers the inline asm ever writes (see slice_products), claimed
   // before anything else so that they are never shared with an MFMA operand.
@@ -255,6 +254,32 @@ page_score_tile_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t
   }
 }
 
+template <int kQ, int kRows, int kSteps, bool kMulti>
+__global__ void __launch_bounds__(256, 2)
+page_score_tile_kernel(const char *__restrict__ q, int64_t q_row_stride, int64_t q_head_stride,
+                       const char *__restrict__ mm, int n_rows, int64_t n_pages,
+                       float *__restrict__ out, int64_t out_row_stride, int64_t out_head_stride,
+                       int round_out, int rounds) {
+  page_score_tile_block<kQ, kRows, kSteps, kMulti>(q, q_row_stride, q_head_stride, mm, n_rows, n_pages, out,
+                                                   out_row_stride, out_head_stride, round_out, rounds,
+                                                   blockIdx.z * kRows);
+}
+
+// Several layers of the same sizes (blockIdx.z), up to kRows query rows each.
+struct ScoreLayers {
+  const char *q[kStepBatch], *mm[kStepBatch];
+  float *out[kStepBatch];
+};
+template <int kQ, int kRows, int kSteps, bool kMulti>
+__global__ void __launch_bounds__(256, 2)
+page_score_tile_layers_kernel(const ScoreLayers l, int64_t q_row_stride, int64_t q_head_stride, int n_rows,
+                              int64_t n_pages, int64_t out_row_stride, int64_t out_head_stride, int round_out,
+                              int rounds) {
+  const int i = blockIdx.z;
+  page_score_tile_block<kQ, kRows, kSteps, kMulti>(l.q[i], q_row_stride, q_head_stride, l.mm[i], n_rows, n_pages,
+                                                   l.out[i], out_row_stride, out_head_stride, round_out, rounds, 0);
+}
+
 // Whether the tile kernel takes the shape, and its launch.
 inline bool page_score_tile_supported(int head_dim, int64_t n_pages, int64_t out_row_stride,
                                       int64_t out_head_stride, const void *out, const void *q,
@@ -268,7 +293,8 @@ inline bool page_score_tile_supported(int head_dim, int64_t n_pages, int64_t out
 template <int kQ, int kRows>
 static void launch_page_score_tile(const void *q, int64_t qrs, int64_t qhs, const void *mm,
                                    int n_rows, int n_heads, int64_t n_pages, float *out,
-                                   int64_t ors, int64_t ohs, int round_out, hipStream_t s) {
+                                   int64_t ors, int64_t ohs, int round_out, hipStream_t s,
+                                   const ScoreLayers *layers = nullptr, int n_layers = 0) {
   constexpr int kP = 16 / kQ;
   const unsigned z = (unsigned)ceil_div(n_rows, kRows);
   // One round per wave while that gives at most ~4 blocks per CU; the rounds of
@@ -277,10 +303,15 @@ static void launch_page_score_tile(const void *q, int64_t qrs, int64_t qhs, cons
   const int64_t total_pages = n_pages * n_heads;
   const int64_t target_blocks = 1024;
   auto blocks_for = [&](int steps) { return ceil_div(n_pages, (int64_t)4 * steps * kP); };
-#define DA_TILE_LAUNCH(steps, multi, grid_x, rounds)                                            \
-  hipLaunchKernelGGL((page_score_tile_kernel<kQ, kRows, steps, multi>),                         \
-                     dim3((unsigned)(grid_x), n_heads, z), dim3(256), 0, s, (const char *)q, qrs, \
-                     qhs, (const char *)mm, n_rows, n_pages, out, ors, ohs, round_out, rounds)
+#define DA_TILE_LAUNCH(steps, multi, grid_x, rounds)                                              \
+  if (layers)                                                                                     \
+    hipLaunchKernelGGL((page_score_tile_layers_kernel<kQ, kRows, steps, multi>),                  \
+                       dim3((unsigned)(grid_x), n_heads, n_layers), dim3(256), 0, s, *layers, qrs, qhs, n_rows, \
+                       n_pages, ors, ohs, round_out, rounds);                                     \
+  else                                                                                            \
+    hipLaunchKernelGGL((page_score_tile_kernel<kQ, kRows, steps, multi>),                         \
+                       dim3((unsigned)(grid_x), n_heads, z), dim3(256), 0, s, (const char *)q, qrs, \
+                       qhs, (const char *)mm, n_rows, n_pages, out, ors, ohs, round_out, rounds)
   // 8 steps per round need 64 registers of page data next to the query operands:
   // with 8 query rows that no longer fits, so those take 4 steps per round.
   constexpr bool kLong = kRows == 4;
@@ -290,7 +321,9 @@ static void launch_page_score_tile(const void *q, int64_t qrs, int64_t qhs, cons
       return;
     }
   } else if (blocks_for(8) * n_heads <= target_blocks) {         // one round of 8 steps
-    if constexpr (kLong) DA_TILE_LAUNCH(8, false, blocks_for(8), 1);
+    if constexpr (kLong) {
+      DA_TILE_LAUNCH(8, false, blocks_for(8), 1);
+    }
     return;
   }
   {

@@ -71,4 +71,7 @@ constexpr int kStepBatch = 8;
 bool topk_lru_in_one_launch(const da_decode_step_args &a);
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s);
 
+// The page scores of those layers (page_score.hip).
+int launch_score_layers(const da_decode_step_args *a, int n, bool *done, hipStream_t s);
+
 }  // namespace da

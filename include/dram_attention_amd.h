@@ -504,7 +504,7 @@ int da_pages_gather_attend(const void *dram, int64_t dram_head_stride_bytes,
  * da_lru_update (DA_LRU_BUMP_STEP) and da_decode_attention_paged (STREAM | FIRST |
  * SECOND) on one argument block, in that order on `stream`, with the operands and results that
  * each has when called alone; top-k and LRU update are one launch where rows are of up to
- * 16384 pages and a head has no more requests than slots (the words of lru_workspace behind the
+ * 4096 pages and a head has no more requests than slots (the words of lru_workspace behind the
  * first two, zeroed once as the rest, then count a head's workgroups in).  For the layout a DRAMAttention layer has: every
  * array contiguous, int64 maps and indexes, fp32 access times and scores.
  * `args_bytes` = sizeof(da_decode_step_args).
@@ -541,8 +541,8 @@ int da_decode_step(const da_decode_step_args *args, size_t args_bytes, void *str
 /*
  * A step of each of n_steps layers whose queries do not depend on each other: the results of
  * da_decode_step on every block, in fewer launches.  The blocks differ in pointers, cache_len, scale,
- * rates and score flags only, top-k and LRU update are one launch (both said by
- * da_decode_steps_supported; DA_ENOTSUP before anything is launched otherwise), and no two share a
+ * rates and score flags only, rows are of up to 16384 pages and a head has no more requests than
+ * slots (all said by da_decode_steps_supported; DA_ENOTSUP before anything is launched otherwise), and no two share a
  * buffer that a step writes.  `args_bytes` = n_steps * sizeof(da_decode_step_args).
  */
 int da_decode_steps_supported(const da_decode_step_args *args, int n_steps, size_t args_bytes);

@@ -196,15 +196,18 @@ def test_stack_argument_checks_and_short_stacks():
     check_step(layers[0], oracles[0], q, k, v, w.prompt_tokens, out, 0, 2e-2, 1e-2)
 
 
-@pytest.mark.parametrize("n,dtype,sizes", [
-    (2, torch.float32, None), (8, torch.bfloat16, None), (9, torch.float16, None),   # a batch of launches, one more
-    (3, torch.bfloat16, (200, 200, 216)),                                            # layers of different sizes
+@pytest.mark.parametrize("n,dtype,heads,sizes", [
+    (2, torch.float32, (8, 2, 64), None),
+    (8, torch.bfloat16, (8, 2, 64), None), (9, torch.float16, (8, 2, 64), None),   # a batch of launches, one more
+    (3, torch.bfloat16, (16, 2, 128), None), (2, torch.float16, (12, 2, 128), None), (2, torch.float32, (4, 4, 128), None),
+    (3, torch.bfloat16, (8, 2, 64), (200, 200, 216)),                              # layers of different sizes
 ])
-def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, sizes):
+def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, heads, sizes):
     """Bits of the serial order for every layer, its caches and what its next step starts from."""
     from dram_attention_amd import AttentionStack, DRAMAttention
 
-    Hq, Hkv, D, S = 8, 2, 64, 1500
+    Hq, Hkv, D = heads
+    S = 1500
     g = torch.Generator(device=DEV).manual_seed(n)
 
     def rand(*shape):
@@ -213,7 +216,7 @@ def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, sizes):
     stacks = []
     prompts = [(rand(1, S, Hkv, D), rand(1, S, Hkv, D)) for _ in range(n)]
     for pipelined in (True, False):
-        layers = [DRAMAttention(6, 480, local, 16, 96, Hkv, D, device=DEV, dtype=dtype)
+        layers = [DRAMAttention(6, 800, local, 16, 96, Hkv, D, device=DEV, dtype=dtype)
                   for local in sizes or [200] * n]
         for m, (k, v) in zip(layers, prompts):
             m.init_cache(k, v)
