@@ -107,6 +107,38 @@ def test_page_score_strided_query_view():
     assert same(out.cpu(), out.cpu().bfloat16().float())
 
 
+@pytest.mark.parametrize("D,rows", [(64, 1), (64, 4), (128, 7), (128, 8), (256, 3)])
+def test_page_score_fp16_terms_are_rounded_products(D, rows):
+    """One channel of the query is not zero, so a score is one term: the larger of the two products, each rounded
+    to fp16, a NaN losing against the other.  Values over fp16's whole range, subnormals, infinities and NaN."""
+    from dram_attention_amd.max_ip_kernel import page_scores
+
+    g = torch.Generator().manual_seed(D + rows)
+    P = 203
+
+    def bits(*shape):
+        return torch.randint(-32768, 32768, shape, generator=g, dtype=torch.int32).to(torch.int16).view(torch.float16)
+
+    q, mm = torch.zeros(rows, 2, D, dtype=torch.float16), torch.zeros(2, P, 2, D, dtype=torch.float16)
+    chans = torch.randint(0, D, (rows, 2), generator=g)
+    terms = bits(2, P, 2)
+    for h in range(2):
+        mm[h].copy_(torch.where(torch.isfinite(terms[h]), terms[h], torch.ones(())).half()[..., None].expand(P, 2, D))
+        for r in range(rows):
+            q[r, h, chans[r, h]] = bits(1)[0]
+            mm[h, :, :, chans[r, h]] = terms[h]
+    # (a channel another row uses holds non-finite terms too, which that row's zero turns into NaN: left out)
+    out = torch.empty(rows, 2, P, dtype=torch.float32, device=DEV)
+    page_scores(q.to(DEV), mm.to(DEV), out, round_to_input=False)
+    for h in range(2):
+        finite = torch.isfinite(terms[h]).all(-1)
+        for r in range(rows):
+            prod = (q[r, h, chans[r, h]].float() * mm[h, :, :, chans[r, h]].float()).half().float()
+            want = torch.fmax(prod[:, 0], prod[:, 1])
+            use = finite if len(set(chans[:, h].tolist())) > 1 else torch.ones_like(finite)
+            assert same(out[r, h].cpu()[use], want[use]), (h, r)
+
+
 def test_page_score_fp16_follows_the_bf16_scheme():
     """fp16 inputs: products rounded to fp16, fp32 maximum and sum, one rounding at the
     end (the oracle's statement).  The reference's Triton kernel would accumulate in
