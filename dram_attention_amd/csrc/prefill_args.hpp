@@ -18,6 +18,7 @@ struct PrefillArgs {
   int n_groups;     // workgroups that share a kv head's rows: rep / kHeads
   int64_t n_row_blocks;
   int n_kv_heads;
+  int late_at, n_late;  // the last n_late pieces of work take the places from late_at on (0: in order)
   float scale_log2;
   // fp32 only: words of which one is not zero where the prompt's operands do not split into three
   // bf16 parts (null: nobody looked); the plain kernel then runs if gate_runs_if_set, the split one if not
@@ -32,6 +33,31 @@ __device__ __forceinline__ bool prefill_gate(const PrefillArgs &a) {
   uint32_t any = 0;
   for (int i = threadIdx.x; i < a.n_gate; i += blockDim.x) any |= a.gate[i];
   return (__syncthreads_or((int)any) != 0) != (a.gate_runs_if_set != 0);
+}
+
+// Which piece of work, numbered longest first, a workgroup takes.  With one workgroup per compute
+// unit, pieces go in grid order to the first unit that is free; workgroups are dealt in turn to the
+// part's 32 shader engines before that, so an engine's eight units share every 32nd.  Longest first,
+// the second 256 pieces pair up with the first, longest with shortest, to sums that are all alike, and
+// if there are two rounds and a part of one, the short pieces of the third prolong as many units.  So those
+// go ahead of the second round and in place of the shortest pieces of the first: the units that take
+// them have time for three.  By 32s, which keeps every engine's share and which head a die works on.
+// us in order / like this, D 128: 4613 tokens of 32/8 heads (584 pieces) 176 / 170, 5200 (656) 222 / 210, 6000
+// (752) 284 / 272; 3600, 40/10 (570) 137 / 131; 2300, 64/8 (576) 94.4 / 87.2; D 64: 10000, 16/4 (628) 246 / 230.  Four
+// rounds and a part gain 1 to 3 % (8700 tokens, 1088 pieces 561 / 552; 9200, 1152 628 / 611); three lose as
+// much as they gain, and a part of less than 32 is not worth it (4613 of 28/4, 532: 159 / 161).
+__device__ __forceinline__ unsigned prefill_piece(const PrefillArgs &a) {
+  const unsigned b = blockIdx.x, at = a.late_at, n = a.n_late;
+  return b < at || n == 0 ? b : b < at + n ? gridDim.x - n + (b - at) : b - n;
+}
+inline void prefill_order(PrefillArgs &a, int64_t pieces) {
+  constexpr int kUnits = 256, kEngines = 32;
+  const int rounds = (int)(pieces / kUnits < 8 ? pieces / kUnits : 8), part = (int)(pieces % kUnits);
+  a.n_late = 0;
+  if ((rounds != 2 && rounds != 4) || part <= kEngines) return;
+  const int n = (int)ceil_div(part, kEngines), ahead = ((rounds == 2 ? 6 : 5) * n + 5) / 10;
+  a.n_late = n * kEngines;
+  a.late_at = kUnits - ahead * kEngines;
 }
 
 // The kernel on fp32 instructions (prefill_attention_f32.hip), head_dim 64 or 128.

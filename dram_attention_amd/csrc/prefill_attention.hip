@@ -133,8 +133,9 @@ prefill_attention_kernel(const PrefillArgs a) {
   // start when the chip is running empty: 4613 tokens, 28/4 heads, D 128: 194.9 -> 157.1 us; 8192
   // tokens, 16/4, D 64: 221.9 -> 151.5; 8192, 40/10, D 128: 716 -> 637; 20000: 3734 -> 3641; 60000: the same.
   const unsigned n_kv_heads = a.n_kv_heads;
-  const int hk = (int)(blockIdx.x % n_kv_heads);
-  const int64_t rem = blockIdx.x / n_kv_heads;
+  const unsigned piece = prefill_piece(a);
+  const int hk = (int)(piece % n_kv_heads);
+  const int64_t rem = piece / n_kv_heads;
   const int64_t rb = a.n_row_blocks - 1 - rem / a.n_groups;
   const int hg = (int)(rem % a.n_groups);
   const int hq = hk * a.rep + hg * kHeads + wave % kHeads;
@@ -406,6 +407,7 @@ static int launch_prefill_split(PrefillArgs a, int heads, hipStream_t s) {
   a.n_row_blocks = ceil_div(a.seq_len, 32 * (kPfWaves / heads / kSplit));
   const int64_t blocks = a.n_row_blocks * a.n_groups * a.n_kv_heads;
   if (blocks > 0x7fffffff) return fail(DA_ENOTSUP, "da_prefill_attention: %lld workgroups", (long long)blocks);
+  prefill_order(a, blocks);
   const dim3 grid((unsigned)blocks);
 #define DA_PREFILL(kHeads) \
   hipLaunchKernelGGL((prefill_attention_kernel<T, kD, kHeads, kSplit>), grid, dim3(kPfThreads), 0, s, a)

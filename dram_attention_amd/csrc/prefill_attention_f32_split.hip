@@ -194,8 +194,9 @@ prefill_attention_f32_split_kernel(const PrefillArgs a, const char *__restrict__
 
   // all heads' longest rows first, the kv heads in turn: see prefill_attention.hip
   const unsigned n_kv_heads = a.n_kv_heads;
-  const int hk = (int)(blockIdx.x % n_kv_heads);
-  const int64_t rem = blockIdx.x / n_kv_heads;
+  const unsigned piece = prefill_piece(a);
+  const int hk = (int)(piece % n_kv_heads);
+  const int64_t rem = piece / n_kv_heads;
   const int64_t rb = a.n_row_blocks - 1 - rem / a.n_groups;
   const int hq = hk * a.rep + (int)(rem % a.n_groups) * kHeads + (wave & 3) % kHeads;
   const int kgroup = wave >> 2;          // which 32 keys of a round
@@ -453,6 +454,7 @@ static int launch_prefill_f32_split(PrefillArgs a, char *workspace, hipStream_t 
   const int64_t blocks = b.n_row_blocks * b.n_groups * a.n_kv_heads;
   if (blocks > 0x7fffffff)
     return fail(DA_ENOTSUP, "da_prefill_attention_f32_split: %lld workgroups", (long long)blocks);
+  prefill_order(b, blocks);
   const dim3 grid((unsigned)blocks);
   if (heads == 4)
     hipLaunchKernelGGL((prefill_attention_f32_split_kernel<kD, 4>), grid, dim3(kPsThreads), 0, s, b, planes, rounds);

@@ -315,6 +315,24 @@ def test_fp32_prefill_splits_to_the_ends_of_its_range():
         assert ((out[0, :, h].double() - want).abs() <= 1e-5 * want.abs().amax(-1, keepdim=True)).all()
 
 
+@pytest.mark.parametrize("dtype,S,Hq,Hkv,D", [
+    (torch.bfloat16, 3600, 40, 40, 64),     # 600 pieces: two rounds and a part
+    (torch.float16, 2050, 66, 66, 128),     # 594, of 66 heads: the part's last 32 are not all of one row block
+    (torch.bfloat16, 6700, 40, 40, 64),     # 1080: four rounds and a part
+    (torch.float32, 2560, 28, 28, 64), (torch.float32, 2300, 8, 2, 128),   # 560 and 144
+])
+def test_prefill_in_the_order_of_parts_of_a_round_covers_every_row(dtype, S, Hq, Hkv, D):
+    """All rows of all heads against torch's blocked form in fp32, where the order of the pieces is not longest
+    first.  Bounds of the other prefill tests: 2e-2 and 1e-2 in 16 bits, 1e-5 in fp32."""
+    from dram_attention_amd.dram_attention import causal_prefill_attention
+
+    xq, xk, xv = draw(S, Hq, Hkv, D, dtype, 5)
+    out = causal_prefill_attention(xq, xk, xv)
+    want = causal_prefill_attention(xq.float(), xk.float(), xv.float(), "blocked")
+    atol, rtol = (1e-5, 1e-5) if dtype == torch.float32 else (2e-2, 1e-2)
+    assert close(out, want, atol, rtol)
+
+
 def test_fp32_prompts_of_other_shapes_are_torchs():
     """Several sequences, and keys that reach beyond the queries (row i looks at keys 0..i), against the
     single-sequence kernel and the blocked form: fp32 both, 1e-5.  Heads that do not split are refused."""
