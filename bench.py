@@ -267,8 +267,8 @@ def stack_leg(w, n_layers, steps, warmup, seed, dev):
             "speedup_of_overlap": res["pipelined"]["layer_steps_per_s"] / res["serial"]["layer_steps_per_s"],
             "distinct_misses_per_layer_last_step": misses,
             "h2d_bytes_per_model_step": misses * n_layers * page_bytes,
-            "what": "pipelined: selection of layer i+1.. on a side stream while layer i's pages cross "
-                    "the host link; serial: the same launches on one stream"}
+            "what": "pipelined: the scores, the selections, the page streams and the merges of eight layers "
+                    "in a launch each; serial: one layer's step after the other"}
 
 
 def algorithmic_bytes(w, local_rows):
