@@ -262,16 +262,20 @@ def store_build_blocks(q_shape, k_shape, dtype: torch.dtype, page_size: int = 16
     there are as many as fill the link but a little, by the bytes each has in flight (a page, up to
     16 KB), or fewer where the store is done in 0.6 of attention's time all the same (20000 tokens in bf16:
     5 3045, 6 2990, 8 3006, 12 3651; 50000 tokens, 28/4 heads: 2 to 16 within 0.5 %, 32 4 % more).  Where
-    the store takes several times as long as attention, it gets the whole link: 12000 tokens, 16/16 heads,
-    D 64: 8 1170, 32 995.  Rates: attention at 1 PFLOP/s, or 190 TFLOP/s in fp32; 5.4 GB/s to the host per
-    workgroup beside it, 4 with pages of 4 KB."""
+    the store takes so much longer than attention that ``whole`` or more were needed for that, it gets the
+    whole link: 12000 tokens, 16/16 heads, D 64, 47 needed: 8 1170, 32 995; 4000, 24/8, D 128, 39 needed: 8
+    404, 32 350; 3000, 64/8, 24 needed: 8 365, 24 342.  With pages of 16 KB a full link costs attention more:
+    3000 of 24/8 heads in fp32, 24 needed: 6 625, 24 680; 6000 of 32/8 in pages of 32 tokens, 22 needed: 6 552,
+    22 593.  Rates: attention at 1 PFLOP/s, or 190 TFLOP/s in fp32; 5.4 GB/s to the host per workgroup beside
+    it, 4 with pages of 4 KB."""
     _, S, Hq, D = q_shape
     flops_per_s, esize = (1.9e14, 4) if dtype == torch.float32 else (1e15, 2)
     attention_s = max(1e-9, 2.0 * S * S * Hq * D / flops_per_s)    # (no queries: attention refuses them)
     page_bytes = page_size * 2 * D * esize
-    bytes_per_s, most = (5.4e9, 6) if page_bytes >= 16384 else (5.4e9, 8) if page_bytes >= 8192 else (4e9, 12)
+    bytes_per_s, most, whole = ((5.4e9, 6, 25) if page_bytes >= 16384 else (5.4e9, 8, 24) if page_bytes >= 8192 else
+                                (4e9, 12, 36))
     blocks = math.ceil(2.0 * k_shape[1] * k_shape[2] * D * esize / bytes_per_s / (0.6 * attention_s))
-    return max(2, min(most if blocks < 3 * most else 32, blocks))
+    return max(2, min(most if blocks < whole else 32, blocks))
 
 
 _build_streams = {}
