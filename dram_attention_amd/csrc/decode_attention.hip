@@ -187,6 +187,7 @@ struct MergeLayer {
   float *part_ml, *part_acc;
   const int32_t *miss_count, *c_len_dev;
   int64_t c_len;
+  const char *new_k;  // null: a step without a token to append
   char *out;
 };
 struct MergeBatch {
@@ -201,6 +202,7 @@ decode_attention_merge_layers_kernel(AttnArgs a, const MergeBatch batch, int hea
   a.miss_count = l.miss_count;
   a.c_len_dev = l.c_len_dev;
   a.c_len = l.c_len;
+  a.new_k = l.new_k;
   merge_block<T>(a, kMergeAll, head_dim, l.out, out_head_stride, nullptr);
 }
 
@@ -311,7 +313,7 @@ int launch_merge_layers(const PreparedAttention *p, const da_decode_step_args *s
   MergeBatch batch;
   for (int i = 0; i < n; ++i) {
     const AttnArgs &a = p[i].a;
-    batch.layer[i] = {a.part_ml, a.part_acc, a.miss_count, a.c_len_dev, a.c_len, (char *)steps[i].out};
+    batch.layer[i] = {a.part_ml, a.part_acc, a.miss_count, a.c_len_dev, a.c_len, a.new_k, (char *)steps[i].out};
   }
   const dim3 grid(p->a.n_q_heads, n);
   const int D = p->head_dim;

@@ -234,3 +234,65 @@ def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, heads, 
             for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
                          "hbm_page_to_dram_page_mapping", "current_step"):
                 assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
+
+
+def stepped_blocks(n, dtype, heads, S=1500):
+    """Two sets of n layers over the same prompts, and for each layer of either set the argument block of a step, as
+    a list in the order of the struct, and the output it points at; the partial results start out as NaN."""
+    from dram_attention_amd import DRAMAttention, _lib
+
+    Hq, Hkv, D = heads
+    g = torch.Generator(device=DEV).manual_seed(n + D)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    prompts = [(rand(1, S, Hkv, D), rand(1, S, Hkv, D)) for _ in range(n)]
+    tokens = [(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D)) for _ in range(n)]
+    sets = []
+    for _ in range(2):
+        layers, blocks, outs = [], [], []
+        for (k, v), (xq, xk, xv) in zip(prompts, tokens):
+            m = DRAMAttention(6, 800, 200, 16, 96, Hkv, D, device=DEV, dtype=dtype)
+            m.init_cache(k, v)
+            args, out = m._step_args(xq, xk, xv, S)
+            m._workspace.fill_(float("nan"))
+            layers.append(m)
+            blocks.append(list(_lib.DECODE_STEP_ARGS.unpack(args)))
+            outs.append(out)
+        sets.append((layers, blocks, outs))
+    torch.cuda.synchronize()
+    return sets, tokens
+
+
+def step_state(m):
+    """What a step leaves behind in a layer."""
+    lru = m.lru_cache
+    return [m.cache_k, m.cache_v, lru.hbm_kv_cache, lru.page_access_time, lru.dram_page_to_hbm_page_mapping,
+            lru.hbm_page_to_dram_page_mapping, lru.current_step]
+
+
+@pytest.mark.parametrize("dtype,heads", [(torch.float32, (8, 2, 64)), (torch.bfloat16, (16, 2, 128))])
+@pytest.mark.parametrize("appends", [(False, True, True), (True, False, True)])
+def test_blocks_with_and_without_a_new_token_in_one_call(dtype, heads, appends):
+    """The C entry: layers that append a token next to layers that do not, with an empty local window, the edge of a
+    chunk; the outputs and caches of a call per block."""
+    from dram_attention_amd import _lib
+
+    lib, pack = _lib.load(), _lib.DECODE_STEP_ARGS.pack
+    ((layers, blocks, outs), (alone, single, wants)), _tokens = stepped_blocks(3, dtype, heads)
+    for block in blocks + single:
+        block[28] = 0                                        # cache_len
+    for i, append in enumerate(appends):
+        if not append:
+            blocks[i][1:3] = single[i][1:3] = [0, 0]         # new_k, new_v
+    args = b"".join(pack(*b) for b in blocks)
+    assert lib.da_decode_steps_supported(args, 3, len(args))
+    stream = _lib.stream_ptr(outs[0].device)
+    _lib.check(lib.da_decode_steps(args, 3, len(args), stream), "steps")
+    for b in single:
+        _lib.check(lib.da_decode_step(pack(*b), len(args) // 3, stream), "step")
+    for i in range(3):
+        assert same(outs[i], wants[i]), i
+        assert not outs[i].isnan().any()
+        assert all(same(a, b) for a, b in zip(step_state(layers[i]), step_state(alone[i]))), i
