@@ -29,6 +29,14 @@ static int check_step(const da_decode_step_args &a) {
   return DA_OK;
 }
 
+// What da_page_score refuses of a step that check_step and prepare_step let pass.
+static int check_scores(const da_decode_step_args &a) {
+  DA_REQUIRE(a.minmax && a.scores, "da_decode_step: null pointer");
+  DA_REQUIRE((a.score_flags & ~(DA_SCORE_ROUND | DA_SCORE_ORDERED_BOUNDS)) == 0,
+             "da_decode_step: unknown score flag bits %d", a.score_flags);
+  return DA_OK;
+}
+
 static int scores_of(const da_decode_step_args &a, void *stream) {
   const int H = a.n_kv_heads, D = a.head_dim, rep = a.n_q_heads / H;
   return da_page_score(a.q, a.q_head_stride, a.q_head_stride * rep, a.minmax, a.n_pages * 2 * D, 2 * D, D, rep, H,
@@ -136,8 +144,10 @@ extern "C" int da_decode_steps(const da_decode_step_args *a, int n_steps, size_t
   if (!da_decode_steps_supported(a, n_steps, args_bytes))
     return fail(DA_ENOTSUP, "da_decode_steps: layers of the same sizes, whose selection and update are one launch");
   PreparedAttention p[kStepBatch];
-  for (int i = 0; i < n_steps; ++i) {     // (every block is looked at before the first launch)
-    const int rc = prepare_step(a[i], p[0]);
+  for (int i = 0; i < n_steps; ++i) {     // (every operand of every block is looked at before the first launch)
+    int rc = prepare_step(a[i], p[0]);
+    if (rc == DA_OK) rc = check_scores(a[i]);
+    if (rc == DA_OK) rc = check_topk_lru(a[i]);
     if (rc) return rc;
   }
   hipStream_t s = (hipStream_t)stream;

@@ -496,6 +496,11 @@ static int topk_lru_layer(const da_decode_step_args &a, TopkLruLayer &l) {
   return DA_OK;
 }
 
+int check_topk_lru(const da_decode_step_args &a) {
+  TopkLruLayer l;
+  return topk_lru_layer(a, l);
+}
+
 template <int kLayers>
 static int launch_topk_lru_batch(const da_decode_step_args *a, int n, hipStream_t s) {
   TopkLruBatch<kLayers> batch;

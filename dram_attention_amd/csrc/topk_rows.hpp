@@ -65,10 +65,11 @@ __device__ __forceinline__ void lru_candidates_block(const LruCandidateArgs &c, 
 }
 
 // Ordered top-k of every row, the list of least recent slots and the LRU update of a decode step
-// as one launch (lru_update.hip).  Whether a step's sizes allow it, and the launch itself, whose
-// operands it checks, of n <= kStepBatch layers of the same sizes.
+// as one launch (lru_update.hip).  Whether a step's sizes allow it, whether its operands are there, and
+// the launch itself, which checks them too, of n <= kStepBatch layers of the same sizes.
 constexpr int kStepBatch = 8;
 bool topk_lru_in_one_launch(const da_decode_step_args &a);
+int check_topk_lru(const da_decode_step_args &a);
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s);
 
 // The page scores of those layers (page_score.hip).

@@ -542,8 +542,9 @@ int da_decode_step(const da_decode_step_args *args, size_t args_bytes, void *str
  * A step of each of n_steps layers whose queries do not depend on each other: the results of
  * da_decode_step on every block, in fewer launches.  The blocks differ in pointers, cache_len, scale,
  * rates and score flags only, rows are of up to 16384 pages and a head has no more requests than
- * slots (all said by da_decode_steps_supported; DA_ENOTSUP before anything is launched otherwise), and no two share a
- * buffer that a step writes.  `args_bytes` = n_steps * sizeof(da_decode_step_args).
+ * slots (all said by da_decode_steps_supported), and no two share a buffer that a step writes.  Blocks of other
+ * kinds (DA_ENOTSUP) and a block with an operand that a call of its own refuses are refused before anything is
+ * launched, so no layer has stepped.  `args_bytes` = n_steps * sizeof(da_decode_step_args).
  */
 int da_decode_steps_supported(const da_decode_step_args *args, int n_steps, size_t args_bytes);
 int da_decode_steps(const da_decode_step_args *args, int n_steps, size_t args_bytes, void *stream);

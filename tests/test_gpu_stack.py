@@ -296,3 +296,23 @@ def test_blocks_with_and_without_a_new_token_in_one_call(dtype, heads, appends):
         assert same(outs[i], wants[i]), i
         assert not outs[i].isnan().any()
         assert all(same(a, b) for a, b in zip(step_state(layers[i]), step_state(alone[i]))), i
+
+
+@pytest.mark.parametrize("field,value", [(4, 0), (5, 0), (6, 0), (8, 0), (18, 0), (19, 0), (40, 64)],
+                         ids=["minmax", "scores", "idx", "access_time", "lru_workspace", "dram", "score_flags"])
+def test_a_bad_block_is_refused_before_any_layer_steps(field, value):
+    """Nine blocks, one more than a batch of launches, the last one not usable: an error and nothing changed."""
+    from dram_attention_amd import _lib
+
+    lib, n = _lib.load(), 9
+    ((layers, blocks, outs), _), _tokens = stepped_blocks(n, torch.bfloat16, (8, 2, 64))
+    blocks[-1][field] = value
+    for out in outs:
+        out.fill_(-7.0)
+    before = [[t.clone() for t in step_state(m)] for m in layers]
+    args = b"".join(_lib.DECODE_STEP_ARGS.pack(*b) for b in blocks)
+    rc = lib.da_decode_steps(args, n, len(args), _lib.stream_ptr(outs[0].device))
+    torch.cuda.synchronize()
+    assert rc == -1 and lib.da_last_error_string()
+    for m, state, out in zip(layers, before, outs):
+        assert all(same(a, b) for a, b in zip(step_state(m), state)) and (out == -7.0).all()
