@@ -12,6 +12,12 @@
 // of D/4, and an output's in one for every 16 keys instead of every 4.  Queries, keys, values
 // and softmax weights are split alike; softmax, its sums and the outputs are fp32.
 //
+// Weights reach down to 2^-126, where second and third parts would fall below the normal numbers (a
+// weight of 2^-121 kept to 2.6e-4), so they are split as 2^24 times themselves: the smallest
+// third part is then a normal number, and the sums of 2^31 weights of 2^8 and values of 2^60 end at 2^123.
+// Exact, and taken back with the division by the sum; us without / with it: 9200 tokens, 8/2 heads,
+// D 64: 457 / 466; 9000, 32/8, D 128: 3196 / 3217.
+//
 // Operands for which that is not so (not finite, above 2^60 or, but for zero, below 2^-100:
 // infinite products, third parts that fp32's own range cuts off) are looked for by the kernel
 // that splits keys and values, which leaves a word per workgroup; if one is set, this file's
@@ -24,8 +30,8 @@
 //
 // Bound: MFMA, six bf16 products at 1024 flops per cycle and SIMD: 171 against the 64 of the
 // fp32 instructions.  us of the plain kernel / of the three launches here: 9200 tokens, 8/2 heads,
-// D 64: 695 / 465 (1.12 PFLOP/s of bf16 products; a large bf16 matrix product of the library: 1.36);
-// 5000, 16/16, D 64: 447 / 312; 9000, 32/8, D 128: 5006 / 3180 (1.25 PFLOP/s); 64/8, 2000, D 128: 532 / 372.
+// D 64: 695 / 466 (1.12 PFLOP/s of bf16 products; a large bf16 matrix product of the library: 1.36);
+// 5000, 16/16, D 64: 447 / 302; 9000, 32/8, D 128: 5006 / 3217 (1.24 PFLOP/s); 64/8, 2000, D 128: 532 / 367.
 //
 // Work split.  prefill_split_kernel writes keys and values once, split and in the order in which
 // the matrix instructions take them: an operand of one instruction, 32 rows x 16 k indices
@@ -53,6 +59,7 @@ constexpr int kPsThreads = 512;
 constexpr int kPsKeys = 64;            // keys of a round, 32 for each group of waves
 constexpr int kPsOperand = 1024;       // bytes of one operand of an MFMA
 constexpr int kPsSplitThreads = 256;
+constexpr float kWeightScale = 0x1p24f;  // of the softmax weights while they are split (see above)
 constexpr int kPsMaxSplitBlocks = 1024;  // workgroups of the splitting kernel, a flag word each
 
 template <int kD>
@@ -311,7 +318,7 @@ prefill_attention_f32_split_kernel(const PrefillArgs a, const char *__restrict__
     for (int j = 0; j < 2; ++j) {
       float p[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = st[8 * j + i];
+      for (int i = 0; i < 8; ++i) p[i] = st[8 * j + i] * kWeightScale;
       split8(p, pt[j]);
     }
   };
@@ -415,7 +422,7 @@ prefill_attention_f32_split_kernel(const PrefillArgs a, const char *__restrict__
   const float mine = fast_exp2(m - mx), theirs = fast_exp2(other.x - mx);
   l = l * mine + other.y * theirs;
   l += __shfl_xor(l, 32, 64);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l > 0.f ? 1.f / l / kWeightScale : 0.f;
   if (my_row < S) {
     float *op = (float *)(a.out + (my_row * a.o_tok_stride + (int64_t)hq * a.o_head_stride) * 4) + 4 * g;
 #pragma unroll

@@ -94,7 +94,8 @@ int da_prefill_attention_f32(const float *q, int64_t q_tok_stride, int64_t q_hea
  * The same, faster for all but short prompts: every operand as the sum of three bf16 numbers,
  * products of those on the bf16 matrix instructions, sums in fp32; no further from float64 than
  * the form above, which does the prompt after all where an operand is not finite, above 2^60 or
- * (but for 0) below 2^-100 (decided on the device).
+ * (but for 0) below 2^-100 (decided on the device).  Softmax weights are taken at fp32 down to 2^-126 of
+ * a row's largest, as there.
  *   workspace: 16-byte aligned, 4096 + ceil(S / 64) * Hkv * 768 * D bytes; contents may be anything.
  *              da_prefill_attention_f32_workspace_bytes is that size, or 0 where the prompt is so
  *              short that the form above is the faster one

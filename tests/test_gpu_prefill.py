@@ -315,6 +315,28 @@ def test_fp32_prefill_splits_to_the_ends_of_its_range():
         assert ((out[0, :, h].double() - want).abs() <= 1e-5 * want.abs().amax(-1, keepdim=True)).all()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_fp32_prefill_small_weights_keep_their_bits(D):
+    """Values that read out the weights (key j has a one in channel j and zeros elsewhere), the first of each 32 keys
+    of weight 1 and the others of 2^-100 to 2^-123: every one within what fp32 scores give.  A score of
+    123 powers of two is off by 123 * 2^-24 for each rounding of the scale (two) and by half its last place, 2^-18,
+    where the reference is subtracted, all times ln 2; the division adds 2^-23."""
+    S = 64
+    q, k, v = torch.zeros(1, S, 1, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV)
+    q[..., 0] = 1.0
+    j = torch.arange(S, device=DEV)
+    k[0, :, 0, 0] = -math.log(2) * math.sqrt(D) * torch.where(j % 32 == 0, 0.0, 100 + 23 * (j % 32) / 31)
+    v[0, j, 0, j] = 1.0
+    out, _ = _split_prefill(q, k, v)
+    mask = torch.ones(S, S, dtype=torch.bool, device=DEV).triu_(1)
+    s_ = (k[0, :, 0, 0].double() / math.sqrt(D)).expand(S, S).masked_fill(mask, float("-inf"))
+    want = torch.softmax(s_, -1)
+    bound = (2 * 123 * 2.0 ** -24 + 2.0 ** -18) * math.log(2) + 2.0 ** -23
+    got = out[0, :, 0, :S].double()
+    worst = ((got - want).abs() / want)[~mask].max().item()
+    assert worst <= bound and (got[mask] == 0).all()
+
+
 @pytest.mark.parametrize("dtype,S,Hq,Hkv,D", [
     (torch.bfloat16, 3600, 40, 40, 64),     # 600 pieces: two rounds and a part
     (torch.float16, 2050, 66, 66, 128),     # 594, of 66 heads: the part's last 32 are not all of one row block
