@@ -254,28 +254,47 @@ def _prefill_operands(xq, xk, xv, lse):
                  xk.stride(2), xv.data_ptr(), xv.stride(1), xv.stride(2))
 
 
-def store_build_blocks(q_shape, k_shape, dtype: torch.dtype, page_size: int = 16) -> int:
-    """Workgroups that write the page store of the keys (and values) of ``k_shape`` next to prefill
-    attention.  Each takes a compute unit from it, and once the writes fill the link (57 GB/s)
-    every miss of attention's caches waits behind them: 9000 tokens, 32/8 heads, D 128, bf16, in us by
-    workgroups: 6 910, 8 755, 12 949, 32 1054; 4000 of those heads in fp32: 5 756, 8 860, 16 973.  So
-    there are as many as fill the link but a little, by the bytes each has in flight (a page, up to
-    16 KB), or fewer where the store is done in 0.6 of attention's time all the same (20000 tokens in bf16:
-    5 3045, 6 2990, 8 3006, 12 3651; 50000 tokens, 28/4 heads: 2 to 16 within 0.5 %, 32 4 % more).  Where
-    the store takes so much longer than attention that ``whole`` or more were needed for that, it gets the
-    whole link: 12000 tokens, 16/16 heads, D 64, 47 needed: 8 1170, 32 995; 4000, 24/8, D 128, 39 needed: 8
-    404, 32 350; 3000, 64/8, 24 needed: 8 365, 24 342.  With pages of 16 KB a full link costs attention more:
-    3000 of 24/8 heads in fp32, 24 needed: 6 625, 24 680; 6000 of 32/8 in pages of 32 tokens, 22 needed: 6 552,
-    22 593.  Rates: attention at 1 PFLOP/s, or 190 TFLOP/s in fp32; 5.4 GB/s to the host per workgroup beside
-    it, 4 with pages of 4 KB."""
+def store_build_blocks(q_shape, k_shape, dtype: torch.dtype, page_size: int = 16, resident: float = 0.0) -> int:
+    """Workgroups that write the page store of the keys (and values) of ``k_shape`` next to prefill attention,
+    the share ``resident`` of whose pages go into slots as well.  Each takes a compute unit from it, and
+    once the writes fill the link (57 GB/s) every miss of attention's caches waits behind them: up to the count
+    ``most`` another workgroup makes the store faster, the next few cost attention a fifth or more.  So up to
+    a ratio of the store's time on a full link to attention's there are ``most`` (fewer where the store is far
+    shorter), and beyond it, as the end of the store decides, the more the larger the ratio is.  A workgroup
+    moves more the larger its pages are, and less beside fp32 attention, beside heads that do not share
+    their keys and values, whose attention uses more of the memory, and where its pages go into slots.
+    us by workgroups (* the one taken here; pages of 16 tokens, up to 0.4 resident where not stated):
+
+      64/8 heads, D 128 (8 KB) 30455 tokens: 2 14103, 3 13413, *5, 7 13234, 10 13523, 28 14523
+      32/8, D 128 20922: 4 3415, 5 3296, *7 3216, 8 3274, 9 3632, 12 3836, 32 4093
+        10357: 6 1066, *7 928, 8 934, 10 1209, 16 1212; 6784: 6 696, *7 633, 8 654, 10 676, 12 630, 16 689, 32 705
+        4910: 7 459, 8 483, 12 447, *16 447, 20 440, 24 445, 32 455; 2778: 8 350, 16 322, 24 307, *32 305
+      40/10, D 128, 0.9 resident 20545: 5 4323, 7 4061, 8 4011, *9, 10 3981, 14 4778
+      16/16, D 128 39023: 6 8325, 7 7144, *8 6144, 9 7223, 12 8664; 20677: 8 3353, 12 3517, 14 3377, *16 3403, 32 3736
+      16/16, D 64 (4 KB) 30548: 8 3347, 9 3011, *10 2757, 12 3134, 16 3124; 15292: 10 1391, 16 1474, *24 1335, 32 1305
+        all resident 39957: 7 6258, 10 4708, 12 4046, *13, 14 4014, 20 5016
+      32/8, D 128, fp32 (16 KB) 3370: 5 676, *6 660, 7 712, 8 763, 12 766, 32 898; 1888: 6 398, 8 411, *12 375, 16 382
+
+    Over 306 prompts of 29 layouts (heads, type, page) that is 1.3 % slower on average than the best of 13 to 16
+    counts, and 11 % at most: 5265 tokens of 24/8 heads, D 128, fp32, *6 1072, 5 969.  Over 140 drawn ones, up to all
+    resident, 0.9 % and 10 %.  (One count two or three off costs 15 to 30 % at the worst places.)"""
     _, S, Hq, D = q_shape
-    flops_per_s, esize = (1.9e14, 4) if dtype == torch.float32 else (1e15, 2)
+    Hkv = k_shape[2]
+    f32, shared = dtype == torch.float32, Hq >= 3 * Hkv
+    flops_per_s, esize = (1.9e14, 4) if f32 else (1e15, 2)
     attention_s = max(1e-9, 2.0 * S * S * Hq * D / flops_per_s)    # (no queries: attention refuses them)
-    page_bytes = page_size * 2 * D * esize
-    bytes_per_s, most, whole = ((5.4e9, 6, 25) if page_bytes >= 16384 else (5.4e9, 8, 24) if page_bytes >= 8192 else
-                                (4e9, 12, 36))
-    blocks = math.ceil(2.0 * k_shape[1] * k_shape[2] * D * esize / bytes_per_s / (0.6 * attention_s))
-    return max(2, min(most if blocks < whole else 32, blocks))
+    store_s = 2e-5 + 2.0 * k_shape[1] * Hkv * D * esize / 57e9    # (20 us until the first pages are across)
+    ratio, page_bytes = store_s / attention_s, page_size * 2 * D * esize
+    if page_bytes >= 16384:
+        most, line, least, slope = 6, 1.3 if shared else 1.5, 12, 4.0
+    elif page_bytes >= 8192:
+        most, line, least, slope = 8 - shared + f32, 1.2 if shared else 1.45, 14, 5.5
+    else:
+        most, line, least, slope = 10, 1.1 if shared else 1.4, 20, 5.5
+    if ratio < line:
+        most = int(most * (1 + (0.2 if f32 or page_bytes >= 16384 else 0.4) * resident))
+        return max(2, min(most, math.ceil(30 * ratio)))
+    return min(32, max(least, 2 * int(slope * ratio)))
 
 
 _build_streams = {}
@@ -516,7 +535,8 @@ class DRAMAttention(torch.nn.Module):
         attends, the page store is written next to it, on a stream of its own: attention is
         bound by the matrix cores, the store by the host link.  An init_cache of somebody's
         own is called, behind attention."""
-        if not (self._paged_tokens(xk.shape[1]) > self.lru_hbm_cache_size
+        paged = self._paged_tokens(xk.shape[1])
+        if not (paged > self.lru_hbm_cache_size
                 and type(self).init_cache is _INIT_CACHE and "init_cache" not in self.__dict__
                 and self.prefill_backend in ("auto", "native") and xk.is_cuda
                 and (prefill_attention_supported(xq) or prefill_attention_f32_supported(xq, xk, xv))):
@@ -526,8 +546,8 @@ class DRAMAttention(torch.nn.Module):
         output = []
         self._build_cache(
             xk, xv, build_stream=build_stream(xk.device),
-            build_blocks=store_build_blocks(xq.shape, (1, self._paged_tokens(xk.shape[1]), *xk.shape[2:]), xq.dtype,
-                                            self.page_size),
+            build_blocks=store_build_blocks(xq.shape, (1, paged, *xk.shape[2:]), xq.dtype, self.page_size,
+                                            self.lru_hbm_cache_size / paged),
             beside=lambda: output.append(causal_prefill_attention(xq, xk, xv, self.prefill_backend)))
         return output[0]
 

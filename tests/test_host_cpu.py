@@ -141,6 +141,42 @@ def test_store_build_blocks_stays_within_its_limits():
             assert 2 <= store_build_blocks((1, S, 4, 64), (1, max(S, 1000), 2, 64), dtype) <= 32
 
 
+@pytest.mark.parametrize("heads,dtype,page,prompts", [
+    # (paged tokens, of the prompt's tokens, workgroups): both sides of a line, a long prompt, a short one
+    ((32, 8, 128), torch.bfloat16, 16, [(131072, 135152, 2), (20000, 21000, 7), (9000, 10000, 7), (6200, 7200, 7), (5400, 6400, 14),
+                                        (4000, 5000, 16), (1800, 2800, 24)]),
+    ((40, 10, 128), torch.bfloat16, 16, [(9248, 10242, 7), (4976, 6000, 14)]),
+    ((16, 16, 128), torch.bfloat16, 16, [(24000, 25000, 8), (23600, 24600, 8), (22000, 23000, 16)]),
+    ((16, 16, 64), torch.bfloat16, 16, [(40000, 41000, 10), (24000, 25000, 10), (22000, 23000, 20), (11000, 12000, 30)]),
+    ((16, 4, 64), torch.bfloat16, 16, [(8000, 9000, 10), (6000, 7000, 20), (4000, 5000, 20), (3000, 4000, 24)]),
+    ((16, 4, 64), torch.bfloat16, 32, [(8000, 9000, 7)]),
+    ((32, 8, 128), torch.bfloat16, 32, [(20000, 21000, 6), (6000, 7000, 6), (4500, 5500, 12), (2000, 3000, 16)]),
+    ((8, 2, 64), torch.float32, 16, [(8192, 9200, 8), (5000, 6000, 8)]),
+    ((16, 16, 64), torch.float32, 16, [(12000, 13000, 9)]),
+    ((24, 8, 128), torch.float32, 16, [(2744, 3000, 12), (4000, 5000, 6)]),
+    ((32, 8, 128), torch.float32, 32, [(4000, 5000, 6)]),
+])
+def test_store_build_blocks_by_ratio_page_size_and_heads(heads, dtype, page, prompts):
+    """The workgroups of the store at the places that its rule was measured at."""
+    from dram_attention_amd.dram_attention import store_build_blocks
+
+    Hq, Hkv, D = heads
+    got = [store_build_blocks((1, S, Hq, D), (1, paged, Hkv, D), dtype, page) for paged, S, _ in prompts]
+    assert got == [n for _, _, n in prompts]
+
+
+def test_store_build_blocks_where_pages_go_into_slots_too():
+    """A workgroup that writes its pages twice moves less: up to 1.4 times as many, for large pages and fp32 1.2."""
+    from dram_attention_amd.dram_attention import store_build_blocks
+
+    def blocks(dtype, page, *shares):
+        return [store_build_blocks((1, 9000, 16, 128), (1, 8000, 4, 128), dtype, page, share) for share in shares]
+
+    assert blocks(torch.bfloat16, 16, 0.0, 0.35, 0.36, 0.9) == [7, 7, 8, 9]
+    assert blocks(torch.float16, 32, 0.0, 0.8, 0.9) == [6, 6, 7]
+    assert blocks(torch.float32, 16, 0.0, 0.8, 0.9) == [6, 6, 7]
+
+
 def test_package_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "dram_attention_amd")
     for name in os.listdir(pkg):
