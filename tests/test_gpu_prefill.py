@@ -186,6 +186,34 @@ def test_module_prefill_stage_values_at_the_layer_shape(backend):
     assert isinstance(m.lru_cache, LRUCache) and m.dram_kv_cache_size == (S - 512 + 16) // 16 * 16
 
 
+def _plain_prefill(xq, xk, xv):
+    """da_prefill_attention_f32 itself, whatever the length."""
+    from dram_attention_amd import _lib
+
+    S, Hq, D = xq.shape[1:]
+    out, lse = torch.empty(1, S, Hq, D, device=DEV), torch.empty(Hq, S, device=DEV)
+    _lib.check(_lib.load().da_prefill_attention_f32(
+        xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1), xk.stride(2), xv.data_ptr(),
+        xv.stride(1), xv.stride(2), S, Hq, xk.shape[2], D, 1 / math.sqrt(D), out.data_ptr(), out.stride(1),
+        out.stride(2), lse.data_ptr(), _lib.stream_ptr(xq.device)), "plain")
+    return out, lse
+
+
+def _split_prefill(xq, xk, xv):
+    """da_prefill_attention_f32_split itself, whatever the length, in a workspace of NaN bytes."""
+    from dram_attention_amd import _lib
+
+    S, Hq, D = xq.shape[1:]
+    Hkv = xk.shape[2]
+    out, lse = torch.empty(1, S, Hq, D, device=DEV), torch.empty(Hq, S, device=DEV)
+    room = torch.full((4096 + -(-S // 64) * Hkv * 768 * D,), 255, dtype=torch.uint8, device=DEV)
+    _lib.check(_lib.load().da_prefill_attention_f32_split(
+        xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1), xk.stride(2), xv.data_ptr(),
+        xv.stride(1), xv.stride(2), S, Hq, Hkv, D, 1 / math.sqrt(D), out.data_ptr(), out.stride(1), out.stride(2),
+        lse.data_ptr(), room.data_ptr(), room.numel(), _lib.stream_ptr(xq.device)), "split")
+    return out, lse
+
+
 @pytest.mark.parametrize("S,Hq,Hkv,D", [
     (1, 4, 1, 64), (15, 8, 2, 64), (16, 4, 4, 128), (17, 6, 3, 64), (31, 2, 1, 128), (32, 3, 1, 64),
     (33, 8, 1, 128), (63, 4, 2, 64), (65, 5, 5, 128), (1000, 8, 2, 64), (2049, 12, 3, 128),
@@ -205,31 +233,34 @@ def test_fp32_prefill_kernel_matches_dense_float64(S, Hq, Hkv, D):
     lse = torch.empty(Hq, S, dtype=torch.float32, device=DEV)
     out = prefill_attention_f32(xq, xk, xv, lse=lse)
     assert same(causal_prefill_attention(xq, xk, xv), out)
+    plain, plain_lse = _plain_prefill(xq, xk, xv)        # (the longer of these prompts takes the other kernel)
     rep = Hq // Hkv
     mask = torch.ones(S, S, dtype=torch.bool, device=DEV).triu_(1)
     for h in range(Hq):
         q, k, v = xq[0, :, h].double(), xk[0, :, h // rep].double(), xv[0, :, h // rep].double()
         s_ = (q @ k.t().contiguous() / math.sqrt(D)).masked_fill_(mask, float("-inf"))
-        assert close(out[0, :, h].double(), torch.softmax(s_, -1) @ v, 1e-5, 1e-5)
-        assert close(lse[h].double(), torch.logsumexp(s_, -1), 1e-5, 1e-5)
+        want, want_lse = torch.softmax(s_, -1) @ v, torch.logsumexp(s_, -1)
+        assert close(out[0, :, h].double(), want, 1e-5, 1e-5) and close(lse[h].double(), want_lse, 1e-5, 1e-5)
+        assert close(plain[0, :, h].double(), want, 1e-5, 1e-5) and close(plain_lse[h].double(), want_lse, 1e-5, 1e-5)
 
 
+@pytest.mark.parametrize("kernel", ["plain", "split"])
 @pytest.mark.parametrize("D", [64, 128])
-def test_fp32_prefill_sums_are_short_chains(D):
+def test_fp32_prefill_sums_are_short_chains(D, kernel):
     """Summands that lose half of what lies below the sum's last place when they are added one
     after the other, seen in the log-sum-exp.  Sum of the weights: one addition to the running sum per tile of
     32 keys (and five in and behind it), half a unit in the last place each, and that of the result
     (9, to 2^-21).  A single score: half the channels in a chain lie a binade below the whole sum and lose
-    nothing; the chains' sum, the scale, the product with ln 2 and the two logarithms remain, half a unit each."""
-    from dram_attention_amd.dram_attention import prefill_attention_f32
-
+    nothing; the chains' sum, the scale, the product with ln 2 and the two logarithms remain, half a unit each.
+    (The kernel on bf16 parts adds to each of two running sums once per 64 keys, and its score is one sum of the
+    large products, exact here, and the small ones: within the same bounds.)"""
+    prefill = _plain_prefill if kernel == "plain" else _split_prefill
     S = 8192
     odd = 1.0 + 502 * 2.0 ** -23
     q, k, v = torch.zeros(1, S, 4, D, device=DEV), torch.zeros(1, S, 1, D, device=DEV), torch.ones(1, S, 1, D, device=DEV)
     q[..., 0] = 1.0
     k[:, 32:, :, 0] = math.log(odd) * math.sqrt(D)       # the first tile's scores, zero, stay the reference
-    lse = torch.empty(4, S, device=DEV)
-    prefill_attention_f32(q, k, v, lse=lse)
+    _, lse = prefill(q, k, v)
     n = torch.arange(1, S + 1, device=DEV, dtype=torch.float64)
     weight = (k[0, 32, 0, 0].double() / math.sqrt(D)).exp()
     want = (n.clamp(max=32) + (n - 32).clamp(min=0) * weight).log()
@@ -237,25 +268,9 @@ def test_fp32_prefill_sums_are_short_chains(D):
 
     term = 1.0 + 0.49 * D * 2.0 ** -24                   # 0.49 of the last place of sums in D/2 .. D
     k = torch.full((1, 1, 1, D), term, device=DEV)
-    lse = torch.empty(4, 1, device=DEV)
-    prefill_attention_f32(torch.ones(1, 1, 4, D, device=DEV), k, v[:, :1].contiguous(), lse=lse)
+    _, lse = prefill(torch.ones(1, 1, 4, D, device=DEV), k, v[:, :1].contiguous())
     want = D * k[0, 0, 0, 0].double().item() / math.sqrt(D)
     assert (lse.double() / want - 1).abs().max().item() < 5 * 2.0 ** -24
-
-
-def _split_prefill(xq, xk, xv):
-    """da_prefill_attention_f32_split itself, whatever the length, in a workspace of NaN bytes."""
-    from dram_attention_amd import _lib
-
-    S, Hq, D = xq.shape[1:]
-    Hkv = xk.shape[2]
-    out, lse = torch.empty(1, S, Hq, D, device=DEV), torch.empty(Hq, S, device=DEV)
-    room = torch.full((4096 + -(-S // 64) * Hkv * 768 * D,), 255, dtype=torch.uint8, device=DEV)
-    _lib.check(_lib.load().da_prefill_attention_f32_split(
-        xq.data_ptr(), xq.stride(1), xq.stride(2), xk.data_ptr(), xk.stride(1), xk.stride(2), xv.data_ptr(),
-        xv.stride(1), xv.stride(2), S, Hq, Hkv, D, 1 / math.sqrt(D), out.data_ptr(), out.stride(1), out.stride(2),
-        lse.data_ptr(), room.data_ptr(), room.numel(), _lib.stream_ptr(xq.device)), "split")
-    return out, lse
 
 
 @pytest.mark.parametrize("S,Hq,Hkv,D", [
@@ -283,21 +298,50 @@ def test_fp32_prefill_in_three_parts_matches_dense_float64(S, Hq, Hkv, D):
 def test_fp32_prefill_operands_that_do_not_split(value, D):
     """One element of the queries, keys or values, first or last, outside what three parts stand for: the bits of
     the kernel on fp32 instructions."""
-    from dram_attention_amd import _lib
-
     S, Hq, Hkv = 70, 4, 2
     for which in range(3):
         for at in (0, -1):
             ops = list(draw(S, Hq, Hkv, D, torch.float32, 3))
             ops[which].view(-1)[at] = value
-            out, lse = _split_prefill(*ops)
-            want, want_lse = torch.empty_like(out), torch.empty_like(lse)
-            q, k, v = ops
-            _lib.check(_lib.load().da_prefill_attention_f32(
-                q.data_ptr(), q.stride(1), q.stride(2), k.data_ptr(), k.stride(1), k.stride(2), v.data_ptr(),
-                v.stride(1), v.stride(2), S, Hq, Hkv, D, 1 / math.sqrt(D), want.data_ptr(), want.stride(1),
-                want.stride(2), want_lse.data_ptr(), _lib.stream_ptr(q.device)), "plain")
+            (out, lse), (want, want_lse) = _split_prefill(*ops), _plain_prefill(*ops)
             assert same(out, want) and same(lse, want_lse)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_fp32_prefill_finds_one_operand_among_all_workgroups(which):
+    """As many workgroups split as there are words for them, several passes each; the one element that does not
+    split lies in the middle, in a late pass, or at the end."""
+    S, H, D = 2560, 28, 64
+    ops = list(draw(S, H, H, D, torch.float32, 6))
+    flat = ops[which].view(-1)
+    clean, _ = _split_prefill(*ops)
+    want, _ = _plain_prefill(*ops)
+    assert not torch.equal(clean, want)                  # (the two kernels are told apart by their bits)
+    for at in (flat.numel() // 2 + 77, flat.numel() - H * D * 40 + 5, flat.numel() - 1):
+        kept = flat[at].item()
+        flat[at] = 2.0 ** -110
+        (out, lse), (want, want_lse) = _split_prefill(*ops), _plain_prefill(*ops)
+        flat[at] = kept
+        assert same(out, want) and same(lse, want_lse), at
+
+
+def test_fp32_prefill_without_memory_for_the_parts(monkeypatch):
+    """The workspace is refused, and only that: the plain kernel's bits."""
+    from dram_attention_amd.dram_attention import prefill_attention_f32
+
+    ops = draw(1500, 4, 2, 64, torch.float32, 8)
+    want, _ = _plain_prefill(*ops)
+    assert not same(prefill_attention_f32(*ops), want)
+    empty, refused = torch.empty, []
+
+    def no_bytes(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", no_bytes)
+    assert same(prefill_attention_f32(*ops), want) and len(refused) == 1
 
 
 def test_fp32_prefill_splits_to_the_ends_of_its_range():

@@ -200,6 +200,8 @@ def test_stack_argument_checks_and_short_stacks():
     (2, torch.float32, (8, 2, 64), None),
     (8, torch.bfloat16, (8, 2, 64), None), (9, torch.float16, (8, 2, 64), None),   # a batch of launches, one more
     (3, torch.bfloat16, (16, 2, 128), None), (2, torch.float16, (12, 2, 128), None), (2, torch.float32, (4, 4, 128), None),
+    # head sizes whose scores, or scores and page streams, go layer by layer
+    (3, torch.bfloat16, (8, 2, 32), None), (2, torch.float32, (8, 2, 32), None), (3, torch.float16, (8, 2, 256), None),
     (3, torch.bfloat16, (8, 2, 64), (200, 200, 216)),                              # layers of different sizes
 ])
 def test_layers_stepped_by_one_call_equal_layers_stepped_alone(n, dtype, heads, sizes):
@@ -316,3 +318,28 @@ def test_a_bad_block_is_refused_before_any_layer_steps(field, value):
     assert rc == -1 and lib.da_last_error_string()
     for m, state, out in zip(layers, before, outs):
         assert all(same(a, b) for a, b in zip(step_state(m), state)) and (out == -7.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_blocks_of_other_score_flags_and_query_strides_in_one_call(dtype):
+    """The C entry: a layer whose page bounds are not said to be ordered, and one whose query rows lie apart; the
+    results of a call per block."""
+    from dram_attention_amd import _lib
+
+    lib, pack = _lib.load(), _lib.DECODE_STEP_ARGS.pack
+    ((layers, blocks, outs), (alone, single, wants)), tokens = stepped_blocks(3, dtype, (8, 2, 64))
+    apart = torch.full((8, 128), float("nan"), dtype=dtype, device=DEV)
+    apart[:, :64] = tokens[2][0][0, 0]
+    for some in (blocks, single):
+        some[1][40] &= 1                                     # DA_SCORE_ROUND alone
+        some[2][0], some[2][25] = apart.data_ptr(), 128      # q, q_head_stride
+    assert blocks[0][40] != blocks[1][40]
+    args = b"".join(pack(*b) for b in blocks)
+    assert lib.da_decode_steps_supported(args, 3, len(args))
+    stream = _lib.stream_ptr(outs[0].device)
+    _lib.check(lib.da_decode_steps(args, 3, len(args), stream), "steps")
+    for b in single:
+        _lib.check(lib.da_decode_step(pack(*b), len(args) // 3, stream), "step")
+    for i in range(3):
+        assert same(outs[i], wants[i]), i
+        assert all(same(a, b) for a, b in zip(step_state(layers[i]), step_state(alone[i]))), i
