@@ -23,6 +23,7 @@ SOURCES = (
     "page_score.hip",
     "topk_pages.hip",
     "lru_update.hip",
+    "select_short.hip",
     "decode_attention.hip",
     "stream_attention.hip",
     "decode_step.hip",

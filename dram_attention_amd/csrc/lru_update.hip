@@ -515,6 +515,13 @@ static int launch_topk_lru_batch(const da_decode_step_args *a, int n, hipStream_
 }
 
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s) {
+  if (topk_lru_short(*a)) {
+    for (int i = 0; i < n; ++i) {
+      const int rc = check_topk_lru(a[i]);
+      if (rc) return rc;
+    }
+    return launch_topk_lru_short(a, n, s);
+  }
   return n == 1 ? launch_topk_lru_batch<1>(a, 1, s) : launch_topk_lru_batch<kStepBatch>(a, n, s);
 }
 

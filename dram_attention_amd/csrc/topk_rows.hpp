@@ -71,6 +71,9 @@ constexpr int kStepBatch = 8;
 bool topk_lru_in_one_launch(const da_decode_step_args &a);
 int check_topk_lru(const da_decode_step_args &a);
 int launch_topk_lru(const da_decode_step_args *a, int n, hipStream_t s);
+// The same for short rows, a workgroup per kv head (select_short.hip); the operands are checked.
+bool topk_lru_short(const da_decode_step_args &a);
+int launch_topk_lru_short(const da_decode_step_args *a, int n, hipStream_t s);
 
 // The page scores of those layers (page_score.hip).
 int launch_score_layers(const da_decode_step_args *a, int n, bool *done, hipStream_t s);

@@ -903,6 +903,50 @@ def test_selection_and_update_in_one_launch(Hq, Hkv, slots, kp, S):
             assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
 
 
+@pytest.mark.parametrize("Hq,Hkv,slots,kp,pages,dtype,levels,step0", [
+    (8, 2, 128, 32, 513, torch.float32, 0, 0),
+    (8, 2, 128, 32, 512, torch.float32, 2, 4000),      # few distinct scores: the threshold is a tie
+    (4, 1, 65, 16, 66, torch.bfloat16, 0, 0),          # two registers of keys, two of slots, each but started
+    (1, 1, 2, 1, 3, torch.float16, 0, 0),              # one request a step
+    (7, 1, 1023, 128, 1024, torch.bfloat16, 1, 16777000),   # the longest row and list, all scores alike
+    (8, 1, 1022, 127, 1024, torch.float16, 0, 255),    # nearly the most requests and slots
+    (16, 2, 1000, 100, 1023, torch.bfloat16, 3, 65535),
+    (12, 2, 600, 65, 1024, torch.float32, 1, 70000),
+    (16, 2, 1024, 128, 1025, torch.bfloat16, 0, 0), (9, 1, 600, 50, 700, torch.bfloat16, 0, 0),   # one page, one row
+    (2, 1, 600, 129, 700, torch.bfloat16, 0, 0),       # and one listed page too many
+])
+def test_selection_and_update_of_short_rows(Hq, Hkv, slots, kp, pages, dtype, levels, step0):
+    """Where a workgroup does a whole head, and one past each of its limits: the bits of the separate
+    launches, step by step; ``levels``: scores of few distinct values, ``step0``: times of a long run."""
+    from dram_attention_amd import DRAMAttention
+
+    D, page, local = 64, 16, 48
+    S = (pages - 1) * page + local
+    g = torch.Generator(device=DEV).manual_seed(11)
+
+    def rand(*shape):
+        if levels:
+            return torch.randint(1 - levels, levels, shape, device=DEV, generator=g).to(dtype)
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    a, b = (DRAMAttention(8, slots * page, local, page, kp * page, Hkv, D, device=DEV, dtype=dtype) for _ in range(2))
+    for m in (a, b):
+        m.init_cache(k, v)
+        m.lru_cache.page_access_time += step0
+        m.lru_cache.current_step += step0
+    assert a.lru_cache.dram_kv_cache.shape[1] == pages
+    for t in range(5):
+        xq, xk, xv = (rand(1, 1, h, D) for h in (Hq, Hkv, Hkv))
+        got = a(xq, xk, xv, start_pos=S + t, stage="generate")
+        assert same(got, b.attend_(xq, xk, xv, S + t, b.select_(xq))), t
+        for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
+                     "hbm_page_to_dram_page_mapping", "current_step", "_topk_idx"):
+            assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
+        for name in ("miss_count", "candidates", "slot_epoch", "hit_mask"):
+            assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
+
+
 def test_an_exchanged_method_of_a_step_is_called(monkeypatch):
     """Whatever the step is made of, on the instances, on the classes or in a subclass."""
     from dram_attention_amd import DRAMAttention, LRUCache
