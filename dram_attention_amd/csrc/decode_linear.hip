@@ -13,11 +13,15 @@
 // the gate and up row of a channel) meets in one wave: 64 lanes x 16 bytes of each row per
 // step, kUnroll steps of loads in flight per wave before the first is used; the input row
 // is read from LDS, packed dot products into fp32, one fold over the wave per pair.
-// Workgroups of four waves; each wave takes consecutive pairs, as many as keep the whole
-// grid resident at once (at most 8 workgroups per compute unit).
+// Workgroups of four waves, no more than are resident at once (98 registers a wave: four
+// workgroups per compute unit, fewer where the input row's LDS says so), every wave a pair in
+// turn: all waves end within a pair of each other.  us, up to 2048 workgroups with consecutive pairs per
+// wave (whose second round found half the chip idle) / this: output projection and
+// feed-forward of 2048 x 7168 26.3 / 24.6, of 4096 x 14336 70.4 / 68.5; vocabulary 32000 x 2048 25.7 / 23.9,
+// 50257 x 1024 26.4 / 23.7, 128256 x 4096 166.6 / 162.7.
 //
 // Measured (bf16, in a decode step, each with its endings; in brackets the library products
-// alone): vocabulary 128256 x 4096 163 us = 6.4 TB/s (188); 2 x 14336 x 4096 40 us = 5.9 TB/s
+// alone): vocabulary 128256 x 4096 160 us = 6.6 TB/s (188); 2 x 14336 x 4096 39 us = 6.0 TB/s
 // (57); 4096 x 14336 22 us (26); queries, keys and values 6144 x 4096 11.5 us (44 in three
 // launches).  A token through four such layers over 32K-token prefixes, one graph: 1.41 -> 1.04 ms;
 // through four layers of dim 2048 from Python, 72 -> 38 launches: 1.38 -> 0.67 ms.
@@ -30,7 +34,8 @@ constexpr int kLinThreads = 256;
 constexpr int kLinWaves = kLinThreads / 64;
 constexpr int kLinUnroll = 4;
 constexpr int kLinMaxRow = 60 * 1024;   // bytes of the input row (LDS)
-constexpr int64_t kLinResident = 256 * 8;  // workgroups of a grid that is resident at once
+constexpr int64_t kLinUnits = 256, kLinPerUnit = 4;  // compute units, resident workgroups of each
+constexpr size_t kLinLds = 160 * 1024;
 
 enum LinearEnd { kEndRope, kEndSwiglu, kEndAdd, kEndLogits };
 
@@ -41,7 +46,6 @@ struct LinearArgs {
   int dim;                  // K
   const char *w[3];         // rope: wq, wk, wv; swiglu: w1, w3; else w[0]
   int64_t n_pairs;
-  int pairs_per_wave;
   // rope: rows of wq and of wk (and of wv), channels of a head, cosine and sine per pair
   int q_rows, kv_rows, head_dim;
   const float *rope;
@@ -59,8 +63,8 @@ decode_linear_kernel(const LinearArgs a) {
   const int vecs = a.dim / T::kVec;
   const int steps = (vecs + 63) / 64;
   const int64_t row_b = (int64_t)a.dim * T::kBytes;
-  int64_t pair = ((int64_t)blockIdx.x * kLinWaves + wave) * a.pairs_per_wave;
-  const int64_t pair_end = pair + a.pairs_per_wave < a.n_pairs ? pair + a.pairs_per_wave : a.n_pairs;
+  int64_t pair = (int64_t)blockIdx.x * kLinWaves + wave;
+  const int64_t n_waves = (int64_t)gridDim.x * kLinWaves;
 
   // the two rows of a pair, and (rope) which matrix they belong to
   auto rows_of = [&](int64_t p, const char *&r0, const char *&r1) {
@@ -163,10 +167,10 @@ decode_linear_kernel(const LinearArgs a) {
     const int64_t done = pair;
     if (s0 >= steps) {
       s0 = 0;
-      ++pair;
-      if (pair < pair_end) rows_of(pair, r0, r1);
+      pair += n_waves;
+      if (pair < a.n_pairs) rows_of(pair, r0, r1);
     }
-    const bool more = pair < pair_end;
+    const bool more = pair < a.n_pairs;
     if (more) load(r0, r1, s0);
     if (pair == done) continue;
     // a pair is complete
@@ -263,9 +267,10 @@ static int launch_linear(const char *what, LinearArgs a, int dtype, hipStream_t 
   for (const void *p : {(const void *)a.x, (const void *)a.norm_weight, (const void *)a.w[0],
                         (const void *)a.w[1], (const void *)a.w[2]})
     DA_REQUIRE((uintptr_t)p % 16 == 0, "%s: operands must be 16-byte aligned", what);
-  a.pairs_per_wave = (int)ceil_div(a.n_pairs, kLinWaves * kLinResident);
-  const int64_t blocks = ceil_div(a.n_pairs, (int64_t)kLinWaves * a.pairs_per_wave);
   const size_t lds = (size_t)ceil_div(row_b, 1024 * kLinUnroll) * 1024 * kLinUnroll;
+  const int64_t fit = (int64_t)(kLinLds / (lds + 64)), most = kLinUnits * (fit < kLinPerUnit ? fit : kLinPerUnit);
+  const int64_t wanted = ceil_div(a.n_pairs, (int64_t)kLinWaves);
+  const int64_t blocks = wanted < most ? wanted : most;
   const dim3 grid((unsigned)blocks);
 #define DA_LINEAR(T) hipLaunchKernelGGL((decode_linear_kernel<T, kEnd>), grid, dim3(kLinThreads), lds, s, a)
   if (dtype == DA_BF16) DA_LINEAR(BF16);
