@@ -197,6 +197,23 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native half of the bindings (csrc/host_calls.cpp); raises if it is missing."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"{LIB_PATH.with_name('_host.so')} is missing or of another torch: build it with "
+                               "`python -m dram_attention_amd.build` (there is no fallback path)") from e
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().da_last_error_string().decode(errors="replace")

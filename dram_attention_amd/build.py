@@ -1,4 +1,4 @@
-"""Compile libdramattn.so (gfx950) from csrc/ with hipcc.
+"""Compile libdramattn.so (gfx950) from csrc/ with hipcc, and the Python module of its host calls.
 
 Run as ``python -m dram_attention_amd.build``; ``__graft_entry__.build()`` calls
 :func:`build_library`.  The library is built in-tree next to this file.
@@ -15,6 +15,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB_PATH = HERE / "libdramattn.so"
+HOST_PATH = HERE / "_host.so"
 SOURCES = (
     "api.hip",
     "page_minmax.hip",
@@ -156,6 +157,25 @@ def check_hand_placed_registers(verbose: bool = False) -> None:
         print(f"hand-placed registers of {n} tile scorer variants are clear of MFMA operands")
 
 
+def build_host_calls() -> None:
+    """Compile the Python module of csrc/host_calls.cpp against this interpreter's torch and
+    the library next to it (already built)."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}",
+           "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
+           str(CSRC / "host_calls.cpp"), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+           f"-L{HERE}", "-ldramattn", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_calls.cpp:\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build_library(verbose: bool = False) -> Path:
     """Compile every kernel source and link the shared library; returns its path."""
     hipcc = _hipcc()
@@ -183,6 +203,7 @@ def build_library(verbose: bool = False) -> Path:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     check_hand_placed_registers(verbose)
     os.replace(tmp, LIB_PATH)
+    build_host_calls()
     return LIB_PATH
 
 

@@ -562,15 +562,29 @@ class DRAMAttention(torch.nn.Module):
         return self.attend_(xq, xk, xv, start_pos, self.select_(xq))
 
     def _step_in_one_call(self, xq, xk, xv, start_pos):
-        """select_ and attend_ as one native call (da_decode_step) where everything has the
-        layout a layer is built with; None where anything differs, and the two methods, which
-        take or refuse it, do the step.  The same results on the same operands."""
+        """select_ and attend_ as one native call (da_decode_step; over a static prefix
+        da_decode_attention) where everything has the layout a layer is built with; None where
+        anything differs, and the two methods, which take or refuse it, do the step.  The same
+        results on the same operands."""
+        lru = self._modules.get("lru_cache")
+        if type(lru) is DummyCache:
+            return self._static_step(lru, xq, xk, xv, start_pos)
         step = self._step_args(xq, xk, xv, start_pos)
         if step is None:
             return None
         args, out = step
         _lib.check(_lib.load().da_decode_step(args, len(args), _lib.stream_ptr(xq.device)), "da_decode_step")
         return out
+
+    def _static_step(self, lru, xq, xk, xv, start_pos):
+        """A step over a static prefix, or None."""
+        cls, layer, own, prefix = type(self), self.__dict__, self._buffers, lru.__dict__
+        if ((cls.select_, cls.attend_, DummyCache.get_kv_cache_) != _STATIC_METHODS or "select_" in layer
+                or "attend_" in layer or "get_kv_cache_" in prefix):
+            return None
+        return _lib.host().static_step(
+            xq, xk, xv, start_pos, prefix.get("k_cache"), prefix.get("v_cache"), own["cache_k"], own["cache_v"],
+            self.dram_kv_cache_size, self._workspace, _lib.stream_ptr(xq.device))
 
     def _step_args(self, xq, xk, xv, start_pos):
         """(argument block of da_decode_step, output) of a step that one native call can do, else None."""
@@ -581,70 +595,34 @@ class DRAMAttention(torch.nn.Module):
         selector, buffers, own = lru.top_k_selector, lru._buffers, self._buffers
         if type(selector) is not IPUpperboundTopKSelector or not self._steps_by_its_own_methods(lru, selector):
             return None
-        minmax, dram, hbm = selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"]
-        H, P, _, D = minmax.shape
-        N, page, dtype = lru.num_hbm_pages, lru.page_size, xq.dtype
-        if xq.dim() != 4:
-            return None
-        Hq = xq.shape[2]
-        rep, kp = Hq // H, min(lru.top_k, P)
-        times, d2h, h2d, step = (buffers["page_access_time"], buffers["dram_page_to_hbm_page_mapping"],
-                                 buffers["hbm_page_to_dram_page_mapping"], buffers["current_step"])
-        cache_k, cache_v = own["cache_k"], own["cache_v"]
-        capacity = cache_k.shape[1]
-        page_dim = page * 2 * D
-        if not (xq.shape == (1, 1, rep * H, D) and xk.shape == xv.shape == (1, 1, H, D) and kp > 0 and N > 0
-                and minmax.shape[2] == 2 and hbm.shape == (H, N, page_dim) and dram.shape == (H, P, page_dim)
-                and times.shape == h2d.shape == (H, N) and d2h.shape == (H, P)
-                and cache_k.shape == cache_v.shape == (1, capacity, H, D)
-                and times.dtype is torch.float32 and d2h.dtype is h2d.dtype is torch.int64
-                and step.dtype is torch.int32 and step.numel() == 1
-                and gather_attend_supported(Hq, H, D, page, dtype)):
-            return None
-        device = xq.device
-        for t in (xq, xk, xv, minmax, hbm, cache_k, cache_v):
-            if t.dtype is not dtype or t.device != device or not t.is_contiguous():
-                return None
-        for t in (times, d2h, h2d, step):
-            if t.device != device or not t.is_contiguous():
-                return None
-        if dram.dtype is not dtype or not dram.is_contiguous():
-            return None
-        if isinstance(start_pos, torch.Tensor):
-            if start_pos.dtype is not torch.int32 or start_pos.device != device:
-                return None
-            cache_len, cache_len_dev = -self.dram_kv_cache_size, start_pos.data_ptr()
-        else:
-            cache_len, cache_len_dev = int(start_pos) - self.dram_kv_cache_size, 0
-            if cache_len < 0 or cache_len >= capacity:
-                return None
-        total = rep * kp
-        scratch, idx, scores = lru._scratch_for(total), lru._topk_idx, selector._scores
-        if idx is None or idx.shape[1] != total:
-            idx = lru._topk_idx = torch.empty(H, total, dtype=torch.int64, device=device)
+        step_args = _lib.host().step_args
+        for _ in range(2):
+            step = step_args(
+                xq, xk, xv, start_pos, selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"],
+                buffers["page_access_time"], buffers["dram_page_to_hbm_page_mapping"],
+                buffers["hbm_page_to_dram_page_mapping"], buffers["current_step"], own["cache_k"], own["cache_v"],
+                lru.num_hbm_pages, lru.page_size, lru.top_k, self.dram_kv_cache_size, lru.page_stores()[1],
+                self.stream_blocks, SCORE_FLAGS[selector.bounds_are_ordered], self.link_gbps, self.block_gbps,
+                lru._scratch, lru._topk_idx, selector._scores, selector._split_ws, self._workspace)
+            if type(step) is not int:
+                return step
+            self._make_room(lru, selector, step, xq)    # (a layer's first step)
+        return None
+
+    def _make_room(self, lru, selector, rep, xq):
+        """What the launches of a step hand to one another, for ``rep`` query rows a kv head."""
+        H, P, _, D = selector.chunk_min_max.shape
+        kp, device, idx, scores = min(lru.top_k, P), xq.device, lru._topk_idx, selector._scores
+        lru._scratch_for(rep * kp)
+        if idx is None or idx.shape[1] != rep * kp:
+            lru._topk_idx = torch.empty(H, rep * kp, dtype=torch.int64, device=device)
         if scores is None or scores.shape[0] != rep:
             scores = selector._scores = torch.empty(rep, H, P, dtype=torch.float32, device=device)
-        if scratch.slot_epoch.shape[1] != N:
-            return None
-        topk_ws = selector._workspace(scores, kp)
+        selector._workspace(scores, kp)
         if self._workspace is None:
-            self._workspace = attention_workspace(Hq, H, D, dtype, N * page, capacity, total * page, device)
-        workspace = self._workspace
-        out = torch.empty(1, 1, Hq, D, dtype=dtype, device=device)
-        args = _lib.DECODE_STEP_ARGS.pack(
-            xq.data_ptr(), xk.data_ptr(), xv.data_ptr(), out.data_ptr(), minmax.data_ptr(), scores.data_ptr(),
-            idx.data_ptr(), 0 if topk_ws is None else topk_ws.data_ptr(), times.data_ptr(),
-            scratch.candidates.data_ptr(), step.data_ptr(), d2h.data_ptr(), h2d.data_ptr(),
-            scratch.hit_mask.data_ptr(), scratch.miss_page.data_ptr(), scratch.miss_slot.data_ptr(),
-            scratch.miss_count.data_ptr(), scratch.slot_epoch.data_ptr(), scratch.workspace.data_ptr(),
-            lru.page_stores()[1], hbm.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), cache_len_dev,
-            workspace.data_ptr(),
-            D, P, capacity, cache_len, 0 if topk_ws is None else topk_ws.numel(), scratch.workspace.numel(),
-            workspace.numel() * 4,
-            Hq, H, D, _lib.dtype_code(dtype), page, kp, N, scratch.candidates.shape[1],
-            SCORE_FLAGS[selector.bounds_are_ordered], max(1, min(self.stream_blocks // H, total)),
-            1.0 / math.sqrt(D), self.link_gbps, self.block_gbps, 0)
-        return args, out
+            self._workspace = attention_workspace(
+                rep * H, H, D, xq.dtype, lru.num_hbm_pages * lru.page_size, self.cache_k.shape[1],
+                rep * kp * lru.page_size, device)
 
     def _steps_by_its_own_methods(self, lru, selector) -> bool:
         """Whether the methods a step is made of are this module's: neither a subclass, nor an
@@ -771,4 +749,5 @@ class DRAMAttention(torch.nn.Module):
 
 _STEP_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, LRUCache.select_, LRUCache.update_, LRUCache.views,
                  IPUpperboundTopKSelector.top_k_for_lru, IPUpperboundTopKSelector.scores)
+_STATIC_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, DummyCache.get_kv_cache_)
 _INIT_CACHE = DRAMAttention.init_cache

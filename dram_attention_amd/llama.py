@@ -222,9 +222,9 @@ class TransformerBlock(nn.Module):
             parts = self._modules
             a, f, norm1, norm2 = (parts["attention"], parts["feed_forward"], parts["attention_norm"],
                                   parts["ffn_norm"])
-            if self._one_token_kernels(a, f, norm1, norm2, x, rope_rows):
-                wq, wk, wv, wo = (a._modules[n]._parameters["weight"] for n in ("wq", "wk", "wv", "wo"))
-                w1, w2, w3 = (f._modules[n]._parameters["weight"] for n in ("w1", "w2", "w3"))
+            weights = self._one_token_kernels(a, f, norm1, norm2, x, rope_rows)
+            if weights is not None:
+                wq, wk, wv, wo, w1, w3, w2 = weights
                 xq, xk, xv = K.linear_qkv_rope(x, norm1, wq, wk, wv, a.n_heads, a.n_kv_heads, a.head_dim,
                                                rope_rows)
                 out = a.dram_attention(xq, xk, xv, start_pos=start_pos, stage="generate")
@@ -244,30 +244,26 @@ class TransformerBlock(nn.Module):
         return h + self.feed_forward(normed)
 
     @staticmethod
-    def _one_token_kernels(a, f, norm1, norm2, x, rope_rows) -> bool:
-        """Whether the one-token kernels may stand for these modules of a block: the modules
-        are the block's own kinds, nobody watches them, and every shape is the one that the
-        kernels take for granted."""
+    def _one_token_kernels(a, f, norm1, norm2, x, rope_rows):
+        """The weights (wq, wk, wv, wo, w1, w3, w2) if the one-token kernels may stand for these
+        modules of a block, else None: the modules are the block's own kinds, nobody watches
+        them, and every shape is the one that the kernels take for granted."""
         if not (type(a) is Attention and type(f) is FeedForward and type(norm1) is type(norm2) is RMSNorm):
-            return False
+            return None
         weight1, weight2 = norm1._parameters.get("weight"), norm2._parameters.get("weight")
         if not (K.takes(x, weight1, weight2) and K.bare(a, f, norm1, norm2)
                 and rope_rows.dtype is torch.float32 and rope_rows.is_contiguous()
                 and rope_rows.device == x.device):
-            return False
-        am, fm, dim = a._modules, f._modules, x.shape[2]
-        wq, wk, wv, wo, w1, w2, w3 = am["wq"], am["wk"], am["wv"], am["wo"], fm["w1"], fm["w2"], fm["w3"]
-        if not K.linears_fit(x, wq, wk, wv, wo, w1, w3, w2):
-            return False
-        q_rows, kv_rows, hidden = a.n_heads * a.head_dim, a.n_kv_heads * a.head_dim, w1.out_features
-        return (dim * x.element_size() % 16 == 0
-                and (wq.out_features, wq.in_features) == (q_rows, dim)
-                and (wk.out_features, wk.in_features) == (wv.out_features, wv.in_features) == (kv_rows, dim)
-                and (wo.out_features, wo.in_features) == (dim, q_rows)
-                and (w3.out_features, w3.in_features) == (hidden, w1.in_features) == (hidden, dim)
-                and (w2.out_features, w2.in_features) == (dim, hidden)
-                and weight1.shape == weight2.shape == (dim,)
-                and rope_rows.shape == (1, a.head_dim // 2, 2) and a.head_dim % 2 == 0)
+            return None
+        am, fm, dim, hd = a._modules, f._modules, x.shape[2], a.head_dim
+        w1 = fm["w1"]
+        q_rows, kv_rows, hidden = a.n_heads * hd, a.n_kv_heads * hd, getattr(w1, "out_features", -1)
+        if not (dim * x.element_size() % 16 == 0 and weight1.shape == weight2.shape == (dim,)
+                and rope_rows.shape == (1, hd // 2, 2) and hd % 2 == 0):
+            return None
+        return K.linears_fit(x, (am["wq"], q_rows, dim), (am["wk"], kv_rows, dim), (am["wv"], kv_rows, dim),
+                             (am["wo"], dim, q_rows), (w1, hidden, dim), (fm["w3"], hidden, dim),
+                             (fm["w2"], dim, hidden))
 
 
 class Transformer(nn.Module):

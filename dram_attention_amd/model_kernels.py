@@ -12,8 +12,6 @@ from torch.utils._device import DeviceContext
 
 from . import _lib
 
-_TYPES = (torch.bfloat16, torch.float16, torch.float32)
-_PLAIN = (torch.Tensor, nn.Parameter)
 # (asked several times for every layer of a token)
 _transform_level = torch._C._functorch.maybe_current_level
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
@@ -40,16 +38,8 @@ def _function_mode_watches() -> bool:
 def takes(*tensors: torch.Tensor) -> bool:
     """Whether the kernels apply: plain, contiguous, aligned GPU tensors of one type, and no
     autograd, autocast or transform that would have to see the operation."""
-    x = tensors[0]
-    if (not x.is_cuda or x.dtype not in _TYPES or torch.is_grad_enabled() or torch.is_autocast_enabled()
-            or not unobserved()):
-        return False
-    dtype, device = x.dtype, x.device
-    for t in tensors:
-        if (type(t) not in _PLAIN or t.dtype is not dtype or t.device != device or not t.is_contiguous()
-                or t.data_ptr() % 16):
-            return False
-    return True
+    return (tensors[0].is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled() and unobserved()
+            and _lib.host().alike(*tensors))
 
 
 def norm_fits(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -109,26 +99,18 @@ def plain_linears(*modules: nn.Module) -> bool:
 MAX_LINEAR_ROW = 60 * 1024  # bytes of an input row the one-token layers hold in LDS
 
 
-def linears_fit(x: torch.Tensor, *linears: nn.Module) -> bool:
-    """Whether the one-token layers may stand for these nn.Linear modules (x: any tensor of
-    the step, for its type and device)."""
+def linears_fit(x: torch.Tensor, *linears) -> tuple | None:
+    """The weights of these nn.Linear modules, if the one-token layers may stand for them (x: any
+    tensor of the step, for its type and device), else None.  Each as a module or as (module,
+    outputs, inputs), where only these sizes will do."""
     # (hooks first: pruning and weight normalisation keep the class, move the parameter and put
     # the weight together in a pre-hook)
-    if not bare(*linears):
-        return False
-    dtype, device, esize = x.dtype, x.device, x.element_size()
+    if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
+        return None
+    args = []
     for m in linears:
-        if type(m) is not nn.Linear:
-            return False
-        p = m._parameters
-        w = p.get("weight")
-        row = m.in_features * esize
-        if (p.get("bias", m) is not None or type(w) not in _PLAIN or w.dtype is not dtype or w.device != device
-                or not w.is_contiguous()
-                or w.shape != (m.out_features, m.in_features) or w.data_ptr() % 16 or row % 16
-                or row > MAX_LINEAR_ROW):
-            return False
-    return True
+        args += m if type(m) is tuple else (m, -1, -1)
+    return _lib.host().linears(x, nn.Linear, MAX_LINEAR_ROW, *args)
 
 
 def row_fits(row, x: torch.Tensor, n: int) -> bool:
@@ -140,15 +122,8 @@ def row_fits(row, x: torch.Tensor, n: int) -> bool:
 
 def linear_qkv_rope(x, norm, wq, wk, wv, n_heads, n_kv_heads, head_dim, rope_row):
     """Rotated queries and keys, and values, of one token: (1,1,Hq,D), (1,1,Hkv,D) x 2."""
-    out = torch.empty(n_heads + 2 * n_kv_heads, head_dim, dtype=x.dtype, device=x.device)
-    q, k, v = out.split((n_heads, n_kv_heads, n_kv_heads))
-    _lib.check(
-        _lib.load().da_linear_qkv_rope(
-            x.data_ptr(), norm.weight.data_ptr(), norm.eps, x.shape[-1], wq.data_ptr(), wk.data_ptr(),
-            wv.data_ptr(), n_heads, n_kv_heads, head_dim, rope_row.data_ptr(), q.data_ptr(), k.data_ptr(),
-            v.data_ptr(), _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
-        "da_linear_qkv_rope")
-    return q[None, None], k[None, None], v[None, None]
+    return _lib.host().qkv_rope(x, norm.weight, norm.eps, wq, wk, wv, n_heads, n_kv_heads, head_dim, rope_row,
+                                _lib.stream_ptr(x.device))
 
 
 def linear_swiglu(x, norm, w1, w3):
@@ -175,17 +150,7 @@ def linear_add(x, w, residual):
 
 def block_tail(attended, wo, x, norm, w1, w3, w2):
     """The rest of a block behind attention's output, residuals included, as one call."""
-    dim, hidden = w2.shape
-    room = torch.empty(dim + hidden, dtype=x.dtype, device=x.device)
-    out = torch.empty_like(x)
-    h = room.data_ptr()
-    _lib.check(
-        _lib.load().da_linear_block_tail(
-            attended.data_ptr(), wo.shape[1], wo.data_ptr(), x.data_ptr(), dim, norm.weight.data_ptr(), norm.eps,
-            w1.data_ptr(), w3.data_ptr(), hidden, w2.data_ptr(), h, h + dim * x.element_size(), out.data_ptr(),
-            _lib.dtype_code(x.dtype), _lib.stream_ptr(x.device)),
-        "da_linear_block_tail")
-    return out
+    return _lib.host().block_tail(attended, wo, x, norm.weight, norm.eps, w1, w3, w2, _lib.stream_ptr(x.device))
 
 
 def linear_logits(x, norm, w):

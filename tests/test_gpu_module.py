@@ -874,6 +874,56 @@ def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
         a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,dtype", [(8, 2, 64, torch.float32), (28, 4, 128, torch.bfloat16),
+                                            (4, 4, 32, torch.float16)])
+def test_static_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, dtype, monkeypatch):
+    """A step over a static prefix is one native call: the bits of select_ + attend_ on a twin, for host
+    and device positions and for strided operands; positions of another kind, a full window and an
+    exchanged method take the two halves, which take or refuse them as before."""
+    from dram_attention_amd import DRAMAttention, DummyCache
+
+    S = 700
+    g = torch.Generator(device=DEV).manual_seed(8)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    a, b = (DRAMAttention(8, 4096, 200, 16, 64, Hkv, D, device=DEV, dtype=dtype) for _ in range(2))
+    a.init_cache(k, v)
+    b.init_cache(k, v)
+    assert type(a.lru_cache) is DummyCache
+    calls = []
+    one_call = a._step_in_one_call
+    a._step_in_one_call = lambda *args: calls.append(one_call(*args)) or calls[-1]
+
+    def check(xq, start, in_one=True):
+        xk, xv = rand(1, 1, Hkv, D), rand(1, 1, Hkv, D)
+        got = a(xq, xk, xv, start_pos=start, stage="generate")
+        assert same(got, b.attend_(xq, xk, xv, start, b.select_(xq)))
+        assert same(a.cache_k, b.cache_k) and same(a.cache_v, b.cache_v)
+        assert (calls.pop() is not None) == in_one
+
+    check(rand(1, 1, Hq, D), S, in_one=False)           # (the first step makes the workspace)
+    check(rand(1, 1, Hq, D), S + 1)
+    check(rand(1, 1, Hq, D), torch.tensor([S + 2], dtype=torch.int32, device=DEV))
+    check(rand(1, 1, Hq, 2 * D)[..., :D], S + 3)        # strided rows
+    check(rand(1, 1, Hq, D), torch.tensor([S + 4], device=DEV), in_one=False)     # int64
+    check(rand(1, 1, Hq, D), torch.tensor(S + 5).numpy()[()], in_one=False)       # a numpy integer
+    with pytest.raises(RuntimeError, match="local cache overflow"):
+        a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
+    with pytest.raises(RuntimeError, match="one token per call"):
+        a(rand(1, 2, Hq, D), rand(1, 2, Hkv, D), rand(1, 2, Hkv, D), start_pos=S, stage="generate")
+    for owner, name in ((a, "attend_"), (a.lru_cache, "get_kv_cache_"), (DummyCache, "get_kv_cache_")):
+        inner, seen = getattr(owner, name), []
+        with monkeypatch.context() as patch:
+            patch.setattr(owner, name, lambda *x, **kw: seen.append(1) or inner(*x, **kw))
+            a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 6, stage="generate")
+        assert seen, name
+        if not isinstance(owner, type):
+            delattr(owner, name)
+
+
 @pytest.mark.parametrize("Hq,Hkv,slots,kp,S", [
     (8, 2, 24, 6, 1500),     # as many requests as slots
     (8, 2, 20, 6, 1500),     # more: the serial walk, a launch of its own
