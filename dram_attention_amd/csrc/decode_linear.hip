@@ -211,47 +211,91 @@ decode_linear_kernel(const LinearArgs a) {
 }
 
 // Index of the largest logit (the lowest of equal ones; a NaN counts as the largest, as in
-// torch.argmax).  One workgroup, eight loads in flight per thread: half a megabyte of logits,
-// just written, comes from cache, without a second launch or a hand-over between workgroups
-// (128256 logits: 13 us; torch's reduction 40 us).
-constexpr int kArgmaxThreads = 1024;
+// torch.argmax).  One workgroup: half a megabyte of logits, just written, comes from cache, without a
+// second launch or a hand-over between workgroups.  Bound: the latency of its loads, 16 in
+// flight per thread, once the arithmetic is short: a thread keeps the best of its vectors of four
+// values, not of its values (a maximum and an index per vector), and whether there was a NaN at all; which
+// value of the best vector it was is looked up at the end, and only a row with a NaN is gone
+// through again.  128256 logits: 9.5 us (a key and an index per value 13.5, torch's reduction 40).
+constexpr int kArgmaxThreads = 1024, kArgmaxLoads = 16;
 __global__ void __launch_bounds__(kArgmaxThreads)
 argmax_kernel(const float *__restrict__ x, int64_t n, int64_t *__restrict__ out) {
-  // (order key, ~index): the larger is the better, and of equal values the lower index
-  unsigned long long best = 0;
-  auto take = [&](float v, int64_t i) {
-    const unsigned long long k = (unsigned long long)float_order_key(v) << 32 | (uint32_t)~(uint32_t)i;
-    best = k > best ? k : best;
-  };
+  constexpr uint32_t kNone = 0xffffffffu;
+  __shared__ float part_best[kArgmaxThreads / 64];
+  __shared__ uint32_t part_at[kArgmaxThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int64_t vecs = n / 4;
-  for (int64_t j0 = threadIdx.x; j0 < vecs; j0 += 8 * kArgmaxThreads) {
-    float4 v[8];
+  float best = -INFINITY;
+  uint32_t at = kNone;        // vector of the best value, the lowest (n < 2^31)
+  bool nan = false;
+  for (int64_t j0 = t; j0 < vecs; j0 += kArgmaxLoads * kArgmaxThreads) {
+    float4 v[kArgmaxLoads];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < kArgmaxLoads; ++u) {
       const int64_t j = j0 + u * kArgmaxThreads;
       v[u] = *(const float4 *)(x + 4 * (j < vecs ? j : j0));
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int64_t j = j0 + u * kArgmaxThreads < vecs ? j0 + u * kArgmaxThreads : j0;
-      take(v[u].x, 4 * j);
-      take(v[u].y, 4 * j + 1);
-      take(v[u].z, 4 * j + 2);
-      take(v[u].w, 4 * j + 3);
+    for (int u = 0; u < kArgmaxLoads; ++u) {
+      const int64_t j = j0 + u * kArgmaxThreads;
+      nan |= __builtin_isunordered(v[u].x, v[u].y) || __builtin_isunordered(v[u].z, v[u].w);
+      const float m = fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w));
+      if (j < vecs && (m > best || at == kNone)) {     // (a row of -inf has a best too)
+        best = m;
+        at = (uint32_t)j;
+      }
     }
   }
-  for (int64_t i = 4 * vecs + threadIdx.x; i < n; i += kArgmaxThreads) take(x[i], i);
+  // the last n % 4 values as a vector of their own
+  if (t == 0)
+    for (int64_t i = 4 * vecs; i < n; ++i) {
+      nan |= x[i] != x[i];
+      if (x[i] > best || at == kNone) {
+        best = x[i];
+        at = (uint32_t)vecs;
+      }
+    }
+  if (__syncthreads_or(nan)) {
+    uint32_t first = kNone;
+    for (int64_t i = t; i < n; i += kArgmaxThreads)
+      if (x[i] != x[i]) {
+        first = (uint32_t)i;
+        break;
+      }
+    for (int m = 32; m >= 1; m >>= 1) first = min(first, (uint32_t)__shfl_xor((int)first, m, 64));
+    if (lane == 0) part_at[wave] = first;
+    __syncthreads();
+    if (t == 0) {
+      for (int i = 1; i < kArgmaxThreads / 64; ++i) first = min(first, part_at[i]);
+      *out = (int64_t)first;
+    }
+    return;
+  }
+  // (a thread without a vector: -inf at kNone, behind every other)
+  auto better = [](float b, uint32_t i, float c, uint32_t k) { return c > b || (c == b && k < i); };
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
-    const unsigned long long o = __shfl_xor(best, m, 64);
-    best = o > best ? o : best;
+    const float c = __shfl_xor(best, m, 64);
+    const uint32_t k = (uint32_t)__shfl_xor((int)at, m, 64);
+    if (better(best, at, c, k)) {
+      best = c;
+      at = k;
+    }
   }
-  __shared__ unsigned long long part[kArgmaxThreads / 64];
-  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = best;
+  if (lane == 0) {
+    part_best[wave] = best;
+    part_at[wave] = at;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < kArgmaxThreads / 64; ++i) best = part[i] > best ? part[i] : best;
-    *out = (int64_t)(uint32_t)~(uint32_t)best;
+  if (t == 0) {
+    for (int i = 1; i < kArgmaxThreads / 64; ++i)
+      if (better(best, at, part_best[i], part_at[i])) {
+        best = part_best[i];
+        at = part_at[i];
+      }
+    int64_t i = 4 * (int64_t)at;
+    while (x[i] != best) ++i;      // (no NaN: the vector, or the rest of the row, holds it)
+    *out = i;
   }
 }
 

@@ -266,6 +266,12 @@ class TransformerBlock(nn.Module):
                              (fm["w2"], dim, hidden))
 
 
+def _index(position: torch.Tensor) -> torch.Tensor:
+    """A device position as one index (32 bits are one as they are: no launch)."""
+    index = position.reshape(1)
+    return index if index.dtype in (torch.int32, torch.int64) else index.long()
+
+
 class Transformer(nn.Module):
     """``forward(tokens (1, S), start_pos) -> logits (1, 1, vocab)`` fp32 of the last
     position (evaluation/dram-attention/model.py:276-317)."""
@@ -291,7 +297,7 @@ class Transformer(nn.Module):
         h = self.tok_embeddings(tokens)
         if isinstance(start_pos, torch.Tensor):
             assert seqlen == 1, "a device-resident position is for single-token decode steps"
-            rows = self.rope.index_select(0, start_pos.reshape(1).long())
+            rows = self.rope.index_select(0, _index(start_pos))
         else:
             rows = self.rope[start_pos: start_pos + seqlen]
         for layer in self.layers:
