@@ -302,10 +302,11 @@ __device__ __forceinline__ void attention_tile_block(const AttnArgs &a, const in
   }
 }
 
-template <typename T, int kD, int kRows>
+template <typename T, int kD, int kRows, bool kStreamLoads>
 __global__ void __launch_bounds__(kAttnThreads)
-decode_attention_tile_kernel(const AttnArgs a) {
-  attention_tile_block<T, kD, kRows>(a, blockIdx.x, blockIdx.y);
+decode_attention_tile_kernel(const AttnArgs a, const bool heads_first) {
+  attention_tile_block<T, kD, kRows, kStreamLoads>(a, heads_first ? blockIdx.y : blockIdx.x,
+                                                   heads_first ? blockIdx.x : blockIdx.y);
 }
 
 }  // namespace da

@@ -206,16 +206,24 @@ decode_attention_merge_layers_kernel(AttnArgs a, const MergeBatch batch, int hea
   merge_block<T>(a, kMergeAll, head_dim, l.out, out_head_stride, nullptr);
 }
 
-// The matrix-core form of the pass, for the shapes it takes.
-template <typename T, int kD>
+// The matrix-core form of the pass, for the shapes it takes.  Two rules on what it reads:
+//   - keys and values laid out token by token (a prompt's own, as a static cache keeps them): blocks that
+//     follow each other take the heads of the same tokens, which lie next to each other.  us a call on
+//     32768 tokens out of the caches, tokens / heads first: 32/8 heads 34.8 / 33.9, 28/4 22.3 / 21.6, 64/8
+//     35.4 / 34.3; laid out head by head 35.5 / 35.5, and 100000 tokens 81.3 / 85.4.
+//   - more than the last-level cache holds: streaming loads (100000 tokens of 32/8 81.3 / 79.0; with
+//     less they are slower where the caches still have it, 32768 tokens 30.3 / 33.3).
+constexpr int64_t kLastLevelBytes = 256 << 20;
+template <typename T, int kD, bool kStream>
 static void launch_tile(const AttnArgs &a, int n_launch, int n_kv_heads, hipStream_t s) {
-  const dim3 grid(n_launch, n_kv_heads, 1);
-  if (a.rep <= 4)
-    hipLaunchKernelGGL((decode_attention_tile_kernel<T, kD, 4>), grid, dim3(kAttnThreads), 0, s, a);
-  else if (a.rep <= 8)
-    hipLaunchKernelGGL((decode_attention_tile_kernel<T, kD, 8>), grid, dim3(kAttnThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL((decode_attention_tile_kernel<T, kD, 16>), grid, dim3(kAttnThreads), 0, s, a);
+  const bool heads_first = a.p_tok_stride > a.p_head_stride;
+  const dim3 grid = heads_first ? dim3(n_kv_heads, n_launch, 1) : dim3(n_launch, n_kv_heads, 1);
+#define DA_TILE(kRows) \
+  hipLaunchKernelGGL((decode_attention_tile_kernel<T, kD, kRows, kStream>), grid, dim3(kAttnThreads), 0, s, a, heads_first)
+  if (a.rep <= 4) DA_TILE(4);
+  else if (a.rep <= 8) DA_TILE(8);
+  else DA_TILE(16);
+#undef DA_TILE
 }
 
 template <typename T, int kLanes, bool kTail>
@@ -227,7 +235,10 @@ static void launch_split(AttnArgs a, int first_chunk, int n_launch, int n_kv_hea
   if constexpr (!kTail && T::kBytes == 2 && (kLanes == 8 || kLanes == 16 || kLanes == 32)) {
     const int dtype = std::is_same<T, BF16>::value ? DA_BF16 : DA_F16;
     if (tile_pass_supported(dtype, kLanes * 8, rep, a.slot_epoch != nullptr, a.page_size)) {
-      launch_tile<T, kLanes * 8>(a, n_launch, n_kv_heads, s);
+      if ((a.p_len + a.c_capacity) * n_kv_heads * 2 * kLanes * 16 > kLastLevelBytes)
+        launch_tile<T, kLanes * 8, true>(a, n_launch, n_kv_heads, s);
+      else
+        launch_tile<T, kLanes * 8, false>(a, n_launch, n_kv_heads, s);
       return;
     }
   }
@@ -429,7 +440,8 @@ int prepare_attention(const void *q, int64_t q_head_stride, int n_q_heads, int n
                overlap->gather_blocks, n_kv_heads, kGatherMaxBlocks);
     a.gather_blocks = overlap->gather_blocks;
   }
-  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
+  const bool tiles_alone = !overlap && tile_pass_supported(dtype, head_dim, a.rep, false, 0);
+  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens, tiles_alone);
   a.chunk = p.chunk;
   a.tail_chunk = p.tail_chunk;
   a.n_pchunks = p.n_p;
@@ -499,8 +511,13 @@ extern "C" size_t da_decode_attention_workspace_bytes(int n_q_heads, int n_kv_he
     return 0;
   const int lanes = lanes_of(head_dim, dtype);
   if (!lanes) return 0;
-  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
-  return attn_workspace_bytes(n_q_heads, head_dim, p.total()) + 16;
+  // (whichever plan it will be)
+  int64_t most = 0;
+  for (const bool tiles_alone : {false, true}) {
+    const int64_t n = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens, tiles_alone).total();
+    if (n > most) most = n;
+  }
+  return attn_workspace_bytes(n_q_heads, head_dim, most) + 16;
 }
 
 extern "C" int da_decode_attention_paged(const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int dtype,

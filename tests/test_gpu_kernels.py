@@ -814,3 +814,37 @@ def test_page_cache_init_kernel(H, P, N):
     assert times.tolist() == [5.0] + [0.0] * (H * N) + [5.0]
     assert h2d.tolist() == [99] + list(range(P - N, P)) * H + [99]
     assert d2h.tolist() == [99] + ([-1] * (P - N) + list(range(N))) * H + [99]
+
+
+@pytest.mark.parametrize("layout", ["token by token", "head by head"])
+@pytest.mark.parametrize("H,rep,D,T,capacity", [
+    (4, 7, 128, 3, 5), (8, 4, 128, 1217, 300), (16, 1, 64, 4097, 64),   # few tokens, a chunk and one, short chunks
+    (8, 2, 128, 65536 - 64, 64), (8, 2, 128, 65536 - 64, 65),            # as much as the last-level cache, and more
+])
+def test_static_pass_by_layout_and_size(layout, H, rep, D, T, capacity):
+    """The attention pass of its own launch: which grid order it takes follows the layout, which loads the
+    size.  Against an fp32 computation of the same inputs: bf16 softmax weights and outputs (2^-9 of a weight
+    and of the result, sums in fp32), the bound of the other passes."""
+    from dram_attention_amd import decode_attention
+
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).bfloat16()
+
+    q, cache_k, cache_v, nk, nv = rand(H * rep, D), rand(capacity, H, D), rand(capacity, H, D), rand(H, D), rand(H, D)
+    if layout == "token by token":
+        k, v = (rand(T, H, D).transpose(0, 1) for _ in range(2))
+    else:
+        k, v = rand(H, T, D), rand(H, T, D)
+    n = capacity - 2
+    lse = torch.empty(H * rep, dtype=torch.float32, device=DEV)
+    out = decode_attention(q, k, v, cache_k, cache_v, n, nk, nv, lse=lse)
+    assert torch.equal(cache_k[n], nk) and torch.equal(cache_v[n], nv)
+    for h in range(H):
+        keys = torch.cat((k[h], cache_k[:n + 1, h])).float()
+        values = torch.cat((v[h], cache_v[:n + 1, h])).float()
+        scores = (q[h * rep:(h + 1) * rep].float() @ keys.t().contiguous()) * D ** -0.5
+        rows = slice(h * rep, (h + 1) * rep)
+        assert torch.allclose(lse[rows], scores.logsumexp(-1), atol=1e-3, rtol=1e-4), h
+        assert torch.allclose(out[rows].float(), scores.softmax(-1) @ values, atol=2e-2, rtol=1e-2), h
