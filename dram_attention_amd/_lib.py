@@ -52,6 +52,10 @@ SIGNATURES = {
     ),
     "da_page_cache_init": (
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]),
+    "da_prompt_cache": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int64, c_int, c_int64, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "da_pages_build": (
         c_int,
         [c_void_p, c_void_p, c_int64, c_int64, c_int, c_int64, c_int, c_int, c_int, c_void_p,

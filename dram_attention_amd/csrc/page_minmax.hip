@@ -6,72 +6,17 @@
 // One lane owns a 16-byte column chunk of one (page, head) and walks the
 // page's rows; adjacent lanes own adjacent chunks, heads vary next, so a wave
 // reads whole contiguous rows when the keys are laid out (token, head, dim).
-#include "common.hpp"
+#include "page_minmax.hpp"
 
 namespace da {
 
-// min/max that let NaN win, as torch.aminmax does.
-__device__ __forceinline__ float nan_min(float m, float x) { return (x < m || x != x) ? x : m; }
-__device__ __forceinline__ float nan_max(float m, float x) { return (x > m || x != x) ? x : m; }
-
-template <typename T>
-__device__ __forceinline__ u32x4 repack(const float *f);
-template <>
-__device__ __forceinline__ u32x4 repack<F32>(const float *f) {
-  u32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = __builtin_bit_cast(uint32_t, f[i]);
-  return v;
-}
-template <>
-__device__ __forceinline__ u32x4 repack<F16>(const float *f) {
-  u32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = pack_f16(f[2 * i], f[2 * i + 1]);
-  return v;
-}
-template <>
-__device__ __forceinline__ u32x4 repack<BF16>(const float *f) {
-  u32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = pack_bf16(f[2 * i], f[2 * i + 1]);
-  return v;
-}
-
-// Vector path: head_dim is a multiple of the 16-byte lane width and every
-// stride keeps 16-byte alignment.
 template <typename T>
 __global__ void __launch_bounds__(256)
 page_minmax_vec_kernel(const char *__restrict__ k, int64_t head_stride, int64_t tok_stride,
                        int n_heads, int64_t n_pages, int page, int chunks_per_row,
                        char *__restrict__ out) {
-  constexpr int V = T::kVec;
-  const int64_t items = n_pages * n_heads * chunks_per_row;
-  for (int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; it < items;
-       it += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(it % chunks_per_row);
-    const int64_t ph = it / chunks_per_row;
-    const int h = (int)(ph % n_heads);
-    const int64_t p = ph / n_heads;
-    const char *src =
-        k + (h * head_stride + p * page * tok_stride + (int64_t)c * V) * T::kBytes;
-    float mn[V], mx[V], f[V];
-    unpack<T>(load16(src), mn);
-#pragma unroll
-    for (int i = 0; i < V; ++i) mx[i] = mn[i];
-    for (int t = 1; t < page; ++t) {
-      unpack<T>(load16(src + (int64_t)t * tok_stride * T::kBytes), f);
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        mn[i] = nan_min(mn[i], f[i]);
-        mx[i] = nan_max(mx[i], f[i]);
-      }
-    }
-    const int64_t d = (int64_t)chunks_per_row * V;
-    char *dst = out + (((int64_t)h * n_pages + p) * 2 * d + (int64_t)c * V) * T::kBytes;
-    store16(dst, repack<T>(mn));
-    store16(dst + d * T::kBytes, repack<T>(mx));
-  }
+  page_minmax_vec<T>(k, head_stride, tok_stride, n_heads, n_pages, page, chunks_per_row, out,
+                     (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x);
 }
 
 // Scalar path for any head_dim / alignment.
@@ -105,9 +50,7 @@ static int launch_page_minmax(const void *k, int64_t head_stride, int64_t tok_st
                               int64_t n_pages, int page, int head_dim, void *out,
                               hipStream_t stream) {
   constexpr int V = T::kVec;
-  const bool vec = head_dim % V == 0 && head_stride % V == 0 && tok_stride % V == 0 &&
-                   ((uintptr_t)k % 16) == 0 && ((uintptr_t)out % 16) == 0;
-  if (vec) {
+  if (minmax_vec_fits(k, head_stride, tok_stride, head_dim, V == 4 ? DA_F32 : DA_F16, out)) {
     const int chunks = head_dim / V;
     const int64_t items = n_pages * n_heads * chunks;
     const int blocks = (int)(ceil_div(items, 256) < 65536 ? ceil_div(items, 256) : 65536);

@@ -437,6 +437,8 @@ class DRAMAttention(torch.nn.Module):
         prefix_k = k_cache[0, :paged].transpose(0, 1)
         prefix_v = v_cache[0, :paged].transpose(0, 1)
         link_gbps = cache = held = None
+        # (a selector of another kind may still refuse the prompt behind the launch)
+        in_one = self._caches_in_one_launch(k_cache, v_cache, paged) and self.page_selector == "bound"
         try:
             if paged > self.lru_hbm_cache_size:
                 if self.page_selector not in ("bound", "token_max"):
@@ -450,6 +452,8 @@ class DRAMAttention(torch.nn.Module):
                     top_k=self.top_k // self.page_size,
                     lru_hbm_cache_size=self.lru_hbm_cache_size,
                     device=self.device,
+                    fill=(lambda cache, summaries: self._fill_caches(k_cache, v_cache, paged, cache, summaries))
+                    if in_one else None,
                     **build,
                 )
                 if self.page_selector == "token_max":
@@ -457,14 +461,17 @@ class DRAMAttention(torch.nn.Module):
                         prefix_k, cache.num_dram_pages, device=self.device)
             else:
                 cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
-            tail = seqlen - paged
-            window_k, window_v = self.cache_k[:, :tail], self.cache_v[:, :tail]
-            tail_k, tail_v = k_cache[:, paged:], v_cache[:, paged:]
-            if not tail_k.shape == tail_v.shape == window_k.shape:
-                # (both are refused here or neither is)
-                tail_k, tail_v = tail_k.expand_as(window_k), tail_v.expand_as(window_v)
-            window_k.copy_(tail_k, non_blocking=True)
-            window_v.copy_(tail_v, non_blocking=True)
+                if in_one:
+                    self._fill_caches(k_cache, v_cache, paged)
+            if not in_one:
+                tail = seqlen - paged
+                window_k, window_v = self.cache_k[:, :tail], self.cache_v[:, :tail]
+                tail_k, tail_v = k_cache[:, paged:], v_cache[:, paged:]
+                if not tail_k.shape == tail_v.shape == window_k.shape:
+                    # (both are refused here or neither is)
+                    tail_k, tail_v = tail_k.expand_as(window_k), tail_v.expand_as(window_v)
+                window_k.copy_(tail_k, non_blocking=True)
+                window_v.copy_(tail_v, non_blocking=True)
             # Nothing refuses the prompt from here on.  The old cache is taken apart while the
             # new store is on its way, but for its own store, in pinned memory, which launches
             # of the last steps may still be reading until finish_build has waited.
@@ -476,6 +483,39 @@ class DRAMAttention(torch.nn.Module):
             if isinstance(cache, LRUCache):
                 cache.finish_build()
         del held
+
+    def _caches_in_one_launch(self, k, v, paged: int) -> bool:
+        """Whether da_prompt_cache may fill this layer's window (and page cache) from a prompt's (1,S,H,D)
+        keys and values: plain GPU tensors of the window's type on its device, aligned, one layout for
+        both, of the size that the window was made for."""
+        own = self._buffers
+        cache_k, cache_v = own["cache_k"], own["cache_v"]
+        tail, esize = k.shape[1] - paged, k.element_size()
+        return (paged >= 0 and 0 <= tail <= cache_k.shape[1] and k.is_cuda and k.shape == v.shape
+                and k.stride() == v.stride() and k.stride(3) == 1
+                and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is cache_k.dtype
+                        and t.device == cache_k.device for t in (k, v, cache_v))
+                and cache_k.shape == cache_v.shape and cache_k.shape[2:] == k.shape[2:]
+                and cache_k.is_contiguous() and cache_v.is_contiguous()
+                and all(n * esize % 16 == 0 for n in (k.stride(1), k.stride(2), k.shape[3]))
+                and all(t.data_ptr() % 16 == 0 for t in (k, v, cache_k, cache_v))
+                and not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad))
+                and torch.device(self.device).type == "cuda" and unobserved())
+
+    def _fill_caches(self, k, v, paged: int, cache=None, summaries=None) -> None:
+        """The local window (and ``cache``'s metadata and page summaries) in one launch."""
+        _, S, H, D = k.shape
+        page = [0, None, None, None, None, None]
+        if cache is not None:
+            b = cache._buffers
+            page = [cache.num_hbm_pages, summaries.data_ptr()] + [b[n].data_ptr() for n in (
+                "current_step", "page_access_time", "dram_page_to_hbm_page_mapping", "hbm_page_to_dram_page_mapping")]
+        _lib.check(
+            _lib.load().da_prompt_cache(
+                k.data_ptr(), v.data_ptr(), k.stride(1), k.stride(2), S, H, D, _lib.dtype_code(k.dtype),
+                paged // self.page_size, self.page_size, *page, self._buffers["cache_k"].data_ptr(),
+                self._buffers["cache_v"].data_ptr(), _lib.stream_ptr(k.device)),
+            "da_prompt_cache")
 
     def _paged_tokens(self, seqlen: int) -> int:
         """Prompt tokens that go to the paged prefix; the rest is the local window."""

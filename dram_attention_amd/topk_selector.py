@@ -103,13 +103,15 @@ class IPUpperboundTopKSelector:
     reference's kernel output is.
     """
 
-    def __init__(self, k_cache: torch.Tensor, num_pages: int, device="cuda"):
+    def __init__(self, k_cache: torch.Tensor, num_pages: int, device="cuda", *,
+                 summaries: torch.Tensor | None = None):
+        """``summaries``: what page_min_max gives for these keys, where somebody else makes it."""
         num_heads, dram_kv_cache_size, head_dim = k_cache.shape
         self.num_kv_heads = num_heads
         assert dram_kv_cache_size % num_pages == 0, "Cache size must be divisible by num_pages."
         self.device = torch.device(device)
         # the summaries are built on the GPU: host-resident keys are moved first
-        self.chunk_min_max = page_min_max(k_cache.to(device=device), num_pages)
+        self.chunk_min_max = page_min_max(k_cache.to(device=device), num_pages) if summaries is None else summaries
         # chunk_min_max comes from page_min_max, so min <= max in every channel and the
         # scorer may pick the bound by the sign of q; clear this after writing other
         # contents into chunk_min_max

@@ -129,6 +129,19 @@ int da_page_cache_init(int32_t *current_step, float *access_time, int64_t *dram_
                        int n_kv_heads, int64_t n_pages, int64_t n_slots, void *stream);
 
 /*
+ * What a prompt leaves behind besides its page store, as one launch: the summaries of its first n_pages
+ * pages (as da_page_minmax), the metadata of a page cache over them (as da_page_cache_init) and a copy
+ * of the other tokens (init_cache's local window, dram_attention.py:113-133).  With current_step NULL
+ * (a static prefix) the copy only.
+ *   k, v     : (n_tokens, Hkv, D), the same element strides (tok_stride, head_stride, 1); 16-byte aligned rows
+ *   window_k, window_v : (n_tokens - n_pages*page_size, Hkv, D), contiguous
+ */
+int da_prompt_cache(const void *k, const void *v, int64_t tok_stride, int64_t head_stride, int64_t n_tokens,
+                    int n_kv_heads, int head_dim, int dtype, int64_t n_pages, int page_size, int64_t n_slots,
+                    void *summaries, int32_t *current_step, float *access_time, int64_t *dram_to_hbm,
+                    int64_t *hbm_to_dram, void *window_k, void *window_v, void *stream);
+
+/*
  * Subsystem 1b — build the paged KV store from the prompt's keys and values.
  * Replaces the torch copies of LRUCache.__init__, dram_attention/lru_cache.py:131-141
  * (interleaved page layout in the pinned store) and :191-209 (initial slots).

@@ -572,3 +572,51 @@ def test_a_prompt_refused_late_leaves_the_layer_decoding_as_before(why, stage, m
     xq, xk, xv = draw(1, 4, 2, 64, torch.bfloat16, 3)
     assert same(m(xq, xk, xv, start_pos=1000, stage="generate"), ref(xq, xk, xv, start_pos=1000, stage="generate"))
     assert same(m.cache_k, ref.cache_k) and same(m.cache_v, ref.cache_v)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S,local,lru,page,kind", [
+    (1500, 200, 320, 16, "plain"), (1511, 200, 320, 16, "plain"),    # pages and a window that ends inside one
+    (3000, 1000, 640, 32, "view"), (700, 203, 4096, 16, "plain"),    # strided prompt; static prefix
+    (150, 160, 4096, 16, "view"), (700, 16, 0, 16, "plain"),         # the window alone, no slots
+    (1500, 200, 320, 16, "odd rows"), (1500, 200, 320, 16, "unlike values"),   # left to the launches of their own
+])
+def test_prompt_caches_in_one_launch_equal_the_separate_ones(dtype, S, local, lru, page, kind, monkeypatch):
+    """Summaries, page cache metadata and window, bit for bit, and which prompts the launch is for."""
+    from dram_attention_amd import DRAMAttention, LRUCache
+
+    H, D = 3, 64
+    g = torch.Generator(device=DEV).manual_seed(S)
+
+    def rand(width):
+        return torch.randn(1, S, H, width, device=DEV, generator=g).to(dtype)
+
+    if kind == "plain":
+        k, v = rand(D), rand(D)
+    elif kind == "view":
+        k, v = rand(2 * D)[..., :D], rand(2 * D)[..., D:]
+    elif kind == "odd rows":
+        k, v = rand(D + 1)[..., :D], rand(D + 1)[..., :D]
+    else:
+        k, v = rand(D), rand(2 * D)[..., :D]
+    launches, fill = [], DRAMAttention._fill_caches
+    monkeypatch.setattr(DRAMAttention, "_fill_caches", lambda *a: launches.append(1) or fill(*a))
+
+    def layer():
+        m = DRAMAttention(8, lru, local, page, 4 * page, H, D, device=DEV, dtype=dtype)
+        m.init_cache(k, v)
+        return m
+
+    one = layer()
+    assert len(launches) == (kind in ("plain", "view"))
+    with monkeypatch.context() as patch:
+        patch.setattr(DRAMAttention, "_caches_in_one_launch", lambda *a: False)
+        many = layer()
+    for name in ("cache_k", "cache_v"):
+        assert torch.equal(getattr(one, name), getattr(many, name)), name
+    assert type(one.lru_cache) is type(many.lru_cache) and one.dram_kv_cache_size == many.dram_kv_cache_size
+    if isinstance(one.lru_cache, LRUCache):
+        for name in ("current_step", "page_access_time", "dram_page_to_hbm_page_mapping",
+                     "hbm_page_to_dram_page_mapping", "dram_kv_cache", "hbm_kv_cache"):
+            assert torch.equal(getattr(one.lru_cache, name), getattr(many.lru_cache, name)), name
+        assert torch.equal(one.lru_cache.top_k_selector.chunk_min_max, many.lru_cache.top_k_selector.chunk_min_max)
