@@ -4,29 +4,31 @@
 //
 // Bound: latency, a chain of dependent steps over a few KB.  What counts is how few of them
 // there are and that they stay inside a wave or, at worst, inside the workgroup:
-//   - a wave selects a row, its keys in registers (key j*64 + lane in register j): the k-th
-//     largest by bisection from the highest bit in which two keys differ (a compare and an add
-//     per register and bit, one sum over the wave per bit; it ends as soon as exactly k keys
-//     reach the threshold), the survivors compacted by ballots and ordered by counting, without
-//     one barrier;
+//   - a wave selects a row, its keys in registers (key j*64 + lane in register j): the k-th largest by
+//     histograms of eight bits from the highest in which two keys differ (bf16 scores: two at
+//     most; it ends as soon as a whole bin is wanted), the survivors compacted by every lane for
+//     itself and ordered by counting, without one barrier;
 //   - another wave meanwhile puts all slots in order of their access times by a stable radix
 //     sort that only it takes part in, so the list of least recent slots is complete;
 //   - both page maps are in LDS by then (a short row has few pages): the update reads nothing
 //     from memory, with one thread per request and one per slot.
 // us a launch (under the profiler; in brackets a workgroup a row): 512 pages of 2 heads in fp32, 4 rows of
-// 32 pages, 128 slots 6.4 (13.1); 445 of 4 heads in bf16, the same lists 6.3 (12.2); 1000 of 8 heads, 4 rows of 64, 256
-// slots 8.8 (12.0), of 128, 512 slots 10.0 (12.8); 8 rows of 60 11.6 (13.6); fp32, 100 of 1000 pages 9.4 (13.6).
+// 32 pages, 128 slots 5.9 (12.9); 445 of 4 heads in bf16, the same lists 6.2 (12.0); 1000 of 8 heads, 4 rows of 64,
+// 256 slots 7.3 (12.1), of 128, 512 slots 9.4 (13.3); 8 rows of 60 10.8 (13.6); 2047 of 8 heads, 4 rows of 128, 512
+// slots 10.5 (13.1); fp32, 100 of 1000 pages 8.7 (13.5), 120 of 1800, 900 slots 12.3 (14.0).  Bisection bit by bit
+// in place of the histograms: 6.4 for the first, 13.0 for 2047 pages.
 //
-// The rule (topk_lru_short): rows of at most 1024 pages (with a register more for every 64, 2047 pages of
-// 8 heads took 12.2 to 13.4 where a workgroup a row takes 12.6 to 14.3, and 1800 pages with 1000
-// slots 13.6 where it takes 12.8: the bisection grows with the row and the sort with the slots, and
-// both have one wave), 8 rows a head, lists of 128 pages (ordering by counting grows with the
-// square), 1024 requests and 1024 slots (a thread each).
+// The rule (topk_lru_short): rows of at most 2048 pages (32 registers of keys), 8 rows a head, lists of
+// 128 pages (ordering by counting grows with the square), 1024 requests and 1024 slots (a thread each);
+// of the slots no more than 896 where the row is longer than 1024 pages: the one wave that sorts them
+// is the last to be done there (1800 pages, 7 rows of 100, 1000 slots 13.5 (13.3)).
+#include <type_traits>
+
 #include "topk_rows.hpp"
 
 namespace da {
 
-constexpr int kShortPages = 1024, kShortRows = 8, kShortList = 128;
+constexpr int kShortPages = 2048, kShortRows = 8, kShortList = 128;
 constexpr int kShortSlots = kSelThreads;
 constexpr int kShortSlotRegs = kShortSlots / 64;
 constexpr int kSlotWave = kSelWaves - 1;   // the wave that orders the slots
@@ -48,8 +50,10 @@ struct ShortBatch {
   ShortLayer layer[kLayers];
 };
 
+constexpr int kShortCopies = 4;   // of a row's histogram
 struct alignas(16) ShortShared {
   uint64_t words[kShortRows][kShortList + 4];   // a row's survivors, while it orders them
+  uint32_t hist[kShortRows][256 * kShortCopies];
   uint32_t slot_key[kShortSlots];
   uint32_t digit_at[256];
   uint16_t order[2][kShortSlots];               // slots, least recent first, by turns
@@ -86,17 +90,16 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
   v = max(v, dpp_u32<0x143, 0xc>(v));
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_inclusive(v), 63);
-}
-
 // The k <= kShortList largest of the n <= 64 * kKeys values of `row`, ties by lowest index, in
-// order: emit(rank, index).  One wave; `words`: its room in LDS.  kRounded: values rounded to a
-// 16-bit type, whose keys below the upper 19 bits say nothing more: key and index fit one word then.
-template <int kKeys, bool kRounded, typename Emit>
-__device__ __forceinline__ void select_row(const float *row, int n, int k, uint64_t *words, const Emit &emit) {
-  constexpr uint32_t kCounts = kRounded ? 0xffffe000u : 0xffffffffu, kIndex = 0x3ffu;
-  static_assert(kKeys * 64 <= kIndex + 1, "an index of 10 bits");
+// order: emit(rank, index).  One wave; `words` and `hist`: its room in LDS.  kLow: the lowest bit
+// of a key that says anything (values rounded to a 16-bit type: 16 for bf16, 13 for fp16; key and
+// index then fit one word).
+template <int kKeys, int kLow, typename Emit>
+__device__ __forceinline__ void select_row(const float *row, int n, int k, uint64_t *words, uint32_t *hist,
+                                           const Emit &emit) {
+  constexpr bool kOneWord = kLow > 0;
+  constexpr uint32_t kCounts = ~0u << kLow, kIndex = 0x7ffu;
+  static_assert(kKeys * 64 <= kIndex + 1 && (!kOneWord || kIndex < (1u << kLow)), "an index of 11 bits");
   const int lane = threadIdx.x & 63;
   uint32_t key[kKeys];
   uint32_t most = 0, not_least = 0;
@@ -117,89 +120,125 @@ __device__ __forceinline__ void select_row(const float *row, int n, int k, uint6
     }
   }
   most = wave_max(most);
-  const uint32_t differ = most ^ ~wave_max(not_least);
-  // bits from the highest in which two keys differ down, and the threshold as far as it is known
-  uint32_t bit = differ == 0 ? 0u : 0x80000000u >> __builtin_clz(differ);
-  uint32_t least = bit == 0 ? most : most & ~(bit | (bit - 1u));
-  bool exact = false;                            // exactly k keys reach `least`
-  for (; bit >= (kCounts & -kCounts) && !exact; bit >>= 1) {
-    // (counted per lane and folded once: a ballot per register costs five times the compare)
-    const uint32_t reach = least | bit;
-    uint32_t n_in = 0;
+  const uint32_t differ = most ^ (~wave_max(not_least) & kCounts);
+  // The k-th largest key, eight bits a pass from the highest in which two keys differ: a histogram of the
+  // keys that share the bits known so far, a few copies of it, and the bin that holds the k-th.
+  int top = differ == 0 ? kLow - 1 : 31 - __builtin_clz(differ);
+  uint32_t least = top >= kLow ? most & ~((2u << top) - 1u) : most;
+  int want = k;                                  // of the keys that begin like `least`
+  bool exact = false;                            // all of those are wanted
+  for (bool first = true; top >= kLow && !exact; first = false) {
+    const int shift = top - 7 > kLow ? top - 7 : kLow;
+    const uint32_t mask = (2u << (top - shift)) - 1u;
 #pragma unroll
-    for (int j = 0; j < kKeys; ++j) n_in += key[j] >= reach ? 1u : 0u;
-    n_in = wave_sum(n_in);
-    if (n_in >= (uint32_t)k) least = reach;
-    exact = n_in == (uint32_t)k;
+    for (int u = 0; u < kShortCopies; ++u) *(u32x4 *)(hist + (u * 64 + lane) * 4) = u32x4{0, 0, 0, 0};
+    wave_step();
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j)
+      if (first || (key[j] ^ least) >> top < 2u)  // (bits above `top` the same)
+        atomicAdd(&hist[(key[j] >> shift & mask) * kShortCopies + (lane & (kShortCopies - 1))], 1u);
+    wave_step();
+    uint32_t c[4], mine = 0;                     // bins 255 - 4 lane and the three below
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      static_assert(kShortCopies == 4, "a bin's copies are one 16-byte read");
+      const u32x4 w = *(const u32x4 *)(hist + (255 - 4 * lane - x) * kShortCopies);
+      c[x] = w[0] + w[1] + w[2] + w[3];
+      mine += c[x];
+    }
+    const uint32_t upto = wave_scan_inclusive(mine), before = upto - mine;
+    const bool here = before < (uint32_t)want && (uint32_t)want <= upto;     // in one lane
+    uint32_t above = before, bin = 255 - 4 * lane, count = c[0];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+      if (bin == 255u - 4 * lane - x && above + c[x] < (uint32_t)want) {
+        above += c[x];
+        count = c[x + 1];
+        --bin;
+      }
+    const int at = __builtin_ctzll(__ballot(here));
+    above = (uint32_t)__builtin_amdgcn_readlane((int)above, at);
+    bin = (uint32_t)__builtin_amdgcn_readlane((int)bin, at);
+    count = (uint32_t)__builtin_amdgcn_readlane((int)count, at);
+    least |= bin << shift;
+    want -= (int)above;
+    exact = want == (int)count;
+    top = shift - 1;
   }
-  // Compaction: keys above the k-th largest, then as many equal to it as are wanted.
+  // Compaction, each lane its own: the keys above the threshold (exact: and those that begin like it), in any
+  // order; then as many equal to it as are wanted, the lowest indices, by ballots where there are any.
   uint32_t *words32 = (uint32_t *)words;
-  auto keep = [&](uint32_t at, int j) {
+  auto keep = [&](uint32_t to, int j) {
     const uint32_t i = (uint32_t)(j * 64 + lane);
-    if constexpr (kRounded) words32[at] = key[j] | (kIndex - i);
-    else words[at] = (uint64_t)key[j] << 32 | (uint64_t)(kIndex - i);
+    if constexpr (kOneWord) words32[to] = key[j] | (kIndex - i);
+    else words[to] = (uint64_t)key[j] << 32 | (uint64_t)(kIndex - i);
   };
-  uint32_t at = 0;
+  auto above_all = [&](auto in) {
+    uint32_t mine = 0;
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j) mine += in(j) ? 1u : 0u;
+    uint32_t to = wave_scan_inclusive(mine) - mine;
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j)
+      if (in(j)) keep(to++, j);
+  };
   if (exact) {
-#pragma unroll
-    for (int j = 0; j < kKeys; ++j) {
-      const uint64_t m = __ballot(key[j] >= least);
-      if (key[j] >= least) keep(at + lanes_below(m), j);
-      at += (uint32_t)__popcll(m);
-    }
+    above_all([&](int j) { return key[j] >= least && j * 64 + lane < n; });
   } else {
-#pragma unroll
-    for (int j = 0; j < kKeys; ++j) {
-      const uint64_t m = __ballot(key[j] > least);
-      if (key[j] > least) keep(at + lanes_below(m), j);
-      at += (uint32_t)__popcll(m);
-    }
+    above_all([&](int j) { return key[j] > least; });
+    uint32_t to = (uint32_t)(k - want);
 #pragma unroll
     for (int j = 0; j < kKeys; ++j) {
       const uint64_t m = __ballot(key[j] == least);
-      const uint32_t mine = at + lanes_below(m);
+      if (m == 0 || to >= (uint32_t)k) continue;
+      const uint32_t mine = to + lanes_below(m);
       if (key[j] == least && mine < (uint32_t)k) keep(mine, j);
-      at += (uint32_t)__popcll(m);
+      to += (uint32_t)__popcll(m);
     }
   }
   if (lane < 4) {                                // (zeroes, which beat nothing, up to a whole read)
-    if constexpr (kRounded) words32[k + lane] = 0;
+    if constexpr (kOneWord) words32[k + lane] = 0;
     else words[k + lane] = 0;
   }
   wave_step();
   // Order: all words are distinct, a word's rank is how many are larger.
-  uint32_t rank[2] = {0, 0}, index[2];
-  if constexpr (kRounded) {
-    uint32_t mine[2];
+  auto order = [&](auto two) {
+    constexpr int kMine = decltype(two)::value;
+    uint32_t rank[kMine] = {}, index[kMine];
+    if constexpr (kOneWord) {
+      uint32_t mine[kMine];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      mine[e] = lane + 64 * e < k ? words32[lane + 64 * e] : 0xffffffffu;
-      index[e] = kIndex - (mine[e] & kIndex);
-    }
+      for (int e = 0; e < kMine; ++e) {
+        mine[e] = lane + 64 * e < k ? words32[lane + 64 * e] : 0xffffffffu;
+        index[e] = kIndex - (mine[e] & kIndex);
+      }
 #pragma unroll 4
-    for (int i = 0; i < k; i += 4) {
-      const u32x4 w = *(const u32x4 *)(words32 + i);
+      for (int i = 0; i < k; i += 4) {
+        const u32x4 w = *(const u32x4 *)(words32 + i);
 #pragma unroll
-      for (int e = 0; e < 2; ++e)
-        rank[e] += (w[0] > mine[e]) + (w[1] > mine[e]) + (w[2] > mine[e]) + (w[3] > mine[e]);
-    }
-  } else {
-    uint64_t mine[2];
+        for (int e = 0; e < kMine; ++e)
+          rank[e] += (w[0] > mine[e]) + (w[1] > mine[e]) + (w[2] > mine[e]) + (w[3] > mine[e]);
+      }
+    } else {
+      uint64_t mine[kMine];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      mine[e] = lane + 64 * e < k ? words[lane + 64 * e] : ~0ull;
-      index[e] = kIndex - (uint32_t)mine[e];
-    }
+      for (int e = 0; e < kMine; ++e) {
+        mine[e] = lane + 64 * e < k ? words[lane + 64 * e] : ~0ull;
+        index[e] = kIndex - (uint32_t)mine[e];
+      }
 #pragma unroll 4
-    for (int i = 0; i < k; i += 2) {
-      const u64x2 w = *(const u64x2 *)(words + i);
+      for (int i = 0; i < k; i += 2) {
+        const u64x2 w = *(const u64x2 *)(words + i);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) rank[e] += (w[0] > mine[e]) + (w[1] > mine[e]);
+        for (int e = 0; e < kMine; ++e) rank[e] += (w[0] > mine[e]) + (w[1] > mine[e]);
+      }
     }
-  }
 #pragma unroll
-  for (int e = 0; e < 2; ++e)
-    if (lane + 64 * e < k) emit(rank[e], index[e]);
+    for (int e = 0; e < kMine; ++e)
+      if (lane + 64 * e < k) emit(rank[e], index[e]);
+  };
+  if (k <= 64) order(std::integral_constant<int, 1>{});
+  else order(std::integral_constant<int, 2>{});
 }
 
 // All slots in eviction order (access time, then slot) into sm.order[sm.ordered].  One wave: a
@@ -216,11 +255,16 @@ __device__ __forceinline__ void order_slots(const float *time, int n_slots, Shor
       const int i = j * 64 + lane;
       v[j] = j * 64 < n_slots ? time[i < n_slots ? i : n_slots - 1] : 0.f;
     }
+    // (step counts: as whole numbers they differ in fewer, lower bits than as floats)
+    bool whole = true;
+#pragma unroll
+    for (int j = 0; j < kShortSlotRegs; ++j) whole = whole && v[j] >= 0.f && v[j] <= 0x1p24f && v[j] == truncf(v[j]);
+    whole = __all(whole);
 #pragma unroll
     for (int j = 0; j < kShortSlotRegs; ++j) {
       const int i = j * 64 + lane;
       if (i < n_slots) {
-        const uint32_t key = float_order_key(v[j]);
+        const uint32_t key = whole ? (uint32_t)v[j] : float_order_key(v[j]);
         sm.slot_key[i] = key;
         sm.order[0][i] = (uint16_t)i;
         ones |= key;
@@ -276,7 +320,7 @@ __device__ __forceinline__ void order_slots(const float *time, int n_slots, Shor
   if (lane == 0) sm.ordered = from;
 }
 
-template <int kKeys, bool kRounded, int kLayers>
+template <int kKeys, int kLow, int kLayers>
 __global__ void __launch_bounds__(kSelThreads)
 select_update_short_kernel(const ShortBatch<kLayers> batch) {
   __shared__ ShortShared sm;
@@ -306,7 +350,7 @@ select_update_short_kernel(const ShortBatch<kLayers> batch) {
     const float *row = l.scores + ((int64_t)wave * n_heads + h) * n_pages;
     int64_t *dst = l.idx + (int64_t)h * K + wave * kp;
     uint16_t *request = sm.request + wave * kp;
-    select_row<kKeys, kRounded>(row, n_pages, kp, sm.words[wave], [=](uint32_t rank, uint32_t page) {
+    select_row<kKeys, kLow>(row, n_pages, kp, sm.words[wave], sm.hist[wave], [=](uint32_t rank, uint32_t page) {
       dst[rank] = (int64_t)page;
       request[rank] = (uint16_t)page;
     });
@@ -372,10 +416,10 @@ select_update_short_kernel(const ShortBatch<kLayers> batch) {
 bool topk_lru_short(const da_decode_step_args &a) {
   const int rep = a.n_q_heads / a.n_kv_heads;
   return a.n_pages <= kShortPages && rep <= kShortRows && a.kp <= kShortList && rep * a.kp <= kSelThreads &&
-         a.n_slots <= kShortSlots && rep * a.kp <= a.n_slots;
+         a.n_slots <= (a.n_pages <= 1024 ? kShortSlots : 896) && rep * a.kp <= a.n_slots;
 }
 
-template <int kKeys, bool kRounded, int kLayers>
+template <int kKeys, int kLow, int kLayers>
 static void launch_short(const da_decode_step_args *a, int n, hipStream_t s) {
   ShortBatch<kLayers> batch;
   for (int i = 0; i < n; ++i)
@@ -383,27 +427,29 @@ static void launch_short(const da_decode_step_args *a, int n, hipStream_t s) {
                       a[i].k_cand, a[i].idx, a[i].access_time, a[i].d2h, a[i].h2d, a[i].step,
                       (int32_t *)a[i].lru_workspace, a[i].candidates, a[i].miss_page, a[i].miss_slot, a[i].miss_count,
                       a[i].slot_epoch, a[i].hit_mask};
-  hipLaunchKernelGGL((select_update_short_kernel<kKeys, kRounded, kLayers>), dim3(a->n_kv_heads, n),
+  hipLaunchKernelGGL((select_update_short_kernel<kKeys, kLow, kLayers>), dim3(a->n_kv_heads, n),
                      dim3(kSelThreads), 0, s, batch);
 }
 
-template <int kKeys, bool kRounded>
+template <int kKeys, int kLow>
 static void launch_short(const da_decode_step_args *a, int n, hipStream_t s) {
-  if (n == 1) launch_short<kKeys, kRounded, 1>(a, n, s);
-  else launch_short<kKeys, kRounded, kStepBatch>(a, n, s);
+  if (n == 1) launch_short<kKeys, kLow, 1>(a, n, s);
+  else launch_short<kKeys, kLow, kStepBatch>(a, n, s);
 }
 
-template <bool kRounded>
+template <int kLow>
 static void launch_short(const da_decode_step_args *a, int n, hipStream_t s) {
-  if (a->n_pages <= 512) launch_short<8, kRounded>(a, n, s);
-  else launch_short<16, kRounded>(a, n, s);
+  if (a->n_pages <= 512) launch_short<8, kLow>(a, n, s);
+  else if (a->n_pages <= 1024) launch_short<16, kLow>(a, n, s);
+  else launch_short<32, kLow>(a, n, s);
 }
 
 int launch_topk_lru_short(const da_decode_step_args *a, int n, hipStream_t s) {
-  bool rounded = true;      // (layers may differ in their flags)
-  for (int i = 0; i < n; ++i) rounded = rounded && a[i].dtype != DA_F32 && (a[i].score_flags & DA_SCORE_ROUND);
-  if (rounded) launch_short<true>(a, n, s);
-  else launch_short<false>(a, n, s);
+  bool rounded = a->dtype != DA_F32;      // (layers may differ in their flags)
+  for (int i = 0; i < n; ++i) rounded = rounded && (a[i].score_flags & DA_SCORE_ROUND);
+  if (!rounded) launch_short<0>(a, n, s);
+  else if (a->dtype == DA_BF16) launch_short<16>(a, n, s);
+  else launch_short<13>(a, n, s);
   return launch_status("da_decode_step(selection of short rows)");
 }
 

@@ -958,11 +958,15 @@ def test_selection_and_update_in_one_launch(Hq, Hkv, slots, kp, S):
     (8, 2, 128, 32, 512, torch.float32, 2, 4000),      # few distinct scores: the threshold is a tie
     (4, 1, 65, 16, 66, torch.bfloat16, 0, 0),          # two registers of keys, two of slots, each but started
     (1, 1, 2, 1, 3, torch.float16, 0, 0),              # one request a step
-    (7, 1, 1023, 128, 1024, torch.bfloat16, 1, 16777000),   # the longest row and list, all scores alike
+    (7, 1, 1023, 128, 1024, torch.bfloat16, 1, 16777000),   # the longest list, all scores alike
+    (7, 1, 896, 128, 2048, torch.bfloat16, 0, 16777100),    # the longest row, the most slots beside it
+    (8, 1, 897, 100, 2048, torch.bfloat16, 0, 0),           # and one more
+    (8, 2, 500, 64, 2048, torch.float32, 2, 0), (14, 2, 900, 65, 2047, torch.float16, 0, 300),
+    (8, 2, 700, 128, 1025, torch.float16, 4, 0),
     (8, 1, 1022, 127, 1024, torch.float16, 0, 255),    # nearly the most requests and slots
     (16, 2, 1000, 100, 1023, torch.bfloat16, 3, 65535),
     (12, 2, 600, 65, 1024, torch.float32, 1, 70000),
-    (16, 2, 1024, 128, 1025, torch.bfloat16, 0, 0), (9, 1, 600, 50, 700, torch.bfloat16, 0, 0),   # one page, one row
+    (16, 2, 1024, 128, 2049, torch.bfloat16, 0, 0), (9, 1, 600, 50, 700, torch.bfloat16, 0, 0),   # one page, one row
     (2, 1, 600, 129, 700, torch.bfloat16, 0, 0),       # and one listed page too many
 ])
 def test_selection_and_update_of_short_rows(Hq, Hkv, slots, kp, pages, dtype, levels, step0):
