@@ -437,8 +437,16 @@ class DRAMAttention(torch.nn.Module):
         prefix_k = k_cache[0, :paged].transpose(0, 1)
         prefix_v = v_cache[0, :paged].transpose(0, 1)
         link_gbps = cache = held = None
-        # (a selector of another kind may still refuse the prompt behind the launch)
-        in_one = self._caches_in_one_launch(k_cache, v_cache, paged) and self.page_selector == "bound"
+        filled = []
+
+        def fill(cache=None):
+            # (looked at when the store and attention are on their way.  A selector of another kind
+            # may still refuse the prompt behind the launch)
+            if self.page_selector != "bound" or not self._caches_in_one_launch(k_cache, v_cache, paged):
+                return None
+            filled.append(True)
+            return self._fill_caches(k_cache, v_cache, paged, cache)
+
         try:
             if paged > self.lru_hbm_cache_size:
                 if self.page_selector not in ("bound", "token_max"):
@@ -452,8 +460,7 @@ class DRAMAttention(torch.nn.Module):
                     top_k=self.top_k // self.page_size,
                     lru_hbm_cache_size=self.lru_hbm_cache_size,
                     device=self.device,
-                    fill=(lambda cache, summaries: self._fill_caches(k_cache, v_cache, paged, cache, summaries))
-                    if in_one else None,
+                    fill=fill,
                     **build,
                 )
                 if self.page_selector == "token_max":
@@ -461,9 +468,8 @@ class DRAMAttention(torch.nn.Module):
                         prefix_k, cache.num_dram_pages, device=self.device)
             else:
                 cache = DummyCache(k_cache=prefix_k, v_cache=prefix_v, device=self.device)
-                if in_one:
-                    self._fill_caches(k_cache, v_cache, paged)
-            if not in_one:
+                fill()
+            if not filled:
                 tail = seqlen - paged
                 window_k, window_v = self.cache_k[:, :tail], self.cache_v[:, :tail]
                 tail_k, tail_v = k_cache[:, paged:], v_cache[:, paged:]
@@ -502,12 +508,13 @@ class DRAMAttention(torch.nn.Module):
                 and not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad))
                 and torch.device(self.device).type == "cuda" and unobserved())
 
-    def _fill_caches(self, k, v, paged: int, cache=None, summaries=None) -> None:
-        """The local window (and ``cache``'s metadata and page summaries) in one launch."""
+    def _fill_caches(self, k, v, paged: int, cache=None):
+        """The local window (and ``cache``'s metadata and the page summaries, returned) in one launch."""
         _, S, H, D = k.shape
-        page = [0, None, None, None, None, None]
+        summaries, page = None, [0, None, None, None, None, None]
         if cache is not None:
             b = cache._buffers
+            summaries = torch.empty(H, cache.num_dram_pages, 2, D, dtype=k.dtype, device=k.device)
             page = [cache.num_hbm_pages, summaries.data_ptr()] + [b[n].data_ptr() for n in (
                 "current_step", "page_access_time", "dram_page_to_hbm_page_mapping", "hbm_page_to_dram_page_mapping")]
         _lib.check(
@@ -516,6 +523,7 @@ class DRAMAttention(torch.nn.Module):
                 paged // self.page_size, self.page_size, *page, self._buffers["cache_k"].data_ptr(),
                 self._buffers["cache_v"].data_ptr(), _lib.stream_ptr(k.device)),
             "da_prompt_cache")
+        return summaries
 
     def _paged_tokens(self, seqlen: int) -> int:
         """Prompt tokens that go to the paged prefix; the rest is the local window."""

@@ -64,15 +64,15 @@ class LRUCache(torch.nn.Module):
         build_stream: Optional[torch.cuda.Stream] = None,
         build_blocks: int = 0,
         beside: Optional[Callable[[], None]] = None,
-        fill: Optional[Callable[["LRUCache", torch.Tensor], None]] = None,
+        fill: Optional[Callable[["LRUCache"], Optional[torch.Tensor]]] = None,
     ):
         """``beside`` (with ``build_stream``): work that the caller issues on the current
         stream as soon as the page store is being written, on ``build_stream`` and by at most
         ``build_blocks`` workgroups; the rest of the construction is issued behind it.  The
         caller then ends the build with :meth:`finish_build` before anything reads or frees
         the keys, the store or the slots.  Without it the store is complete on return.
-        ``fill``: issues the page summaries and this cache's metadata (da_prompt_cache) into the
-        buffers it is given."""
+        ``fill``, called behind ``beside``: issues this cache's metadata and the page summaries
+        (da_prompt_cache) and returns these, or does nothing and returns None."""
         super().__init__()
         assert k_cache.shape == v_cache.shape, "Key and value cache shapes must match."
         num_kv_heads, dram_kv_cache_size, head_dim = k_cache.shape
@@ -147,12 +147,9 @@ class LRUCache(torch.nn.Module):
         try:
             if beside is not None:
                 beside()
-            summaries = None if fill is None else torch.empty(
-                num_kv_heads, num_dram_pages, 2, head_dim, dtype=dtype, device=self.hbm_kv_cache.device)
+            summaries = None if fill is None else fill(self)
             self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device, summaries=summaries)
-            if fill is not None:
-                fill(self, summaries)
-            else:
+            if summaries is None:
                 _lib.check(
                     _lib.load().da_page_cache_init(
                         self.current_step.data_ptr(), self.page_access_time.data_ptr(),
