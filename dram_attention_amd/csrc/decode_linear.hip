@@ -23,8 +23,8 @@
 // Measured (bf16, in a decode step, each with its endings; in brackets the library products
 // alone): vocabulary 128256 x 4096 160 us = 6.6 TB/s (188); 2 x 14336 x 4096 39 us = 6.0 TB/s
 // (57); 4096 x 14336 22 us (26); queries, keys and values 6144 x 4096 11.5 us (44 in three
-// launches).  A token through four such layers over 32K-token prefixes, one graph: 1.41 -> 1.04 ms;
-// through four layers of dim 2048 from Python, 72 -> 38 launches: 1.38 -> 0.67 ms.
+// launches).  A token through four such layers over 32K-token prefixes, one graph, library products /
+// these: 1.41 / 1.04 ms; through four layers of dim 2048 from Python, 72 / 38 launches: 1.38 / 0.67 ms.
 #include "attention_core.hpp"
 #include "model_math.hpp"
 

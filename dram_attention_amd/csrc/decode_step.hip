@@ -4,10 +4,10 @@
 // reference).  Host code only: it issues the launches of the entry points it stands for, on the
 // operands of one argument block, selection and LRU update as one where their sizes allow.
 //
-// What it saves is the caller's time: a step of the small layers takes 35 us of the GPU and
-// 86 us of Python that marshals five calls of 18 to 33 arguments.  With one call: 34 us a step
-// for the fp32 layer over 8K tokens (85 before), 435 us a token for four 2048-wide model layers
-// launched from Python (674 before).
+// What it saves is the caller's time: five calls of 18 to 33 arguments take 86 us to marshal from
+// Python, where a step of the small layers takes 25 us of the GPU.  Five calls / this one: the fp32
+// layer over 8K tokens 85 / 34 us a step, four 2048-wide model layers launched from Python
+// 674 / 435 us a token (25 and 277 since, by what the one call is made of).
 //
 // Several layers whose queries do not depend on each other (da_decode_steps): all scores in a
 // launch, all selections and updates in a launch, all page streams in a launch
@@ -46,7 +46,7 @@ static int scores_of(const da_decode_step_args &a, void *stream) {
 
 // (Rows of more than 4096 pages keep the two launches: their steps stream for so long that the caller's
 // time is hidden, and on the GPU the hand-over is 0.4 us slower there than a launch: 128K tokens 160.8 /
-// 161.5 us; 3064 pages 81.2 / 81.0; 513 pages 32.5 / 31.6.)
+// 161.5 us; 3064 pages 81.2 / 81.0.  Rows of up to 2048 pages are select_short.hip's in most cases.)
 static int select_and_update(const da_decode_step_args &a, void *stream) {
   if (a.n_pages <= 4096 && topk_lru_in_one_launch(a)) return launch_topk_lru(&a, 1, (hipStream_t)stream);
   const int H = a.n_kv_heads, rep = a.n_q_heads / H, K = rep * a.kp;

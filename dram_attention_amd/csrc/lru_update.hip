@@ -416,10 +416,9 @@ static void launch_lru_time(int time_type, dim3 grid, hipStream_t s, const void 
 // row, one for the list of least recent slots, and whichever of them is done last goes on to the
 // update.  What they hand over, the requests and the list, is written through to memory and read
 // from there (a few KB per head), which takes almost as long as the launch of the update that it
-// saves; the caller, who has one launch less to issue, gains more.  A step of the fp32 layer over
-// 8K tokens, two launches / one in three pairs of runs: 32.8 / 31.7, 32.9 / 31.5, 32.8 / 31.8 us (a host thread's part
-// of it 36 / 33).  A token of four 2048-wide layers launched from Python 348 / 335, 334 / 333, 351 / 333, where two runs of
-// one form differ by 2 to 7 %; steps that stream for 60 us and more gain nothing (decode_step.hip).
+// saves; the caller, who has one launch less to issue, gains 3 us of 36 a step.  Steps that stream for
+// 60 us and more gain nothing (decode_step.hip).  Short rows have a kernel whose one workgroup per head hands
+// nothing over (select_short.hip: 512 pages 5.9 us a launch, here 12.9); this one is for the others.
 struct TopkLruLayer {
   const float *scores;  // (rows, heads, pages)
   int n_rows, n_pages, kp;
