@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -113,8 +114,37 @@ PyObject *raise(int rc, const char *what) {
   PyErr_Format(PyExc_RuntimeError, "%s failed (code %d): %s", what, rc, da_last_error_string());
   return nullptr;
 }
-at::Tensor empty_like(at::IntArrayRef sizes, const at::Tensor &x) { return at::empty(sizes, x.options().requires_grad(false)); }
+// Other Python threads run while this one allocates or launches: either may wait, an allocation for
+// another thread that holds the allocator, a launch for room in its queue.
+struct Released {
+  PyThreadState *state = PyEval_SaveThread();
+  ~Released() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+int unlocked(F call) {
+  const Released others;
+  return call();
+}
+at::Tensor empty_like(at::IntArrayRef sizes, const at::Tensor &x) {
+  const Released others;
+  return at::empty(sizes, x.options().requires_grad(false));
+}
 PyObject *wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
+// A tuple that takes these over; null, with the error that is set, if one is.
+PyObject *tuple_of(std::initializer_list<PyObject *> items) {
+  PyObject *result = PyTuple_New((Py_ssize_t)items.size());
+  bool whole = result != nullptr;
+  Py_ssize_t n = 0;
+  for (PyObject *o : items) {
+    whole = whole && o != nullptr;
+    if (result)
+      PyTuple_SET_ITEM(result, n++, o);
+    else
+      Py_XDECREF(o);
+  }
+  if (!whole) Py_CLEAR(result);
+  return result;
+}
 
 // The position of the token: a Python int, or one int32 on the device.
 struct Position {
@@ -247,12 +277,7 @@ PyObject *step_args(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   a.scale = (float)(1.0 / std::sqrt((double)D));
   a.link_gbps = (float)link;
   a.block_gbps = (float)block;
-  PyObject *bytes = PyBytes_FromStringAndSize((const char *)&a, sizeof(a));
-  if (!bytes) return nullptr;
-  PyObject *result = PyTuple_New(2);
-  PyTuple_SET_ITEM(result, 0, bytes);
-  PyTuple_SET_ITEM(result, 1, wrap(std::move(out)));
-  return result;
+  return tuple_of({PyBytes_FromStringAndSize((const char *)&a, sizeof(a)), wrap(std::move(out))});
   END_HANDLE_TH_ERRORS
 }
 
@@ -282,11 +307,13 @@ PyObject *static_step(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   Position pos;
   if (!position(start, paged, *xq, pos)) Py_RETURN_NONE;
   at::Tensor out = empty_like({1, 1, Hq, D}, *xq);
-  const int rc = da_decode_attention(
-      xq->data_ptr(), xq->stride(2), (int)Hq, (int)H, (int)D, dtype, pk->data_ptr(), pv->data_ptr(), pk->stride(1),
-      pk->stride(0), T, ck->data_ptr(), cv->data_ptr(), ck->stride(1), ck->stride(2), capacity, pos.len, pos.len_dev,
-      xk->data_ptr(), xv->data_ptr(), xk->stride(2), (float)(1.0 / std::sqrt((double)D)), out.data_ptr(), D, nullptr,
-      workspace->data_ptr(), workspace->nbytes(), stream);
+  const int rc = unlocked([&] {
+    return da_decode_attention(
+        xq->data_ptr(), xq->stride(2), (int)Hq, (int)H, (int)D, dtype, pk->data_ptr(), pv->data_ptr(), pk->stride(1),
+        pk->stride(0), T, ck->data_ptr(), cv->data_ptr(), ck->stride(1), ck->stride(2), capacity, pos.len, pos.len_dev,
+        xk->data_ptr(), xv->data_ptr(), xk->stride(2), (float)(1.0 / std::sqrt((double)D)), out.data_ptr(), D, nullptr,
+        workspace->data_ptr(), workspace->nbytes(), stream);
+  });
   if (rc) return raise(rc, "da_decode_attention");
   return wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -378,16 +405,14 @@ PyObject *qkv_rope(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   void *stream = in.pointer();
   if (!in.ok) return PyErr_Format(PyExc_TypeError, "qkv_rope: bad argument");
   at::Tensor q = empty_like({1, 1, Hq, D}, *x), k = empty_like({1, 1, H, D}, *x), v = empty_like({1, 1, H, D}, *x);
-  const int rc = da_linear_qkv_rope(x->data_ptr(), norm->data_ptr(), (float)eps, (int)x->size(-1), wq->data_ptr(),
-                                    wk->data_ptr(), wv->data_ptr(), (int)Hq, (int)H, (int)D,
-                                    (const float *)rope->data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                    dtype_code(*x), stream);
+  const int rc = unlocked([&] {
+    return da_linear_qkv_rope(x->data_ptr(), norm->data_ptr(), (float)eps, (int)x->size(-1), wq->data_ptr(),
+                              wk->data_ptr(), wv->data_ptr(), (int)Hq, (int)H, (int)D,
+                              (const float *)rope->data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                              dtype_code(*x), stream);
+  });
   if (rc) return raise(rc, "da_linear_qkv_rope");
-  PyObject *result = PyTuple_New(3);
-  PyTuple_SET_ITEM(result, 0, wrap(std::move(q)));
-  PyTuple_SET_ITEM(result, 1, wrap(std::move(k)));
-  PyTuple_SET_ITEM(result, 2, wrap(std::move(v)));
-  return result;
+  return tuple_of({wrap(std::move(q)), wrap(std::move(k)), wrap(std::move(v))});
   END_HANDLE_TH_ERRORS
 }
 
@@ -404,10 +429,12 @@ PyObject *block_tail(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   const int64_t dim = w2->size(0), hidden = w2->size(1);
   at::Tensor room = empty_like({dim + hidden}, *x), out = empty_like(x->sizes(), *x);
   char *h = (char *)room.data_ptr();
-  const int rc = da_linear_block_tail(attended->data_ptr(), (int)wo->size(1), wo->data_ptr(), x->data_ptr(), (int)dim,
-                                      norm->data_ptr(), (float)eps, w1->data_ptr(), w3->data_ptr(), (int)hidden,
-                                      w2->data_ptr(), h, h + dim * x->element_size(), out.data_ptr(), dtype_code(*x),
-                                      stream);
+  const int rc = unlocked([&] {
+    return da_linear_block_tail(attended->data_ptr(), (int)wo->size(1), wo->data_ptr(), x->data_ptr(), (int)dim,
+                                norm->data_ptr(), (float)eps, w1->data_ptr(), w3->data_ptr(), (int)hidden,
+                                w2->data_ptr(), h, h + dim * x->element_size(), out.data_ptr(), dtype_code(*x),
+                                stream);
+  });
   if (rc) return raise(rc, "da_linear_block_tail");
   return wrap(std::move(out));
   END_HANDLE_TH_ERRORS
