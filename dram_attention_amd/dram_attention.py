@@ -442,7 +442,8 @@ class DRAMAttention(torch.nn.Module):
         def fill(cache=None):
             # (looked at when the store and attention are on their way.  A selector of another kind
             # may still refuse the prompt behind the launch)
-            if self.page_selector != "bound" or not self._caches_in_one_launch(k_cache, v_cache, paged):
+            if (self.page_selector != "bound" or not self._caches_in_one_launch(k_cache, v_cache, paged)
+                    or cache is not None and cache.current_step.device != k_cache.device):
                 return None
             filled.append(True)
             return self._fill_caches(k_cache, v_cache, paged, cache)
