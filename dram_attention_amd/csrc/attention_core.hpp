@@ -400,20 +400,17 @@ __device__ __forceinline__ StreamRange stream_range(int b, int n_blocks, int64_t
   return {b * total / n_eff, (b + 1) * total / n_eff};
 }
 
-// want_blocks: every block pays a fixed prologue and a merge epilogue, so few long chunks beat many
-// short ones (measured on the 128K workload with the vector pass: 31.9 us at 512 blocks, 32.6 us at
-// 2048).  One block per CU where the matrix cores do the pass and it is a launch of its own: one wave
-// per SIMD keeps the memory busy.  Two per CU for the vector pass, which needs them for its arithmetic, and
-// next to a page stream, which hides the pass (128K shape 158.9 / 159.9 us a step with one, the LRU
-// update behind it 6.5 / 7.1; 50K tokens, fp16 79.4 / 78.7).  us a call, pass and merge,
-// on keys and values out of the caches, 512 blocks / 256: tile pass, D 128, 32768 tokens of 32/8 heads
-// 36.2 / 34.8, of 28/4 23.6 / 22.3, of 64/8 36.8 / 35.4, 8192 of 32/8 18.4 / 17.6, 100000 84.8 / 81.3; 32768 of 16/16,
-// D 64 36.1 / 33.8 (128 blocks 42.3, 192 35.1, 240 34.9, 320 41.0, 384 38.5 for the first); vector
-// pass, fp32: 20000 of 32/8, D 128 42.5 / 53.0, 60000 of 8/2, D 64 21.7 / 23.0.
-constexpr int kTileBlocks = 256, kVectorBlocks = 512;
-
-inline int pick_chunk(int64_t p_len, int64_t c_capacity, int n_kv_heads, int step_tokens, int64_t want_blocks) {
-  // (never below one unrolled round)
+inline int pick_chunk(int64_t p_len, int64_t c_capacity, int n_kv_heads, int step_tokens) {
+  // ~2 blocks per CU on a 256-CU part: every block pays a fixed prologue and a
+  // merge epilogue, so few long chunks beat many short ones (measured on the
+  // 128K workload: 31.9 us at 512 blocks, 32.6 us at 2048); never below one
+  // unrolled round.  Not one per CU, which a pass of its own over a full window would have faster: blocks over rows
+  // that the window only has room for leave at once, so half the units stand idle where it is mostly empty,
+  // and longer chunks round the softmax weights to 16 bits further from float64.  us a call out of the caches, 512
+  // blocks / 256, error against float64 of bf16 in brackets: 32768 tokens of 32/8 heads, D 128, 4100 in a window
+  // of 4136 36.2 / 33.8 (2.32e-3 / 2.36e-3), of 36864 45.7 / 48.4; 70000 of 16/16, D 64 71.8 / 102.6; 2048 of
+  // 32/8 11.6 / 10.1 (1.92e-3 / 2.12e-3).
+  const int64_t want_blocks = 256 * 2;
   int64_t chunk = (p_len + c_capacity) * n_kv_heads / want_blocks;
   const int round = step_tokens * kAttnUnroll;
   if (chunk < round) chunk = round;
@@ -446,13 +443,13 @@ struct ChunkPlan {
   int pre_chunk() const { return n_p + n_l + n_t; }
   int gather_chunk0() const { return n_p + n_l + n_t + 1; }
 };
-// The chunk geometry of a launch; a function of the shapes only (tiles_alone: the matrix cores
-// do the pass, without a page stream), so that every phase of a step agrees on it.
+// The chunk geometry of a launch; a function of the shapes only, so that the
+// workspace query and every phase of a step agree on it.
 inline ChunkPlan plan_chunks(int n_kv_heads, int lanes, int64_t p_len, int64_t c_capacity,
-                             int64_t miss_tokens, bool tiles_alone) {
+                             int64_t miss_tokens) {
   const int step_tokens = kAttnWaves * (64 / lanes);
   ChunkPlan p;
-  p.chunk = pick_chunk(p_len, c_capacity, n_kv_heads, step_tokens, tiles_alone ? kTileBlocks : kVectorBlocks);
+  p.chunk = pick_chunk(p_len, c_capacity, n_kv_heads, step_tokens);
   p.n_p = (int)ceil_div(p_len, p.chunk);
   p.n_l = (int)ceil_div(c_capacity, p.chunk);
   // the tail is short and every block starts with a dependent slot lookup:

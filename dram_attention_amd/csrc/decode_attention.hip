@@ -208,9 +208,10 @@ decode_attention_merge_layers_kernel(AttnArgs a, const MergeBatch batch, int hea
 
 // The matrix-core form of the pass, for the shapes it takes.  Two rules on what it reads:
 //   - keys and values laid out token by token (a prompt's own, as a static cache keeps them): blocks that
-//     follow each other take the heads of the same tokens, which lie next to each other.  us a call on
-//     32768 tokens out of the caches, tokens / heads first: 32/8 heads 34.8 / 33.9, 28/4 22.3 / 21.6, 64/8
-//     35.4 / 34.3; laid out head by head 35.5 / 35.5, and 100000 tokens 81.3 / 85.4.
+//     follow each other take the heads of the same tokens, which lie next to each other.  us a call out of the
+//     caches, tokens / heads first: 32768 tokens of 32/8 heads 36.2 / 34.7, of 28/4 23.5 / 23.4, of 16/16, D 64
+//     36.9 / 35.4, 16384 of 32/8, D 256 44.2 / 39.7, 8192 of 32/8 16.8 / 16.6, 2048 11.6 / 11.8.  Laid out
+//     head by head the order by tokens stays (100000 of 32/8, 256 blocks: 81.3 / 85.4).
 //   - more than the last-level cache holds: streaming loads (100000 tokens of 32/8 81.3 / 79.0; with
 //     less they are slower where the caches still have it, 32768 tokens 30.3 / 33.3).
 constexpr int64_t kLastLevelBytes = 256 << 20;
@@ -440,8 +441,7 @@ int prepare_attention(const void *q, int64_t q_head_stride, int n_q_heads, int n
                overlap->gather_blocks, n_kv_heads, kGatherMaxBlocks);
     a.gather_blocks = overlap->gather_blocks;
   }
-  const bool tiles_alone = !overlap && tile_pass_supported(dtype, head_dim, a.rep, false, 0);
-  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens, tiles_alone);
+  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
   a.chunk = p.chunk;
   a.tail_chunk = p.tail_chunk;
   a.n_pchunks = p.n_p;
@@ -511,13 +511,8 @@ extern "C" size_t da_decode_attention_workspace_bytes(int n_q_heads, int n_kv_he
     return 0;
   const int lanes = lanes_of(head_dim, dtype);
   if (!lanes) return 0;
-  // (whichever plan it will be)
-  int64_t most = 0;
-  for (const bool tiles_alone : {false, true}) {
-    const int64_t n = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens, tiles_alone).total();
-    if (n > most) most = n;
-  }
-  return attn_workspace_bytes(n_q_heads, head_dim, most) + 16;
+  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, miss_tokens);
+  return attn_workspace_bytes(n_q_heads, head_dim, p.total()) + 16;
 }
 
 extern "C" int da_decode_attention_paged(const void *q, int64_t q_head_stride, int n_q_heads, int n_kv_heads, int head_dim, int dtype,

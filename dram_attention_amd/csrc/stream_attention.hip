@@ -330,7 +330,7 @@ extern "C" int da_pages_gather_attend(
                  (uintptr_t)dram % 16 == 0 && (uintptr_t)hbm % 16 == 0 && (uintptr_t)q % 16 == 0 &&
                  q_head_stride % vec == 0 && (uintptr_t)workspace % 16 == 0,
              "da_pages_gather_attend: operands must be 16-byte aligned");
-  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, (int64_t)k * page_size, false);
+  const ChunkPlan p = plan_chunks(n_kv_heads, lanes, p_len, c_capacity, (int64_t)k * page_size);
   const size_t need = attn_workspace_bytes(n_q_heads, head_dim, p.total());
   DA_REQUIRE(workspace_bytes >= need, "da_pages_gather_attend: workspace %zu < %zu bytes",
              workspace_bytes, need);

@@ -848,3 +848,25 @@ def test_static_pass_by_layout_and_size(layout, H, rep, D, T, capacity):
         rows = slice(h * rep, (h + 1) * rep)
         assert torch.allclose(lse[rows], scores.logsumexp(-1), atol=1e-3, rtol=1e-4), h
         assert torch.allclose(out[rows].float(), scores.softmax(-1) @ values, atol=2e-2, rtol=1e-2), h
+
+
+@pytest.mark.parametrize("H,D,T,capacity,n", [
+    (8, 128, 32768, 4096 + 32768, 4100), (8, 128, 8192, 1024 + 8192, 1030),   # room reserved for a long answer
+    (8, 128, 32768, 4096 + 40, 4100), (2, 64, 60000, 1064, 1030),
+])
+def test_static_pass_fills_the_chip_whatever_is_reserved(H, D, T, capacity, n):
+    """Workgroups over rows that the window only has room for leave at once: the others, which leave a partial
+    result each, are still about one per compute unit (256) or more, and no more than the 512 that are
+    resident together."""
+    from dram_attention_amd import decode_attention
+    from dram_attention_amd.dram_attention import attention_workspace
+
+    q = torch.randn(H, D, device=DEV).bfloat16()
+    k, v = (torch.randn(T, H, D, device=DEV).bfloat16().transpose(0, 1) for _ in range(2))
+    cache_k, cache_v = (torch.randn(capacity, H, D, device=DEV).bfloat16() for _ in range(2))
+    workspace = attention_workspace(H, H, D, torch.bfloat16, T, capacity, 0, DEV).fill_(float("nan"))
+    decode_attention(q, k, v, cache_k, cache_v, n, cache_k[0], cache_v[0], workspace=workspace)
+    chunks = (workspace.numel() - 4) // (H * (D + 2))
+    written = ~workspace[:chunks * H * D].view(chunks, H, D).isnan().any(-1)
+    written[-1] = False                          # (room for a merged state)
+    assert 240 <= int(written.sum()) <= 512
