@@ -212,9 +212,12 @@ decode_attention_merge_layers_kernel(AttnArgs a, const MergeBatch batch, int hea
 //     caches, tokens / heads first: 32768 tokens of 32/8 heads 36.2 / 34.7, of 28/4 23.5 / 23.4, of 16/16, D 64
 //     36.9 / 35.4, 16384 of 32/8, D 256 44.2 / 39.7, 8192 of 32/8 16.8 / 16.6, 2048 11.6 / 11.8.  Laid out
 //     head by head the order by tokens stays (100000 of 32/8, 256 blocks: 81.3 / 85.4).
-//   - more than the last-level cache holds: streaming loads (100000 tokens of 32/8 81.3 / 79.0; with
-//     less they are slower where the caches still have it, 32768 tokens 30.3 / 33.3).
-constexpr int64_t kLastLevelBytes = 256 << 20;
+//   - a prefix well beyond the last-level cache (256 MiB): streaming loads.  Of the prefix alone, which is all
+//     read: the window is mostly room.  us a call without / with, on keys and values out of the caches and on the same
+//     ones again: 85000 tokens of 32/8 heads (332 MiB) 72.0 / 68.4 and 71.8 / 69.6, laid out head by head 70.2 /
+//     62.3 and 69.8 / 64.2; 75000 (293 MiB) 64.4 / 61.3 and 61.2 / 62.0; 66000 (258 MiB) 57.1 / 54.8 and 50.4 / 55.9;
+//     32768 with room for as many 45.7 / 49.3 and 36.0 / 49.8; 200000 152.8 / 144.5 and 152.5 / 146.0.
+constexpr int64_t kStreamedBytes = 320 << 20;
 template <typename T, int kD, bool kStream>
 static void launch_tile(const AttnArgs &a, int n_launch, int n_kv_heads, hipStream_t s) {
   const bool heads_first = a.p_tok_stride > a.p_head_stride;
@@ -236,7 +239,7 @@ static void launch_split(AttnArgs a, int first_chunk, int n_launch, int n_kv_hea
   if constexpr (!kTail && T::kBytes == 2 && (kLanes == 8 || kLanes == 16 || kLanes == 32)) {
     const int dtype = std::is_same<T, BF16>::value ? DA_BF16 : DA_F16;
     if (tile_pass_supported(dtype, kLanes * 8, rep, a.slot_epoch != nullptr, a.page_size)) {
-      if ((a.p_len + a.c_capacity) * n_kv_heads * 2 * kLanes * 16 > kLastLevelBytes)
+      if (a.p_len * n_kv_heads * 2 * kLanes * 16 > kStreamedBytes)
         launch_tile<T, kLanes * 8, true>(a, n_launch, n_kv_heads, s);
       else
         launch_tile<T, kLanes * 8, false>(a, n_launch, n_kv_heads, s);

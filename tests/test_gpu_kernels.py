@@ -820,6 +820,7 @@ def test_page_cache_init_kernel(H, P, N):
 @pytest.mark.parametrize("H,rep,D,T,capacity", [
     (4, 7, 128, 3, 5), (8, 4, 128, 1217, 300), (16, 1, 64, 4097, 64),   # few tokens, a chunk and one, short chunks
     (8, 2, 128, 65536 - 64, 64), (8, 2, 128, 65536 - 64, 65),            # as much as the last-level cache, and more
+    (8, 2, 128, 81920, 20000), (8, 2, 128, 81921, 64),                   # a prefix up to the streaming loads' line, and beyond
 ])
 def test_static_pass_by_layout_and_size(layout, H, rep, D, T, capacity):
     """The attention pass of its own launch: which grid order it takes follows the layout, which loads the
