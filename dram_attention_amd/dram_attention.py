@@ -496,7 +496,9 @@ class DRAMAttention(torch.nn.Module):
         keys and values: plain GPU tensors of the window's type on its device, aligned, one layout for
         both, of the size that the window was made for."""
         own = self._buffers
-        cache_k, cache_v = own["cache_k"], own["cache_v"]
+        cache_k, cache_v = own.get("cache_k"), own.get("cache_v")
+        if cache_k is None or cache_v is None:      # (a window that is no buffer any more)
+            return False
         tail, esize = k.shape[1] - paged, k.element_size()
         return (paged >= 0 and 0 <= tail <= cache_k.shape[1] and k.is_cuda and k.shape == v.shape
                 and k.stride() == v.stride() and k.stride(3) == 1
@@ -632,8 +634,8 @@ class DRAMAttention(torch.nn.Module):
                 or "attend_" in layer or "get_kv_cache_" in prefix):
             return None
         return _lib.host().static_step(
-            xq, xk, xv, start_pos, prefix.get("k_cache"), prefix.get("v_cache"), own["cache_k"], own["cache_v"],
-            self.dram_kv_cache_size, self._workspace, _lib.stream_ptr(xq.device))
+            xq, xk, xv, start_pos, prefix.get("k_cache"), prefix.get("v_cache"), own.get("cache_k"),
+            own.get("cache_v"), self.dram_kv_cache_size, self._workspace, _lib.stream_ptr(xq.device))
 
     def _step_args(self, xq, xk, xv, start_pos):
         """(argument block of da_decode_step, output) of a step that one native call can do, else None."""
@@ -649,8 +651,8 @@ class DRAMAttention(torch.nn.Module):
             step = step_args(
                 xq, xk, xv, start_pos, selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"],
                 buffers["page_access_time"], buffers["dram_page_to_hbm_page_mapping"],
-                buffers["hbm_page_to_dram_page_mapping"], buffers["current_step"], own["cache_k"], own["cache_v"],
-                lru.num_hbm_pages, lru.page_size, lru.top_k, self.dram_kv_cache_size, lru.page_stores()[1],
+                buffers["hbm_page_to_dram_page_mapping"], buffers["current_step"], own.get("cache_k"),
+                own.get("cache_v"), lru.num_hbm_pages, lru.page_size, lru.top_k, self.dram_kv_cache_size, lru.page_stores()[1],
                 self.stream_blocks, SCORE_FLAGS[selector.bounds_are_ordered], self.link_gbps, self.block_gbps,
                 lru._scratch, lru._topk_idx, selector._scores, selector._split_ws, self._workspace)
             if type(step) is not int:

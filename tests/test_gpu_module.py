@@ -1001,6 +1001,31 @@ def test_selection_and_update_of_short_rows(Hq, Hkv, slots, kp, pages, dtype, le
             assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
 
 
+@pytest.mark.parametrize("lru", [4096, 320])     # a static prefix, a paged one
+def test_a_window_that_became_a_parameter_still_works(lru):
+    """cache_k and cache_v as Parameters instead of buffers: prompt and steps go the general way, to the
+    same bits."""
+    from dram_attention_amd import DRAMAttention
+
+    S, Hq, Hkv, D = 700, 8, 2, 64
+    g = torch.Generator(device=DEV).manual_seed(3)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).bfloat16()
+
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    a, b = (DRAMAttention(8, lru, 200, 16, 64, Hkv, D, device=DEV) for _ in range(2))
+    for name in ("cache_k", "cache_v"):
+        window = a._buffers.pop(name)
+        setattr(a, name, torch.nn.Parameter(window, requires_grad=False))
+    for m in (a, b):
+        m.init_cache(k, v)
+    for t in range(3):
+        x = rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D)
+        got, want = (m(*x, start_pos=S + t, stage="generate") for m in (a, b))
+        assert same(got, want) and same(a.cache_k, b.cache_k) and same(a.cache_v, b.cache_v), t
+
+
 def test_an_exchanged_method_of_a_step_is_called(monkeypatch):
     """Whatever the step is made of, on the instances, on the classes or in a subclass."""
     from dram_attention_amd import DRAMAttention, LRUCache
