@@ -440,8 +440,8 @@ class DRAMAttention(torch.nn.Module):
         filled = []
 
         def fill(cache=None):
-            # (looked at when the store and attention are on their way.  A selector of another kind
-            # may still refuse the prompt behind the launch)
+            # (looked at when the store and attention are on their way.  Another kind of page cache or
+            # selector may still refuse the prompt behind the launch, or may not take what it makes)
             if (self.page_selector != "bound" or not self._caches_in_one_launch(k_cache, v_cache, paged)
                     or cache is not None and cache.current_step.device != k_cache.device):
                 return None
@@ -454,6 +454,8 @@ class DRAMAttention(torch.nn.Module):
                     raise RuntimeError(f"Unsupported page selector: {self.page_selector}")
                 # (measured ahead of the store, which may be crossing the link when LRUCache returns)
                 link_gbps = 0.95 * host_link_gbps(self.cache_k.device)
+                if LRUCache.__init__ is _LRU_CACHE_INIT:
+                    build["fill"] = fill
                 cache = LRUCache(
                     k_cache=prefix_k,
                     v_cache=prefix_v,
@@ -461,7 +463,6 @@ class DRAMAttention(torch.nn.Module):
                     top_k=self.top_k // self.page_size,
                     lru_hbm_cache_size=self.lru_hbm_cache_size,
                     device=self.device,
-                    fill=fill,
                     **build,
                 )
                 if self.page_selector == "token_max":
@@ -802,3 +803,4 @@ _STEP_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, LRUCache.select_,
                  IPUpperboundTopKSelector.top_k_for_lru, IPUpperboundTopKSelector.scores)
 _STATIC_METHODS = (DRAMAttention.select_, DRAMAttention.attend_, DummyCache.get_kv_cache_)
 _INIT_CACHE = DRAMAttention.init_cache
+_LRU_CACHE_INIT = LRUCache.__init__

@@ -17,6 +17,9 @@ from .lru_kernel import (LruScratch, lru_update, lru_update_and_gather, pages_ga
 from .topk_selector import IPUpperboundTopKSelector
 
 
+_SELECTOR_INIT = IPUpperboundTopKSelector.__init__
+
+
 class CacheOutput(NamedTuple):
     k_cache: torch.Tensor
     v_cache: torch.Tensor
@@ -72,7 +75,8 @@ class LRUCache(torch.nn.Module):
         caller then ends the build with :meth:`finish_build` before anything reads or frees
         the keys, the store or the slots.  Without it the store is complete on return.
         ``fill``, called behind ``beside``: issues this cache's metadata and the page summaries
-        (da_prompt_cache) and returns these, or does nothing and returns None."""
+        (da_prompt_cache) and returns these, or does nothing and returns None.  Not called where the
+        selector is of another kind, which makes its own."""
         super().__init__()
         assert k_cache.shape == v_cache.shape, "Key and value cache shapes must match."
         num_kv_heads, dram_kv_cache_size, head_dim = k_cache.shape
@@ -147,9 +151,12 @@ class LRUCache(torch.nn.Module):
         try:
             if beside is not None:
                 beside()
-            summaries = None if fill is None else fill(self)
-            self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device, summaries=summaries)
-            if summaries is None:
+            summaries = fill(self) if fill is not None and IPUpperboundTopKSelector.__init__ is _SELECTOR_INIT else None
+            if summaries is not None:
+                self.top_k_selector = IPUpperboundTopKSelector(
+                    k_cache, num_dram_pages, device=device, summaries=summaries)
+            else:
+                self.top_k_selector = IPUpperboundTopKSelector(k_cache, num_dram_pages, device=device)
                 _lib.check(
                     _lib.load().da_page_cache_init(
                         self.current_step.data_ptr(), self.page_access_time.data_ptr(),

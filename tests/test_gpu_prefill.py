@@ -620,3 +620,53 @@ def test_prompt_caches_in_one_launch_equal_the_separate_ones(dtype, S, local, lr
                      "hbm_page_to_dram_page_mapping", "dram_kv_cache", "hbm_kv_cache"):
             assert torch.equal(getattr(one.lru_cache, name), getattr(many.lru_cache, name)), name
         assert torch.equal(one.lru_cache.top_k_selector.chunk_min_max, many.lru_cache.top_k_selector.chunk_min_max)
+
+
+@pytest.mark.parametrize("what,stage", [
+    ("page cache", "init_cache"),       # (a prompt tells its page cache where to write the store, too)
+    ("selector", "init_cache"), ("selector", "prefill"),
+    ("selector that refuses", "init_cache"), ("selector that refuses", "prefill"),
+])
+def test_stand_ins_for_the_page_cache_and_its_selector(what, stage, monkeypatch):
+    """Classes put in their places with the signatures of the reference's: init_cache calls the page cache
+    with its parameters and no others, the page cache its selector; one that refuses the prompt leaves the layer
+    as it was."""
+    from dram_attention_amd import DRAMAttention, IPUpperboundTopKSelector, LRUCache, dram_attention, lru_cache
+
+    class Cache(LRUCache):
+        def __init__(self, k_cache, v_cache, page_size, top_k, lru_hbm_cache_size=None, hbm_kv_cache_fraction=0.2,
+                     device="cuda"):
+            made.append(self)
+            super().__init__(k_cache, v_cache, page_size, top_k, lru_hbm_cache_size, hbm_kv_cache_fraction, device)
+
+    class Selector(IPUpperboundTopKSelector):
+        def __init__(self, k_cache, num_pages, device="cuda"):
+            made.append(self)
+            if what == "selector that refuses":
+                raise RuntimeError("not these keys")
+            super().__init__(k_cache, num_pages, device)
+
+    made, (q, k, v) = [], draw(1000, 4, 2, 64, torch.bfloat16, 1)
+    m, ref = (DRAMAttention(max_output_length=4, lru_hbm_cache_size=256, local_cache_size=256, page_size=16, top_k=64,
+                            n_kv_heads=2, head_dim=64, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    m.init_cache(k, v)
+    window = m.cache_k.clone(), m.cache_v.clone()
+    _, k, v = draw(1100, 4, 2, 64, torch.bfloat16, 2)
+    ref.init_cache(k, v)
+    if what == "page cache":
+        monkeypatch.setattr(dram_attention, "LRUCache", Cache)
+    else:
+        monkeypatch.setattr(lru_cache, "IPUpperboundTopKSelector", Selector)
+    q = draw(1100, 4, 2, 64, torch.bfloat16, 2)[0]
+    prompt = (lambda: m.init_cache(k, v)) if stage == "init_cache" else (lambda: m(q, k, v, start_pos=0, stage="prefill"))
+    if what == "selector that refuses":
+        with pytest.raises(RuntimeError, match="not these keys"):
+            prompt()
+        assert made and same(m.cache_k, window[0]) and same(m.cache_v, window[1])
+        return
+    prompt()
+    assert len(made) == 1
+    assert same(m.cache_k, ref.cache_k) and same(m.cache_v, ref.cache_v)
+    assert same(m.lru_cache.top_k_selector.chunk_min_max, ref.lru_cache.top_k_selector.chunk_min_max)
+    for name in ("current_step", "page_access_time", "dram_page_to_hbm_page_mapping", "hbm_page_to_dram_page_mapping"):
+        assert same(getattr(m.lru_cache, name), getattr(ref.lru_cache, name)), name
