@@ -252,7 +252,7 @@ class TransformerBlock(nn.Module):
             return None
         weight1, weight2 = norm1._parameters.get("weight"), norm2._parameters.get("weight")
         if not (K.takes(x, weight1, weight2) and K.bare(a, f, norm1, norm2)
-                and rope_rows.dtype is torch.float32 and rope_rows.is_contiguous()
+                and type(rope_rows) in (torch.Tensor, nn.Parameter) and rope_rows.dtype is torch.float32 and rope_rows.is_contiguous()
                 and rope_rows.device == x.device):
             return None
         am, fm, dim, hd = a._modules, f._modules, x.shape[2], a.head_dim

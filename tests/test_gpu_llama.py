@@ -617,3 +617,20 @@ def test_transforms_see_the_norm_as_torch_operators():
         assert tangent is not None and torch.isfinite(tangent).all() and tangent.abs().max() > 0
         traced = torch.jit.trace(norm, (x,), check_trace=False)
         assert torch.allclose(traced(t), norm(t), atol=1e-6)
+
+
+def test_a_rotation_table_of_a_class_of_its_own_is_left_to_the_modules(monkeypatch):
+    """A token through a model whose table is a subclass of Tensor: the bits of the modules one by one."""
+    class Table(torch.Tensor):
+        pass
+
+    args = small_args(torch.bfloat16)
+    model, ref = (build(args, 5) for _ in range(2))
+    prompt = torch.arange(600, device="cuda")[None] % args.vocab_size
+    for m in (model, ref):
+        m(prompt, 0)
+    model.rope = model.rope.as_subclass(Table)
+    got = model(prompt[:, :1], 600)
+    with monkeypatch.context() as patch:
+        patch.setattr(L.TransformerBlock, "_one_token_kernels", staticmethod(lambda *a: None))
+        assert torch.equal(got, ref(prompt[:, :1], 600))
