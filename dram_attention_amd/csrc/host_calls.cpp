@@ -48,6 +48,18 @@ bool like(const at::Tensor &t, const at::Tensor &x) {
 bool aligned(const at::Tensor &t) { return (uintptr_t)t.data_ptr() % 16 == 0; }
 bool is_shape(const at::Tensor &t, at::IntArrayRef want) { return t.sizes() == want; }
 
+// A whole number of any kind (numpy's too); `ok` is left false by anything else.
+int64_t whole_number(PyObject *o, bool &ok) {
+  PyObject *n = PyNumber_Index(o);
+  const long long v = n ? PyLong_AsLongLong(n) : -1;
+  Py_XDECREF(n);
+  if (v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    ok = false;
+  }
+  return v;
+}
+
 // Positional arguments, read in order; what is not what it should be leaves `ok` false.
 struct Args {
   PyObject *const *at;
@@ -73,19 +85,7 @@ struct Args {
     ok = ok && t != nullptr;
     return t;
   }
-  int64_t integer() {
-    PyObject *o = next();
-    if (!PyLong_Check(o)) {
-      ok = false;
-      return 0;
-    }
-    const long long v = PyLong_AsLongLong(o);
-    if (v == -1 && PyErr_Occurred()) {
-      PyErr_Clear();
-      ok = false;
-    }
-    return v;
-  }
+  int64_t integer() { return whole_number(next(), ok); }
   double number() {
     PyObject *o = next();
     const double v = PyFloat_AsDouble(o);
@@ -362,7 +362,9 @@ PyObject *linears(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   };
   auto features = [&](PyObject *dict, PyObject *name) -> int64_t {
     PyObject *o = item(dict, name);
-    return o && PyLong_CheckExact(o) ? PyLong_AsLongLong(o) : -2;
+    bool ok = o != nullptr;
+    const int64_t n = ok ? whole_number(o, ok) : 0;
+    return ok ? n : -2;
   };
   for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject *m = in.next();

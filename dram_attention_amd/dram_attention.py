@@ -648,6 +648,8 @@ class DRAMAttention(torch.nn.Module):
         if type(selector) is not IPUpperboundTopKSelector or not self._steps_by_its_own_methods(lru, selector):
             return None
         step_args = _lib.host().step_args
+        if not isinstance(start_pos, torch.Tensor):
+            start_pos = int(start_pos)
         for _ in range(2):
             step = step_args(
                 xq, xk, xv, start_pos, selector.chunk_min_max, buffers["dram_kv_cache"], buffers["hbm_kv_cache"],

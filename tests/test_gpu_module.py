@@ -874,6 +874,30 @@ def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
         a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
 
 
+def test_numpy_sizes_and_positions_step_in_one_call():
+    """A layer built from numpy's integers, stepped at numpy's positions: one native call a step, the bits of a
+    twin of Python's."""
+    from dram_attention_amd import DRAMAttention
+
+    S, Hq, Hkv, D = 1500, 8, 2, 64
+    g = torch.Generator(device=DEV).manual_seed(6)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).bfloat16()
+
+    sizes = 8, 480, 200, 16, 96, Hkv, D
+    a, b = (DRAMAttention(*(kind(n) for n in sizes), device=DEV) for kind in (np.int64, int))
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    for m in (a, b):
+        m.init_cache(k, v)
+    calls, one_call = [], a._step_in_one_call
+    a._step_in_one_call = lambda *args: calls.append(one_call(*args)) or calls[-1]
+    for t in np.arange(3):
+        x = rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D)
+        got, want = (m(*x, start_pos=p, stage="generate") for m, p in ((a, S + t), (b, S + int(t))))
+        assert calls.pop() is not None and same(got, want), t
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,dtype", [(8, 2, 64, torch.float32), (28, 4, 128, torch.bfloat16),
                                             (4, 4, 32, torch.float16)])
 def test_static_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, dtype, monkeypatch):

@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -100,6 +101,17 @@ def test_linears_that_make_their_weights_are_left_to_torch(change):
         dict(weight_norm=weight_norm, spectral_norm=spectral_norm)[change](m)
     assert type(m) is torch.nn.Linear and m(x).shape == (1, 1, 8)
     assert not K.linears_fit(x, plain, m)
+
+
+def test_linears_of_numpy_sizes_are_taken():
+    from dram_attention_amd import model_kernels as K
+
+    x, m = torch.zeros(1, 1, 16), torch.nn.Linear(16, 8, bias=False)
+    m.in_features, m.out_features = np.int64(16), np.int32(8)
+    assert K.linears_fit(x, m) == (m.weight,) == K.linears_fit(x, (m, np.int64(8), 16))
+    for wrong in (9, 2 ** 70, "8", 8.0, None):
+        m.out_features = wrong
+        assert K.linears_fit(x, m) is None
 
 
 def test_compiled_code_is_asked_for_its_operators_without_a_graph_break():
