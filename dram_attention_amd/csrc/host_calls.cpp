@@ -211,21 +211,32 @@ PyObject *step_args(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   if (!position(start, paged, *xq, pos)) Py_RETURN_NONE;
   if (!pos.len_dev && (pos.len < 0 || pos.len >= capacity)) Py_RETURN_NONE;
 
+  // (the room is looked at like the operands: the kernels write to all of it)
   const int64_t total = rep * kp;
+  auto fits = [&](const at::Tensor *t, at::IntArrayRef shape, at::ScalarType type) {
+    return t && t->scalar_type() == type && t->device() == xq->device() && t->is_contiguous() && is_shape(*t, shape);
+  };
   const at::Tensor *idx = in.tensor_or_none(), *scores = in.tensor_or_none(), *topk_ws = in.tensor_or_none(),
                    *workspace = in.tensor_or_none();
   if (!in.ok) Py_RETURN_NONE;
   const size_t topk_need = da_topk_pages_workspace_bytes((int)rep, (int)H, P, (int)kp);
-  if (!PyTuple_Check(scratch) || PyTuple_GET_SIZE(scratch) != 7 || !idx || !scores || !workspace ||
-      (topk_need && (!topk_ws || (size_t)topk_ws->nbytes() < topk_need)))
+  if (!PyTuple_Check(scratch) || PyTuple_GET_SIZE(scratch) != 7 || !fits(idx, {H, total}, at::kLong) ||
+      !fits(scores, {rep, H, P}, at::kFloat) || !workspace || !fits(workspace, workspace->sizes(), at::kFloat) ||
+      (topk_need && (!topk_ws || !fits(topk_ws, topk_ws->sizes(), at::kByte) ||
+                     (size_t)topk_ws->nbytes() < topk_need)))
     return PyLong_FromLongLong(rep);
   const at::Tensor *room[7];   // miss_page, miss_slot, miss_count, hit_mask, workspace, slot_epoch, candidates
   for (int i = 0; i < 7; ++i)
     if (!(room[i] = tensor_of(PyTuple_GET_ITEM(scratch, i)))) Py_RETURN_NONE;
-  if (room[0]->dim() != 2 || room[0]->size(1) != total || idx->dim() != 2 || idx->size(1) != total ||
-      scores->dim() != 3 || scores->size(0) != rep)
-    return PyLong_FromLongLong(rep);
-  if (room[5]->dim() != 2 || room[5]->size(1) != N || room[6]->dim() != 2) Py_RETURN_NONE;
+  if (room[0]->dim() != 2 || room[0]->size(1) != total) return PyLong_FromLongLong(rep);
+  const at::Tensor &list = *room[6];
+  if (list.dim() != 2 || list.size(1) < 1) Py_RETURN_NONE;
+  const int64_t stamps_end = list.storage_offset() + H * (list.size(1) + 1);   // (a word per head behind the lists)
+  if (!(fits(room[0], {H, total}, at::kInt) && fits(room[1], {H, total}, at::kInt) && fits(room[2], {H}, at::kInt) &&
+        fits(room[3], {H, total}, at::kByte) && fits(room[4], room[4]->sizes(), at::kByte) &&
+        fits(room[5], {H, N}, at::kInt) && fits(&list, {H, list.size(1)}, at::kInt) &&
+        (int64_t)list.storage().nbytes() >= stamps_end * 4))
+    Py_RETURN_NONE;
 
   at::Tensor out = empty_like({1, 1, Hq, D}, *xq);
   da_decode_step_args a = {};

@@ -666,13 +666,17 @@ class DRAMAttention(torch.nn.Module):
     def _make_room(self, lru, selector, rep, xq):
         """What the launches of a step hand to one another, for ``rep`` query rows a kv head."""
         H, P, _, D = selector.chunk_min_max.shape
-        kp, device, idx, scores = min(lru.top_k, P), xq.device, lru._topk_idx, selector._scores
+        kp, device = min(lru.top_k, P), xq.device
+
+        def room(t, shape, dtype):
+            if t is not None and t.shape == shape and t.dtype is dtype and t.device == device and t.is_contiguous():
+                return t
+            return torch.empty(shape, dtype=dtype, device=device)
+
         lru._scratch_for(rep * kp)
-        if idx is None or idx.shape[1] != rep * kp:
-            lru._topk_idx = torch.empty(H, rep * kp, dtype=torch.int64, device=device)
-        if scores is None or scores.shape[0] != rep:
-            scores = selector._scores = torch.empty(rep, H, P, dtype=torch.float32, device=device)
-        selector._workspace(scores, kp)
+        lru._topk_idx = room(lru._topk_idx, (H, rep * kp), torch.int64)
+        selector._scores = room(selector._scores, (rep, H, P), torch.float32)
+        selector._workspace(selector._scores, kp)
         if self._workspace is None:
             self._workspace = attention_workspace(
                 rep * H, H, D, xq.dtype, lru.num_hbm_pages * lru.page_size, self.cache_k.shape[1],

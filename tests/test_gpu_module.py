@@ -874,6 +874,50 @@ def test_step_in_one_call_equals_its_two_halves(Hq, Hkv, D, page, dtype):
         a(rand(1, 1, Hq, D), rand(1, 1, Hkv, D), rand(1, 1, Hkv, D), start_pos=S + 4000, stage="generate")
 
 
+def test_room_of_other_sizes_is_not_handed_to_a_step():
+    """What the launches of a step write into is looked at like the operands: lists and scores of another
+    shape, type or device are made anew, scratch of another shape leaves the step to the two halves.  (Nothing is
+    launched here: the argument block alone is asked for.)"""
+    from dram_attention_amd import DRAMAttention
+
+    S, Hq, Hkv, D = 1500, 8, 2, 64
+    m = DRAMAttention(8, 480, 200, 16, 96, Hkv, D, device=DEV)
+    k, x = torch.randn(1, S, Hkv, D, device=DEV).bfloat16(), torch.randn(1, 1, Hq, D, device=DEV).bfloat16()
+    m.init_cache(k, k)
+    lru, step = m.lru_cache, lambda: m._step_args(x, k[:, :1], k[:, :1], S)
+    assert step() is not None
+    total, pages = lru._topk_idx.shape[1], lru.num_dram_pages
+
+    def owner(name):
+        return lru if name == "_topk_idx" else lru.top_k_selector
+
+    for name, wrong in (("_topk_idx", torch.empty(Hkv - 1, total, dtype=torch.int64, device=DEV)),
+                        ("_topk_idx", torch.empty(Hkv, total, dtype=torch.int32, device=DEV)),
+                        ("_topk_idx", torch.empty(Hkv, total, dtype=torch.int64)),
+                        ("_scores", torch.empty(Hq // Hkv, Hkv, pages - 1, device=DEV)),
+                        ("_scores", torch.empty(Hq // Hkv, Hkv - 1, pages, device=DEV)),
+                        ("_scores", torch.empty(Hq // Hkv, Hkv, pages, device=DEV, dtype=torch.float16))):
+        right = getattr(owner(name), name)
+        setattr(owner(name), name, wrong)
+        assert step() is not None
+        now = getattr(owner(name), name)
+        assert now is not wrong and (now.shape, now.dtype, now.device) == (right.shape, right.dtype, right.device)
+    scratch = lru._scratch
+    assert scratch.candidates.shape[0] == Hkv
+    for name in scratch._fields:
+        right = getattr(scratch, name)
+        shorter = right[:-1] if right.shape[0] > 1 else right[:, :-1]
+        for wrong in (right.cpu(), right.to(torch.int64), shorter.contiguous()):
+            if name == "workspace" and wrong.is_cuda and wrong.dtype is right.dtype:
+                continue                # (its size is what the library asks for, and checks)
+            lru._scratch = scratch._replace(**{name: wrong})
+            assert step() is None, (name, wrong.shape, wrong.dtype, wrong.device)
+    lru._scratch = scratch._replace(candidates=scratch.candidates.clone())      # without the stamps behind it
+    assert step() is None
+    lru._scratch = scratch
+    assert step() is not None
+
+
 def test_numpy_sizes_and_positions_step_in_one_call():
     """A layer built from numpy's integers, stepped at numpy's positions: one native call a step, the bits of a
     twin of Python's."""
