@@ -294,12 +294,10 @@ __device__ __forceinline__ void order_slots(const float *time, int n_slots, Shor
           peers &= bit ? with : ~with;
         }
         const uint32_t below = lanes_below(peers);
-        uint32_t seen = 0;
-        if (valid) {
-          // (every peer reads the counter before the lowest of them raises it)
-          seen = sm.digit_at[digit];
-          if (below == 0) sm.digit_at[digit] = seen + (uint32_t)__popcll(peers);
-        }
+        // (every peer reads the counter before the lowest of them raises it)
+        const uint32_t seen = sm.digit_at[digit];
+        wave_step();
+        if (valid && below == 0) sm.digit_at[digit] = seen + (uint32_t)__popcll(peers);
         wave_step();
         word[j] = slot | (seen + below) << 10 | digit << 20;
       }
