@@ -1069,6 +1069,61 @@ def test_selection_and_update_of_short_rows(Hq, Hkv, slots, kp, pages, dtype, le
             assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
 
 
+@pytest.mark.parametrize("dtype,pages,slots,kp", [(torch.float32, 445, 200, 40), (torch.bfloat16, 1001, 700, 100),
+                                                  (torch.float16, 2047, 640, 128), (torch.bfloat16, 70, 66, 9)])
+@pytest.mark.parametrize("what", ["fractions of a step", "steps beyond 2^24", "scores"])
+def test_selection_and_update_of_short_rows_of_special_values(what, dtype, pages, slots, kp):
+    """Access times that are no whole numbers or too large for one (put in order as floats, in more passes), and
+    scores that are NaN, +inf and -inf, in rows that end inside a wave's register: the bits of the separate launches."""
+    from dram_attention_amd import DRAMAttention
+
+    Hq, Hkv, D, page, local = 8, 2, 64, 16, 48
+    S = (pages - 1) * page + local
+    g = torch.Generator(device=DEV).manual_seed(pages)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(dtype)
+
+    k, v = rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    a, b = (DRAMAttention(8, slots * page, local, page, kp * page, Hkv, D, device=DEV, dtype=dtype) for _ in range(2))
+    times = torch.rand(Hkv, slots, device=DEV, generator=g)
+    special = torch.randint(0, 16, (Hkv, pages), device=DEV, generator=g)
+    for m in (a, b):
+        m.init_cache(k, v)
+        lru, minmax = m.lru_cache, m.lru_cache.top_k_selector.chunk_min_max
+        if what == "fractions of a step":
+            lru.page_access_time.copy_(times * 9000 - 100)
+            lru.page_access_time[:, ::7] = 0.5                   # (ties, in the order of the slots)
+            lru.current_step.fill_(9000)
+        elif what == "steps beyond 2^24":
+            lru.page_access_time.copy_((times * 2 ** 23).round() * 4)
+            lru.current_step.fill_(2 ** 25)
+        else:
+            # the bound of a channel whose minimum and maximum are both +inf or -inf has a sign of its own; two of
+            # opposite signs make NaN
+            for value, sign in ((1, float("inf")), (2, float("-inf"))):
+                minmax[..., 0][(special == value)[..., None].expand(-1, -1, 2)] = sign
+            minmax[..., 0][(special == 3)[..., None].expand(-1, -1, 2)] = float("inf")
+            minmax[..., 1][(special == 3)[..., None].expand(-1, -1, 2)] = float("-inf")
+    for t in range(5):
+        xq, xk, xv = (rand(1, 1, h, D) for h in (Hq, Hkv, Hkv))
+        xq[..., :2] = xq[..., :2].abs() + 0.5
+        if t % 2:
+            xq[..., 0] *= -1
+        got = a(xq, xk, xv, start_pos=S + t, stage="generate")
+        assert same(got, b.attend_(xq, xk, xv, S + t, b.select_(xq))), t
+        for name in ("hbm_kv_cache", "page_access_time", "dram_page_to_hbm_page_mapping",
+                     "hbm_page_to_dram_page_mapping", "current_step", "_topk_idx"):
+            assert same(getattr(a.lru_cache, name), getattr(b.lru_cache, name)), (t, name)
+        for name in ("miss_count", "candidates", "slot_epoch", "hit_mask"):
+            assert same(getattr(a.lru_cache._scratch, name), getattr(b.lru_cache._scratch, name)), (t, name)
+        scores = a.lru_cache.top_k_selector._scores
+        if what == "scores":
+            assert scores.isnan().any() == (t % 2 == 0) and (scores == float("inf")).any() and scores.isneginf().any()
+        for m in (a, b):
+            m.lru_cache.current_step += 7        # (a step of its own as a float, too)
+
+
 @pytest.mark.parametrize("lru", [4096, 320])     # a static prefix, a paged one
 def test_a_window_that_became_a_parameter_still_works(lru):
     """cache_k and cache_v as Parameters instead of buffers: prompt and steps go the general way, to the
