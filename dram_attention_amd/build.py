@@ -157,27 +157,29 @@ def check_hand_placed_registers(verbose: bool = False) -> None:
         print(f"hand-placed registers of {n} tile scorer variants are clear of MFMA operands")
 
 
-def build_host_calls() -> None:
+def build_host_calls(library: Path) -> Path:
     """Compile the Python module of csrc/host_calls.cpp against this interpreter's torch and
-    the library next to it (already built)."""
+    ``library``, beside it; returns its path."""
     import sysconfig
 
     import torch
 
     root = Path(torch.__file__).resolve().parent
-    tmp = HOST_PATH.with_suffix(".so.tmp")
+    out = library.with_name(HOST_PATH.name)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}",
            "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
-           str(CSRC / "host_calls.cpp"), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
-           f"-L{HERE}", "-ldramattn", "-Wl,-rpath,$ORIGIN"]
+           str(CSRC / "host_calls.cpp"), "-o", str(out), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+           f"-L{library.parent}", "-ldramattn", "-Wl,-rpath,$ORIGIN"]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed on host_calls.cpp:\n{proc.stderr}")
-    os.replace(tmp, HOST_PATH)
+    return out
 
 
 def build_library(verbose: bool = False) -> Path:
-    """Compile every kernel source and link the shared library; returns its path."""
+    """Compile every kernel source, link the shared library and compile the module of its host calls,
+    which calls it by the argument lists of the same header: the two take the places of the last
+    build's when both are made.  Returns the library's path."""
     hipcc = _hipcc()
     objdir = HERE / "build"
     objdir.mkdir(exist_ok=True)
@@ -196,14 +198,15 @@ def build_library(verbose: bool = False) -> Path:
 
     with ThreadPoolExecutor(max_workers=min(6, os.cpu_count() or 1)) as pool:
         objs = list(pool.map(compile_one, SOURCES))
-    tmp = LIB_PATH.with_suffix(".so.tmp")
-    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
+    made = objdir / LIB_PATH.name
+    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(made)]
     proc = subprocess.run(link, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     check_hand_placed_registers(verbose)
-    os.replace(tmp, LIB_PATH)
-    build_host_calls()
+    host = build_host_calls(made)
+    os.replace(made, LIB_PATH)
+    os.replace(host, HOST_PATH)
     return LIB_PATH
 
 

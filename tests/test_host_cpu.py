@@ -356,6 +356,36 @@ def test_tile_scorer_hazard_check_on_doctored_listings():
         mfma="v_mfma_f32_16x16x32_bf16 v[166:169], v[142:145], v[90:93], v[166:169]")) == 1
 
 
+@pytest.mark.parametrize("fails", ["host_calls.cpp", "-shared", "page_score.hip", None])
+def test_a_failing_build_leaves_the_last_library_and_its_module(fails, tmp_path, monkeypatch):
+    """The library and the module that calls it by the same header change together or not at all
+    (compilers that only write their output, or fail)."""
+    from types import SimpleNamespace
+
+    from dram_attention_amd import build
+
+    def compiler(cmd, **kwargs):
+        if fails is not None and any(fails in word for word in cmd):
+            return SimpleNamespace(returncode=1, stderr="no")
+        with open(cmd[cmd.index("-o") + 1], "w") as f:
+            f.write("new")
+        return SimpleNamespace(returncode=0, stderr="")
+
+    for name in ("LIB_PATH", "HOST_PATH"):
+        path = tmp_path / getattr(build, name).name
+        path.write_text("old")
+        monkeypatch.setattr(build, name, path)
+    monkeypatch.setattr(build, "HERE", tmp_path)
+    monkeypatch.setattr(build.subprocess, "run", compiler)
+    monkeypatch.setattr(build, "check_hand_placed_registers", lambda verbose: None)
+    if fails is None:
+        assert build.build_library() == build.LIB_PATH
+    else:
+        with pytest.raises(RuntimeError, match="failed"):
+            build.build_library()
+    assert [p.read_text() for p in (build.LIB_PATH, build.HOST_PATH)] == ["old" if fails else "new"] * 2
+
+
 def test_bench_roofline_traffic_constant_matches_the_committed_counter_summary():
     """bench.py reports the roofline kernel's HBM bytes per launch from the committed
     counter summary and keeps the same figure as a constant for when the file is not
