@@ -629,7 +629,9 @@ class DRAMAttention(torch.nn.Module):
         return out
 
     def _static_step(self, lru, xq, xk, xv, start_pos):
-        """A step over a static prefix, or None."""
+        """A step over a static prefix, or None (a prompt's first, too, by which the workspace is sized)."""
+        if self._workspace is None:
+            return None
         cls, layer, own, prefix = type(self), self.__dict__, self._buffers, lru.__dict__
         if ((cls.select_, cls.attend_, DummyCache.get_kv_cache_) != _STATIC_METHODS or "select_" in layer
                 or "attend_" in layer or "get_kv_cache_" in prefix):

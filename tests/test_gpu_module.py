@@ -918,6 +918,25 @@ def test_room_of_other_sizes_is_not_handed_to_a_step():
     assert step() is not None
 
 
+def test_a_static_layers_first_step_is_not_tried_natively(monkeypatch):
+    """Before there is a workspace the native call could only refuse the step."""
+    from types import SimpleNamespace
+
+    from dram_attention_amd import DRAMAttention, _lib
+
+    S, Hq, Hkv, D = 700, 8, 2, 64
+    host, calls = _lib.host(), []
+    monkeypatch.setattr(_lib, "host", lambda: SimpleNamespace(
+        static_step=lambda *args: calls.append(host.static_step(*args)) or calls[-1]))
+    m, k = DRAMAttention(8, 4096, 200, 16, 64, Hkv, D, device=DEV), torch.randn(1, S, Hkv, D, device=DEV).bfloat16()
+    x = torch.randn(1, 1, Hq, D, device=DEV).bfloat16()
+    for prompt in range(2):
+        m.init_cache(k, k)
+        for t in range(3):
+            m(x, k[:, :1], k[:, :1], start_pos=S + t, stage="generate")
+    assert len(calls) == 4 and all(c is not None for c in calls)
+
+
 def test_numpy_sizes_and_positions_step_in_one_call():
     """A layer built from numpy's integers, stepped at numpy's positions: one native call a step, the bits of a
     twin of Python's."""
