@@ -313,11 +313,11 @@ def test_rope_kernel_matches_torch(S, Hq, Hkv, D, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("dim,n", [(8, 1), (256, 2), (520, 7), (2048, 66), (2056, 33), (4096, 257), (30720, 5),
-                                   (136, 8201), (30720, 2059)])
+                                   (136, 8201), (30720, 4099)])
 def test_one_token_linear_kernels_match_torch(dim, n, dtype):
     """The one-token layers at the edges of a wave's step (512 elements of 16 bits), of its
     unrolled steps (2048) and at the longest row, odd and single output rows, more pairs of rows than the
-    grid has waves (8192 and 2048 of them, by the length of the row), against fp64
+    grid has waves (4096, or 2048 where two workgroups' rows fill a unit's LDS), against fp64
     products of the same inputs.  Bound: sums of `dim` fp32 terms, then one turn of each
     rounding to the type (a unit in the last place: 2^-7 of the value in bf16, 2^-10 in
     fp16); silu and the product add one more each."""
@@ -349,9 +349,10 @@ def test_one_token_linear_kernels_match_torch(dim, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-def test_one_token_qkv_kernel_matches_the_modules(dtype):
+@pytest.mark.parametrize("Hq,Hkv,D,dim", [(6, 2, 64, 264),
+                                          (72, 8, 128, 136)])   # waves go on in each of the three matrices
+def test_one_token_qkv_kernel_matches_the_modules(Hq, Hkv, D, dim, dtype):
     g = torch.Generator().manual_seed(3)
-    Hq, Hkv, D, dim = 6, 2, 64, 264
     x = torch.randn(1, 1, dim, generator=g).to(dtype).cuda()
     wq, wk, wv = ((torch.randn(h * D, dim, generator=g) / 16).to(dtype).cuda() for h in (Hq, Hkv, Hkv))
     row = L.rope_table(D, 20, 1e4, False, device="cuda")[13:14]
