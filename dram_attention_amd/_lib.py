@@ -23,7 +23,8 @@ _DTYPES = {torch.float32: DA_F32, torch.float16: DA_F16, torch.bfloat16: DA_BF16
 _ITYPES = {torch.int32: DA_I32, torch.int64: DA_I64}
 _TIME_TYPES = {torch.float32: DA_TIME_F32, torch.int32: DA_TIME_I32}
 
-# name -> (restype, argtypes); one line per symbol of the header
+# name -> (restype, argtypes); one line per symbol of the header (those that _host calls natively, da_decode_attention,
+# da_linear_qkv_rope and da_linear_block_tail, are for other callers here)
 SIGNATURES = {
     "da_version": (c_int, []),
     "da_last_error_string": (c_char_p, []),
@@ -176,7 +177,8 @@ class PagedOverlap(ctypes.Structure):
     ]
 
 
-# struct da_decode_step_args of the header: 25 pointers, 7 int64, 10 int32, 3 floats, 1 int32
+# struct da_decode_step_args of the header: 25 pointers, 7 int64, 10 int32, 3 floats, 1 int32.  A layer's blocks are
+# made natively (_host.step_args); this is for callers of da_decode_step(s) that read, change or make them
 DECODE_STEP_ARGS = struct.Struct("=25Q7q10i3fi")
 
 _lib = None

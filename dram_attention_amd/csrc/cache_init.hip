@@ -104,9 +104,8 @@ extern "C" int da_prompt_cache(const void *k, const void *v, int64_t tok_stride,
   DA_REQUIRE(!paged || (summaries && dram_to_hbm && n_pages > 0 && (n_slots == 0 || (access_time && hbm_to_dram))),
              "da_prompt_cache: null pointer of a page cache, or none of its pages");
   const int vec = 16 / elem_size(dtype);
-  DA_REQUIRE(head_dim % vec == 0 && tok_stride % vec == 0 && head_stride % vec == 0 && (uintptr_t)k % 16 == 0 &&
-                 (uintptr_t)v % 16 == 0 && (uintptr_t)window_k % 16 == 0 && (uintptr_t)window_v % 16 == 0 &&
-                 (uintptr_t)summaries % 16 == 0,
+  DA_REQUIRE(minmax_vec_fits(k, head_stride, tok_stride, head_dim, dtype, summaries) && (uintptr_t)v % 16 == 0 &&
+                 (uintptr_t)window_k % 16 == 0 && (uintptr_t)window_v % 16 == 0,
              "da_prompt_cache: rows must be 16-byte aligned");
   PromptCacheArgs a = {};
   a.k = (const char *)k;
