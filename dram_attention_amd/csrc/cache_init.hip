@@ -33,8 +33,9 @@ page_cache_init_kernel(int32_t *__restrict__ step, float *__restrict__ access_ti
 // [0, minmax_blocks)), the metadata of the page cache and the local window's copy of the last tokens.  Bound:
 // HBM for the summaries, launches for the rest: four of them in a row, 12 + 5 + 5.5 + 5.5 us behind the
 // attention of 9200 tokens in fp32, whatever their size; a static prefix has the two copies only.
-// us a prompt, launch by launch / in one: 9200 tokens of 8/2 heads in fp32 487.5 / 478.7; 8192 through two layers of
-// a model 6348 / 6327; 4613 of 32/8, a static prefix 179.9 / 179.3.
+// us a prompt, the separate launches / this one (two runs of one side differ by up to 0.4 %): 9200 tokens of 8/2 heads in
+// fp32 473.3 / 465.2; no difference shown for 8192 through two layers of a model (6366 / 6357) and 4613 of
+// 32/8, a static prefix (173.7 / 173.0).
 struct PromptCacheArgs {
   const char *k, *v;                  // (tokens, heads, head_dim)
   int64_t tok_stride, head_stride;    // elements

@@ -11,7 +11,7 @@
 //   - another wave meanwhile puts all slots in order of their access times by a stable radix
 //     sort that only it takes part in, so the list of least recent slots is complete;
 //   - both page maps are in LDS by then (a short row has few pages): the update reads nothing
-//     from memory, with one thread per request and one per slot.
+//     from memory but the ticket of the step counter, with one thread per request and one per slot.
 // us a launch (under the profiler; in brackets a workgroup a row): 512 pages of 2 heads in fp32, 4 rows of
 // 32 pages, 128 slots 5.9 (12.9); 445 of 4 heads in bf16, the same lists 6.2 (12.0); 1000 of 8 heads, 4 rows of 64,
 // 256 slots 7.3 (12.1), of 128, 512 slots 9.4 (13.3); 8 rows of 60 10.8 (13.6); 2047 of 8 heads, 4 rows of 128, 512
